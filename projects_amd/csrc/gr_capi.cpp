@@ -954,13 +954,11 @@ int gr_ring_correct(float *sino, long slice_stride, long row_stride, int n_slice
     if (!(fabsf(ring_coeff) < 1e30f)) return fail(GR_EINVAL, "ring coefficient not finite");
     if (iterations == 0) return GR_OK;
     hipStream_t s = (hipStream_t)stream;
-    float *rm = nullptr, *cm = nullptr;
-    hipError_t e = hipMallocAsync((void **)&rm, sizeof(float) * (size_t)n_slices * n_ang, s);
-    if (e == hipSuccess) e = hipMallocAsync((void **)&cm, sizeof(float) * (size_t)n_slices * n_det, s);
+    void *scratch = nullptr;
+    hipError_t e = hipMallocAsync(&scratch, gr_ring_scratch_bytes(n_slices, n_ang, n_det), s);
     if (e == hipSuccess)
-        e = gr_launch_ring(sino, slice_stride, row_stride, n_slices, n_ang, n_det, ring_coeff, iterations, rm, cm, s);
-    if (rm) (void)hipFreeAsync(rm, s);
-    if (cm) (void)hipFreeAsync(cm, s);
+        e = gr_launch_ring(sino, slice_stride, row_stride, n_slices, n_ang, n_det, ring_coeff, iterations, scratch, s);
+    if (scratch) (void)hipFreeAsync(scratch, s);
     if (e != hipSuccess) return hip_fail(e, "ring correction");
     return GR_OK;
 }

@@ -100,3 +100,29 @@ def test_ring_correction_vs_oracle():
         # the correction reduces the column-to-column ripple
         ripple = lambda a: np.std(np.diff(a.mean(axis=0)))
         assert ripple(out[s]) < ripple(sino[s])
+
+
+# the edges of the one-pass kernel: rows narrower than a wave, the widths
+# where a thread holds 4, 8 and 16 values and one past each (the last: rows
+# read again for the column sums), 16-byte pieces and single values, the
+# 62-column groups of the estimate, one to several workgroups per slice
+@pytest.mark.parametrize("ns,n_ang,n_det,row,zeros", [
+    (1, 1, 1, 1, ()), (1, 3, 2, 2, ()), (2, 5, 62, 62, (2,)), (1, 37, 63, 64, (0, 36)), (3, 90, 1024, 1024, (5,)),
+    (2, 41, 1025, 1028, ()), (1, 64, 2048, 2048, (63,)), (2, 33, 2051, 2060, (7,)), (1, 20, 4096, 4096, ()),
+    (1, 19, 4099, 4099, (3,)), (40, 70, 200, 200, (1, 2))])
+def test_ring_correction_sizes(ns, n_ang, n_det, row, zeros):
+    """Against the oracle, whose float column sums run over the rows in order:
+    rounding of at most about n_ang + 3 additions per mean and iteration, a
+    few 1e-6 over six iterations; rows of zero mean keep their values."""
+    rng = np.random.default_rng(n_det)
+    sino = (1.0 + rng.random((ns, n_ang, n_det)) + 0.1 * rng.standard_normal(n_det)).astype(np.float32)
+    for i in zeros:
+        sino[:, i] = 0.0
+    buf = torch.full((ns, n_ang, row), float("nan"), device="cuda")
+    g = buf[:, :, :n_det]
+    g.copy_(torch.from_numpy(sino))
+    gr.ring_correct(g, 0.8, iterations=6)
+    out = g.cpu().numpy()
+    for s in range(0, ns, max(1, ns // 3)):
+        assert O.rel_l2(out[s], O.ring_correct(sino[s], 0.8, iterations=6)) < 1e-5, s
+    assert torch.isnan(buf[:, :, n_det:]).all()

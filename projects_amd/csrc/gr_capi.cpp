@@ -396,7 +396,7 @@ void free_plan(gr_plan *pl) {
     void *ptrs[] = {pl->d_cose, pl->d_sine, pl->d_roi, pl->d_wtbl, pl->d_winv, pl->d_filphase, pl->d_akey,
                     pl->d_aord, pl->d_ang, pl->d_gop, pl->d_gop_n, pl->d_gop_off, pl->d_dwtbl, pl->d_rowtiles,
                     pl->d_sop_tile, pl->d_sop_ch, pl->d_sop_keys, pl->d_sop_ent, pl->d_hmeta, pl->d_hseg,
-                    pl->d_hsplit, pl->d_hitems};
+                    pl->d_hsplit, pl->d_hitems, pl->d_sweep};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     shared_release(pl->d_tw_row);
@@ -765,17 +765,9 @@ namespace {
 // geometry passes) has paid for itself.
 constexpr long kGopAutoPairs = 16;
 
-// The chunk loop of gr_recon_device / gr_recon_device_raw: K1..K4 per chunk
-// of max_pairs pairs; K1 reads float rows (pre null) or detector counts.
-int recon_chunks(gr_plan *pl, const float *sino, long sino_slice_stride, long sino_row_stride, const GrPre *pre,
-                 float *out, long out_slice_stride, long out_row_stride, int n_slices, void *stream) {
-    if (!pl->d_spec1) return fail(GR_EINVAL, "plan has no workspace");
-    const GrGeom &g = pl->g;
-    if (out_row_stride < g.out_n || out_slice_stride < out_row_stride * g.out_n)
-        return fail(GR_EINVAL, "image strides smaller than the window they hold");
-    GR_HIP(hipSetDevice(pl->prm.device));
-    hipStream_t s = (hipStream_t)stream;  // NULL: the null stream
-    const int n_pairs = (n_slices + 1) / 2;
+// Count n_pairs pairs about to be reconstructed on stream s and build the
+// operator of a plan in GR_GRIDOP_AUTO when they reach the trigger.
+int count_pairs(gr_plan *pl, int n_pairs, hipStream_t s) {
     if (pl->gop_state == 0 && pl->prm.grid_op == GR_GRIDOP_AUTO && pl->pairs_done + n_pairs >= kGopAutoPairs) {
         // not while a graph is being captured: the build synchronises
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -786,6 +778,25 @@ int recon_chunks(gr_plan *pl, const float *sino, long sino_slice_stride, long si
         }
     }
     pl->pairs_done += n_pairs;
+    return GR_OK;
+}
+
+// The chunk loop of gr_recon_device / gr_recon_device_raw: K1..K4 per chunk
+// of max_pairs pairs; K1 reads float rows (pre null) or detector counts.
+int recon_chunks(gr_plan *pl, const float *sino, long sino_slice_stride, long sino_row_stride, const GrPre *pre,
+                 float *out, long out_slice_stride, long out_row_stride, int n_slices, void *stream,
+                 bool counted = false) {
+    if (!pl->d_spec1) return fail(GR_EINVAL, "plan has no workspace");
+    const GrGeom &g = pl->g;
+    if (out_row_stride < g.out_n || out_slice_stride < out_row_stride * g.out_n)
+        return fail(GR_EINVAL, "image strides smaller than the window they hold");
+    GR_HIP(hipSetDevice(pl->prm.device));
+    hipStream_t s = (hipStream_t)stream;  // NULL: the null stream
+    const int n_pairs = (n_slices + 1) / 2;
+    if (!counted) {
+        const int rc = count_pairs(pl, n_pairs, s);
+        if (rc) return rc;
+    }
     const GrDevTables t = pl->tables();
     for (int p0 = 0; p0 < n_pairs; p0 += pl->max_pairs) {
         const int np = std::min(pl->max_pairs, n_pairs - p0);
@@ -976,26 +987,42 @@ int gr_center_entropy(gr_plan *pl, const float *sino, long sino_slice_stride, lo
         return fail(GR_EINVAL, "sinogram strides smaller than the rows they hold");
     GR_HIP(hipSetDevice(pl->prm.device));
     hipStream_t s = (hipStream_t)stream;
+    if (!pl->d_spec1) return fail(GR_EINVAL, "plan has no workspace");
     const long on = g.out_n, nb1 = n_bins + 1;
-    float *d_shift = nullptr, *d_img = nullptr;
-    unsigned *d_hist = nullptr;
-    hipError_t e = hipMallocAsync((void **)&d_shift, sizeof(float) * n_shifts, s);
-    if (e == hipSuccess) e = hipMallocAsync((void **)&d_img, sizeof(float) * 2 * on * on * n_shifts, s);
-    if (e == hipSuccess) e = hipMallocAsync((void **)&d_hist, sizeof(unsigned) * nb1 * n_shifts, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(d_shift, shifts, sizeof(float) * n_shifts, hipMemcpyHostToDevice, s);
-    int rc = GR_OK;
-    if (e == hipSuccess) {
-        GrPre p{3, nullptr, 0, 0, nullptr, nullptr, nullptr, 0, 0.0f, d_shift};
-        rc = recon_chunks(pl, sino, sino_slice_stride, sino_row_stride, &p, d_img, on * on, on, 2 * n_shifts, s);
+    // shifts and histograms: kept by the plan (allocated and freed per call
+    // they are given back to the system at every synchronisation)
+    const size_t shift_bytes = (sizeof(float) * n_shifts + 255) / 256 * 256;
+    const size_t sweep_bytes = shift_bytes + sizeof(unsigned) * nb1 * n_shifts;
+    if (sweep_bytes > pl->sweep_bytes) {
+        if (pl->d_sweep) {
+            GR_HIP(hipFree(pl->d_sweep));
+            pl->d_sweep = nullptr;
+            pl->dev_bytes -= pl->sweep_bytes;
+            pl->sweep_bytes = 0;
+        }
+        const int rc = dev_alloc(pl, (char **)&pl->d_sweep, sweep_bytes);
+        if (rc) return rc;
+        pl->sweep_bytes = sweep_bytes;
+    }
+    float *d_shift = (float *)pl->d_sweep;
+    unsigned *d_hist = (unsigned *)((char *)pl->d_sweep + shift_bytes);
+    GR_HIP(hipMemcpyAsync(d_shift, shifts, sizeof(float) * n_shifts, hipMemcpyHostToDevice, s));
+    int rc = count_pairs(pl, n_shifts, s);
+    // a chunk's images go to the gridding step's grid, which is free once the
+    // row transform has read it and larger than the images (M > out_n: 8 M^2
+    // bytes per pair against 8 out_n^2), and are counted before the next chunk
+    float *img = (float *)pl->d_ht;
+    hipError_t e = hipSuccess;
+    for (int c0 = 0; c0 < n_shifts && rc == GR_OK && e == hipSuccess; c0 += pl->max_pairs) {
+        const int np = std::min(pl->max_pairs, n_shifts - c0);
+        GrPre p{3, nullptr, 0, 0, nullptr, nullptr, nullptr, 0, 0.0f, d_shift + c0};
+        rc = recon_chunks(pl, sino, sino_slice_stride, sino_row_stride, &p, img, on * on, on, 2 * np, s, true);
+        if (rc == GR_OK)
+            e = gr_launch_hist(img, 2 * on * on, np, hist_min, hist_max, n_bins, d_hist + nb1 * c0, s);
     }
     std::vector<unsigned> h((size_t)nb1 * n_shifts);
     if (e == hipSuccess && rc == GR_OK)
-        e = gr_launch_hist(d_img, 2 * on * on, on * on, on, (int)on, n_shifts, hist_min, hist_max, n_bins, d_hist, s);
-    if (e == hipSuccess && rc == GR_OK)
         e = hipMemcpyAsync(h.data(), d_hist, sizeof(unsigned) * h.size(), hipMemcpyDeviceToHost, s);
-    if (d_shift) (void)hipFreeAsync(d_shift, s);
-    if (d_img) (void)hipFreeAsync(d_img, s);
-    if (d_hist) (void)hipFreeAsync(d_hist, s);
     const hipError_t w = hipStreamSynchronize(s);
     if (rc) return rc;
     if (e != hipSuccess) return hip_fail(e, "centre sweep");

@@ -204,11 +204,10 @@ hipError_t gr_launch_phantom(float *sino, long slice_stride, int n_slices, long 
                              int n_ell, float photons, int density, float gauss_rel, int n_tex, float tex_amp,
                              float tex_fmax, hipStream_t s);
 
-// Histograms for the entropy metric: n_cand candidates, each two on x on
-// images (slice_stride / row_stride floats apart, candidates cand_stride
-// apart); hist receives n_cand x (n_bins + 1) counts.
-hipError_t gr_launch_hist(const float *img, long cand_stride, long slice_stride, long row_stride, int on,
-                          int n_cand, float vmin, float vmax, int n_bins, unsigned *hist, hipStream_t s);
+// Histograms for the entropy metric: n_cand candidates of npix values each,
+// one after another; hist receives n_cand x (n_bins + 1) counts.
+hipError_t gr_launch_hist(const float *img, long npix, int n_cand, float vmin, float vmax, int n_bins,
+                          unsigned *hist, hipStream_t s);
 
 // Ring-artefact correction in place (tomo_recon.cpp:3905-3972); scratch:
 // gr_ring_scratch_bytes, 256-byte aligned.

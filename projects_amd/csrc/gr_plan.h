@@ -49,6 +49,9 @@ struct gr_plan {
     bool owns_workspace = true;
     float2 *d_spec1 = nullptr, *d_spec2 = nullptr, *d_ht = nullptr, *d_z = nullptr;
     size_t dev_bytes = 0;
+    // centre sweeps: shifts and histograms, grown to the largest sweep so far
+    void *d_sweep = nullptr;
+    size_t sweep_bytes = 0;
     // launch tuning (0 = automatic)
     int cols_per_block = 0;
     // host-row entry points (gr_exec_pairs, gr_recon_host): two staging slots

@@ -65,3 +65,27 @@ def test_entropy_sweep_matches_oracle_and_finds_the_axis():
     assert abs(best - (-true_off)) <= 0.25, best
     assert int(np.argmin(ent)) == int(np.argmin(ref))
     plan.close()
+
+
+@pytest.mark.parametrize("n,max_pairs,nb", [(65, 1, 3), (64, 2, 512), (127, 8, 2048), (96, 3, 16383)])
+def test_entropy_sweep_chunks_and_bins(n, max_pairs, nb):
+    """Sweeps cut into chunks of max_pairs candidates (the last one partial),
+    odd and even windows, histograms with 16 copies down to one: the counts of
+    a chunked sweep are those of each candidate alone (same images, integer
+    counts), so the entropies are equal bit for bit; and near the oracle's."""
+    sino = np.stack([phantom.sinogram(5, s, 60, n, n / 2.0, 8) for s in range(2)]).astype(np.float32)
+    g = torch.from_numpy(sino).cuda()
+    crop = (((1 << (2 * n - 1).bit_length()) - 1 - n) // 2, n)
+    shifts = np.arange(-2.0, 2.01, 0.8, dtype=np.float32)
+    lo, hi = -0.25, 1.0
+    plan = gr.Plan(n_ang=60, n_det=n, center=n / 2.0, pad="half", crop=crop, max_pairs=max_pairs, grid_op="off")
+    ent = plan.center_entropy(g, shifts, lo, hi, nb)
+    one = gr.Plan(n_ang=60, n_det=n, center=n / 2.0, pad="half", crop=crop, max_pairs=1, grid_op="off")
+    each = np.concatenate([one.center_entropy(g, shifts[i:i + 1], lo, hi, nb) for i in range(len(shifts))])
+    assert np.array_equal(ent, each)
+    imgs = [one.recon(torch.from_numpy(np.stack([np.stack([O_shift(r, s) for r in sino[k]]) for k in (0, 1)])).cuda())
+            for s in shifts]
+    ref = np.array([O.entropy(im.cpu().numpy().ravel(), lo, hi, nb) for im in imgs])
+    assert np.max(np.abs(ent - ref)) <= 1e-5 * np.max(ref)
+    plan.close()
+    one.close()

@@ -86,6 +86,12 @@ struct GrDevTables {
     const uint4 *sop_tile = nullptr;
     const uint2 *sop_ch = nullptr;
     const unsigned *sop_keys = nullptr, *sop_ent = nullptr;
+    // the centre tiles as the geometry kernel grids them (compensated sums):
+    // the first split_slots slots of every sector, one work item {tile slot,
+    // window position of its first line, index} per merge group, a wave each,
+    // and per tile {tile slot, first item, items}
+    const uint4 *sitems = nullptr, *smeta = nullptr;
+    int n_sitems = 0, n_smeta = 0, split_slots = 0;
     // per tile row (M / 8 rows) the interval [lo, hi] of tiles that can hold
     // a nonzero cell (gr_active_tile_range), evaluated once on the device
     const int2 *row_tiles = nullptr;
@@ -143,6 +149,16 @@ constexpr unsigned kGridNoTile = 0xffffffffu;
 hipError_t gr_launch_grid(const GrGeom &g, const GrDevTables &t, int n_ang, long ltbl,
                           const float2 *spec1, const float2 *spec2, float2 *ht, float2 *scratch, int pairs,
                           int accum, hipStream_t s);
+
+// The split of the centre tiles (GrDevTables::sitems): lines per tile of the
+// first `slots` slots of every sector into lines[sector * slots + slot]; the
+// items of those tiles, tile w's from first[w] on.  kGridMergeLines: sample
+// lines per merge group.
+constexpr int kGridMergeLines = 16;
+hipError_t gr_launch_split_lines(const GrGeom &g, const GrDevTables &t, int n_ang, long ltbl, int slots,
+                                 unsigned *lines, hipStream_t s);
+hipError_t gr_launch_split_items(const GrGeom &g, const GrDevTables &t, int n_ang, long ltbl, int slots,
+                                 const unsigned *first, uint4 *items, hipStream_t s);
 
 // The precomputed operator: whether the geometry's sample indices fit its
 // entries; the count pass (rows per tile of the ragged layout into tile_n,

@@ -43,6 +43,9 @@ struct gr_plan {
     uint2 *d_hseg = nullptr;
     unsigned *d_hsplit = nullptr;
     int n_hitems = 0, n_split = 0, split_groups = 0;
+    // the centre tiles' merge groups for the geometry kernel (GrDevTables::sitems)
+    uint4 *d_sitems = nullptr, *d_smeta = nullptr;
+    int n_sitems = 0, n_smeta = 0, split_slots = 0;
     long pairs_done = 0;  // pairs reconstructed so far (the automatic build's trigger)
     // workspace for max_pairs pairs: owned, or a region bound by a queue
     int max_pairs = 1;
@@ -91,6 +94,11 @@ struct gr_plan {
         t.ntiles = ntiles;
         t.sector_len = sector_len;
         t.row_tiles = d_rowtiles;
+        t.sitems = d_sitems;
+        t.smeta = d_smeta;
+        t.n_sitems = n_sitems;
+        t.n_smeta = n_smeta;
+        t.split_slots = split_slots;
         if (gop_state == 1) {
             t.gop = d_gop;
             t.gop_n = d_gop_n;

@@ -57,7 +57,7 @@
 namespace {
 
 constexpr int kTile = 8;        // cells per tile side; one tile per wavefront
-constexpr int kMergeAngles = 16;  // sample lines per compensated partial
+constexpr int kMergeAngles = kGridMergeLines;  // sample lines per compensated partial
 
 struct GridArgs {
     const float2 *spec1, *spec2;
@@ -71,6 +71,11 @@ struct GridArgs {
     int ntiles, sector_len, n_ang, half, lds_wtbl, pair_base, pair_end;
     GrGatherGeom g;
     float L2m, dmax, rmax;
+    // split centre tiles (GrDevTables): items, slots they take in each
+    // sector, and their partials [item][pair][lane]
+    const uint4 *sitems;
+    int n_sitems, split_slots, part_pairs;
+    float2 *part;
 };
 
 // Slot of the tile list for wave `wave` of workgroup `block` in a launch of
@@ -174,47 +179,104 @@ __device__ __forceinline__ void chunk_taps(const float2 (*stage)[P], int c0, int
     }
 }
 
+// A tile as walk_tile sees it: its centre relative to the grid's, how far a
+// sample of it may be from the centre, and its window of sorted angles, two
+// ranges of keys laid end to end (positions 0 .. n - 1).
+struct TileLines {
+    float cu, cv, reach;
+    int r0, n0, r2, n;
+    __device__ __forceinline__ int key(int pos) const { return pos < n0 ? r0 + pos : r2 + (pos - n0); }
+};
+
+__device__ __forceinline__ TileLines tile_lines(const GridArgs &A, int tx, int ty) {
+    const float M2 = A.g.fM2;
+    TileLines t;
+    t.cu = (float)(tx * kTile) + 3.5f - M2;
+    t.cv = (float)(ty * kTile) + 3.5f - M2;
+    t.reach = 3.5f + A.L2m;  // tile half-width plus box half-width
+    int r1, r3;
+    gr_angle_window(tx, ty, M2, A.dmax, A.akey, A.n_ang, t.r0, r1, t.r2, r3);
+    t.n0 = max(r1 - t.r0, 0);
+    t.n = t.n0 + max(r3 - t.r2, 0);
+    return t;
+}
+
+// Whether the sample line of direction cs passes the tile, and the samples of
+// it that can reach the tile: direct [td0, td1], mirrored [tm0, tm1].
+__device__ __forceinline__ bool line_hits(const GridArgs &A, const TileLines &t, float4 cs, int &td0, int &td1,
+                                          int &tm0, int &tm1) {
+    // does the line pass through the tile grown by the box half-width?
+    if (fabsf(t.cu * cs.y - t.cv * cs.x) > t.reach * (fabsf(cs.x) + fabsf(cs.y)) + 0.05f) return false;
+    gr_candidates_r(t.cu, t.cv, cs.z, cs.w, t.reach, A.g, td0, td1, tm0, tm1);
+    return td0 <= td1 || tm0 <= tm1;
+}
+
 // Walk the sample lines that can reach the wave's tile, in the kernel's fixed
 // order (sorted angle keys, the window's two ranges in turn; per line the
 // direct samples, then the mirrored ones, in chunks of at most 64 ascending
 // j), calling on_chunk(mirror, row_off, c0, nj, j0, j1, C, S) per chunk --
 // [c0, c0+nj) the tile's samples of the chunk, [j0, j1] the lane's own
 // candidates among them -- and on_line() after each line that passed the
-// tile tests.  Tiles beyond the largest sample radius visit nothing.
+// tile tests.  Tiles beyond the largest sample radius visit nothing.  pos0,
+// max_lines: start at window position pos0, stop after that many lines.
 template <class ChunkFn, class LineFn>
 __device__ __forceinline__ void walk_tile(const GridArgs &A, int tx, int ty, bool valid, float du, float dv,
-                                          ChunkFn &&on_chunk, LineFn &&on_line) {
-    const float M2 = A.g.fM2;
-    if (!gr_tile_active(tx, ty, M2, A.rmax)) return;
-    const float cu = (float)(tx * kTile) + 3.5f - M2, cv = (float)(ty * kTile) + 3.5f - M2;
-    const float reach = 3.5f + A.L2m;  // tile half-width plus box half-width
-    int r0, r1, r2, r3;
-    gr_angle_window(tx, ty, M2, A.dmax, A.akey, A.n_ang, r0, r1, r2, r3);
-    for (int side = 0; side < 2; side++) {
-        const int k0 = side ? r2 : r0, k1 = side ? r3 : r1;
-        for (int k = k0; k < k1; k++) {
-            const float4 cs = table_load(A.ang, k);
-            // does the line pass through the tile grown by the box half-width?
-            if (fabsf(cu * cs.y - cv * cs.x) > reach * (fabsf(cs.x) + fabsf(cs.y)) + 0.05f) continue;
+                                          ChunkFn &&on_chunk, LineFn &&on_line, int pos0 = 0,
+                                          int max_lines = 0x7fffffff) {
+    if (!gr_tile_active(tx, ty, A.g.fM2, A.rmax)) return;
+    const TileLines t = tile_lines(A, tx, ty);
+    for (int pos = pos0; pos < t.n && max_lines > 0; pos++) {
+        const int k = t.key(pos);
+        const float4 cs = table_load(A.ang, k);
+        int td0, td1, tm0, tm1;
+        if (!line_hits(A, t, cs, td0, td1, tm0, tm1)) continue;
+        max_lines--;
+        int jd0, jd1, jm0, jm1;
+        gr_candidates_r(du, dv, cs.z, cs.w, A.L2m, A.g, jd0, jd1, jm0, jm1);
+        if (!valid) {
+            jd1 = jd0 - 1;
+            jm1 = jm0 - 1;
+        }
+        const long row_off = (long)table_load(A.aord, k) * A.half;
+        for (int c0 = td0; c0 <= td1; c0 += 64)
+            on_chunk(0, row_off, c0, min(64, td1 - c0 + 1), max(jd0, c0), min(min(jd1, td1), c0 + 63), cs.x, cs.y);
+        for (int c0 = tm0; c0 <= tm1; c0 += 64)
+            on_chunk(1, row_off, c0, min(64, tm1 - c0 + 1), max(jm0, c0), min(min(jm1, tm1), c0 + 63), cs.x, cs.y);
+        on_line();
+    }
+}
+
+// The merge groups (kMergeAngles lines) of the first `slots` tiles of every
+// sector, a wave per tile, 64 lines tested at once.  MODE 0: lines per tile
+// into lines[sector * slots + slot].  MODE 1: the items of the tiles
+// (gr_launch_split_items), tile t's from first[t] on.
+template <int MODE>
+__global__ void __launch_bounds__(256) k_split_lines(GridArgs A, int slots, unsigned *lines, const unsigned *first,
+                                                     uint4 *items) {
+    const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    if (w >= kGridSectors * slots) return;
+    const int ti = (w / slots) * A.sector_len + w % slots;
+    const unsigned tt = table_load(A.tiles, ti);
+    unsigned n = 0;
+    const int tx = (int)(tt & 0xffffu), ty = (int)(tt >> 16);
+    if (tt != kGridNoTile && gr_tile_active(tx, ty, A.g.fM2, A.rmax)) {
+        const TileLines t = tile_lines(A, tx, ty);
+        for (int p0 = 0; p0 < t.n; p0 += 64) {
+            const int pos = p0 + lane;
             int td0, td1, tm0, tm1;
-            gr_candidates_r(cu, cv, cs.z, cs.w, reach, A.g, td0, td1, tm0, tm1);
-            if (td0 > td1 && tm0 > tm1) continue;
-            int jd0, jd1, jm0, jm1;
-            gr_candidates_r(du, dv, cs.z, cs.w, A.L2m, A.g, jd0, jd1, jm0, jm1);
-            if (!valid) {
-                jd1 = jd0 - 1;
-                jm1 = jm0 - 1;
+            const bool hit = pos < t.n && line_hits(A, t, A.ang[t.key(min(pos, t.n - 1))], td0, td1, tm0, tm1);
+            const unsigned long long mask = __ballot(hit);
+            if (MODE == 1 && hit) {
+                const unsigned rank = n + (unsigned)__popcll(mask & ((1ull << lane) - 1));
+                if (rank % kMergeAngles == 0) {
+                    const unsigned i = first[w] + rank / kMergeAngles;
+                    items[i] = make_uint4((unsigned)ti, (unsigned)pos, i, 0u);
+                }
             }
-            const long row_off = (long)table_load(A.aord, k) * A.half;
-            for (int c0 = td0; c0 <= td1; c0 += 64)
-                on_chunk(0, row_off, c0, min(64, td1 - c0 + 1), max(jd0, c0), min(min(jd1, td1), c0 + 63), cs.x,
-                         cs.y);
-            for (int c0 = tm0; c0 <= tm1; c0 += 64)
-                on_chunk(1, row_off, c0, min(64, tm1 - c0 + 1), max(jm0, c0), min(min(jm1, tm1), c0 + 63), cs.x,
-                         cs.y);
-            on_line();
+            n += (unsigned)__popcll(mask);
         }
     }
+    if (MODE == 0 && lane == 0) lines[w] = n;
 }
 
 // Write the wave's 64 cells for the P pairs -- only for tiles that can hold
@@ -235,6 +297,12 @@ __device__ __forceinline__ void store_cells(const GridArgs &A, int pair0, int nv
     }
 }
 
+// Workgroups of k_grid given to the merge groups of split tiles (a multiple of
+// the sector count, so the other workgroups keep their XCD-to-sector map).
+__host__ __device__ __forceinline__ int split_blocks(int n_items, int wpb) {
+    return (n_items + wpb * kGridSectors - 1) / (wpb * kGridSectors) * kGridSectors;
+}
+
 template <int ACCUM, int P>
 __global__ void __launch_bounds__(256) k_grid(GridArgs A) {
     extern __shared__ float smem[];
@@ -251,9 +319,23 @@ __global__ void __launch_bounds__(256) k_grid(GridArgs A) {
     // the tile slot as a wave-uniform value: the tile, its angle window and
     // each line's angle record then come through scalar loads, which do not
     // wait behind the spectra loads in the vector memory counter
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int ti = __builtin_amdgcn_readfirstlane(sector_slot(A, blockIdx.x, blockDim.x >> 6, wave, 0));
-    if (ti < 0) return;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, wpb = blockDim.x >> 6;
+    // the first workgroups take the merge groups of the split tiles, one per wave
+    const int sb = split_blocks(A.n_sitems, wpb);
+    int ti, pos0 = 0, max_lines = 0x7fffffff;
+    float2 *part_out = nullptr;
+    if ((int)blockIdx.x < sb) {
+        const int item = __builtin_amdgcn_readfirstlane((int)blockIdx.x * wpb + wave);
+        if (item >= A.n_sitems) return;
+        const uint4 it = table_load(A.sitems, item);
+        ti = (int)it.x;
+        pos0 = (int)it.y;
+        max_lines = kMergeAngles;
+        part_out = A.part + (size_t)it.z * A.part_pairs * 64;
+    } else {
+        ti = __builtin_amdgcn_readfirstlane(sector_slot(A, (int)blockIdx.x - sb, wpb, wave, A.split_slots));
+        if (ti < 0) return;
+    }
     const unsigned tt = table_load(A.tiles, ti);
     if (tt == kGridNoTile) return;
     float2(*stage)[P] = reinterpret_cast<float2(*)[P]>(smem + A.lds_wtbl) + wave * 128;  // two buffers of 64 slots
@@ -314,10 +396,49 @@ __global__ void __launch_bounds__(256) k_grid(GridArgs A) {
             p_C = C;
             p_S = S;
         },
-        [&]() { p_eol = true; });  // the pending chunk ends its line
+        [&]() { p_eol = true; },  // the pending chunk ends its line
+        pos0, max_lines);
+    if (part_out) {  // a merge group of a split tile: its partials, unmerged
+        if (have) {
+            p_eol = false;
+            add_pending();
+        }
+#pragma unroll
+        for (int p = 0; p < P; p++)
+            if (p < nvalid) part_out[(pair0 + p) * 64 + lane] = part[p];
+        return;
+    }
     if (have) add_pending();
     if (ACCUM == GR_ACCUM_COMPENSATED && lines) merge<P>(acc, part);
     store_cells<ACCUM, P>(A, pair0, nvalid, a, b, acc);
+}
+
+// The split tiles' sums: per (tile, pair) wave, the partials merged in the
+// order of their groups -- the merges k_grid would have done -- and the cells
+// stored.  meta: {tile slot, first item, items} per tile.  Sixteen partials
+// load at a time.
+__global__ void __launch_bounds__(256) k_split_merge(GridArgs A, const uint4 *meta, int n_tiles, int pairs) {
+    const int w = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (w >= n_tiles * pairs) return;
+    const uint4 m = meta[w / pairs];
+    const int pair = w % pairs;
+    const unsigned tt = A.tiles[m.x], n = m.z;
+    if (tt == kGridNoTile) return;
+    const int a = (int)(tt & 0xffffu) * kTile + (lane & 7), b = (int)(tt >> 16) * kTile + (lane >> 3);
+    const size_t stride = (size_t)A.part_pairs * 64;
+    const float2 *in = A.part + m.y * stride + (size_t)pair * 64 + lane;
+    float4 acc[1] = {make_float4(0.0f, 0.0f, 0.0f, 0.0f)};
+    for (unsigned k0 = 0; k0 < n; k0 += 16) {
+        float2 q[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) q[i] = in[min(k0 + i, n - 1u) * stride];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            float2 part[1] = {k0 + i < n ? q[i] : make_float2(0.0f, 0.0f)};
+            merge<1>(acc, part);
+        }
+    }
+    store_cells<GR_ACCUM_COMPENSATED, 1>(A, pair, 1, a, b, acc);
 }
 
 // ---- the precomputed gather operator ----------------------------------------
@@ -1068,7 +1189,7 @@ hipError_t launch(const GridArgs &A, const GopArgs *O, int groups, size_t lds_ba
     const size_t lds = lds_base + sizeof(float2) * 128 * wpb * P;  // two staging buffers per wave
     hipError_t e = gr_allow_lds(k_grid<ACCUM, P>, lds);
     if (e != hipSuccess) return e;
-    const int blocks = kGridSectors * ((A.sector_len + wpb - 1) / wpb);
+    const int blocks = split_blocks(A.n_sitems, wpb) + kGridSectors * ((A.sector_len - A.split_slots + wpb - 1) / wpb);
     hipLaunchKernelGGL((k_grid<ACCUM, P>), dim3(blocks, groups), dim3(64 * wpb), lds, s, A);
     return hipGetLastError();
 }
@@ -1130,6 +1251,9 @@ GridArgs make_args(const GrGeom &g, const GrDevTables &t, int n_ang, long ltbl) 
     A.L2m = g.L2 + 0.01f;
     A.dmax = 3.5f * 1.41421356f + A.L2m * 1.41421356f + 0.05f;
     A.rmax = gr_grid_rmax(g);
+    A.sitems = nullptr;
+    A.n_sitems = A.split_slots = A.part_pairs = 0;
+    A.part = nullptr;
     return A;
 }
 
@@ -1167,13 +1291,43 @@ hipError_t gr_launch_grid(const GrGeom &g, const GrDevTables &t, int n_ang, long
     const GopArgs *op = t.gop ? &O : nullptr;
     const size_t lds_base = sizeof(float) * A.lds_wtbl;
     const int wpb = g.grid_wpb == 1 || g.grid_wpb == 2 ? g.grid_wpb : 4;
+    const bool split = !op && t.n_sitems > 0 && accum == GR_ACCUM_COMPENSATED;
+    if (split) {
+        A.sitems = t.sitems;
+        A.n_sitems = t.n_sitems;
+        A.split_slots = t.split_slots;
+        A.part = scratch;
+        A.part_pairs = pairs;
+    }
     hipError_t e = accum == GR_ACCUM_PLAIN ? launch_all<GR_ACCUM_PLAIN>(A, op, pairs, lds_base, wpb, s)
                                            : launch_all<GR_ACCUM_COMPENSATED>(A, op, pairs, lds_base, wpb, s);
-    if (e != hipSuccess || !op || !cut) return e;
+    if (e != hipSuccess) return e;
     A.pair_base = 0;
     A.pair_end = pairs;
+    if (split) {
+        hipLaunchKernelGGL(k_split_merge, dim3((t.n_smeta * pairs + 3) / 4), dim3(256), 0, s, A, t.smeta, t.n_smeta,
+                           pairs);
+        return hipGetLastError();
+    }
+    if (!cut) return e;
     const int waves = O.n_split * pairs;
     hipLaunchKernelGGL(k_gop_merge, dim3((waves + 3) / 4), dim3(256), 0, s, A, O, pairs);
+    return hipGetLastError();
+}
+
+hipError_t gr_launch_split_lines(const GrGeom &g, const GrDevTables &t, int n_ang, long ltbl, int slots,
+                                 unsigned *lines, hipStream_t s) {
+    const GridArgs A = make_args(g, t, n_ang, ltbl);
+    hipLaunchKernelGGL(k_split_lines<0>, dim3((kGridSectors * slots + 3) / 4), dim3(256), 0, s, A, slots, lines,
+                       (const unsigned *)nullptr, (uint4 *)nullptr);
+    return hipGetLastError();
+}
+
+hipError_t gr_launch_split_items(const GrGeom &g, const GrDevTables &t, int n_ang, long ltbl, int slots,
+                                 const unsigned *first, uint4 *items, hipStream_t s) {
+    const GridArgs A = make_args(g, t, n_ang, ltbl);
+    hipLaunchKernelGGL(k_split_lines<1>, dim3((kGridSectors * slots + 3) / 4), dim3(256), 0, s, A, slots,
+                       (unsigned *)nullptr, first, items);
     return hipGetLastError();
 }
 

@@ -152,3 +152,33 @@ def test_operator_precision_geometry_pair():
     print(f"M=8192 pair: rel-L2 vs oracle {e:.2e}", flush=True)
     assert e < 1e-5
     p.close()
+
+
+# Centre tiles cut at their merge groups (compensated sums, no operator): one
+# line short of a split, exactly and one more than a whole number of groups,
+# angles that all coincide or crowd one window end, a full circle
+SPLIT_ANGLES = {
+    "lines48": dict(geom=1, n_ang=48), "lines49": dict(geom=1, n_ang=49), "groups4": dict(geom=1, n_ang=64),
+    "groups4+1": dict(geom=1, n_ang=65), "full": dict(geom=2, n_ang=130),
+    "equal": dict(geom=0, angles=[33.0] * 90), "crowded": dict(geom=0, angles=list(np.linspace(0, 1, 200)) + [179.99] * 60),
+}
+
+
+@pytest.mark.parametrize("name", sorted(SPLIT_ANGLES))
+@pytest.mark.parametrize("ns", [1, 10])
+def test_split_centre_tiles_are_bitwise_neutral(name, ns):
+    """A window of two columns leaves no room for the partials, so that plan
+    grids whole tiles; its images are bitwise the window of a split plan's,
+    and the operator's."""
+    kw = dict(SPLIT_ANGLES[name])
+    kw["n_ang"] = kw.get("n_ang") or len(kw["angles"])
+    n_det = 60
+    sino = torch.from_numpy(np.random.default_rng(3).standard_normal((ns, kw["n_ang"], n_det)).astype(np.float32)).cuda()
+    imgs = []
+    for crop, op in (((0, 63), "off"), ((0, 63), "on"), ((30, 2), "off")):
+        plan = gr.Plan(n_det=n_det, center=30.2, crop=crop, grid_op=op, **kw)
+        imgs.append(plan.recon(sino))
+        torch.cuda.synchronize()
+        plan.close()
+    assert torch.equal(imgs[0], imgs[1])
+    assert torch.equal(imgs[0][:, 30:32, 30:32], imgs[2])

@@ -73,6 +73,18 @@ __host__ __device__ __forceinline__ bool gr_tap(int j, float C, float S, float q
     return true;
 }
 
+// gr_tap without a branch: whether the sample deposits into the cell, and the
+// weight it has then (some table product otherwise).
+__host__ __device__ __forceinline__ bool gr_tap_weight(int j, float C, float S, float qa, float qb,
+                                                       const GrGatherGeom &g, const float *wtbl, float &w) {
+    float U, V;
+    gr_sample_uv(j, C, S, g, U, V);
+    int iu = gr_nn_index(fabsf(U - qa) * g.tblspcg), iv = gr_nn_index(fabsf(V - qb) * g.tblspcg);
+    iu = iu > g.ltbl ? g.ltbl : iu;
+    iv = iv > g.ltbl ? g.ltbl : iv;
+    w = wtbl[iu] * wtbl[iv];
+    return U - g.L2 <= qa && qa <= U + g.L2 && V - g.L2 <= qb && qb <= V + g.L2;
+}
 
 // Convolvent of the reference's compile-time INTERP variant (grid.cpp:18-24)
 // with its argument parenthesised (as written the macro does not compile:
@@ -157,9 +169,11 @@ __host__ __device__ __forceinline__ int gr_upper_bound(const float *a, int n, fl
     return lo;
 }
 
-__host__ __device__ __forceinline__ void gr_angle_window(int tx, int ty, float M2, float dmax,
-                                                         const float *akey, int n_ang, int &r0,
-                                                         int &r1, int &r2, int &r3) {
+// lower(x), upper(x): the lower and upper bound of x among the sorted keys.
+template <class Lower, class Upper>
+__host__ __device__ __forceinline__ void gr_angle_window_by(int tx, int ty, float M2, float dmax, int n_ang,
+                                                            Lower &&lower, Upper &&upper, int &r0, int &r1, int &r2,
+                                                            int &r3) {
     const float cu = (float)(tx * 8) + 3.5f - M2, cv = (float)(ty * 8) + 3.5f - M2;
     const float Rt = sqrtf(cu * cu + cv * cv);
     r0 = 0;
@@ -173,16 +187,19 @@ __host__ __device__ __forceinline__ void gr_angle_window(int tx, int ty, float M
     if (phi >= kPi) phi -= kPi;
     const float alpha = asinf(fminf(1.0f, dmax / Rt)) + 1e-4f;
     const float lo = phi - alpha, hi = phi + alpha;
-    if (lo < 0.0f) {
-        r0 = gr_lower_bound(akey, n_ang, lo + kPi);
-        r3 = gr_upper_bound(akey, n_ang, hi);
-    } else if (hi >= kPi) {
-        r0 = gr_lower_bound(akey, n_ang, lo);
-        r3 = gr_upper_bound(akey, n_ang, hi - kPi);
-    } else {
-        r0 = gr_lower_bound(akey, n_ang, lo);
-        r1 = gr_upper_bound(akey, n_ang, hi);
-    }
+    const bool under = lo < 0.0f, over = !under && hi >= kPi;  // the window wraps around
+    const int a = lower(under ? lo + kPi : lo), b = upper(over ? hi - kPi : hi);
+    r0 = a;
+    if (under || over) r3 = b;
+    else r1 = b;
+}
+
+__host__ __device__ __forceinline__ void gr_angle_window(int tx, int ty, float M2, float dmax,
+                                                         const float *akey, int n_ang, int &r0,
+                                                         int &r1, int &r2, int &r3) {
+    gr_angle_window_by(
+        tx, ty, M2, dmax, n_ang, [&](float x) { return gr_lower_bound(akey, n_ang, x); },
+        [&](float x) { return gr_upper_bound(akey, n_ang, x); }, r0, r1, r2, r3);
 }
 
 // Candidate samples of one angle for a cell at offset (du, dv) from the grid

@@ -29,8 +29,8 @@
 //
 // Per angle, the samples that can reach the tile form one contiguous range of
 // j for the direct term and one for the mirrored term; the wave stages the P
-// pairs' spectra of that range in its own LDS slot (64 samples at a time) and
-// each lane then runs its own exact candidate range against LDS.
+// pairs' spectra of those ranges in its own LDS slots, several lines at a time,
+// and each lane then tests its own candidates of each line exactly.
 //
 // Accumulation: GR_ACCUM_PLAIN adds each tap's float product in float, in a
 // fixed order (the tile's sample lines by sorted angle key, per line the
@@ -141,44 +141,6 @@ __device__ __forceinline__ void load_pairs(const float2 *src, float2 (&v)[P]) {
     }
 }
 
-template <int P>
-__device__ __forceinline__ void store_pairs(float2 *dst, const float2 (&v)[P]) {
-    if (P == 1) {
-        dst[0] = v[0];
-    } else {
-#pragma unroll
-        for (int i = 0; i < P / 2; i++)
-            reinterpret_cast<float4 *>(dst)[i] = make_float4(v[2 * i].x, v[2 * i].y, v[2 * i + 1].x, v[2 * i + 1].y);
-    }
-}
-
-// Add the taps of samples [j0, j1] into cell (qa, qb) from one chunk of a
-// sample row staged in the wave's LDS buffer stage (slot l: the P pairs'
-// values of sample c0 + l).  In a partial group the spare slots hold other
-// data: their accumulators are never stored.
-template <int ACCUM, int P>
-__device__ __forceinline__ void chunk_taps(const float2 (*stage)[P], int c0, int j0, int j1, float C, float S,
-                                           float qa, float qb, const GrGatherGeom &g, const float *wtbl,
-                                           const float *dwtbl, float4 (&acc)[P], float2 (&part)[P]) {
-    for (int j = j0; j <= j1; j++) {
-        float w;
-        if (dwtbl ? gr_tap_interp(j, C, S, qa, qb, g, wtbl, dwtbl, w) : gr_tap(j, C, S, qa, qb, g, wtbl, w)) {
-            float2 u[P];
-            load_pairs<P>(stage[j - c0], u);
-#pragma unroll
-            for (int p = 0; p < P; p++) {
-                if (ACCUM == GR_ACCUM_COMPENSATED) {
-                    part[p].x = __builtin_fmaf(w, u[p].x, part[p].x);
-                    part[p].y = __builtin_fmaf(w, u[p].y, part[p].y);
-                } else {
-                    acc[p].x += w * u[p].x;
-                    acc[p].z += w * u[p].y;
-                }
-            }
-        }
-    }
-}
-
 // A tile as walk_tile sees it: its centre relative to the grid's, how far a
 // sample of it may be from the centre, and its window of sorted angles, two
 // ranges of keys laid end to end (positions 0 .. n - 1).
@@ -188,6 +150,25 @@ struct TileLines {
     __device__ __forceinline__ int key(int pos) const { return pos < n0 ? r0 + pos : r2 + (pos - n0); }
 };
 
+// Number of the n sorted keys a[] that lie below x (upper: at or below), by
+// the whole wave, 64 keys a step: two loads for up to 4096 angles instead of a
+// chain of a dozen.
+__device__ __forceinline__ int wave_bound(const float *a, int n, float x, bool upper) {
+    const int lane = threadIdx.x & 63;
+    int lo = 0, hi = n;
+    while (lo < hi) {
+        const int step = (hi - lo + 63) >> 6, i = lo + lane * step;
+        const float v = a[min(i, n - 1)];
+        const int c = __popcll(__ballot(i < hi && (upper ? v <= x : v < x)));
+        if (c == 0) return lo;
+        if (step == 1) return lo + c;
+        hi = min(lo + c * step, hi);
+        lo += (c - 1) * step + 1;
+    }
+    return lo;
+}
+
+// By a whole wave (all 64 lanes active).
 __device__ __forceinline__ TileLines tile_lines(const GridArgs &A, int tx, int ty) {
     const float M2 = A.g.fM2;
     TileLines t;
@@ -195,9 +176,14 @@ __device__ __forceinline__ TileLines tile_lines(const GridArgs &A, int tx, int t
     t.cv = (float)(ty * kTile) + 3.5f - M2;
     t.reach = 3.5f + A.L2m;  // tile half-width plus box half-width
     int r1, r3;
-    gr_angle_window(tx, ty, M2, A.dmax, A.akey, A.n_ang, t.r0, r1, t.r2, r3);
-    t.n0 = max(r1 - t.r0, 0);
-    t.n = t.n0 + max(r3 - t.r2, 0);
+    gr_angle_window_by(
+        tx, ty, M2, A.dmax, A.n_ang, [&](float x) { return wave_bound(A.akey, A.n_ang, x, false); },
+        [&](float x) { return wave_bound(A.akey, A.n_ang, x, true); }, t.r0, r1, t.r2, r3);
+    // uniform, and known to be: the loops over the window are scalar then
+    t.r0 = __builtin_amdgcn_readfirstlane(t.r0);
+    t.r2 = __builtin_amdgcn_readfirstlane(t.r2);
+    t.n0 = __builtin_amdgcn_readfirstlane(max(r1 - t.r0, 0));
+    t.n = t.n0 + __builtin_amdgcn_readfirstlane(max(r3 - t.r2, 0));
     return t;
 }
 
@@ -211,38 +197,65 @@ __device__ __forceinline__ bool line_hits(const GridArgs &A, const TileLines &t,
     return td0 <= td1 || tm0 <= tm1;
 }
 
+// A sample line that hits a tile, as a lane holds it: direction and
+// reciprocals, angle index, the tile's samples of it.
+struct Line {
+    float4 cs;
+    int ang, td0, td1, tm0, tm1;
+    __device__ __forceinline__ int direct() const { return max(td1 - td0 + 1, 0); }
+    __device__ __forceinline__ int mirrored() const { return max(tm1 - tm0 + 1, 0); }
+    // lane l's line in every lane
+    __device__ __forceinline__ Line of_lane(int l) const {
+        auto f = [&](float x) { return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(x), l)); };
+        auto i = [&](int x) { return __builtin_amdgcn_readlane(x, l); };
+        return Line{make_float4(f(cs.x), f(cs.y), f(cs.z), f(cs.w)), i(ang), i(td0), i(td1), i(tm0), i(tm1)};
+    }
+};
+
+// The lines of window positions p0 .. p0 + 63, one per lane, and which of
+// them hit the tile.
+__device__ __forceinline__ unsigned long long batch_lines(const GridArgs &A, const TileLines &t, int p0, Line &ln) {
+    const int pos = p0 + (int)(threadIdx.x & 63), k = t.key(min(pos, t.n - 1));
+    ln.cs = A.ang[k];
+    ln.ang = A.aord[k];
+    ln.td0 = ln.tm0 = 1;
+    ln.td1 = ln.tm1 = 0;
+    return __ballot(pos < t.n && line_hits(A, t, ln.cs, ln.td0, ln.td1, ln.tm0, ln.tm1));
+}
+
 // Walk the sample lines that can reach the wave's tile, in the kernel's fixed
 // order (sorted angle keys, the window's two ranges in turn; per line the
 // direct samples, then the mirrored ones, in chunks of at most 64 ascending
 // j), calling on_chunk(mirror, row_off, c0, nj, j0, j1, C, S) per chunk --
 // [c0, c0+nj) the tile's samples of the chunk, [j0, j1] the lane's own
 // candidates among them -- and on_line() after each line that passed the
-// tile tests.  Tiles beyond the largest sample radius visit nothing.  pos0,
-// max_lines: start at window position pos0, stop after that many lines.
+// tile tests.  Tiles beyond the largest sample radius visit nothing.  The
+// lines are tested 64 at a time, one per lane.
 template <class ChunkFn, class LineFn>
 __device__ __forceinline__ void walk_tile(const GridArgs &A, int tx, int ty, bool valid, float du, float dv,
-                                          ChunkFn &&on_chunk, LineFn &&on_line, int pos0 = 0,
-                                          int max_lines = 0x7fffffff) {
+                                          ChunkFn &&on_chunk, LineFn &&on_line) {
     if (!gr_tile_active(tx, ty, A.g.fM2, A.rmax)) return;
     const TileLines t = tile_lines(A, tx, ty);
-    for (int pos = pos0; pos < t.n && max_lines > 0; pos++) {
-        const int k = t.key(pos);
-        const float4 cs = table_load(A.ang, k);
-        int td0, td1, tm0, tm1;
-        if (!line_hits(A, t, cs, td0, td1, tm0, tm1)) continue;
-        max_lines--;
-        int jd0, jd1, jm0, jm1;
-        gr_candidates_r(du, dv, cs.z, cs.w, A.L2m, A.g, jd0, jd1, jm0, jm1);
-        if (!valid) {
-            jd1 = jd0 - 1;
-            jm1 = jm0 - 1;
+    for (int p0 = 0; p0 < t.n; p0 += 64) {
+        Line mine;
+        unsigned long long mask = batch_lines(A, t, p0, mine);
+        for (; mask; mask &= mask - 1) {
+            const Line l = mine.of_lane(__builtin_ctzll(mask));
+            int jd0, jd1, jm0, jm1;
+            gr_candidates_r(du, dv, l.cs.z, l.cs.w, A.L2m, A.g, jd0, jd1, jm0, jm1);
+            if (!valid) {
+                jd1 = jd0 - 1;
+                jm1 = jm0 - 1;
+            }
+            const long row_off = (long)l.ang * A.half;
+            for (int c0 = l.td0; c0 <= l.td1; c0 += 64)
+                on_chunk(0, row_off, c0, min(64, l.td1 - c0 + 1), max(jd0, c0), min(min(jd1, l.td1), c0 + 63), l.cs.x,
+                         l.cs.y);
+            for (int c0 = l.tm0; c0 <= l.tm1; c0 += 64)
+                on_chunk(1, row_off, c0, min(64, l.tm1 - c0 + 1), max(jm0, c0), min(min(jm1, l.tm1), c0 + 63), l.cs.x,
+                         l.cs.y);
+            on_line();
         }
-        const long row_off = (long)table_load(A.aord, k) * A.half;
-        for (int c0 = td0; c0 <= td1; c0 += 64)
-            on_chunk(0, row_off, c0, min(64, td1 - c0 + 1), max(jd0, c0), min(min(jd1, td1), c0 + 63), cs.x, cs.y);
-        for (int c0 = tm0; c0 <= tm1; c0 += 64)
-            on_chunk(1, row_off, c0, min(64, tm1 - c0 + 1), max(jm0, c0), min(min(jm1, tm1), c0 + 63), cs.x, cs.y);
-        on_line();
     }
 }
 
@@ -263,10 +276,9 @@ __global__ void __launch_bounds__(256) k_split_lines(GridArgs A, int slots, unsi
         const TileLines t = tile_lines(A, tx, ty);
         for (int p0 = 0; p0 < t.n; p0 += 64) {
             const int pos = p0 + lane;
-            int td0, td1, tm0, tm1;
-            const bool hit = pos < t.n && line_hits(A, t, A.ang[t.key(min(pos, t.n - 1))], td0, td1, tm0, tm1);
-            const unsigned long long mask = __ballot(hit);
-            if (MODE == 1 && hit) {
+            Line mine;
+            const unsigned long long mask = batch_lines(A, t, p0, mine);
+            if (MODE == 1 && (mask >> lane & 1)) {
                 const unsigned rank = n + (unsigned)__popcll(mask & ((1ull << lane) - 1));
                 if (rank % kMergeAngles == 0) {
                     const unsigned i = first[w] + rank / kMergeAngles;
@@ -303,8 +315,74 @@ __host__ __device__ __forceinline__ int split_blocks(int n_items, int wpb) {
     return (n_items + wpb * kGridSectors - 1) / (wpb * kGridSectors) * kGridSectors;
 }
 
+// A wave's sample slots in LDS: plane q holds piece q of every slot (16 bytes
+// of the P pairs' values for P >= 2, the real and the imaginary float for P =
+// 1), so the 16-byte reads of 64 lanes at random slots spread over all banks
+// (a 64-byte record stride would leave them a quarter of them).  Records
+// reach the slots by global-to-LDS loads, which write lane l's piece at the
+// load's LDS base + l * piece: slot l (l + 64, ...) of each plane, no
+// registers in between.  (Loading whole records per lane group instead --
+// coalesced reads, pieces rotated within a slot against bank conflicts --
+// took fewer texture-addresser cycles but more VALU work and was slower.)
+template <int P, int S>
+struct Slots {
+    static constexpr int piece = P >= 2 ? 16 : 4;  // bytes per lane and load
+    static constexpr int planes = P * 8 / piece;
+    static constexpr int plane_bytes = S * piece;
+    static __device__ __forceinline__ void read(const char *stg, unsigned slot, float2 (&v)[P]) {
+        if (P >= 2) {
+#pragma unroll
+            for (int q = 0; q < P / 2; q++) {
+                const float4 x = *reinterpret_cast<const float4 *>(stg + q * plane_bytes + 16 * slot);
+                v[2 * q] = make_float2(x.x, x.y);
+                v[2 * q + 1] = make_float2(x.z, x.w);
+            }
+        } else {
+            v[0] = make_float2(*reinterpret_cast<const float *>(stg + 4 * slot),
+                               *reinterpret_cast<const float *>(stg + plane_bytes + 4 * slot));
+        }
+    }
+};
+
+// Lane l's record into slot slot0 + l.
+template <class St>
+__device__ __forceinline__ void slots_load(const float2 *rec, char *stg, int slot0) {
+#if defined(__HIP_DEVICE_COMPILE__)  // a device builtin: the host pass sees no body
+#pragma unroll
+    for (int q = 0; q < St::planes; q++)
+        __builtin_amdgcn_global_load_lds(
+            (const void *)(reinterpret_cast<const char *>(rec) + q * St::piece),
+            (__attribute__((address_space(3))) void *)(stg + q * St::plane_bytes + slot0 * St::piece), St::piece, 0, 0);
+#else
+    (void)rec;
+    (void)stg;
+    (void)slot0;
+#endif
+}
+
+// k_grid's slots per wave, a multiple of 64: the samples of several lines are
+// staged in one round trip to memory (a light tile's are ~100).
+template <int P>
+constexpr int grid_slots() {
+    return P >= 4 ? 128 : 256;
+}
+template <int P>
+constexpr size_t grid_wave_lds() {  // bytes per wave: slots, keys
+    return (size_t)grid_slots<P>() * (P * sizeof(float2) + sizeof(unsigned));
+}
+
+// A wave grids its tile, or one merge group of a split tile, for P pairs: the
+// window's lines are tested 64 at a time, one per lane; the samples of the
+// lines that hit the tile are laid end to end and loaded up to grid_slots at
+// once into the wave's LDS slots (a light tile's ~100 samples in one round
+// trip; a line at a time, the loads' latency and the scalar loads of each
+// line's record bound the kernel); then each lane adds its own taps line by
+// line.  VALU bound: of a line's candidates a lane holds four on average, and
+// the wave runs until its last lane is done.  At 1500 x 2048 on MI355X: one
+// pair 868 -> 620 us, eight pairs 1799 -> 1130; three waves per SIMD (four
+// spill: 1620).
 template <int ACCUM, int P>
-__global__ void __launch_bounds__(256) k_grid(GridArgs A) {
+__global__ void __launch_bounds__(256, 3) k_grid(GridArgs A) {
     extern __shared__ float smem[];
     // the convolvent table (and its differences for INTERP) in LDS, then the
     // waves' staging areas from lds_wtbl on
@@ -316,32 +394,36 @@ __global__ void __launch_bounds__(256) k_grid(GridArgs A) {
     }
     __syncthreads();
 
-    // the tile slot as a wave-uniform value: the tile, its angle window and
-    // each line's angle record then come through scalar loads, which do not
-    // wait behind the spectra loads in the vector memory counter
+    // the tile slot as a wave-uniform value: the tile and its item come
+    // through scalar loads
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, wpb = blockDim.x >> 6;
     // the first workgroups take the merge groups of the split tiles, one per wave
     const int sb = split_blocks(A.n_sitems, wpb);
-    int ti, pos0 = 0, max_lines = 0x7fffffff;
-    float2 *part_out = nullptr;
-    if ((int)blockIdx.x < sb) {
+    const bool split = (int)blockIdx.x < sb;
+    int ti, pos0 = 0, left = 0x7fffffff, slot_out = 0;  // window position to start from, lines to take
+    if (split) {
         const int item = __builtin_amdgcn_readfirstlane((int)blockIdx.x * wpb + wave);
         if (item >= A.n_sitems) return;
         const uint4 it = table_load(A.sitems, item);
         ti = (int)it.x;
         pos0 = (int)it.y;
-        max_lines = kMergeAngles;
-        part_out = A.part + (size_t)it.z * A.part_pairs * 64;
+        left = kMergeAngles;
+        slot_out = (int)it.z;
     } else {
         ti = __builtin_amdgcn_readfirstlane(sector_slot(A, (int)blockIdx.x - sb, wpb, wave, A.split_slots));
         if (ti < 0) return;
     }
     const unsigned tt = table_load(A.tiles, ti);
     if (tt == kGridNoTile) return;
-    float2(*stage)[P] = reinterpret_cast<float2(*)[P]>(smem + A.lds_wtbl) + wave * 128;  // two buffers of 64 slots
+    const int tx = (int)(tt & 0xffffu), ty = (int)(tt >> 16);
+    // a tile that holds only zeros is not written
+    if (!__builtin_amdgcn_readfirstlane((int)gr_tile_active(tx, ty, A.g.fM2, A.rmax))) return;
+    using St = Slots<P, grid_slots<P>()>;
+    constexpr int NS = grid_slots<P>();
+    char *stg = reinterpret_cast<char *>(smem + A.lds_wtbl) + wave * grid_wave_lds<P>();
+    unsigned *keys = reinterpret_cast<unsigned *>(stg + (size_t)NS * P * sizeof(float2));
     const int pair0 = A.pair_base + blockIdx.y * P;
     const int nvalid = min(P, A.pair_end - pair0);
-    const int tx = (int)(tt & 0xffffu), ty = (int)(tt >> 16);
     const int a = tx * kTile + (lane & 7), b = ty * kTile + (lane >> 3);
     const int M = A.g.M;
     const float M2 = A.g.fM2;
@@ -355,60 +437,124 @@ __global__ void __launch_bounds__(256) k_grid(GridArgs A) {
         acc[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         part[p] = make_float2(0.0f, 0.0f);
     }
-
-    int lines = 0;  // sample lines in the open partial
     const long group = spec_group_offset(A, pair0);
     const float2 *base1 = A.spec1 + group, *base2 = A.spec2 + group;
-    // one chunk in flight: a chunk's samples are loaded when walk_tile hands
-    // it over, the taps of the chunk before are added from the other LDS
-    // buffer while the loads travel, and only then do the new values go to
-    // LDS -- the loaded registers never live past their chunk.  Every lane
-    // loads (past the chunk's end it repeats its last sample, never read), so
-    // no load sits in a branch.  The taps and the merges after each line
-    // keep their order.
-    bool have = false, p_eol = false;
-    int cur = 0, p_mirror = 0, p_c0 = 0, p_j0 = 0, p_j1 = -1;
-    float p_C = 0.0f, p_S = 0.0f;
-    auto add_pending = [&]() {
-        chunk_taps<ACCUM, P>(stage + cur * 64, p_c0, p_j0, p_j1, p_C, p_S, p_mirror ? ma : pa, p_mirror ? mb : pb,
-                             A.g, s_wtbl, s_dwtbl, acc, part);
-        if (p_eol && ACCUM == GR_ACCUM_COMPENSATED && ++lines == kMergeAngles) {
-            merge<P>(acc, part);
-            lines = 0;
+    // The lane's taps of samples [j0, j1] of a line, sample j in slot sb + j.
+    // A sample outside the box counts with weight zero, which changes no bit
+    // of a sum of finite samples (sums start at +0 and are never -0; a sample
+    // that is not finite leaves no pixel of its pair's images finite anyway):
+    // cheaper than a branch around the additions, which also doubles the
+    // registers of the sums.
+    auto run_taps = [&](int j0, int j1, int sb_, float C, float S, float qa, float qb) {
+#pragma unroll 1
+        for (int j = j0; j <= j1; j++) {
+            float w = 0.0f;
+            float2 u[P];
+            St::read(stg, (unsigned)(sb_ + j), u);
+            bool ok;
+            if (s_dwtbl) ok = gr_tap_interp(j, C, S, qa, qb, A.g, s_wtbl, s_dwtbl, w);
+            else ok = gr_tap_weight(j, C, S, qa, qb, A.g, s_wtbl, w);
+            if (!ok) w = 0.0f;
+#pragma unroll
+            for (int p = 0; p < P; p++) {
+                if (ACCUM == GR_ACCUM_COMPENSATED) {
+                    part[p].x = __builtin_fmaf(w, u[p].x, part[p].x);
+                    part[p].y = __builtin_fmaf(w, u[p].y, part[p].y);
+                } else {
+                    acc[p].x += w * u[p].x;
+                    acc[p].z += w * u[p].y;
+                }
+            }
         }
     };
-    walk_tile(
-        A, tx, ty, valid, pa - M2, pb - M2,
-        [&](int mirror, long row_off, int c0, int nj, int j0, int j1, float C, float S) {
-            float2 v[P];
-            load_pairs<P>((mirror ? base2 : base1) + (row_off + c0 + min(lane, nj - 1)) * kSpecGroup, v);
-            if (have) add_pending();
-            cur ^= 1;
-            __builtin_amdgcn_wave_barrier();
-            store_pairs<P>(stage[cur * 64 + lane], v);
-            __builtin_amdgcn_wave_barrier();
-            have = true;
-            p_eol = false;
-            p_mirror = mirror;
-            p_c0 = c0;
-            p_j0 = j0;
-            p_j1 = j1;
-            p_C = C;
-            p_S = S;
-        },
-        [&]() { p_eol = true; },  // the pending chunk ends its line
-        pos0, max_lines);
-    if (part_out) {  // a merge group of a split tile: its partials, unmerged
-        if (have) {
-            p_eol = false;
-            add_pending();
+    // the samples are in the slots (the compiler does not see that the loads
+    // above write what run_taps reads) / every read of them is done and the
+    // next may be loaded over them
+    auto slots_filled = [&]() {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto slots_read = [&]() {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+    };
+    int lines = 0;  // sample lines in the open partial
+    const int merge_at = split ? kMergeAngles + 1 : kMergeAngles;  // a split tile's group is not merged here
+    // samples per cell along an axis of direction cosine c, r = 1 / c (0 for
+    // |c| <= 1e-6: then no sample leaves the cell's column, all or none reach it)
+    const float per_cell = 1.0f / A.g.scale;
+    auto axis = [&](float r) { return r != 0.0f ? r * per_cell : 1e7f * per_cell; };
+    const TileLines t = tile_lines(A, tx, ty);
+    for (int p0 = pos0; p0 < t.n && left > 0; p0 += 64) {
+        Line mine;
+        unsigned long long mask = batch_lines(A, t, p0, mine);
+        // a merge group takes its first lines only
+        while (left < 64 && __popcll(mask) > left) mask &= ~(1ull << (63 - __builtin_clzll(mask)));
+        left -= __popcll(mask);
+        // the lines' samples (direct, then mirrored) laid end to end, the
+        // lane's line at [off, end); they are staged NS at a time, and a line
+        // that crosses the border of two rounds is taken in two parts
+        const int nd = mine.direct(), cnt = mask >> lane & 1 ? nd + mine.mirrored() : 0;
+        int end = cnt;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int x = __shfl_up(end, o);
+            end += lane >= o ? x : 0;
         }
+        const int off = end - cnt, total = __builtin_amdgcn_readlane(end, 63);
+        for (int start = 0; start < total; start += NS) {
+            const int n = min(NS, total - start);
+            // each line's lane writes its samples' keys (lane, side, j), then
+            // slot k's lane loads its record
+#pragma unroll 1
+            for (int i = max(start - off, 0); i < min(cnt, start + n - off); i++)
+                keys[off - start + i] = (unsigned)lane << 16 | (unsigned)(i < nd ? mine.td0 + i : (mine.tm0 + i - nd) | 0x8000);
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int k = 0; k < NS; k += 64)
+                if (k < n) {
+                    const unsigned key = keys[min(k + lane, n - 1)];
+                    const long rec = ((long)__shfl(mine.ang, (int)(key >> 16)) * A.half + (int)(key & 0x7fffu)) * kSpecGroup;
+                    slots_load<St>((key & 0x8000u ? base2 : base1) + rec, stg, k);
+                }
+            slots_filled();
+#pragma unroll 1
+            for (unsigned long long m = __ballot(cnt > 0 && end > start && off < start + n); m; m &= m - 1) {
+                const int first = __builtin_ctzll(m);
+                const Line l = mine.of_lane(first);
+                const int o = __builtin_amdgcn_readlane(off, first) - start;  // slot of the line's first sample
+                // the lane's candidates: s = scale j within L2m of the cell in
+                // both axes (a superset of its taps; run_taps tests each)
+                const float ax = axis(l.cs.z), ay = axis(l.cs.w);
+                const float cx = (pa - M2) * ax, cy = (pb - M2) * ay;
+                const float hx = A.L2m * fabsf(ax) + 1e-3f, hy = A.L2m * fabsf(ay) + 1e-3f;
+                const float lo = fmaxf(cx - hx, cy - hy), hi = fminf(cx + hx, cy + hy);
+#pragma unroll 1
+                for (int side = l.td0 <= l.td1 ? 0 : 1; side < (l.tm0 <= l.tm1 ? 2 : 1); side++) {
+                    const int s0 = side ? l.tm0 : l.td0, s1 = side ? l.tm1 : l.td1;
+                    const int sb = (side ? o + l.direct() : o) - s0;  // sample j in slot sb + j
+                    // of the tile's samples in the slots
+                    const float f0 = (float)max(s0, -sb), f1 = valid ? (float)min(s1, n - 1 - sb) : -1.0f;
+                    const int j0 = (int)fmaxf(f0, ceilf(side ? -hi : lo));
+                    const int j1 = (int)fminf(f1, floorf(side ? -lo : hi));
+                    run_taps(j0, j1, sb, l.cs.x, l.cs.y, side ? ma : pa, side ? mb : pb);
+                }
+                lines += __builtin_amdgcn_readlane(end, first) <= start + n ? 1 : 0;
+                if (ACCUM == GR_ACCUM_COMPENSATED && __builtin_amdgcn_readfirstlane(lines) == merge_at) {
+                    merge<P>(acc, part);
+                    lines = 0;
+                }
+            }
+            slots_read();
+        }
+    }
+    if (split) {  // a merge group of a split tile: its partials, unmerged
+        float2 *part_out = A.part + (size_t)slot_out * A.part_pairs * 64;
 #pragma unroll
         for (int p = 0; p < P; p++)
             if (p < nvalid) part_out[(pair0 + p) * 64 + lane] = part[p];
         return;
     }
-    if (have) add_pending();
     if (ACCUM == GR_ACCUM_COMPENSATED && lines) merge<P>(acc, part);
     store_cells<ACCUM, P>(A, pair0, nvalid, a, b, acc);
 }
@@ -807,56 +953,10 @@ __device__ __forceinline__ void grid_op_heavy(const GridArgs &A, const GopArgs &
     store_cells<ACCUM, 1>(A, pair, 1, a, b, acc);
 }
 
-// A wave's record slots in LDS: plane q holds piece q of every slot (16
-// bytes of the P pairs' values for P >= 2, the real and the imaginary float
-// for P = 1), so the 16-byte reads of 64 lanes at random slots spread over
-// all banks (a 64-byte record stride would leave them a quarter of them).
-// Records reach the slots by global-to-LDS loads, which write lane l's piece
-// at the load's LDS base + l * piece: slot l (or l + 64) of each plane, no
-// registers in between.  (Loading whole records per lane group instead --
-// coalesced reads, pieces rotated within a slot against bank conflicts --
-// took fewer texture-addresser cycles but more VALU work and was slower.)
-template <int P>
-struct SopStage {
-    static constexpr int piece = P >= 2 ? 16 : 4;  // bytes per lane and load
-    static constexpr int planes = P * 8 / piece;
-    static constexpr int plane_bytes = kSopSlots * piece;
-};
-
 template <int P>
 __device__ __forceinline__ void sop_stage(unsigned key, const float2 *base1, const float2 *base2, char *stg,
                                           int slot0) {
-    const char *rec = reinterpret_cast<const char *>(((key & kGopMirror) ? base2 : base1) +
-                                                     (long)(key & kGopIdx) * kSpecGroup);
-#if defined(__HIP_DEVICE_COMPILE__)  // a device builtin: the host pass sees no body
-    using St = SopStage<P>;
-#pragma unroll
-    for (int q = 0; q < St::planes; q++)
-        __builtin_amdgcn_global_load_lds(
-            (const void *)(rec + q * St::piece),
-            (__attribute__((address_space(3))) void *)(stg + q * St::plane_bytes + slot0 * St::piece), St::piece,
-            0, 0);
-#else
-    (void)rec;
-    (void)stg;
-    (void)slot0;
-#endif
-}
-
-template <int P>
-__device__ __forceinline__ void sop_read(const char *stg, unsigned slot, float2 (&v)[P]) {
-    using St = SopStage<P>;
-    if (P >= 2) {
-#pragma unroll
-        for (int q = 0; q < P / 2; q++) {
-            const float4 x = *reinterpret_cast<const float4 *>(stg + q * St::plane_bytes + 16 * slot);
-            v[2 * q] = make_float2(x.x, x.y);
-            v[2 * q + 1] = make_float2(x.z, x.w);
-        }
-    } else {
-        v[0] = make_float2(*reinterpret_cast<const float *>(stg + 4 * slot),
-                           *reinterpret_cast<const float *>(stg + St::plane_bytes + 4 * slot));
-    }
+    slots_load<Slots<P, kSopSlots>>(((key & kGopMirror) ? base2 : base1) + (long)(key & kGopIdx) * kSpecGroup, stg, slot0);
 }
 
 // The light tiles of one sector for the P pairs of a group from the staged
@@ -909,7 +1009,7 @@ __device__ __forceinline__ void grid_sop_light(const GridArgs &A, const GopArgs 
         auto consume = [&](unsigned e) {
             const float w = s_w[(e >> 8) & 0xfffu] * s_w[e >> 20];
             float2 v[P];
-            sop_read<P>(stg, e & 0xffu, v);
+            Slots<P, kSopSlots>::read(stg, e & 0xffu, v);
 #pragma unroll
             for (int p = 0; p < P; p++) {
                 if (ACCUM == GR_ACCUM_COMPENSATED) {
@@ -1186,7 +1286,7 @@ hipError_t launch(const GridArgs &A, const GopArgs *O, int groups, size_t lds_ba
             hipLaunchKernelGGL((k_grid_op<ACCUM, P, true>), dim3(sblocks, groups), dim3(256), lds, s, A, o);
         return hipGetLastError();
     }
-    const size_t lds = lds_base + sizeof(float2) * 128 * wpb * P;  // two staging buffers per wave
+    const size_t lds = lds_base + grid_wave_lds<P>() * wpb;
     hipError_t e = gr_allow_lds(k_grid<ACCUM, P>, lds);
     if (e != hipSuccess) return e;
     const int blocks = split_blocks(A.n_sitems, wpb) + kGridSectors * ((A.sector_len - A.split_slots + wpb - 1) / wpb);

@@ -182,3 +182,32 @@ def test_split_centre_tiles_are_bitwise_neutral(name, ns):
         plan.close()
     assert torch.equal(imgs[0], imgs[1])
     assert torch.equal(imgs[0][:, 30:32, 30:32], imgs[2])
+
+
+# Rounds of the geometry kernel's sample slots: a tenth of a cell per sample
+# (lines of more samples than slots, cut between rounds), a twentieth, and more
+# angles than two steps of the wave's key search cover
+ROUNDS = {
+    "long-lines": dict(n_ang=37, n_det=2000, center=1000.3, R=0.1),
+    "longer-lines": dict(n_ang=20, n_det=3000, center=1499.0, R=0.05, geom=2),
+    "many-angles": dict(n_ang=4300, n_det=40, center=20.1),
+}
+
+
+@pytest.mark.parametrize("name", sorted(ROUNDS))
+@pytest.mark.parametrize("ns,accum", [(2, "compensated"), (7, "compensated"), (16, "compensated"), (3, "plain")])
+def test_geometry_kernel_slot_rounds(name, ns, accum):
+    """Bitwise the operator's images, and rel-L2 1e-5 from the oracle inside the disk."""
+    case = ROUNDS[name]
+    sino = sinos(case, ns, 4)
+    ref = gr.Plan(**case, accum=accum, grid_op="off").recon(sino)
+    out = gr.Plan(**case, accum=accum, grid_op="on").recon(sino)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)
+    s = sino[:2].cpu().numpy()
+    r1, r2 = O.recon_f32(O.Geometry(**case), s[0], s[1])
+    m = r1.shape[0]
+    yy, xx = np.mgrid[:m, :m] - (m - 1) / 2
+    disk = (yy * yy + xx * xx) < (0.45 * m) ** 2
+    for img, r in ((ref[0], r1), (ref[1], r2)):
+        assert O.rel_l2(img.cpu().numpy()[disk], r[disk]) < 1e-5

@@ -11,18 +11,15 @@
 // (taps ky*3+kx, correlation, zero padding).
 //
 // The three 32 -> 32 layers run on MFMA (v_mfma_f32_16x16x32_bf16): a block
-// owns an 8 x 32 pixel tile; its input with a one-pixel halo is staged in
-// LDS with an 80-byte pixel stride (the 16 lanes of a 16-byte read then hit
-// 16 disjoint 4-bank groups).  Forward: D[co][pixel] = W_t[co][ci] x
-// X_t[ci][pixel] summed over the 9 taps; each lane keeps its weight fragments
-// (2 x 9 x 8 bf16) in registers for the whole block.  The input gradient is
-// the same kernel with the taps flipped and the channel roles swapped
-// (packed by k_pack), the ReLU mask of the layer input fused into its
-// epilogue.  The weight gradient is D[co][ci] = dZ[co][pixel] x A_t[pixel][ci]
-// with K running over the pixels of a tile row; dZ and three pre-shifted
-// copies of A (one per kx, so every 16-byte read is aligned) are staged
-// transposed in LDS.  Blocks loop over tiles and write per-block partial sums
-// that k_reduce adds in a fixed order: results are bitwise repeatable.
+// owns a tile of pixels; its input with a one-pixel halo is staged in
+// LDS.  Forward: D[co][pixel] = W_t[co][ci] x X_t[ci][pixel] summed over the 9
+// taps; each lane keeps its weight fragments (2 x 9 x 8 bf16) in registers for
+// the whole block.  The input gradient is the same with the taps flipped and
+// the channel roles swapped (packed by k_pack), the ReLU mask of the layer
+// input in its epilogue.  The weight gradient is D[co][ci] = dZ[co][pixel] x
+// A_t[pixel][ci] with K running over the pixels of a tile row, the operands
+// read transposed from LDS.  Blocks loop over tiles and write per-block partial
+// sums that k_reduce adds in a fixed order: results are bitwise repeatable.
 //
 // The 1 -> 32 and 32 -> 1 layers run on MFMA as well: K over the 9 taps of
 // the single input channel, and W5 in row 0 of A.
@@ -207,18 +204,16 @@ __device__ __forceinline__ void put_tile(uint16_t *sx, int tid, const uint4 (&v)
 }
 
 // ---------------------------------------------------------------------------
-// 32 -> 32 convolution on MFMA.  MODE 0: y = bf16(relu(acc + bias));
-// MODE 1 (input gradient): y = bf16(acc * (mask > 0)).  PF (MODE 0, an
+// 32 -> 32 convolution on MFMA: y = bf16(relu(acc + bias)).  PF (an
 // image under 2^31 bytes): the next tile's activations are loaded into
 // registers while this tile's MFMAs run (the bias is held in registers, so
 // no global load sits between them and the wait), on tiles of TR = 16 rows
 // (the halo 1.2x the output rows instead of 1.33x, half the barriers per
 // pixel); same values, same arithmetic.
-template <int MODE, bool PF = false, int TR = TH>
+template <bool PF, int TR = TH>
 __global__ void __launch_bounds__(256) k_conv32(const uint16_t *__restrict__ x, const uint16_t *__restrict__ wp,
-                                                const float *__restrict__ bias, const uint16_t *__restrict__ mask,
-                                                uint16_t *__restrict__ y, int H, int W, int ntiles, TileMap tm) {
-    static_assert(!PF || MODE == 0, "prefetch: forward only");
+                                                const float *__restrict__ bias, uint16_t *__restrict__ y, int H, int W,
+                                                int ntiles, TileMap tm) {
     static_assert(PF || TR == TH, "staged tiles are TH rows");
     __shared__ __align__(16) uint16_t sx[(TR + 2) * WS * PSTR];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -284,18 +279,10 @@ __global__ void __launch_bounds__(256) k_conv32(const uint16_t *__restrict__ x, 
                 const floatx4 a = nb ? acc1 : acc0;
                 const int co0 = nb * 16 + 4 * g;
                 float v[4] = {a[0], a[1], a[2], a[3]};
-                if (MODE == 0) {
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const float z = v[e] + (PF ? bz[nb][e] : bias[co0 + e]);
-                        v[e] = z > 0.0f ? z : 0.0f;
-                    }
-                } else {
-                    const uint2 m = *reinterpret_cast<const uint2 *>(mask + p * CH + co0);
-                    const uint16_t mm[4] = {(uint16_t)(m.x & 0xffff), (uint16_t)(m.x >> 16), (uint16_t)(m.y & 0xffff),
-                                            (uint16_t)(m.y >> 16)};
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = positive_bf16(mm[e]) ? v[e] : 0.0f;
+                for (int e = 0; e < 4; e++) {
+                    const float z = v[e] + (PF ? bz[nb][e] : bias[co0 + e]);
+                    v[e] = z > 0.0f ? z : 0.0f;
                 }
                 uint2 o;
                 o.x = (uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16);
@@ -444,114 +431,209 @@ __global__ void __launch_bounds__(256) k_conv12(const float *__restrict__ x, flo
     }
 }
 
-// Weight gradient of a 32 -> 32 layer: partial[block] = (dW[t][co][ci], db[co])
-// over the tiles blockIdx.x, blockIdx.x + gridDim.x, ...
-constexpr int DZ_CO = TH * TW + 8;     // sdz channel stride (bf16)
-constexpr int SA_CI = HS * TW + 8;     // sa channel stride (bf16)
-constexpr size_t WGRAD_LDS = sizeof(uint16_t) * (CH * DZ_CO + 3 * CH * SA_CI) + sizeof(float) * 256 * 8;
+// ---------------------------------------------------------------------------
+// Backward of a 32 -> 32 layer in one pass: the input gradient
+// dzn = bf16(conv^T(dz) * (a > 0)) and the weight gradient's partial sums, from
+// one read of dz (with its halo) and a.  Bound by HBM: dz, a and dzn once each
+// (1.7 GB per layer of the 32 x 512^2 batch); as two kernels dz and a came
+// twice, and the weight gradient staged four transposed copies by 16-bit LDS
+// stores: 734 + 322 us per layer, now 400.
+//
+// A workgroup of eight waves per CU walks a contiguous range of 16 x 32 pixel
+// tiles, the next tile's records on their way into the other of two LDS
+// buffers (global-to-LDS, no registers) while this one is computed.  Per
+// pixel 64 bytes as in memory, piece s of a pixel in slot s ^ (column / 4 mod
+// 4): the 16-byte fragment reads of 16 neighbouring pixels and the transposing
+// reads touch every bank alike, and since the swizzle depends on the column
+// only, every read of a lane is one of a few addresses plus a constant.
+// * Input gradient: wave w takes rows 2w and 2w + 1; a fragment of a halo row
+//   serves both.  The MFMAs of an output are those of the forward kernel on
+//   the flipped weights, tap by tap.
+// * Weight gradient, dW[t][co][ci] = sum_q dz[q - off_t][co] a[q][ci]: K runs
+//   over the 32 pixels q of a tile row, both operands by transposing LDS reads
+//   (ds_read_b64_tr_b16: lane l of 16 receives channel l of four pixels); wave
+//   w takes the channel quadrant w mod 4 of rows 8 (w / 4) .., the fragments
+//   of three dz rows held in registers while a's rows pass.
+//   db is one more MFMA against ones.  Every wave keeps its sums over all its
+//   tiles and writes them once: records 2 b and 2 b + 1 of workgroup b.
+constexpr int BK_TH = 16, BK_WS = TW + 2, BK_NP = (BK_TH + 2) * BK_WS;  // tile rows, halo columns, halo pixels
+constexpr int BK_DZ_LOADS = (BK_NP * 4 + 63) / 64, BK_A_LOADS = BK_TH * TW * 4 / 64;  // of a wave, 1 KB each
+constexpr int BK_BUF = (BK_DZ_LOADS + BK_A_LOADS) * 1024;
+constexpr size_t BK_LDS = 2 * (size_t)BK_BUF;
+constexpr int BK_THREADS = 512;
 
-__global__ void __launch_bounds__(256) k_conv32_wgrad(const uint16_t *__restrict__ a, const uint16_t *__restrict__ dz,
-                                                      float *__restrict__ part, int H, int W, int ntiles, TileMap tm) {
+__device__ const uint4 zero_piece = {0u, 0u, 0u, 0u};  // what pixels outside the image read
+
+// Lane l's 16 bytes at p into lds + 16 l.
+__device__ __forceinline__ void load_piece(const void *p, unsigned char *lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_global_load_lds(p, (__attribute__((address_space(3))) void *)lds, 16, 0, 0);
+#else
+    (void)p;
+    (void)lds;
+#endif
+}
+
+// Eight K values of a lane by two transposing reads of four.
+__device__ __forceinline__ bf16x8 read_tr(const unsigned char *p0, const unsigned char *p1) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef short s4 __attribute__((ext_vector_type(4)));
+    struct {
+        s4 lo, hi;
+    } v = {__builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4 *)p0),
+           __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4 *)p1)};
+    return __builtin_bit_cast(bf16x8, v);
+#else
+    (void)p0;
+    (void)p1;
+    return bf16x8{};
+#endif
+}
+
+__global__ void __launch_bounds__(BK_THREADS, 2) k_conv32_back(const uint16_t *__restrict__ a,
+                                                              const uint16_t *__restrict__ dz,
+                                                              const uint16_t *__restrict__ wp,
+                                                              uint16_t *__restrict__ dzn, float *__restrict__ part,
+                                                              int H, int W, int ntiles, TileMap tm) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    uint16_t *sdz = reinterpret_cast<uint16_t *>(smem_raw);      // [co][r*TW + c]
-    uint16_t *sa = sdz + CH * DZ_CO;                             // [kx][ci][r*TW + c]
-    float *sdb = reinterpret_cast<float *>(sa + 3 * CH * SA_CI); // [256][8]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 15, g = lane >> 4;
-    floatx4 acc[9];
-#pragma unroll
-    for (int i = 0; i < 9; i++) acc[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    float db[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    const int ch = tid & 3;  // the channel chunk this thread stages (256 % 4 == 0)
-    // The next tile's records are loaded into registers while this tile's are
-    // added (its loads are in flight during the MFMAs): DZ_N pieces of dz and
-    // A_N of a per thread.
-    constexpr int DZ_N = TH * TW * 4 / 256, A_N = (HS * WS * 4 + 255) / 256;
-    uint4 pdz[DZ_N], pa[A_N];
-    auto fetch = [&](int tile) {
+    // workgroup b (on XCD b mod 8) takes range (b mod 8) nb / 8 + b / 8 of the
+    // tiles: neighbouring ranges, and so most shared halos, on one XCD
+    const int nb = (int)gridDim.x;
+    const int rank = nb % 8 ? (int)blockIdx.x : (int)(blockIdx.x % 8) * (nb / 8) + (int)blockIdx.x / 8;
+    const int t0 = (int)((long)ntiles * rank / nb), t1 = (int)((long)ntiles * (rank + 1) / nb);
+
+    auto load = [&](int tile, unsigned char *buf) {
         int img, y0, x0;
-        tm.of(tile, img, y0, x0);
-        const long ibase = (long)img * H * W;
+        tm.of_rows(tile, BK_TH, img, y0, x0);
+        const uint16_t *di = dz + (long)img * H * W * CH, *ai = a + (long)img * H * W * CH;
 #pragma unroll
-        for (int k = 0; k < DZ_N; k++) {
-            const int pix = (tid + 256 * k) >> 2, r = pix / TW, c = pix - r * TW, gy = y0 + r, gx = x0 + c;
-            pdz[k] = make_uint4(0u, 0u, 0u, 0u);
-            if (gy < H && gx < W) pdz[k] = *reinterpret_cast<const uint4 *>(dz + ((ibase + (long)gy * W + gx) * CH + ch * 8));
+        for (int k = 0; k < (BK_DZ_LOADS + 7) / 8; k++) {
+            const int i = wave + 8 * k;
+            if (i >= BK_DZ_LOADS) break;
+            const int s = i * 64 + lane, p = s >> 2, r = p / BK_WS, c = p - r * BK_WS;
+            const int gy = y0 + r - 1, gx = x0 + c - 1;
+            const bool in = p < BK_NP && (unsigned)gy < (unsigned)H && (unsigned)gx < (unsigned)W;
+            const void *src = di + (((long)gy * W + gx) * CH + ((s ^ (c >> 2)) & 3) * 8);
+            load_piece(in ? src : &zero_piece, buf + i * 1024);
         }
 #pragma unroll
-        for (int k = 0; k < A_N; k++) {
-            const int i = tid + 256 * k, pix = i >> 2, r = pix / WS, cc = pix - r * WS;
-            const int gy = y0 + r - 1, gx = x0 + cc - 1;
-            pa[k] = make_uint4(0u, 0u, 0u, 0u);
-            if (i < HS * WS * 4 && gy >= 0 && gy < H && gx >= 0 && gx < W)
-                pa[k] = *reinterpret_cast<const uint4 *>(a + ((ibase + (long)gy * W + gx) * CH + ch * 8));
+        for (int k = 0; k < BK_A_LOADS / 8; k++) {
+            const int i = wave + 8 * k;
+            const int s = i * 64 + lane, p = s >> 2, r = p / TW, c = p - r * TW;
+            const int gy = y0 + r, gx = x0 + c;
+            const void *src = ai + (((long)gy * W + gx) * CH + ((s ^ (c >> 2)) & 3) * 8);
+            load_piece(gy < H && gx < W ? src : &zero_piece, buf + (BK_DZ_LOADS + i) * 1024);
         }
     };
-    if (blockIdx.x < ntiles) fetch(blockIdx.x);
+    if (t0 < t1) load(t0, smem_raw);
 
-    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        __syncthreads();  // previous tile's reads done
+    bf16x8 A[2][9];
 #pragma unroll
-        for (int k = 0; k < DZ_N; k++) {
-            const int pix = (tid + 256 * k) >> 2;
-            const uint32_t w[4] = {pdz[k].x, pdz[k].y, pdz[k].z, pdz[k].w};
+    for (int n = 0; n < 2; n++)
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const uint16_t h = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
-                sdz[(ch * 8 + e) * DZ_CO + pix] = h;
-                db[e] += from_bf16(h);
-            }
-        }
+        for (int t = 0; t < 9; t++)
+            A[n][t] = *reinterpret_cast<const bf16x8 *>(wp + ((t * CH + n * 16 + j) * CH + 8 * g));
+    bf16x8 ones;
 #pragma unroll
-        for (int k = 0; k < A_N; k++) {
-            const int i = tid + 256 * k, pix = i >> 2;
-            if (i >= HS * WS * 4) break;
-            const int r = pix / WS, cc = pix - r * WS;
-            const uint32_t w[4] = {pa[k].x, pa[k].y, pa[k].z, pa[k].w};
+    for (int e = 0; e < 8; e++) ones[e] = (__bf16)1.0f;
+    const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    floatx4 dw[9], db = zero;
 #pragma unroll
-            for (int kx = 0; kx < 3; kx++) {
-                const int c = cc - kx;  // sa[kx] column c holds input column x0 + c + kx - 1
-                if (c < 0 || c >= TW) continue;
+    for (int t = 0; t < 9; t++) dw[t] = zero;
+    const int nbo = (wave >> 1) & 1, nbi = wave & 1, rh = wave >> 2;  // wgrad: quadrant and row half
+
+    // a lane's addresses within a row: 16-byte piece g of column cb + j + kx
+    // (a column 16 further has the same slot), the transposed four channels of
+    // column kx + 8 g + 4 h + j / 4
+    auto slot = [](int c, int piece) { return c * 64 + ((piece ^ (c >> 2)) & 3) * 16; };
+    int o_b[3], o_z[3][2], o_a[2], o_m[2];
 #pragma unroll
-                for (int e = 0; e < 8; e++)
-                    sa[(kx * CH + ch * 8 + e) * SA_CI + r * TW + c] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
-            }
-        }
-        if (tile + (int)gridDim.x < ntiles) fetch(tile + gridDim.x);
+    for (int k = 0; k < 3; k++) {
+        o_b[k] = 2 * wave * BK_WS * 64 + slot(j + k, g);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            o_z[k][h] = rh * 8 * BK_WS * 64 + slot(k + 8 * g + 4 * h + (j >> 2), nbo * 2 + ((j & 3) >> 1)) + 8 * (j & 1);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        o_a[h] = BK_DZ_LOADS * 1024 + rh * 8 * TW * 64 + slot(8 * g + 4 * h + (j >> 2), nbi * 2 + ((j & 3) >> 1)) + 8 * (j & 1);
+        o_m[h] = BK_DZ_LOADS * 1024 + 2 * wave * TW * 64 + slot(j, h * 2 + (g >> 1)) + 8 * (g & 1);
+    }
+
+    for (int tile = t0; tile < t1; tile++) {
+        const unsigned char *cur = smem_raw + ((tile - t0) & 1) * BK_BUF;
+        // this tile's records have arrived, and every wave is done with the other buffer
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-#pragma unroll 1
-        for (int r = 0; r < TH; r++) {
+        if (tile + 1 < t1) load(tile + 1, smem_raw + ((tile + 1 - t0) & 1) * BK_BUF);
+        int img, y0, x0;
+        tm.of_rows(tile, BK_TH, img, y0, x0);
+        const long ibase = (long)img * H * W;
 #pragma unroll
-            for (int i = 0; i < 9; i++) {
-                const int b = wave * 9 + i;  // 36 blocks: tap t, co half, ci half
-                const int t = b >> 2, nbo = (b >> 1) & 1, nbi = b & 1;
-                const int ky = t / 3, kx = t - ky * 3;
-                const bf16x8 Av = *reinterpret_cast<const bf16x8 *>(sdz + (nbo * 16 + j) * DZ_CO + r * TW + 8 * g);
-                const bf16x8 Bv =
-                    *reinterpret_cast<const bf16x8 *>(sa + (kx * CH + nbi * 16 + j) * SA_CI + (r + ky) * TW + 8 * g);
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Av, Bv, acc[i], 0, 0, 0);
+        for (int cb = 0; cb < TW; cb += 16) {
+            floatx4 acc[2][2] = {{zero, zero}, {zero, zero}};
+#pragma unroll
+            for (int hr = 0; hr < 4; hr++)
+#pragma unroll
+                for (int kx = 0; kx < 3; kx++) {
+                    const bf16x8 B = *reinterpret_cast<const bf16x8 *>(cur + o_b[kx] + (hr * BK_WS + cb) * 64);
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        const int ky = hr - i;
+                        if (ky < 0 || ky > 2) continue;
+                        acc[i][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[0][ky * 3 + kx], B, acc[i][0], 0, 0, 0);
+                        acc[i][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[1][ky * 3 + kx], B, acc[i][1], 0, 0, 0);
+                    }
+                }
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int gy = y0 + 2 * wave + i, gx = x0 + cb + j;
+                if (gy < H && gx < W) {
+                    uint16_t *dst = dzn + (ibase + (long)gy * W + gx) * CH + 4 * g;
+#pragma unroll
+                    for (int n = 0; n < 2; n++) {
+                        const uint2 m = *reinterpret_cast<const uint2 *>(cur + o_m[n] + (i * TW + cb) * 64);
+                        const uint16_t mm[4] = {(uint16_t)(m.x & 0xffff), (uint16_t)(m.x >> 16),
+                                                (uint16_t)(m.y & 0xffff), (uint16_t)(m.y >> 16)};
+                        float v[4];
+#pragma unroll
+                        for (int e = 0; e < 4; e++) v[e] = positive_bf16(mm[e]) ? acc[i][n][e] : 0.0f;
+                        uint2 o;
+                        o.x = (uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16);
+                        o.y = (uint32_t)to_bf16(v[2]) | ((uint32_t)to_bf16(v[3]) << 16);
+                        *reinterpret_cast<uint2 *>(dst + n * 16) = o;
+                    }
+                }
             }
         }
-    }
-    float *out = part + (long)blockIdx.x * WG_REC;
+        bf16x8 z[3][3];  // dz halo rows r, r + 1, r + 2 (slot row mod 3) at columns 0, 1, 2 on
 #pragma unroll
-    for (int i = 0; i < 9; i++) {
-        const int b = wave * 9 + i;
-        const int t = b >> 2, nbo = (b >> 1) & 1, nbi = b & 1;
+        for (int r = 0; r < 2; r++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int co = nbo * 16 + 4 * g + e, ci = nbi * 16 + j;
-            out[(t * CH + co) * CH + ci] = acc[i][e];
+            for (int k = 0; k < 3; k++)
+                z[r][k] = read_tr(cur + o_z[k][0] + r * BK_WS * 64, cur + o_z[k][1] + r * BK_WS * 64);
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                z[(r + 2) % 3][k] = read_tr(cur + o_z[k][0] + (r + 2) * BK_WS * 64, cur + o_z[k][1] + (r + 2) * BK_WS * 64);
+            const bf16x8 av = read_tr(cur + o_a[0] + r * TW * 64, cur + o_a[1] + r * TW * 64);
+#pragma unroll
+            for (int t = 0; t < 9; t++)
+                dw[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(z[(r + 2 - t / 3) % 3][2 - t % 3], av, dw[t], 0, 0, 0);
+            if (nbi == 0) db = __builtin_amdgcn_mfma_f32_16x16x32_bf16(z[(r + 1) % 3][1], ones, db, 0, 0, 0);
         }
     }
-    __syncthreads();
+    float *out = part + (long)(2 * blockIdx.x + rh) * WG_REC;
 #pragma unroll
-    for (int e = 0; e < 8; e++) sdb[tid * 8 + e] = db[e];
-    __syncthreads();
-    if (tid < CH) {  // channel tid: chunk tid/8, element tid%8, summed over the threads of that chunk in order
-        float s = 0.0f;
-        for (int k = tid >> 3; k < 256; k += 4) s += sdb[k * 8 + (tid & 7)];
-        out[9 * CH * CH + tid] = s;
+    for (int t = 0; t < 9; t++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) out[(t * CH + nbo * 16 + 4 * g + e) * CH + nbi * 16 + j] = dw[t][e];
+    if (nbi == 0 && j == 0) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) out[9 * CH * CH + nbo * 16 + 4 * g + e] = db[e];
     }
 }
 
@@ -1321,7 +1403,7 @@ int gr_cnn_forward(const float *params, const unsigned short *packed, const floa
     int npf = 0;
     if (pf) {
         int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_conv32<0, true, 16>, 256, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_conv32<true, 16>, 256, 0) !=
                 hipSuccess ||
             per_cu < 1)
             per_cu = 1;
@@ -1330,11 +1412,10 @@ int gr_cnn_forward(const float *params, const unsigned short *packed, const floa
     }
     auto conv32 = [&](const uint16_t *in, const uint16_t *wl, const float *b, uint16_t *out) {
         if (pf)
-            hipLaunchKernelGGL((k_conv32<0, true, 16>), dim3(npf), dim3(256), 0, s, in, wl, b,
-                               (const uint16_t *)nullptr, out, H, W, nt16, tm16);
+            hipLaunchKernelGGL((k_conv32<true, 16>), dim3(npf), dim3(256), 0, s, in, wl, b, out, H, W, nt16,
+                               tm16);
         else
-            hipLaunchKernelGGL((k_conv32<0, false>), dim3(nconv), dim3(256), 0, s, in, wl, b,
-                               (const uint16_t *)nullptr, out, H, W, ntiles, tm);
+            hipLaunchKernelGGL((k_conv32<false>), dim3(nconv), dim3(256), 0, s, in, wl, b, out, H, W, ntiles, tm);
     };
     // inference (a3 aliasing a1 and a4 aliasing a2: the caller keeps no
     // activation): the first layer fused into the second
@@ -1448,16 +1529,17 @@ int gr_cnn_backward(const float *params, const unsigned short *packed, const flo
     // layers 4, 3, 2
     const unsigned short *acts[4] = {a1, a2, a3, a4};
     const int woff[3] = {OFF_W2, OFF_W3, OFF_W4}, boff[3] = {OFF_B2, OFF_B3, OFF_B4};
-    CNN_HIP(gr_allow_lds(k_conv32_wgrad, WGRAD_LDS));
+    CNN_HIP(gr_allow_lds(k_conv32_back, BK_LDS));
+    const TileMap tmb{tm.tiles_x, (H + BK_TH - 1) / BK_TH};
+    const int ntb = tmb.tiles_x * tmb.tiles_y * n;
+    const int nback = std::min(ntb, std::min(MAX_WG_BLOCKS / 2, gr_cu_count() > 0 ? gr_cu_count() : 256));
     uint16_t *dz = dzA, *dzn = dzB;
     for (int l = 2; l >= 0; l--) {  // layer l+2: input acts[l], output gradient dz
-        const uint16_t *ain = reinterpret_cast<const uint16_t *>(acts[l]);
-        hipLaunchKernelGGL(k_conv32_wgrad, dim3(nwg), dim3(256), WGRAD_LDS, s, ain, dz, part, H, W, ntiles, tm);
-        hipLaunchKernelGGL(k_reduce, dim3((WG_REC + 63) / 64), dim3(64 * RED_WAVES), 0, s, part, nwg, WG_REC, 0,
+        hipLaunchKernelGGL(k_conv32_back, dim3(nback), dim3(BK_THREADS), BK_LDS, s,
+                           reinterpret_cast<const uint16_t *>(acts[l]), dz, pk + (long)l * PACK_LAYER + 9 * CH * CH, dzn,
+                           part, H, W, ntb, tmb);
+        hipLaunchKernelGGL(k_reduce, dim3((WG_REC + 63) / 64), dim3(64 * RED_WAVES), 0, s, part, 2 * nback, WG_REC, 0,
                            grads + woff[l], grads + boff[l]);
-        hipLaunchKernelGGL(k_conv32<1>, dim3(ntiles < MAX_CONV_BLOCKS ? ntiles : MAX_CONV_BLOCKS), dim3(256), 0, s,
-                           dz, pk + (long)l * PACK_LAYER + 9 * CH * CH, (const float *)nullptr, ain, dzn, H, W,
-                           ntiles, tm);
         std::swap(dz, dzn);
     }
     // layer 1

@@ -303,3 +303,29 @@ def test_backward_on_512_gridrec_pairs():
         e = rel(gg[k], g[k])
         print(f"grad {k}: rel-L2 {e:.2e}", flush=True)
         assert e < 1e-2, k
+
+
+# the fused backward's 16 x 32 tiles, two rows per wave and eight-row halves:
+# single pixels, rows and columns, one short of, exactly and one past a tile,
+# several tiles and images
+@pytest.mark.parametrize("n,H,W", [(1, 1, 1), (3, 1, 40), (2, 33, 1), (1, 15, 31), (2, 16, 32), (1, 17, 33), (5, 8, 64),
+                                   (1, 50, 97)])
+def test_backward_tile_edges(n, H, W):
+    """Every gradient against the oracle's backward on the GPU's activations.
+    Both round dz to bf16, so they differ where an accumulation order moves a
+    value across a rounding boundary: one in some hundreds of values by one
+    part in 2^8, far below the 2e-3 that one wrong halo pixel would exceed."""
+    net, pd, x, t = make(n + H + W, n, H, W)
+    xg, tg = torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda()
+    net.forward(xg, train=True)
+    net.backward(xg, tg)
+    torch.cuda.synchronize()
+    c = K.forward(pd, x, net.scale)
+    for l, act in enumerate(net._buffers(*x.shape, True)[0]):
+        c[f"a{l + 1}"] = bf16_bits_to_f32(act)
+    c["y"] = net._buffers(*x.shape, True)[2].cpu().numpy()
+    loss, g = K.loss_and_backward(pd, c, t, net.scale)
+    assert abs(float(net.loss.cpu()) - loss) <= 1e-5 * loss
+    gg = Lrn.unflatten(net.grads.cpu().numpy())
+    for k in g:
+        assert np.linalg.norm(gg[k] - g[k]) <= 2e-3 * np.linalg.norm(g[k]), k

@@ -42,22 +42,20 @@ size_t gr_cnn_work_bytes(int n, int H, int W);
  * after every change of params. */
 int gr_cnn_pack(const float *params, unsigned short *packed, void *stream);
 
-/* Forward pass.  a1..a4 receive the activations.  For inference a3 may alias
- * a1 and a4 a2: then the first layer runs fused into the second, a1 is never
- * written (a1's buffer ends holding a3, a2's a4), and y, yn and slice_stats
- * are bitwise those of distinct buffers.  y (may be NULL): the corrected images in the input's units;
- * yn (may be NULL): the same in network units (x/scale + residual), needed by
- * gr_cnn_backward.  slice_stats (may be NULL, needs work): per image, the sums
- * of residual^2 and (x/scale)^2 in network units (2n floats) -- the
- * correction norm of the fallback test. */
+/* Forward pass, all layers in one kernel.  a1..a4 receive the activations;
+ * consecutive ones must be distinct, and a buffer named for two layers ends
+ * holding the later one (a3 may alias a1 and a4 a2).  y (may be NULL): the
+ * corrected images in the input's units; yn (may be NULL): the same in network
+ * units (x/scale + residual), needed by gr_cnn_backward.  slice_stats (may be
+ * NULL, needs work): per image, the sums of residual^2 and (x/scale)^2 in
+ * network units (2n floats) -- the correction norm of the fallback test. */
 int gr_cnn_forward(const float *params, const unsigned short *packed, const float *x, int n, int H, int W,
                    float scale, unsigned short *a1, unsigned short *a2, unsigned short *a3,
                    unsigned short *a4, float *y, float *yn, float *slice_stats, void *work, void *stream);
 
-/* Inference: gr_cnn_forward's y (bitwise) with the five layers fused in one
- * kernel and no activation buffers; slice_stats as there (values may differ
- * in the last bits: another summation order).  work: gr_cnn_infer_work_bytes(n,
- * H, W) bytes when slice_stats is given, else may be NULL. */
+/* Inference: gr_cnn_forward's y and slice_stats (bitwise) with no activation
+ * buffers.  work: gr_cnn_infer_work_bytes(n, H, W) bytes when slice_stats is
+ * given, else may be NULL. */
 size_t gr_cnn_infer_work_bytes(int n, int H, int W);
 int gr_cnn_infer(const float *params, const unsigned short *packed, const float *x, int n, int H, int W,
                  float scale, float *y, float *slice_stats, void *work, void *stream);

@@ -27,6 +27,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 
 #include "gr_fft.hpp"
@@ -45,7 +46,6 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 constexpr int CH = 32;
 constexpr int TH = 8, TW = 32;            // output tile (rows x columns)
 constexpr int HS = TH + 2, WS = TW + 2;   // with the halo
-constexpr int PSTR = 40;                  // LDS pixel stride in bf16 (80 bytes)
 constexpr int OFF_W1 = 0, OFF_B1 = 288, OFF_W2 = 320, OFF_B2 = OFF_W2 + 9216, OFF_W3 = OFF_B2 + 32,
               OFF_B3 = OFF_W3 + 9216, OFF_W4 = OFF_B3 + 32, OFF_B4 = OFF_W4 + 9216, OFF_W5 = OFF_B4 + 32,
               OFF_B5 = OFF_W5 + 288, N_PARAMS = OFF_B5 + 1;
@@ -54,7 +54,6 @@ constexpr int WG_REC = 9 * CH * CH + CH;     // weight-gradient partial record o
 constexpr int IN_REC = 9 * CH + CH;          // of the 1->32 layer
 constexpr int OUT_REC = 9 * CH + 1;          // of the 32->1 layer
 constexpr int MAX_WG_BLOCKS = 512;
-constexpr int MAX_CONV_BLOCKS = 2048;  // 8 per CU: each loops over tiles with its weights in registers
 
 static_assert(N_PARAMS == 28353, "parameter layout");
 
@@ -71,37 +70,6 @@ __device__ __forceinline__ float round_bf16(float f) { return from_bf16(to_bf16(
 __device__ __forceinline__ bool positive_bf16(uint16_t h) { return !(h & 0x8000u) && h != 0; }
 
 __device__ __forceinline__ __bf16 bf16_of(float f) { return __builtin_bit_cast(__bf16, to_bf16(f)); }
-
-// Stage a tile's activations with their one-pixel halo (HS x WS pixels of 32
-// bf16 channels, four 16-byte pieces each; zeros outside the image) from HBM
-// into LDS at pixel stride PSTR, by a workgroup of 256 threads: a thread's
-// loads go out in batches of BATCH, each batch issued before its LDS stores,
-// so the tile costs ceil(6 / BATCH) memory latencies instead of one per loop
-// trip (BATCH bounds the registers the staging holds).
-template <int BATCH>
-__device__ __forceinline__ void stage_tile(const uint16_t *__restrict__ x, uint16_t *sx, long ibase, int H, int W,
-                                           int y0, int x0, int tid) {
-    constexpr int N = HS * WS * 4, PER = (N + 255) / 256;
-#pragma unroll
-    for (int k0 = 0; k0 < PER; k0 += BATCH) {
-        uint4 v[BATCH];
-#pragma unroll
-        for (int k = 0; k < BATCH; k++) {
-            const int i = tid + (k0 + k) * 256;
-            const int pix = i >> 2, ch = i & 3;
-            const int r = pix / WS, c = pix - r * WS;
-            const int gy = y0 + r - 1, gx = x0 + c - 1;
-            v[k] = make_uint4(0u, 0u, 0u, 0u);
-            if (k0 + k < PER && i < N && gy >= 0 && gy < H && gx >= 0 && gx < W)
-                v[k] = *reinterpret_cast<const uint4 *>(x + ((ibase + (long)gy * W + gx) * CH + ch * 8));
-        }
-#pragma unroll
-        for (int k = 0; k < BATCH; k++) {
-            const int i = tid + (k0 + k) * 256;
-            if (k0 + k < PER && i < N) *reinterpret_cast<uint4 *>(sx + (i >> 2) * PSTR + (i & 3) * 8) = v[k];
-        }
-    }
-}
 
 // The 1 -> 32 and 32 -> 1 layers on MFMA too (v_mfma_f32_16x16x32_bf16, the
 // lane layout of the 32 -> 32 layers: A row = lane & 15, B column = lane & 15,
@@ -120,18 +88,6 @@ __device__ __forceinline__ void conv_in_frag(const float *w1, int lane, bf16x8 (
         }
 }
 
-// B of the 1 -> 32 layer for the pixel whose 3 x 3 neighbourhood starts at
-// xs[r * pitch + c] (bf16 values held as floats).
-__device__ __forceinline__ bf16x8 conv_in_b(const float *xs, int pitch, int r, int c, int lane) {
-    bf16x8 B;
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        const int k = 8 * (lane >> 4) + e;
-        B[e] = bf16_of(k < 9 ? xs[(r + k / 3) * pitch + c + k % 3] : 0.0f);
-    }
-    return B;
-}
-
 // 32 -> 1: nine MFMAs (one per tap, K over the 32 input channels) with W5 in
 // row 0 of A and zeros in rows 1..15; the result D[0][pixel] sits in element 0
 // of lanes 0..15.  w5 holds the bf16 values of W5 as floats, [ci * 9 + t].
@@ -141,20 +97,6 @@ __device__ __forceinline__ void conv_out_frag(const float *w5, int lane, bf16x8 
 #pragma unroll
         for (int e = 0; e < 8; e++)
             A[t][e] = bf16_of((lane & 15) == 0 ? w5[(8 * (lane >> 4) + e) * 9 + t] : 0.0f);
-}
-
-// D of the 32 -> 1 layer for the pixel whose neighbourhood starts at record
-// (r, c) of an LDS region of `pitch` records (PSTR bf16 each).
-__device__ __forceinline__ floatx4 conv_out_mfma(const uint16_t *in, int pitch, int r, int c, int lane,
-                                                 const bf16x8 (&A)[9]) {
-    floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int t = 0; t < 9; t++) {
-        const bf16x8 B = *reinterpret_cast<const bf16x8 *>(in + ((r + t / 3) * pitch + c + t % 3) * PSTR +
-                                                           8 * (lane >> 4));
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[t], B, acc, 0, 0, 0);
-    }
-    return acc;
 }
 
 struct TileMap {
@@ -170,264 +112,295 @@ struct TileMap {
     }
 };
 
-// A tile of TR rows: its activations with their halo (TR + 2 rows of WS
-// pixels, stage_tile's pieces) loaded into registers through a buffer bounded
-// to the tile's image: pieces outside the image read zeros with no branch,
-// so all the loads are in flight together and none is waited for until the
-// pieces are stored (needs H W 64 < 2^31).
-template <int TR>
-struct Stage {
-    static constexpr int rows = TR + 2, n = rows * WS * 4, per = (n + 255) / 256;
+// ---------------------------------------------------------------------------
+// The whole forward pass in one kernel.  A workgroup walks down a strip of 56
+// output columns, two image rows a step, all five layers at once: in step s
+// layer 1 computes rows 2s, 2s + 1 of a1, layer 2 rows 2s - 3 .. of a2, layer 3
+// rows 2s - 6, layer 4 rows 2s - 9, and layer 5 rows 2s - 12 of the output, each
+// from rows that earlier steps left in LDS: rings of six rows per activation,
+// one barrier per step.  So a pixel's activations never come back from HBM
+// (layer by layer they went out and in at 64 bytes per pixel and layer), rows
+// are computed once and columns 64 / 56 times; a training pass writes them as
+// they are made, inference writes none.
+//
+// Columns: 64 in every layer, of which layer l is right in columns l - 1 ..
+// 64 - l (columns depend on their neighbours only); LDS rows hold 66, so every
+// read stays inside.  Pixels outside the image are zero, the padding of the
+// next layer.  Twelve waves, one workgroup per CU: wave w holds the weights of
+// layer 2 + w / 4 in registers and takes columns 16 (w mod 4) .., so each SIMD
+// has a wave of each layer; the waves of layer 2 also compute layer 1, those of
+// layer 3 layer 5 (its weights in LDS), those of layer 4 bring x.  A fragment of
+// an input row serves the output rows of all its taps in the wave's two rows,
+// and in the next step's.  LDS records as in k_conv32_back, piece s of a pixel in
+// slot s ^ (column / 4 mod 4).
+//
+// Per output the MFMAs run tap by tap into one accumulator, then bias, ReLU
+// and rounding, whichever buffers are written.  Bound by MFMA (130 per step and
+// SIMD, half of the time) and what a barrier per step leaves exposed around
+// them: 4 x 2048^2 inference 1.05 ms where five layer kernels took 1.93, of
+// which 6.4 GB of activations 1.36 at the rate of a copy; 32 x 512^2 training
+// 0.87 ms (2.2 GB written) against 1.02.
+constexpr int FW_COLS = 64, FW_OUT = 56, FW_RING = 6, FW_PITCH = FW_COLS + 2;
+constexpr int FW_ROW = FW_PITCH * 64, FW_BUF = FW_RING * FW_ROW;  // bytes of a ring's row, of a ring
+constexpr int FW_XP = 68;                                        // floats per x row
+constexpr int FW_THREADS = 768;
+constexpr size_t FW_LDS = 4 * (size_t)FW_BUF + 9 * 1024 + sizeof(float) * (FW_RING * FW_XP + 4 * CH);
+
+struct FwdArgs {
+    const float *x, *prm;
+    const uint16_t *packed;
+    uint16_t *act[4];  // a1 .. a4, null: not written
+    float *y, *yn, *stats;
+    float scale;
+    int H, W, strips, segs, seg_rows;
 };
-constexpr int STAGE_PER = Stage<TH>::per;
-template <int TR>
-__device__ __forceinline__ void prefetch_tile(const uint16_t *__restrict__ x, int H, int W, int img, int y0, int x0,
-                                              int tid, uint4 (&v)[Stage<TR>::per]) {
-    const GrBuf b = gr_buf(x + (long)img * H * W * CH, (unsigned)((long)H * W * CH * sizeof(uint16_t)));
-#pragma unroll
-    for (int k = 0; k < Stage<TR>::per; k++) {
-        const int i = tid + k * 256;
-        const int pix = i >> 2, ch = i & 3;
-        const int r = pix / WS, c = pix - r * WS;
-        const int gy = y0 + r - 1, gx = x0 + c - 1;
-        const bool in = i < Stage<TR>::n && gy >= 0 && gy < H && gx >= 0 && gx < W;
-        v[k] = gr_buf_ld16(b, in ? (unsigned)(((gy * W + gx) * CH + ch * 8) * sizeof(uint16_t)) : kGrBufNone);
-    }
-}
-template <int TR>
-__device__ __forceinline__ void put_tile(uint16_t *sx, int tid, const uint4 (&v)[Stage<TR>::per]) {
-#pragma unroll
-    for (int k = 0; k < Stage<TR>::per; k++) {
-        const int i = tid + k * 256;
-        if (i < Stage<TR>::n) *reinterpret_cast<uint4 *>(sx + (i >> 2) * PSTR + (i & 3) * 8) = v[k];
-    }
+
+// relu(acc + bias) of four channels as bf16 (NaN gives zero, as z > 0 ? z : 0).
+__device__ __forceinline__ uint2 act_of(floatx4 a, float4 b) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const float v[4] = {fmaxf(a[0] + b.x, 0.0f), fmaxf(a[1] + b.y, 0.0f), fmaxf(a[2] + b.z, 0.0f),
+                        fmaxf(a[3] + b.w, 0.0f)};
+    const bf16x2 lo = {(__bf16)v[0], (__bf16)v[1]}, hi = {(__bf16)v[2], (__bf16)v[3]};
+    return make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
 }
 
-// ---------------------------------------------------------------------------
-// 32 -> 32 convolution on MFMA: y = bf16(relu(acc + bias)).  PF (an
-// image under 2^31 bytes): the next tile's activations are loaded into
-// registers while this tile's MFMAs run (the bias is held in registers, so
-// no global load sits between them and the wait), on tiles of TR = 16 rows
-// (the halo 1.2x the output rows instead of 1.33x, half the barriers per
-// pixel); same values, same arithmetic.
-template <bool PF, int TR = TH>
-__global__ void __launch_bounds__(256) k_conv32(const uint16_t *__restrict__ x, const uint16_t *__restrict__ wp,
-                                                const float *__restrict__ bias, uint16_t *__restrict__ y, int H, int W,
-                                                int ntiles, TileMap tm) {
-    static_assert(PF || TR == TH, "staged tiles are TH rows");
-    __shared__ __align__(16) uint16_t sx[(TR + 2) * WS * PSTR];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // weight fragments, loaded once per wave for all its tiles: lane holds
-    // row co = nb*16 + (lane & 15), k = ci = 8*(lane >> 4) + e
+__global__ void __launch_bounds__(FW_THREADS) k_forward(FwdArgs P) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    bf16x8 *w5 = reinterpret_cast<bf16x8 *>(smem_raw + 4 * FW_BUF);  // layer 5's weight fragments, [tap][lane]
+    float *xr = reinterpret_cast<float *>(w5 + 9 * 64);              // ring of six rows of bf16(x / scale)
+    float *sb = xr + FW_RING * FW_XP;                              // b1 .. b4
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 15, g = lane >> 4, q = wave & 3, c = 16 * q + j;
+    const int H = P.H, W = P.W, per = P.strips * P.segs;
+    const int img = (int)blockIdx.x / per, ws = (int)blockIdx.x - img * per;
+    const int X0 = (ws % P.strips) * FW_OUT - 4, Y0 = (ws / P.strips) * P.seg_rows;
+    const int rows = min(P.seg_rows, H - Y0), top = Y0 - 4;  // relative row r is image row top + r
+    const long ibase = (long)img * H * W;
+    const int gx = X0 + c;
+    const bool col_in = (unsigned)gx < (unsigned)W, col_out = col_in && c >= 4 && c < 4 + FW_OUT;
+
+    const float *xim = P.x + ibase;
+    // x rows r, r + 1 (relative), columns -1 .. 64, by the 256 threads of layer
+    // 4's waves; loads are clamped into the image and their values dropped
+    // where they are used (a load inside a branch is waited for there)
+    const int xt = tid - 512, xi = xt >= FW_PITCH ? 1 : 0, xc = xt - xi * FW_PITCH, xgx = X0 + xc - 1;
+    const int xcl = min(max(xgx, 0), W - 1);
+    auto row_of = [&](int r) { return (long)min(max(top + r, 0), H - 1) * W; };  // uniform
+    auto load_x = [&](int r) {
+        const long r0 = row_of(r);
+        const int d = (int)(row_of(r + 1) - r0);
+        return (xim + r0)[xcl + (xi ? d : 0)];
+    };
+    auto put_x = [&](int r, int slot, float v) {
+        const bool in = (unsigned)xgx < (unsigned)W && (unsigned)(top + r + xi) < (unsigned)H;
+        if (xt >= 0 && xt < 2 * FW_PITCH) xr[slot * FW_XP + xc] = in ? round_bf16(v / P.scale) : 0.0f;
+    };
+    put_x(-1, xi ? 0 : 5, load_x(-1));
+    put_x(1, xi ? 2 : 1, load_x(1));
+    float x_next = load_x(3);
+    if (tid < 4 * CH) {
+        const int l = tid >> 5, off[4] = {OFF_B1, OFF_B2, OFF_B3, OFF_B4};
+        sb[tid] = P.prm[off[l] + (tid & 31)];
+    }
+    if (wave == 4) {
+        bf16x8 A5[9];
+        conv_out_frag(P.prm + OFF_W5, lane, A5);
+#pragma unroll
+        for (int t = 0; t < 9; t++) w5[t * 64 + lane] = A5[t];
+    }
+    auto slot = [](int col, int piece) { return col * 64 + ((piece ^ (col >> 2)) & 3) * 16; };
+    // the wave's layer l + 2 reads ring l and writes ring l + 1
+    const int l = wave >> 2;
+    const unsigned char *o_b[3];  // input fragments at column c + kx - 1
+    int o_w[2];                   // the lane's output channels
+#pragma unroll
+    for (int k = 0; k < 3; k++) o_b[k] = smem_raw + l * FW_BUF + slot(c + k, g);
+#pragma unroll
+    for (int n = 0; n < 2; n++) o_w[n] = slot(c + 1, 2 * n + (g >> 1)) + 8 * (g & 1);
+    const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int last = (rows + 15) / 2;  // step of the last output row
+    // activation row r of the lane's pixel and channels into slot rs of ring
+    // k and, where the caller keeps it, to dst
+    auto put = [&](int k, int r, int rs, uint16_t *dst, floatx4 v0, floatx4 v1, float4 b0, float4 b1) {
+        uint2 h0 = act_of(v0, b0), h1 = act_of(v1, b1);
+        const unsigned m = col_in && (unsigned)(top + r) < (unsigned)H ? ~0u : 0u;  // zeros outside the image
+        h0 = make_uint2(h0.x & m, h0.y & m);
+        h1 = make_uint2(h1.x & m, h1.y & m);
+        unsigned char *ring = smem_raw + k * FW_BUF + rs * FW_ROW;
+        *reinterpret_cast<uint2 *>(ring + o_w[0]) = h0;
+        *reinterpret_cast<uint2 *>(ring + o_w[1]) = h1;
+        if (P.act[k] && r >= 4 && r < rows + 4 && col_out) {
+            *reinterpret_cast<uint2 *>(dst) = h0;
+            *reinterpret_cast<uint2 *>(dst + 16) = h1;
+        }
+    };
+    // the lane's place in row r of a kept activation
+    auto place = [&](int k, int r) {
+        return P.act[k] ? P.act[k] + (ibase + (long)(top + r) * W + gx) * CH + 4 * g : nullptr;
+    };
+    const uint16_t *wp = P.packed + (long)l * PACK_LAYER;
     bf16x8 A[2][9];
 #pragma unroll
-    for (int nb = 0; nb < 2; nb++)
+    for (int n = 0; n < 2; n++)
 #pragma unroll
         for (int t = 0; t < 9; t++)
-            A[nb][t] = *reinterpret_cast<const bf16x8 *>(wp + ((t * CH + nb * 16 + (lane & 15)) * CH + 8 * (lane >> 4)));
-    float bz[2][4];
-    if (PF) {
-#pragma unroll
-        for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) bz[nb][e] = bias[nb * 16 + 4 * (lane >> 4) + e];
-        if ((int)blockIdx.x < ntiles) {
-            int img, y0, x0;
-            tm.of_rows(blockIdx.x, TR, img, y0, x0);
-            uint4 pv[Stage<TR>::per];
-            prefetch_tile<TR>(x, H, W, img, y0, x0, tid, pv);
-            put_tile<TR>(sx, tid, pv);
-        }
-    }
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    int img, y0, x0;
-    tm.of_rows(tile, TR, img, y0, x0);
-    const long ibase = (long)img * H * W;
-    uint4 pv[Stage<TR>::per];
-    const int next = tile + (int)gridDim.x;
-    if (PF) {
-        __syncthreads();  // this tile's pieces are in sx
-        if (next < ntiles) {
-            int ni, ny, nx;
-            tm.of_rows(next, TR, ni, ny, nx);
-            prefetch_tile<TR>(x, H, W, ni, ny, nx, tid, pv);
-        }
-    } else {
-        __syncthreads();  // the previous tile's reads of sx are done
-        stage_tile<3>(x, sx, ibase, H, W, y0, x0, tid);
-        __syncthreads();
-    }
+            A[n][t] = *reinterpret_cast<const bf16x8 *>(wp + ((t * CH + n * 16 + j) * CH + 8 * g));
+    __syncthreads();
 
-    const int j = lane & 15, g = lane >> 4;
-#pragma unroll 1
-    for (int q = 0; q < TR / 2; q++) {
-        const int r = wave * (TR / 4) + (q >> 1), cb = (q & 1) * 16;
-        floatx4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = {0.0f, 0.0f, 0.0f, 0.0f};
+    // Layer l + 2's step: rows 2s - 3 (l + 1) and the next.  Ring k's row r sits
+    // in slot (r + 3 (k + 1)) mod 6, so with 2s mod 6 = M2 every layer reads
+    // slots M2 - 1 .. M2 + 2 and writes M2 + 3, M2 + 4: constants, the steps
+    // going by threes.  The upper two input rows are the lower two of the step
+    // before, kept in registers (Bk): their MFMAs start at once while the others
+    // arrive.
+    const int lag = 3 * (l + 1);
+    const float *bias = sb + (l + 1) * CH + 4 * g;
+    const bool act_kept = P.act[l + 1] != nullptr;
+    uint16_t *act = place(l + 1, -lag);
+    bf16x8 Bk[2][3];
 #pragma unroll
-        for (int t = 0; t < 9; t++) {
-            const int ky = t / 3, kx = t - ky * 3;
-            const bf16x8 B = *reinterpret_cast<const bf16x8 *>(sx + ((r + ky) * WS + cb + j + kx) * PSTR + 8 * g);
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[0][t], B, acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[1][t], B, acc1, 0, 0, 0);
-        }
-        // lane holds D[co = nb*16 + 4g + e][pixel j]
-        const int gy = y0 + r, gx = x0 + cb + j;
-        if (gy < H && gx < W) {
-            const long p = ibase + (long)gy * W + gx;
+    for (int hr = 0; hr < 2; hr++)
 #pragma unroll
-            for (int nb = 0; nb < 2; nb++) {
-                const floatx4 a = nb ? acc1 : acc0;
-                const int co0 = nb * 16 + 4 * g;
-                float v[4] = {a[0], a[1], a[2], a[3]};
+        for (int kx = 0; kx < 3; kx++) Bk[hr][kx] = bf16x8{};
+    auto conv = [&](auto m2, int s) {
+        constexpr int M2 = decltype(m2)::value;
+        const int r = 2 * s - lag;
+        bf16x8 Bn[2][3];
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float z = v[e] + (PF ? bz[nb][e] : bias[co0 + e]);
-                    v[e] = z > 0.0f ? z : 0.0f;
+        for (int hr = 0; hr < 2; hr++)
+#pragma unroll
+            for (int kx = 0; kx < 3; kx++)
+                Bn[hr][kx] = *reinterpret_cast<const bf16x8 *>(o_b[kx] + (M2 + 7 + hr) % 6 * FW_ROW);
+        floatx4 acc[2][2] = {{zero, zero}, {zero, zero}};
+#pragma unroll
+        for (int hr = 0; hr < 4; hr++)
+#pragma unroll
+            for (int kx = 0; kx < 3; kx++) {
+                const bf16x8 B = hr < 2 ? Bk[hr][kx] : Bn[hr - 2][kx];
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const int ky = hr - i;
+                    if (ky < 0 || ky > 2) continue;
+                    acc[i][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[0][ky * 3 + kx], B, acc[i][0], 0, 0, 0);
+                    acc[i][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[1][ky * 3 + kx], B, acc[i][1], 0, 0, 0);
                 }
-                uint2 o;
-                o.x = (uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16);
-                o.y = (uint32_t)to_bf16(v[2]) | ((uint32_t)to_bf16(v[3]) << 16);
-                *reinterpret_cast<uint2 *>(y + p * CH + co0) = o;
             }
-        }
-    }
-    if (PF && next < ntiles) {
-        __syncthreads();  // this tile's reads of sx are done
-        put_tile<TR>(sx, tid, pv);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Inference with the first layer fused into the second (a1 never reaches
-// HBM), on 16 x 32 output tiles: the 1 -> 32 layer runs on the tile grown
-// by one pixel -- R12 x RC = 18 x 34 pixels in 39 groups of 16 (1.2x the
-// output pixels; 8 x 32 tiles grew 1.33x and had twice the barriers per
-// pixel) -- into LDS, zeros outside the image (the padding the second
-// layer's staging gives), then the second layer on the 16 x 32 tile from
-// there.
-// Every value is computed by the same MFMA sequence and rounding as in the
-// layer-by-layer kernels: bitwise.  (The last layer fused into the fourth the
-// same way was slower: recomputing the 32 -> 32 layer on the grown tile costs
-// 1.9x its MFMA work and the 62 KB workgroup halved the occupancy.)
-constexpr int TH12 = 16;                     // output tile rows of the fused layers 1 + 2
-constexpr int R12 = TH12 + 2, RC = TW + 2;   // the grown tile
-constexpr int XR12 = TH12 + 4, XC2 = TW + 4; // its input (x) region, two-pixel halo
-
-// Store lane's four channels co0..co0+3 of grown-tile pixel (r, c) as bf16 of
-// relu(acc + bias) -- or zeros for a pixel outside the image.
-__device__ __forceinline__ void put_grown(uint16_t *dst, int r, int c, int co0, floatx4 a, const float *bias,
-                                          bool inside) {
-    float v[4];
+        const float4 b0 = *reinterpret_cast<const float4 *>(bias), b1 = *reinterpret_cast<const float4 *>(bias + 16);
+        put(l + 1, r, (M2 + 3) % 6, act, acc[0][0], acc[0][1], b0, b1);
+        put(l + 1, r + 1, (M2 + 4) % 6, act + (long)W * CH, acc[1][0], acc[1][1], b0, b1);
+        if (act_kept) act += 2L * W * CH;
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const float z = a[e] + bias[co0 + e];
-        v[e] = inside && z > 0.0f ? z : 0.0f;
-    }
-    uint2 o;
-    o.x = (uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16);
-    o.y = (uint32_t)to_bf16(v[2]) | ((uint32_t)to_bf16(v[3]) << 16);
-    *reinterpret_cast<uint2 *>(dst + (r * RC + c) * PSTR + co0) = o;
-}
-
-// Layers 1 and 2: a2 = layer2(layer1(x)) on 8 x 32 tiles, persistent as
-// k_conv32: bf16(x/scale) with a two-pixel halo in LDS, a1 on the grown tile
-// in LDS (k_conv_in's arithmetic), then k_conv32<0>'s.
-__global__ void __launch_bounds__(256) k_conv12(const float *__restrict__ x, float scale,
-                                                const float *__restrict__ prm, const uint16_t *__restrict__ wp,
-                                                uint16_t *__restrict__ y, int H, int W, int ntiles, TileMap tm) {
-    __shared__ float sxs[XR12 * XC2];
-    __shared__ __align__(16) uint16_t sx[R12 * RC * PSTR];
-    __shared__ float sw[9 * CH + 2 * CH];  // W1 (bf16 values), b1, b2
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int i = tid; i < 9 * CH; i += 256) sw[i] = round_bf16(prm[OFF_W1 + i]);
-    if (tid < CH) {
-        sw[9 * CH + tid] = prm[OFF_B1 + tid];
-        sw[10 * CH + tid] = prm[OFF_B2 + tid];
+        for (int hr = 0; hr < 2; hr++)
+#pragma unroll
+            for (int kx = 0; kx < 3; kx++) Bk[hr][kx] = Bn[hr][kx];
+    };
+    auto run = [&](auto &&step) {
+        for (int s = 0; s <= last; s += 3) {
+            step(std::integral_constant<int, 0>{}, s);
+            __syncthreads();
+            if (s + 1 > last) break;
+            step(std::integral_constant<int, 2>{}, s + 1);
+            __syncthreads();
+            if (s + 2 > last) break;
+            step(std::integral_constant<int, 4>{}, s + 2);
+            __syncthreads();
+        }
+    };
+    // the longest chain of a step first: layer 3's wave of each SIMD has half as
+    // many MFMAs again (1105 -> 1050 us at 4 x 2048^2)
+    if (l == 1) __builtin_amdgcn_s_setprio(2);
+    else if (l == 0) __builtin_amdgcn_s_setprio(1);
+    if (l == 0) {  // and layer 1
+        bf16x8 A1[2];
+        conv_in_frag(P.prm + OFF_W1, lane, A1);
+        // its taps 0 .. 7 in lanes 0 .. 15, tap 8 in lanes 16 .. 31
+        const unsigned use0 = g < 2 ? ~0u : 0u, use = g == 0 ? ~0u : 0u;
+        const float *xl = xr + c, *xl0 = xl + (g > 0 ? 2 : 0);  // element 0: tap 0, or tap 8
+        uint16_t *act1 = place(0, 0);
+        run([&](auto m2, int s) {
+            constexpr int M2 = decltype(m2)::value;
+            const float4 b0 = *reinterpret_cast<const float4 *>(sb + 4 * g), b1 = *reinterpret_cast<const float4 *>(sb + 16 + 4 * g);
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                // row 2s + i - 1 + ky of x in slot (M2 + i + 5 + ky) mod 6
+                const int rx[3] = {(M2 + i + 5) % 6 * FW_XP, (M2 + i) % 6 * FW_XP, (M2 + i + 1) % 6 * FW_XP};
+                float v[8];
+                v[0] = xl0[g > 0 ? rx[2] : rx[0]];
+#pragma unroll
+                for (int e = 1; e < 8; e++) v[e] = xl[rx[e / 3] + e % 3];
+                bf16x8 B;
+#pragma unroll
+                for (int e = 0; e < 8; e++) B[e] = bf16_of(__uint_as_float(__float_as_uint(v[e]) & (e ? use : use0)));
+                const floatx4 v0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A1[0], B, zero, 0, 0, 0);
+                const floatx4 v1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A1[1], B, zero, 0, 0, 0);
+                put(0, 2 * s + i, (M2 + 3 + i) % 6, act1 + (long)i * W * CH, v0, v1, b0, b1);
+            }
+            if (P.act[0]) act1 += 2L * W * CH;
+            conv(m2, s);
+        });
+    } else if (l == 2) {  // and x, a step ahead: rows 2s + 3, 2s + 4 into LDS and 2s + 5, 2s + 6 on
+                          // their way into the same register (two would meet in a copy that waits)
+        run([&](auto m2, int s) {
+            constexpr int M2 = decltype(m2)::value;
+            put_x(2 * s + 3, xi ? (M2 + 4) % 6 : (M2 + 3) % 6, x_next);
+            x_next = load_x(2 * s + 5);
+            conv(m2, s);
+        });
+    } else {  // and layer 5
+        const float b5 = P.prm[OFF_B5];
+        const bf16x8 *A5 = w5 + lane;
+        const unsigned char *in5[3] = {smem_raw + 3 * FW_BUF + slot(c, g), smem_raw + 3 * FW_BUF + slot(c + 1, g),
+                                       smem_raw + 3 * FW_BUF + slot(c + 2, g)};
+        const int gxc = min(max(gx, 0), W - 1);
+        float xv[2] = {0.0f, 0.0f};  // x of rows r, r + 1 (rows -12, -11 are outside), loaded a step ahead
+        double r2 = 0.0, x2 = 0.0;   // the lane's sums of residual^2 and (x / scale)^2
+        run([&](auto m2, int s) {
+            constexpr int M2 = decltype(m2)::value;
+            const int r = 2 * s - 12;  // output rows r, r + 1
+            floatx4 acc[2] = {zero, zero};
+#pragma unroll
+            for (int hr = 0; hr < 4; hr++)
+#pragma unroll
+                for (int kx = 0; kx < 3; kx++) {
+                    const bf16x8 B = *reinterpret_cast<const bf16x8 *>(in5[kx] + (M2 + 5 + hr) % 6 * FW_ROW);
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        const int ky = hr - i;
+                        if (ky < 0 || ky > 2) continue;
+                        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A5[(ky * 3 + kx) * 64], B, acc[i], 0, 0, 0);
+                    }
+                }
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                if (lane < 16 && col_out && r + i >= 4 && r + i < rows + 4) {
+                    const float res = acc[i][0] + b5;
+                    const long p = ibase + (long)(top + r + i) * W + gx;
+                    const float xn = xv[i] / P.scale;
+                    const float v = xn + res;
+                    if (P.yn) P.yn[p] = v;
+                    if (P.y) P.y[p] = v * P.scale;
+                    r2 += (double)(res * res);
+                    x2 += (double)(xn * xn);
+                }
+#pragma unroll
+            for (int i = 0; i < 2; i++) xv[i] = (xim + row_of(r + 2 + i))[gxc];
+            conv(m2, s);
+        });
+#pragma unroll
+        for (int h = 8; h > 0; h >>= 1) {
+            r2 += __shfl_down(r2, h, 64);
+            x2 += __shfl_down(x2, h, 64);
+        }
+        if (lane == 0) {  // the rings are free after the last step
+            double *red = reinterpret_cast<double *>(smem_raw);
+            red[2 * q] = r2;
+            red[2 * q + 1] = x2;
+        }
     }
     __syncthreads();
-    bf16x8 A1[2];
-    conv_in_frag(sw, lane, A1);
-    bf16x8 A[2][9];
-#pragma unroll
-    for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-        for (int t = 0; t < 9; t++)
-            A[nb][t] = *reinterpret_cast<const bf16x8 *>(wp + ((t * CH + nb * 16 + (lane & 15)) * CH + 8 * (lane >> 4)));
-    const int j = lane & 15, g = lane >> 4;
-    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        int img, y0, x0;
-        tm.of_rows(tile, TH12, img, y0, x0);
-        const long ibase = (long)img * H * W;
-        __syncthreads();  // the previous tile's reads of sxs and sx are done
-        {
-            constexpr int PER = (XR12 * XC2 + 255) / 256;
-            float v[PER];
-#pragma unroll
-            for (int k = 0; k < PER; k++) {
-                const int i = tid + k * 256;
-                const int r = i / XC2, c = i - r * XC2, gy = y0 + r - 2, gx = x0 + c - 2;
-                v[k] = i < XR12 * XC2 && gy >= 0 && gy < H && gx >= 0 && gx < W ? x[ibase + (long)gy * W + gx] : 0.0f;
-            }
-#pragma unroll
-            for (int k = 0; k < PER; k++) {
-                const int i = tid + k * 256;
-                const int r = i / XC2, c = i - r * XC2, gy = y0 + r - 2, gx = x0 + c - 2;
-                if (i < XR12 * XC2) sxs[i] = (gy >= 0 && gy < H && gx >= 0 && gx < W) ? round_bf16(v[k] / scale) : 0.0f;
-            }
-        }
-        __syncthreads();
-        // a1 on the grown tile: its 612 pixels packed row after row into 39
-        // groups of 16 over the 4 waves (a pixel's MFMA column depends on its
-        // own inputs only, so the packing changes no value)
-        constexpr int NG1 = (R12 * RC + 15) / 16;
-#pragma unroll 1
-        for (int q = wave; q < NG1; q += 4) {
-            const int pix = q * 16 + j, pp = pix < R12 * RC ? pix : R12 * RC - 1;
-            const int r = pp / RC, c = pp - r * RC;
-            const bf16x8 B = conv_in_b(sxs, XC2, r, c, lane);
-            const floatx4 z = {0.0f, 0.0f, 0.0f, 0.0f};
-            const floatx4 acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A1[0], B, z, 0, 0, 0);
-            const floatx4 acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A1[1], B, z, 0, 0, 0);
-            if (pix < R12 * RC) {
-                const int gy = y0 + r - 1, gx = x0 + c - 1;
-                const bool inside = gy >= 0 && gy < H && gx >= 0 && gx < W;
-                put_grown(sx, r, c, 4 * g, acc0, sw + 9 * CH, inside);
-                put_grown(sx, r, c, 16 + 4 * g, acc1, sw + 9 * CH, inside);
-            }
-        }
-        __syncthreads();
-#pragma unroll 1
-        for (int q = 0; q < TH12 / 2; q++) {
-            const int r = wave * (TH12 / 4) + (q >> 1), cb = (q & 1) * 16;
-            floatx4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int t = 0; t < 9; t++) {
-                const int ky = t / 3, kx = t - ky * 3;
-                const bf16x8 B = *reinterpret_cast<const bf16x8 *>(sx + ((r + ky) * WS + cb + j + kx) * PSTR + 8 * g);
-                acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[0][t], B, acc0, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[1][t], B, acc1, 0, 0, 0);
-            }
-            const int gy = y0 + r, gx = x0 + cb + j;
-            if (gy < H && gx < W) {
-                const long p = ibase + (long)gy * W + gx;
-#pragma unroll
-                for (int nb = 0; nb < 2; nb++) {
-                    const floatx4 a = nb ? acc1 : acc0;
-                    const int co0 = nb * 16 + 4 * g;
-                    float v[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const float zz = a[e] + sw[10 * CH + co0 + e];
-                        v[e] = zz > 0.0f ? zz : 0.0f;
-                    }
-                    uint2 o;
-                    o.x = (uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16);
-                    o.y = (uint32_t)to_bf16(v[2]) | ((uint32_t)to_bf16(v[3]) << 16);
-                    *reinterpret_cast<uint2 *>(y + p * CH + co0) = o;
-                }
-            }
-        }
+    if (tid < 2 && P.stats) {
+        const double *red = reinterpret_cast<const double *>(smem_raw);
+        P.stats[2L * blockIdx.x + tid] = (float)(((red[tid] + red[2 + tid]) + red[4 + tid]) + red[6 + tid]);
     }
 }
 
@@ -637,74 +610,6 @@ __global__ void __launch_bounds__(BK_THREADS, 2) k_conv32_back(const uint16_t *_
     }
 }
 
-// ---------------------------------------------------------------------------
-// 1 -> 32 layer: a1 = bf16(relu(W1 * bf16(x/scale) + b1)) on MFMA: a block
-// owns an 8 x 32 pixel tile (persistent over tiles), stages bf16(x/scale)
-// with a one-pixel halo in LDS, and each wave computes 4 groups of 16 pixels.
-__global__ void __launch_bounds__(256) k_conv_in(const float *__restrict__ x, float scale,
-                                                 const float *__restrict__ prm, uint16_t *__restrict__ a1, int H,
-                                                 int W, int ntiles, TileMap tm) {
-    __shared__ float sxs[HS * WS];
-    __shared__ float sw[9 * CH + CH];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int i = tid; i < 9 * CH; i += 256) sw[i] = round_bf16(prm[OFF_W1 + i]);
-    if (tid < CH) sw[9 * CH + tid] = prm[OFF_B1 + tid];
-    __syncthreads();
-    bf16x8 A[2];
-    conv_in_frag(sw, lane, A);
-    const int j = lane & 15, g = lane >> 4;
-    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        int img, y0, x0;
-        tm.of(tile, img, y0, x0);
-        const long ibase = (long)img * H * W;
-        __syncthreads();  // the previous tile's reads of sxs are done
-        {  // both loads of a thread in flight before the stores
-            constexpr int PER = (HS * WS + 255) / 256;
-            float v[PER];
-#pragma unroll
-            for (int k = 0; k < PER; k++) {
-                const int i = tid + k * 256;
-                const int r = i / WS, c = i - r * WS, gy = y0 + r - 1, gx = x0 + c - 1;
-                v[k] = i < HS * WS && gy >= 0 && gy < H && gx >= 0 && gx < W ? x[ibase + (long)gy * W + gx] : 0.0f;
-            }
-#pragma unroll
-            for (int k = 0; k < PER; k++) {
-                const int i = tid + k * 256;
-                const int r = i / WS, c = i - r * WS, gy = y0 + r - 1, gx = x0 + c - 1;
-                if (i < HS * WS) sxs[i] = (gy >= 0 && gy < H && gx >= 0 && gx < W) ? round_bf16(v[k] / scale) : 0.0f;
-            }
-        }
-        __syncthreads();
-#pragma unroll 1
-        for (int q = 0; q < 4; q++) {
-            const int r = wave * 2 + (q >> 1), cb = (q & 1) * 16;
-            const bf16x8 B = conv_in_b(sxs, WS, r, cb + j, lane);
-            const floatx4 z = {0.0f, 0.0f, 0.0f, 0.0f};
-            const floatx4 acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[0], B, z, 0, 0, 0);
-            const floatx4 acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[1], B, z, 0, 0, 0);
-            const int gy = y0 + r, gx = x0 + cb + j;
-            if (gy < H && gx < W) {
-                const long p = ibase + (long)gy * W + gx;
-#pragma unroll
-                for (int nb = 0; nb < 2; nb++) {
-                    const floatx4 a = nb ? acc1 : acc0;
-                    const int co0 = nb * 16 + 4 * g;
-                    float v[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const float zz = a[e] + sw[9 * CH + co0 + e];
-                        v[e] = zz > 0.0f ? zz : 0.0f;
-                    }
-                    uint2 o;
-                    o.x = (uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16);
-                    o.y = (uint32_t)to_bf16(v[2]) | ((uint32_t)to_bf16(v[3]) << 16);
-                    *reinterpret_cast<uint2 *>(a1 + p * CH + co0) = o;
-                }
-            }
-        }
-    }
-}
-
 // Sum acc[9][8] (tap, channel of the thread's group of 8) and extra[8] over
 // the threads of the block that share a channel group (tid mod 4), in a fixed
 // order: lanes of a wave by a butterfly over lane bits 2..5, then the four
@@ -802,303 +707,6 @@ __global__ void __launch_bounds__(256) k_conv_in_wgrad(const float *__restrict__
         }
     }
     block_sum_groups(acc, db, red, part + (long)blockIdx.x * IN_REC, true);
-}
-
-// ---------------------------------------------------------------------------
-// 32 -> 1 layer with the residual: r = W5 * a4 + b5, yn = x/scale + r,
-// y = yn * scale; per-tile sums of r^2 and (x/scale)^2 for the fallback test.
-// An 8 x 32 tile at a time: a4 with a one-pixel halo staged in LDS, each wave
-// 4 groups of 16 pixels on MFMA (conv_out_mfma), lanes 0..15 finishing them;
-// the tile's sums by a pairwise tree (sred[i] += sred[i + h], h = 128 .. 1:
-// the two steps across waves through LDS, the rest inside wave 0 by lane
-// shuffles, the same additions in the same order).  PF (an image under 2^31
-// bytes of activations): persistent workgroups, the next tile's a4 pieces and
-// x values loaded into registers while this tile is computed; otherwise one
-// tile per workgroup.  The same values either way.
-template <bool PF>
-__global__ void __launch_bounds__(256) k_conv_out(const uint16_t *__restrict__ a4, const float *__restrict__ x,
-                                                  float scale, const float *__restrict__ prm, float *__restrict__ y,
-                                                  float *__restrict__ yn, float *__restrict__ stats, int H, int W,
-                                                  int ntiles, TileMap tm) {
-    __shared__ __align__(16) uint16_t sx[HS * WS * PSTR];
-    __shared__ float sw[9 * CH + 1];
-    __shared__ float sred[2][TH * TW];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int j = lane & 15;
-    for (int i = tid; i < 9 * CH; i += 256) sw[i] = round_bf16(prm[OFF_W5 + i]);
-    if (tid == 0) sw[9 * CH] = prm[OFF_B5];
-    // x of the lane's four pixels (lanes 0..15; zero outside the image)
-    auto load_x = [&](int img, int y0, int x0, float (&xv)[4]) {
-        const GrBuf b = gr_buf(x + (long)img * H * W, (unsigned)((long)H * W * sizeof(float)));
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int gy = y0 + wave * 2 + (q >> 1), gx = x0 + (q & 1) * 16 + j;
-            const bool in = lane < 16 && gy < H && gx < W;
-            xv[q] = gr_buf_ldf(b, in ? (unsigned)((gy * W + gx) * sizeof(float)) : kGrBufNone);
-        }
-    };
-    float xv[4];
-    int tile = PF ? (int)blockIdx.x : 0;
-    if (PF) {
-        if (tile < ntiles) {
-            int img, y0, x0;
-            tm.of(tile, img, y0, x0);
-            uint4 pv[STAGE_PER];
-            prefetch_tile<TH>(a4, H, W, img, y0, x0, tid, pv);
-            load_x(img, y0, x0, xv);
-            put_tile<TH>(sx, tid, pv);
-        }
-    } else {
-        tile = (int)blockIdx.x;
-        int img, y0, x0;
-        tm.of(tile, img, y0, x0);
-        stage_tile<6>(a4, sx, (long)img * H * W, H, W, y0, x0, tid);
-    }
-    __syncthreads();
-    bf16x8 A[9];
-    conv_out_frag(sw, lane, A);
-    const float b5 = sw[9 * CH];
-    for (; tile < ntiles; tile += PF ? (int)gridDim.x : ntiles) {
-        int img, y0, x0;
-        tm.of(tile, img, y0, x0);
-        const long ibase = (long)img * H * W;
-        __syncthreads();  // this tile's pieces in sx; the previous tile's sums read
-        const int next = tile + (int)gridDim.x;
-        uint4 pv[STAGE_PER];
-        float xn_next[4];
-        if (PF && next < ntiles) {
-            int ni, ny, nx;
-            tm.of(next, ni, ny, nx);
-            prefetch_tile<TH>(a4, H, W, ni, ny, nx, tid, pv);
-            load_x(ni, ny, nx, xn_next);
-        }
-#pragma unroll 1
-        for (int q = 0; q < 4; q++) {
-            const int r = wave * 2 + (q >> 1), c = (q & 1) * 16 + j;
-            const floatx4 acc = conv_out_mfma(sx, WS, r, c, lane, A);
-            const int gy = y0 + r, gx = x0 + c;
-            if (lane < 16) {  // every pixel of the tile writes its sums: zeros outside the image
-                float s2 = 0.0f, x2 = 0.0f;
-                if (gy < H && gx < W) {
-                    const float s = acc[0] + b5;
-                    const long p = ibase + (long)gy * W + gx;
-                    const float xn = (PF ? xv[q] : x[p]) / scale;
-                    const float v = xn + s;
-                    if (yn) yn[p] = v;
-                    if (y) y[p] = v * scale;
-                    s2 = s * s;
-                    x2 = xn * xn;
-                }
-                sred[0][r * TW + c] = s2;
-                sred[1][r * TW + c] = x2;
-            }
-        }
-        __syncthreads();  // sx reads and sred writes done
-        if (PF && next < ntiles) put_tile<TH>(sx, tid, pv);
-        if (tid < 128) {
-            sred[0][tid] += sred[0][tid + 128];
-            sred[1][tid] += sred[1][tid + 128];
-        }
-        __syncthreads();
-        if (tid < 64) {
-            float r0 = sred[0][tid] + sred[0][tid + 64], r1 = sred[1][tid] + sred[1][tid + 64];
-#pragma unroll
-            for (int h = 32; h > 0; h >>= 1) {
-                r0 += __shfl_down(r0, h, 64);
-                r1 += __shfl_down(r1, h, 64);
-            }
-            if (tid == 0 && stats) {
-                stats[2L * tile] = r0;
-                stats[2L * tile + 1] = r1;
-            }
-        }
-        if (PF) {
-#pragma unroll
-            for (int q = 0; q < 4; q++) xv[q] = xn_next[q];
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Inference, all five layers fused: a block owns an FH x FW output tile and
-// computes each layer on the tile grown by the halo the later layers need
-// (x: 5 pixels, a1: 4, a2: 3, a3: 2, a4: 1), keeping every activation in LDS
-// (a1/a3 and a2/a4 share two buffers), so HBM sees x once and y once instead
-// of four 64-byte activation records per pixel each way.  Per pixel the
-// arithmetic and its order are those of k_conv_in, k_conv32<0> and
-// k_conv_out, so y is bitwise the unfused forward's; activations of pixels
-// outside the image are zero, the unfused path's zero padding.
-constexpr int FH = 16, FW = 32;
-constexpr int XR = FH + 10, XC = FW + 10;
-constexpr int R1 = FH + 8, C1 = FW + 8;
-constexpr int R2 = FH + 6, C2 = FW + 6;
-constexpr size_t FUSED_LDS = sizeof(float) * XR * XC + sizeof(uint16_t) * (size_t)(R1 * C1 + R2 * C2) * PSTR +
-                             sizeof(float) * (IN_REC + OUT_REC) + sizeof(float) * 2 * FH * FW;
-
-// One 32 -> 32 layer from an (Ri x Ci) input region to the (Ri-2 x Ci-2)
-// output region, LDS to LDS; (oy, ox) is the image position of output (0, 0).
-__device__ __forceinline__ void fused_conv32(const uint16_t *in, int Ci, uint16_t *out, int Ro, int Co,
-                                             const uint16_t *__restrict__ wp, const float *__restrict__ bias,
-                                             int oy, int ox, int H, int W, int lane, int wave, int nwaves) {
-    bf16x8 A[2][9];
-#pragma unroll
-    for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-        for (int t = 0; t < 9; t++)
-            A[nb][t] = *reinterpret_cast<const bf16x8 *>(wp + ((t * CH + nb * 16 + (lane & 15)) * CH + 8 * (lane >> 4)));
-    const int j = lane & 15, g = lane >> 4;
-    const int npix = Ro * Co, ngroups = (npix + 15) / 16;
-    // two 16-pixel groups per trip: four independent accumulation chains
-    for (int grp0 = 2 * wave; grp0 < ngroups; grp0 += 2 * nwaves) {
-        int pp[2], rr[2], cc[2];
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            pp[h] = (grp0 + h) * 16 + j;
-            const int pc = pp[h] < npix ? pp[h] : npix - 1;
-            rr[h] = pc / Co;
-            cc[h] = pc - rr[h] * Co;
-        }
-        floatx4 acc[2][2];
-#pragma unroll
-        for (int h = 0; h < 2; h++) acc[h][0] = acc[h][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int t = 0; t < 9; t++) {
-            const int ky = t / 3, kx = t - ky * 3;
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const bf16x8 B =
-                    *reinterpret_cast<const bf16x8 *>(in + ((rr[h] + ky) * Ci + cc[h] + kx) * PSTR + 8 * g);
-                acc[h][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[0][t], B, acc[h][0], 0, 0, 0);
-                acc[h][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[1][t], B, acc[h][1], 0, 0, 0);
-            }
-        }
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-        const int p = pp[h], r = rr[h], c = cc[h];
-        if (p < npix) {
-            const int gy = oy + r, gx = ox + c;
-            const bool inside = gy >= 0 && gy < H && gx >= 0 && gx < W;
-#pragma unroll
-            for (int nb = 0; nb < 2; nb++) {
-                const floatx4 a = acc[h][nb];
-                const int co0 = nb * 16 + 4 * g;
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float z = a[e] + bias[co0 + e];
-                    v[e] = inside && z > 0.0f ? z : 0.0f;
-                }
-                uint2 o;
-                o.x = (uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16);
-                o.y = (uint32_t)to_bf16(v[2]) | ((uint32_t)to_bf16(v[3]) << 16);
-                *reinterpret_cast<uint2 *>(out + p * PSTR + co0) = o;
-            }
-        }
-      }
-    }
-}
-
-__global__ void __launch_bounds__(512) k_cnn_fused(const float *__restrict__ x, float scale,
-                                                   const float *__restrict__ prm, const uint16_t *__restrict__ packed,
-                                                   float *__restrict__ y, float *__restrict__ stats, int H, int W,
-                                                   int tiles_x, int tiles_y) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    float *sx = reinterpret_cast<float *>(smem_raw);                 // [XR][XC] bf16(x/scale) as float
-    uint16_t *bufA = reinterpret_cast<uint16_t *>(sx + XR * XC);     // a1 [R1][C1], then a3
-    uint16_t *bufB = bufA + R1 * C1 * PSTR;                          // a2 [R2][C2], then a4
-    float *sw1 = reinterpret_cast<float *>(bufB + R2 * C2 * PSTR);   // W1 (bf16 values), b1
-    float *sw5 = sw1 + IN_REC;                                       // W5 (bf16 values), b5
-    float *sred = sw5 + OUT_REC;                                     // [2][FH*FW]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
-    const int per = tiles_x * tiles_y;
-    const int img = blockIdx.x / per, rt = blockIdx.x - img * per;
-    const int y0 = (rt / tiles_x) * FH, x0 = (rt % tiles_x) * FW;
-    const long ibase = (long)img * H * W;
-
-    for (int i = tid; i < 9 * CH; i += blockDim.x) sw1[i] = round_bf16(prm[OFF_W1 + i]);
-    for (int i = tid; i < CH; i += blockDim.x) sw1[9 * CH + i] = prm[OFF_B1 + i];
-    for (int i = tid; i < 9 * CH; i += blockDim.x) sw5[i] = round_bf16(prm[OFF_W5 + i]);
-    if (tid == 0) sw5[9 * CH] = prm[OFF_B5];
-    for (int i = tid; i < XR * XC; i += blockDim.x) {
-        const int r = i / XC, c = i - r * XC, gy = y0 - 5 + r, gx = x0 - 5 + c;
-        sx[i] = (gy >= 0 && gy < H && gx >= 0 && gx < W) ? round_bf16(x[ibase + (long)gy * W + gx] / scale) : 0.0f;
-    }
-    __syncthreads();
-    // layer 1 on the a1 region, 16 pixels per MFMA group (as k_conv_in)
-    {
-        bf16x8 A1[2];
-        conv_in_frag(sw1, lane, A1);
-        const int j = lane & 15, g = lane >> 4, npix = R1 * C1;
-        for (int grp = wave; grp * 16 < npix; grp += nwaves) {
-            const int p = grp * 16 + j, pc = p < npix ? p : npix - 1;
-            const int r = pc / C1, c = pc - r * C1;
-            const bf16x8 B = conv_in_b(sx, XC, r, c, lane);
-            const floatx4 z = {0.0f, 0.0f, 0.0f, 0.0f};
-            const floatx4 acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A1[0], B, z, 0, 0, 0);
-            const floatx4 acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A1[1], B, z, 0, 0, 0);
-            if (p < npix) {
-                const int gy = y0 - 4 + r, gx = x0 - 4 + c;
-                const bool inside = gy >= 0 && gy < H && gx >= 0 && gx < W;
-#pragma unroll
-                for (int nb = 0; nb < 2; nb++) {
-                    const floatx4 a = nb ? acc1 : acc0;
-                    const int co0 = nb * 16 + 4 * g;
-                    float v[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const float zz = a[e] + sw1[9 * CH + co0 + e];
-                        v[e] = inside && zz > 0.0f ? zz : 0.0f;
-                    }
-                    uint2 o;
-                    o.x = (uint32_t)to_bf16(v[0]) | ((uint32_t)to_bf16(v[1]) << 16);
-                    o.y = (uint32_t)to_bf16(v[2]) | ((uint32_t)to_bf16(v[3]) << 16);
-                    *reinterpret_cast<uint2 *>(bufA + p * PSTR + co0) = o;
-                }
-            }
-        }
-    }
-    __syncthreads();
-    fused_conv32(bufA, C1, bufB, R2, C2, packed, prm + OFF_B2, y0 - 3, x0 - 3, H, W, lane, wave, nwaves);
-    __syncthreads();
-    fused_conv32(bufB, C2, bufA, R2 - 2, C2 - 2, packed + PACK_LAYER, prm + OFF_B3, y0 - 2, x0 - 2, H, W, lane, wave,
-                 nwaves);
-    __syncthreads();
-    fused_conv32(bufA, C2 - 2, bufB, R2 - 4, C2 - 4, packed + 2 * PACK_LAYER, prm + OFF_B4, y0 - 1, x0 - 1, H, W,
-                 lane, wave, nwaves);
-    __syncthreads();
-    // layer 5 + residual, 16 pixels per MFMA group (as k_conv_out)
-    const int C4 = C2 - 4;
-    for (int i = tid; i < 2 * FH * FW; i += blockDim.x) sred[i] = 0.0f;
-    __syncthreads();
-    {
-        bf16x8 A5[9];
-        conv_out_frag(sw5, lane, A5);
-        const int j = lane & 15;
-        for (int grp = wave; grp * 16 < FH * FW; grp += nwaves) {
-            const int q = grp * 16 + j, r = q / FW, c = q - r * FW, gy = y0 + r, gx = x0 + c;
-            const floatx4 acc = conv_out_mfma(bufB, C4, r, c, lane, A5);
-            if (lane < 16 && gy < H && gx < W) {
-                const float s = acc[0] + sw5[9 * CH];
-                const long p = ibase + (long)gy * W + gx;
-                const float xn = x[p] / scale;
-                y[p] = (xn + s) * scale;
-                sred[q] = s * s;
-                sred[FH * FW + q] = xn * xn;
-            }
-        }
-    }
-    __syncthreads();
-    for (int h = FH * FW / 2; h > 0; h >>= 1) {
-        for (int i = tid; i < h; i += blockDim.x) {
-            sred[i] += sred[i + h];
-            sred[FH * FW + i] += sred[FH * FW + i + h];
-        }
-        __syncthreads();
-    }
-    if (tid == 0 && stats) {
-        stats[2 * blockIdx.x] = sred[0];
-        stats[2 * blockIdx.x + 1] = sred[FH * FW];
-    }
 }
 
 // Loss: dy = 2 (yn - t/scale) / N; per-block partial sums of (yn - t/scale)^2.
@@ -1351,6 +959,40 @@ int check_dims(int n, int H, int W) {
     return GR_OK;
 }
 
+// Segments of rows a strip is cut into: the fewest steps of the busiest CU
+// (one workgroup each at a time); a segment of k rows takes k / 2 + 8 steps,
+// the pipeline's fill and the four halo rows on either side among them.  At
+// least 16 rows each (what gr_cnn_infer_work_bytes counts on).
+int forward_segments(int n, int H, int strips) {
+    const long cus = gr_cu_count() > 0 ? gr_cu_count() : 256;
+    int best = 1;
+    long best_cost = 0;
+    for (int v = 1; v <= std::min(64, (H + 15) / 16); v++) {
+        const long rows = (H + v - 1) / v, groups = (long)n * strips * ((H + rows - 1) / rows);
+        const long cost = (groups + cus - 1) / cus * ((rows + 1) / 2 + 8);
+        if (v == 1 || cost < best_cost) {
+            best = v;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+int run_forward(const float *params, const unsigned short *packed, const float *x, int n, int H, int W, float scale,
+                uint16_t *const (&act)[4], float *y, float *yn, float *slice_stats, float *stats, hipStream_t s) {
+    const int strips = (W + FW_OUT - 1) / FW_OUT, v = forward_segments(n, H, strips);
+    const int rows = (H + v - 1) / v, segs = (H + rows - 1) / rows;
+    if ((long)n * strips * segs > (1L << 31) - 1) return cnn_fail(GR_EINVAL, "too many tiles");
+    FwdArgs A{x, params, reinterpret_cast<const uint16_t *>(packed), {act[0], act[1], act[2], act[3]}, y, yn,
+              slice_stats ? stats : nullptr, scale, H, W, strips, segs, rows};
+    CNN_HIP(gr_allow_lds(k_forward, FW_LDS));
+    hipLaunchKernelGGL(k_forward, dim3((unsigned)(n * strips * segs)), dim3(FW_THREADS), FW_LDS, s, A);
+    if (slice_stats)
+        hipLaunchKernelGGL(k_sum_groups, dim3(2 * n), dim3(256), 0, s, stats, n, strips * segs, 2, 1.0, slice_stats);
+    CNN_HIP(hipGetLastError());
+    return GR_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1388,83 +1030,23 @@ int gr_cnn_forward(const float *params, const unsigned short *packed, const floa
     int rc = check_dims(n, H, W);
     if (rc) return rc;
     if (slice_stats && !work) return cnn_fail(GR_EINVAL, "slice statistics need the work buffer");
-    hipStream_t s = (hipStream_t)stream;
-    const TileMap tm = tiles_of(H, W);
-    const int ntiles = tm.tiles_x * tm.tiles_y * n;
-    const long npx = (long)n * H * W;
-    const uint16_t *pk = reinterpret_cast<const uint16_t *>(packed);
-    const int nconv = ntiles < MAX_CONV_BLOCKS ? ntiles : MAX_CONV_BLOCKS;
-    // a 32 -> 32 forward layer, with the next-tile prefetch when an image's
-    // activations fit a buffer view (< 2^31 bytes)
-    // (its workgroups: exactly those resident at once, each looping over tiles)
-    const bool pf = (long)H * W * CH * (long)sizeof(uint16_t) < (1L << 31);
-    const TileMap tm16{tm.tiles_x, (H + 15) / 16};
-    const int nt16 = tm16.tiles_x * tm16.tiles_y * n;
-    int npf = 0;
-    if (pf) {
-        int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_conv32<true, 16>, 256, 0) !=
-                hipSuccess ||
-            per_cu < 1)
-            per_cu = 1;
-        const long want = (long)per_cu * (gr_cu_count() > 0 ? gr_cu_count() : 256);
-        npf = (int)std::min<long>(nt16, want);
-    }
-    auto conv32 = [&](const uint16_t *in, const uint16_t *wl, const float *b, uint16_t *out) {
-        if (pf)
-            hipLaunchKernelGGL((k_conv32<true, 16>), dim3(npf), dim3(256), 0, s, in, wl, b, out, H, W, nt16,
-                               tm16);
-        else
-            hipLaunchKernelGGL((k_conv32<false>), dim3(nconv), dim3(256), 0, s, in, wl, b, out, H, W, ntiles, tm);
-    };
-    // inference (a3 aliasing a1 and a4 aliasing a2: the caller keeps no
-    // activation): the first layer fused into the second
-    const bool fused = a3 == a1 && a4 == a2;
-    if (fused) {
-        const TileMap tm12{tm.tiles_x, (H + TH12 - 1) / TH12};
-        const int nt12 = tm12.tiles_x * tm12.tiles_y * n;
-        hipLaunchKernelGGL(k_conv12, dim3(nt12 < MAX_CONV_BLOCKS ? nt12 : MAX_CONV_BLOCKS), dim3(256), 0, s, x, scale,
-                           params, pk, a2, H, W, nt12, tm12);
-        conv32(a2, pk + PACK_LAYER, params + OFF_B3, a3);
-        conv32(a3, pk + 2L * PACK_LAYER, params + OFF_B4, a4);
-    } else {
-        hipLaunchKernelGGL(k_conv_in, dim3(nconv), dim3(256), 0, s, x, scale, params, a1, H, W, ntiles, tm);
-        uint16_t *acts[4] = {a1, a2, a3, a4};
-        const int boff[3] = {OFF_B2, OFF_B3, OFF_B4};
-        for (int l = 0; l < 3; l++) conv32(acts[l], pk + (long)l * PACK_LAYER, params + boff[l], acts[l + 1]);
-    }
     float *stats = nullptr;
     if (slice_stats) {
         char *wb = (char *)work;
+        const long npx = (long)n * H * W;
         auto al = [](size_t b) { return (b + 255) / 256 * 256; };
         wb += 2 * al(sizeof(float) * npx) + 2 * al(sizeof(uint16_t) * npx * CH) +
               al(sizeof(float) * (size_t)MAX_WG_BLOCKS * WG_REC);
         stats = (float *)wb;
     }
-    if (pf) {
-        int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_conv_out<true>, 256, 0) !=
-                hipSuccess ||
-            per_cu < 1)
-            per_cu = 1;
-        const int nout = (int)std::min<long>(ntiles, (long)per_cu * (gr_cu_count() > 0 ? gr_cu_count() : 256));
-        hipLaunchKernelGGL(k_conv_out<true>, dim3(nout), dim3(256), 0, s, a4, x, scale, params, y, yn, stats, H, W,
-                           ntiles, tm);
-    } else {
-        hipLaunchKernelGGL(k_conv_out<false>, dim3(ntiles), dim3(256), 0, s, a4, x, scale, params, y, yn, stats, H, W,
-                           ntiles, tm);
-    }
-    if (slice_stats) {
-        const int per = tm.tiles_x * tm.tiles_y;
-        hipLaunchKernelGGL(k_sum_groups, dim3(2 * n), dim3(256), 0, s, stats, n, per, 2, 1.0,
-                           slice_stats);
-    }
-    CNN_HIP(hipGetLastError());
-    return GR_OK;
+    // a buffer named for two layers ends holding the later one
+    uint16_t *act[4] = {a1 == a3 || a1 == a4 ? nullptr : a1, a2 == a4 ? nullptr : a2, a3, a4};
+    return run_forward(params, packed, x, n, H, W, scale, act, y, yn, slice_stats, stats, (hipStream_t)stream);
 }
 
 size_t gr_cnn_infer_work_bytes(int n, int H, int W) {
-    return sizeof(float) * 2 * (size_t)((W + FW - 1) / FW) * ((H + FH - 1) / FH) * (n > 0 ? n : 0);
+    // two floats per workgroup: at most one per 16 rows and 32 columns
+    return sizeof(float) * 2 * (size_t)((W + 31) / 32) * ((H + 15) / 16) * (n > 0 ? n : 0);
 }
 
 int gr_cnn_infer(const float *params, const unsigned short *packed, const float *x, int n, int H, int W, float scale,
@@ -1473,20 +1055,9 @@ int gr_cnn_infer(const float *params, const unsigned short *packed, const float 
     int rc = check_dims(n, H, W);
     if (rc) return rc;
     if (slice_stats && !work) return cnn_fail(GR_EINVAL, "slice statistics need the work buffer");
-    hipStream_t s = (hipStream_t)stream;
-    const int tx = (W + FW - 1) / FW, ty = (H + FH - 1) / FH;
-    const long nblocks = (long)tx * ty * n;
-    const long npx = (long)n * H * W;
-    (void)npx;
-    float *stats = slice_stats ? (float *)work : nullptr;
-    CNN_HIP(gr_allow_lds(k_cnn_fused, FUSED_LDS));
-    hipLaunchKernelGGL(k_cnn_fused, dim3((unsigned)nblocks), dim3(FH * FW), FUSED_LDS, s, x, scale, params,
-                       reinterpret_cast<const uint16_t *>(packed), y, stats, H, W, tx, ty);
-    if (slice_stats)
-        hipLaunchKernelGGL(k_sum_groups, dim3(2 * n), dim3(256), 0, s, stats, n, tx * ty, 2, 1.0,
-                           slice_stats);
-    CNN_HIP(hipGetLastError());
-    return GR_OK;
+    uint16_t *act[4] = {nullptr, nullptr, nullptr, nullptr};
+    return run_forward(params, packed, x, n, H, W, scale, act, y, nullptr, slice_stats, (float *)work,
+                       (hipStream_t)stream);
 }
 
 int gr_cnn_backward(const float *params, const unsigned short *packed, const float *x, const float *target, int n,

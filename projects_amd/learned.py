@@ -82,15 +82,14 @@ class Corrector:
         self.pack()
 
     # -- buffers ----------------------------------------------------------------
-    def _buffers(self, n, H, W, train, acts=True):
-        key = (n, H, W, train, acts)
+    def _buffers(self, n, H, W, train):
+        key = (n, H, W, train)
         if key not in self._bufs:
             torch = self.torch
             for k in [k for k in self._bufs if k[3] == train]:  # keep one shape per mode
                 del self._bufs[k]
-            na = 0 if not acts else (4 if train else 2)
-            acts_l = [torch.empty((n, H, W, CH), dtype=torch.int16, device=self.dev) for _ in range(na)]
-            wb = gr.lib().gr_cnn_work_bytes(n, H, W) if na else gr.lib().gr_cnn_infer_work_bytes(n, H, W)
+            acts_l = [torch.empty((n, H, W, CH), dtype=torch.int16, device=self.dev) for _ in range(4 if train else 0)]
+            wb = gr.lib().gr_cnn_work_bytes(n, H, W) if train else gr.lib().gr_cnn_infer_work_bytes(n, H, W)
             work = torch.empty(wb, dtype=torch.uint8, device=self.dev)
             yn = torch.empty((n, H, W), dtype=torch.float32, device=self.dev) if train else None
             stats = torch.empty((n, 2), dtype=torch.float32, device=self.dev)
@@ -106,27 +105,27 @@ class Corrector:
         """x: cuda float32 [n, H, W] gridrec images.  Returns (y, stats) with
         y = the corrected images and stats [n, 2] = (sum residual^2, sum
         (x/scale)^2) per image."""
+        if not train:
+            return self.infer(x, out, stream)
         torch = self.torch
         assert x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.is_contiguous()
         n, H, W = x.shape
-        acts, work, yn, stats = self._buffers(n, H, W, train)
-        a = acts if train else [acts[0], acts[1], acts[0], acts[1]]
+        acts, work, yn, stats = self._buffers(n, H, W, True)
         if out is None:
             out = torch.empty_like(x)
         rc = gr.lib().gr_cnn_forward(_ptr(self.params), _ptr(self.packed), _ptr(x), n, H, W, self.scale,
-                                     *[_ptr(t) for t in a], _ptr(out), _ptr(yn), _ptr(stats), _ptr(work),
+                                     *[_ptr(t) for t in acts], _ptr(out), _ptr(yn), _ptr(stats), _ptr(work),
                                      C.c_void_p(gr._stream_handle(stream)))
         gr._check(rc, "gr_cnn_forward")
         return out, stats
 
     def infer(self, x, out=None, stream=None):
-        """Inference in one fused kernel, bitwise forward()'s y, with no
-        activation buffers (for memory-tight callers; forward() is faster on
-        MI355X at 2048^2): returns (y, stats)."""
+        """Inference: the training forward's kernel (bitwise its y and stats)
+        writing no activations.  Returns (y, stats)."""
         torch = self.torch
         assert x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.is_contiguous()
         n, H, W = x.shape
-        _, work, _, stats = self._buffers(n, H, W, False, acts=False)
+        _, work, _, stats = self._buffers(n, H, W, False)
         if out is None:
             out = torch.empty_like(x)
         rc = gr.lib().gr_cnn_infer(_ptr(self.params), _ptr(self.packed), _ptr(x), n, H, W, self.scale, _ptr(out),

@@ -329,3 +329,58 @@ def test_backward_tile_edges(n, H, W):
     gg = Lrn.unflatten(net.grads.cpu().numpy())
     for k in g:
         assert np.linalg.norm(gg[k] - g[k]) <= 2e-3 * np.linalg.norm(g[k]), k
+
+
+# the forward kernel's strips of 56 columns (16-column groups, guard columns)
+# and segments of rows (pairs of rows, odd ends): one short of, exactly and one
+# past a strip, several segments, images smaller than the halo
+FORWARD_SHAPES = [(1, 1, 1), (2, 3, 55), (1, 4, 56), (1, 17, 57), (1, 33, 113), (3, 130, 4), (1, 300, 61), (40, 18, 60)]
+
+
+@pytest.mark.parametrize("shape", FORWARD_SHAPES)
+def test_forward_strips_and_segments(shape):
+    """Each layer against the convolution of the GPU's own previous activations:
+    equal up to the rounding of a float sum at a bf16 boundary (tolerances of
+    test_forward_layers_match_oracle); inference bitwise the training output."""
+    net, pd, x, _ = make(sum(shape), *shape)
+    xg = torch.from_numpy(x).cuda()
+    y, stats = net.forward(xg, train=True)
+    torch.cuda.synchronize()
+    a = [bf16_bits_to_f32(t) for t in net._buffers(*shape, True)[0]]
+    xn = x / np.float32(net.scale)
+    prev = K.bf16(xn)[..., None]
+    for l in range(4):
+        w = K.bf16(pd[f"W{l + 1}"])
+        w = w[:, None, :] if l == 0 else w
+        e = K.bf16(np.maximum(K.conv3x3(prev, w) + pd[f"b{l + 1}"], 0.0)).astype(np.float32)
+        tol = np.maximum(np.abs(e) * 2.0 ** -7, 1e-3 * np.sqrt(np.mean(e.astype(np.float64) ** 2)))
+        d = ulp_diff(np.ascontiguousarray(a[l]), np.ascontiguousarray(e))
+        assert np.mean(d > 0) < 0.01 and (np.abs(a[l] - e) <= tol).all(), l
+        prev = a[l]
+    r = K.conv3x3(prev, K.bf16(pd["W5"])[None])[..., 0] + pd["b5"][0]
+    assert rel(y.cpu().numpy(), (xn + r) * net.scale) < 1e-5
+    s = stats.cpu().numpy().astype(np.float64)
+    assert np.allclose(s[:, 0], (r ** 2).reshape(shape[0], -1).sum(1), rtol=1e-4)
+    y2, stats2 = net.infer(xg)
+    torch.cuda.synchronize()
+    assert torch.equal(y, y2) and torch.equal(stats, stats2)
+
+
+def test_forward_aliased_activations():
+    """gr_cnn_forward with a3 in a1's buffer and a4 in a2's: they end holding
+    a3 and a4."""
+    import ctypes as C
+
+    from projects_amd import gridrec as gr
+
+    net, _, x, _ = make(9, 2, 40, 70)
+    xg = torch.from_numpy(x).cuda()
+    y, _ = net.forward(xg, train=True)
+    acts = net._buffers(2, 40, 70, True)[0]
+    b = [torch.zeros_like(acts[0]) for _ in range(2)]
+    y2 = torch.empty_like(xg)
+    p = lambda t: C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p(None)
+    gr._check(gr.lib().gr_cnn_forward(p(net.params), p(net.packed), p(xg), 2, 40, 70, net.scale, p(b[0]), p(b[1]),
+                                      p(b[0]), p(b[1]), p(y2), p(None), p(None), p(None), C.c_void_p(0)), "forward")
+    torch.cuda.synchronize()
+    assert torch.equal(y, y2) and torch.equal(b[0], acts[2]) and torch.equal(b[1], acts[3])

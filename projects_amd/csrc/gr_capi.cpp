@@ -737,8 +737,18 @@ int gr_plan_create_impl(const gr_params *params, gr_plan **plan_out, bool alloc_
         CK(dev_alloc(pl, &pl->d_rowtiles, (size_t)nt));
         hipStream_t rs;
         CK(plan_stream(pl, &rs));
+        std::vector<int2> rt(nt);
         hipError_t e = gr_launch_row_tiles(g, pl->d_rowtiles, rs);
+        if (e == hipSuccess) e = hipMemcpyAsync(rt.data(), pl->d_rowtiles, sizeof(int2) * nt, hipMemcpyDeviceToHost, rs);
         if (e == hipSuccess) e = hipStreamSynchronize(rs);
+        // the disk of samples leaves the first and last rows of the grid empty
+        // where the padded detector is narrower than the grid (37% of them at
+        // 2560 detectors): at least one tile row is kept
+        int lo = 0, hi = nt;
+        while (lo + 1 < hi && rt[lo].x > rt[lo].y) lo++;
+        while (hi - 1 > lo && rt[hi - 1].x > rt[hi - 1].y) hi--;
+        pl->row_lo = lo * ts;
+        pl->row_hi = hi * ts;
         if (e != hipSuccess) {
             free_plan(pl);
             return hip_fail(e, "row tile intervals");

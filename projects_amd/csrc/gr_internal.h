@@ -95,6 +95,9 @@ struct GrDevTables {
     // per tile row (M / 8 rows) the interval [lo, hi] of tiles that can hold
     // a nonzero cell (gr_active_tile_range), evaluated once on the device
     const int2 *row_tiles = nullptr;
+    // rows [row_lo, row_hi) of the grid hold them all; the others are zeros
+    // that no kernel writes, transforms or reads
+    int row_lo = 0, row_hi = 0;
 };
 
 // Compute units of the current device, and the most LDS one workgroup may

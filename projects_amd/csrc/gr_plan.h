@@ -20,6 +20,7 @@ struct gr_plan {
     float4 *d_ang = nullptr;
     unsigned *d_tiles = nullptr;
     int2 *d_rowtiles = nullptr;  // active-tile interval per tile row (K3)
+    int row_lo = 0, row_hi = 0;  // the rows with active tiles
     int ntiles = 0;      // slots: kGridSectors * sector_len
     int sector_len = 0;
     // K2's precomputed gather operator (GR_GRIDOP_*): entries, taps per tile,
@@ -94,6 +95,8 @@ struct gr_plan {
         t.ntiles = ntiles;
         t.sector_len = sector_len;
         t.row_tiles = d_rowtiles;
+        t.row_lo = row_lo;
+        t.row_hi = row_hi;
         t.sitems = d_sitems;
         t.smeta = d_smeta;
         t.n_sitems = n_sitems;

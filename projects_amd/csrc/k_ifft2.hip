@@ -33,6 +33,7 @@ struct RowsArgs {
     const int2 *row_tiles;  // per tile row the written tiles [lo, hi]; the others are zeros
     int M, radix;
     long M02, out_off, out_n;
+    int row_lo, row_hi;  // the grid rows that are not all zeros
 };
 
 // Output hook of the row transform: FFT output i lands in window column
@@ -72,7 +73,7 @@ __global__ void __launch_bounds__(1024) k_ifft_rows(RowsArgs A) {
     constexpr int EPT = 4 * MAXB;
     const int nthr = (int)blockDim.x / CW;
     const int grp = (int)threadIdx.x / nthr, tid = (int)threadIdx.x % nthr;
-    const int b = row_group((int)blockIdx.x, (int)gridDim.x, CW) * CW + grp, p = blockIdx.y;
+    const int b = A.row_lo + row_group((int)blockIdx.x, (int)gridDim.x, CW) * CW + grp, p = blockIdx.y;
     const int M = A.M;
     float2 *row = lds + (long)grp * M;
     const float2 *src = A.ht + ((long)p * M + b) * M;
@@ -118,6 +119,7 @@ struct ColsArgs {
     long out_slice_stride, out_row_stride;
     int M, cw, n_slices, pair0, radix;
     long M02, out_off, out_n;
+    int row_lo, row_hi;  // rows of Z that the row transform wrote; the others read as zeros
 };
 
 // Output hook of the column transform: FFT output i is image column
@@ -184,7 +186,7 @@ __global__ void __launch_bounds__(1024) k_ifft_cols(ColsArgs A) {
         for (int r = 0; r < EPT; r++) {
             const int idx = (int)threadIdx.x + r * (int)blockDim.x;
             const int b = idx / CW, c = idx - b * CW;
-            const bool in = b < M && c0 + c < out_n;
+            const bool in = b >= A.row_lo && b < A.row_hi && c0 + c < out_n;
             v[r] = gr_buf_ld2(zb, in ? (unsigned)(gr_z_index(M, b, c0 + c) * sizeof(float2)) : kGrBufNone);
         }
 #pragma unroll
@@ -195,12 +197,13 @@ __global__ void __launch_bounds__(1024) k_ifft_cols(ColsArgs A) {
         }
     } else if (cw == 1) {
         for (int b = tid; b < M; b += nthr)
-            cols[gr_lds_idx(b)] = c0 < out_n ? zp[gr_z_index(M, b, c0)] : make_float2(0.0f, 0.0f);
+            cols[gr_lds_idx(b)] =
+                c0 < out_n && b >= A.row_lo && b < A.row_hi ? zp[gr_z_index(M, b, c0)] : make_float2(0.0f, 0.0f);
     } else {
         for (int idx = threadIdx.x; idx < cw * M; idx += blockDim.x) {  // CW: cw * M <= 20480; else <= 16384
             const int b = idx / cw, c = idx - b * cw;
             cols[c * gr_lds_len(M) + gr_lds_idx(b)] =
-                (c0 + c < out_n) ? zp[gr_z_index(M, b, c0 + c)] : make_float2(0.0f, 0.0f);
+                c0 + c < out_n && b >= A.row_lo && b < A.row_hi ? zp[gr_z_index(M, b, c0 + c)] : make_float2(0.0f, 0.0f);
         }
     }
     __syncthreads();
@@ -300,9 +303,19 @@ __global__ void __launch_bounds__(kPfThreads) k_ifft_cols_pf(ColsArgs A, int n_i
         const GrBuf zb = gr_buf(A.z + (long)p * kPfM * gr_z_cols(out_n) + (long)c0 * kPfM,
                                 (unsigned)(kPfM * kPfCw * sizeof(float2)));
         const bool in = c0 + lc < out_n;
-        const unsigned o0 = in ? (unsigned)(((t / kPfCw) * kPfCw + lc) * sizeof(float2)) : kGrBufNone;
+        const int b0 = t / kPfCw;
+        if (A.row_hi - A.row_lo == kPfM) {
+            const unsigned o0 = in ? (unsigned)((b0 * kPfCw + lc) * sizeof(float2)) : kGrBufNone;
 #pragma unroll
-        for (int r = 0; r < 16; r++) v[r] = gr_buf_ld2(zb, o0, (unsigned)(r * kPfNthr * kPfCw * sizeof(float2)));
+            for (int r = 0; r < 16; r++) v[r] = gr_buf_ld2(zb, o0, (unsigned)(r * kPfNthr * kPfCw * sizeof(float2)));
+        } else {  // rows outside [row_lo, row_hi) were not written
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int b = b0 + r * kPfNthr;
+                v[r] = gr_buf_ld2(zb, in && b >= A.row_lo && b < A.row_hi ? (unsigned)((b * kPfCw + lc) * sizeof(float2))
+                                                                          : kGrBufNone);
+            }
+        }
         const int grp = t / kPfNthr;
         cu_next = A.winv[off + (c0 + grp < out_n ? c0 + grp : out_n - 1)];
     };
@@ -366,7 +379,7 @@ __global__ void __launch_bounds__(kPfThreads) k_ifft_rows_pf(RowsArgs A, int n_i
     extern __shared__ float2 lds[];
     float2 *tw = lds + kPfCw * kPfColStride;
     const int out_n = (int)A.out_n, off = (int)A.out_off, m02 = (int)A.M02;
-    const int groups = kPfM / kPfCw;  // items per pair
+    const int groups = (A.row_hi - A.row_lo) / kPfCw;  // items per pair
     for (int i = (int)threadIdx.x; i < kPfTw; i += kPfThreads) tw[i] = A.tw[i];
     float2 v[16];
     // the active-tile interval of an item's tile row (its four rows share
@@ -374,11 +387,11 @@ __global__ void __launch_bounds__(kPfThreads) k_ifft_rows_pf(RowsArgs A, int n_i
     // before it are waited for anyway
     auto interval = [&](int item) {
         const int p = item / groups;
-        return item < n_items ? A.row_tiles[((item - p * groups) * kPfCw) >> 3] : make_int2(1, 0);
+        return item < n_items ? A.row_tiles[(A.row_lo + (item - p * groups) * kPfCw) >> 3] : make_int2(1, 0);
     };
     auto load = [&](int item, int2 lh, int t) {  // t: threadIdx.x (an opaque copy inside the loop)
         const int grp = t / kPfNthr, tid = t % kPfNthr;
-        const int p = item / groups, b0 = (item - p * groups) * kPfCw;
+        const int p = item / groups, b0 = A.row_lo + (item - p * groups) * kPfCw;
         const GrBuf hb = gr_buf(A.ht + ((long)p * kPfM + b0) * kPfM, (unsigned)(kPfCw * kPfM * sizeof(float2)));
 #pragma unroll
         for (int r = 0; r < 16; r++) {
@@ -405,7 +418,7 @@ __global__ void __launch_bounds__(kPfThreads) k_ifft_rows_pf(RowsArgs A, int n_i
             lh_next = interval(item + (int)gridDim.x);
         }
         gr_lds_fft<-1, 4, GrFftToLds, true>(row, kPfM, tw, tid, kPfNthr, 16, GrFftToLds(), true);
-        const int p = cur / groups, b0 = (cur - p * groups) * kPfCw;
+        const int p = cur / groups, b0 = A.row_lo + (cur - p * groups) * kPfCw;
         float2 *zp = A.z + (long)p * kPfM * gr_z_cols(out_n);
 #pragma unroll
         for (int r = 0; r < 8; r++) {  // 4 rows x up to 2048 columns = 8192 outputs
@@ -473,10 +486,11 @@ constexpr int kRowsPerBlock = 1;
 
 hipError_t gr_launch_ifft_rows(const GrGeom &g, const GrDevTables &t, const float2 *ht, float2 *z,
                                int pairs, hipStream_t s) {
-    RowsArgs A{ht, z, t.tw_grid, t.row_tiles, (int)g.M, g.fft_radix, g.M02, g.out_off, g.out_n};
+    RowsArgs A{ht, z, t.tw_grid, t.row_tiles, (int)g.M, g.fft_radix, g.M02, g.out_off, g.out_n,
+               t.row_lo, t.row_hi};
     const int nthr = gr_fft_threads(g.M);
     if (g.M == kPfM && nthr == kPfNthr && g.fft_radix == 16 && g.out_n <= 8 * kPfNthr && pf_fits()) {
-        const int n_items = (int)(g.M / kPfCw) * pairs;
+        const int n_items = (t.row_hi - t.row_lo) / kPfCw * pairs;
         const int nblk = std::min(n_items, gr_cu_count());
         hipError_t e = gr_allow_lds(k_ifft_rows_pf, kPfLds);
         if (e != hipSuccess) return e;
@@ -485,7 +499,7 @@ hipError_t gr_launch_ifft_rows(const GrGeom &g, const GrDevTables &t, const floa
     }
     int cw = kRowsPerBlock;  // rows side by side: a power of two dividing M, within 1024 threads and the LDS
     while (cw > 1 && ((long)cw * nthr > 1024 || (long)cw * g.M * 8 > 163840 || g.M % cw)) cw /= 2;
-    const dim3 grid((unsigned)(g.M / cw), pairs), block(cw * nthr);
+    const dim3 grid((unsigned)((t.row_hi - t.row_lo) / cw), pairs), block(cw * nthr);
     const size_t lds = sizeof(float2) * cw * gr_lds_len(g.M);
 #define GR_ROWS_K(MB, CW)                                                          \
     do {                                                                           \
@@ -554,6 +568,8 @@ hipError_t gr_launch_ifft_cols(const GrGeom &g, const GrDevTables &t, const floa
     A.M02 = g.M02;
     A.out_off = g.out_off;
     A.out_n = g.out_n;
+    A.row_lo = t.row_lo;
+    A.row_hi = t.row_hi;
     const int nthr = gr_fft_threads(g.M);
     const bool side = cols_side_by_side(g.M, A.cw);
     if (side && A.cw == kPfCw && g.M == kPfM && nthr == kPfNthr && g.fft_radix == 16 && g.out_n <= 8 * kPfNthr &&

@@ -499,6 +499,11 @@ std::vector<float2> pass_twiddles(long n, int sign) {
                 for (long k = 0; k < Ns; k++) out.push_back(w[r * k * (n / (Ns * 16))]);
             Ns *= 16;
         }
+        if (max_radix >= 16 && Ns * 8 == n) {
+            for (int r = 1; Ns > 1 && r < 8; r++)
+                for (long k = 0; k < Ns; k++) out.push_back(w[r * k * (n / (Ns * 8))]);
+            Ns *= 8;
+        }
         while (Ns * 4 <= n) {
             for (int r = 1; Ns > 1 && r < 4; r++)
                 for (long k = 0; k < Ns; k++) out.push_back(w[r * k * (n / (Ns * 4))]);

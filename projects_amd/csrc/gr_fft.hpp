@@ -3,8 +3,8 @@
 // Stockham autosort formulation (N. K. Govindaraju et al., "High performance
 // discrete Fourier transforms on graphics processors", SC'08): passes of
 // radix 16 (a 4 x 4 decomposition in registers) while 16 divides what is left,
-// then radix 4, then one radix-2 pass when needed (max_radix 4 skips the
-// radix-16 passes: a launch-tuning choice); output in natural order.
+// then one of radix 8, 4 or 2 as needed (max_radix 4: radix 4 and 2 only, a
+// launch-tuning choice); output in natural order.
 // Each pass reads all of a thread's butterfly inputs into registers, crosses a
 // barrier, and writes the outputs back into the same LDS row, so one buffer of
 // N complex values suffices.  SIGN = +1 computes sum_k x_k e^{+2 pi i jk/N},
@@ -96,6 +96,10 @@ __host__ __device__ __forceinline__ long gr_twp_len(long N, int max_radix) {
         if (Ns > 1) len += 15 * Ns;
         Ns *= 16;
     }
+    if (max_radix >= 16 && Ns * 8 == N) {
+        if (Ns > 1) len += 7 * Ns;
+        Ns *= 8;
+    }
     while (Ns * 4 <= N) {
         if (Ns > 1) len += 3 * Ns;
         Ns *= 4;
@@ -132,6 +136,29 @@ __device__ __forceinline__ void gr_dft4(float2 &v0, float2 &v1, float2 &v2, floa
     v3 = make_float2(a1.x - a3.x, a1.y - a3.y);
 }
 
+// 8-point DFT in place, natural order: two 4-point DFTs over the even and the
+// odd inputs, joined with the roots e^{SIGN 2 pi i k/8}.
+template <int SIGN>
+__device__ __forceinline__ void gr_dft8(float2 (&v)[8]) {
+    constexpr float R2 = 0.707106781186547524f;
+    constexpr float s = (float)SIGN;
+    gr_dft4<SIGN>(v[0], v[2], v[4], v[6]);
+    gr_dft4<SIGN>(v[1], v[3], v[5], v[7]);
+    const float2 t0 = v[1];
+    const float2 t1 = make_float2((v[3].x - s * v[3].y) * R2, (v[3].y + s * v[3].x) * R2);
+    const float2 t2 = make_float2(-s * v[5].y, s * v[5].x);
+    const float2 t3 = make_float2((-v[7].x - s * v[7].y) * R2, (s * v[7].x - v[7].y) * R2);
+    const float2 e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6];
+    v[0] = make_float2(e0.x + t0.x, e0.y + t0.y);
+    v[1] = make_float2(e1.x + t1.x, e1.y + t1.y);
+    v[2] = make_float2(e2.x + t2.x, e2.y + t2.y);
+    v[3] = make_float2(e3.x + t3.x, e3.y + t3.y);
+    v[4] = make_float2(e0.x - t0.x, e0.y - t0.y);
+    v[5] = make_float2(e1.x - t1.x, e1.y - t1.y);
+    v[6] = make_float2(e2.x - t2.x, e2.y - t2.y);
+    v[7] = make_float2(e3.x - t3.x, e3.y - t3.y);
+}
+
 // 16-point DFT in place with root w = e^{SIGN 2 pi i/16}: slots r = 4a + b
 // hold x[r]; a 4-point DFT over a for each b, the twiddle w^(bc), a 4-point
 // DFT over b for each c; X[c + 4d] ends in slot 4c + d.
@@ -161,16 +188,6 @@ struct GrFftToLds {
     __device__ void operator()(int, float2, int) const {}
 };
 
-// The first radix-16 pass of butterfly j (Ns = 1, no twiddles) on values
-// already in registers, v[r] = x[j + r N/16], and its outputs stored to buf
-// where gr_lds_fft's own first pass puts them.
-template <int SIGN>
-__device__ __forceinline__ void gr_fft_first_pass16(float2 *buf, float2 (&v)[16], int j) {
-    gr_dft16<SIGN>(v);
-#pragma unroll
-    for (int q = 0; q < 16; q++) buf[gr_lds_idx((j << 4) + q)] = v[4 * (q & 3) + (q >> 2)];
-}
-
 // Returns true when an enabled output hook `out` received the result instead
 // of buf: when the last pass is a radix-16 one, out(i, X[i], s) is called for
 // every output i straight from the registers of that pass (no LDS store, no
@@ -179,14 +196,11 @@ __device__ __forceinline__ void gr_fft_first_pass16(float2 *buf, float2 (&v)[16]
 // hook issues the loads its outputs need there, all in flight together).
 // Otherwise the result is in buf as usual and false is returned.  Every output
 // i is handed over exactly once; for a fixed pass slot the threads hand over
-// consecutive i.  first_done: the caller ran the first radix-16 pass
-// (gr_fft_first_pass16 for every butterfly, then a barrier); only with
-// max_radix 16 and N >= 16.  TW_LDS: tw is a copy of the radix-16 part of
-// the table in LDS (only with max_radix 16 and N a power of 16).
-template <int SIGN, int MAXB, class Out = GrFftToLds, bool TW_LDS = false>
+// consecutive i.
+template <int SIGN, int MAXB, class Out = GrFftToLds>
 __device__ __forceinline__ bool gr_lds_fft(float2 *buf, int N, const float2 *__restrict__ tw, int tid, int nthr,
-                                           int max_radix = 16, Out out = Out(), bool first_done = false) {
-    int Ns = first_done ? 16 : 1;  // the Ns = 1 pass reads no twiddles: tofs stays at the table's start
+                                           int max_radix = 16, Out out = Out()) {
+    int Ns = 1;
     // twiddles by buffer loads: one lane offset (8 k) for all of a pass's
     // loads, the entry's row in the scalar offset, tofs = the pass's table
     const GrBuf twb = gr_buf(tw, (unsigned)((gr_twp_len(N, 16) + gr_twp_len(N, 4)) * sizeof(float2)));
@@ -207,8 +221,7 @@ __device__ __forceinline__ bool gr_lds_fft(float2 *buf, int N, const float2 *__r
                 if (Ns > 1) {
 #pragma unroll
                     for (int r = 1; r < 16; r++)
-                        w[r - 1] = TW_LDS ? tw[tofs / 8u + (unsigned)((r - 1) * Ns + k)]
-                                          : gr_buf_ld2(twb, 8u * (unsigned)k, tofs + 8u * (unsigned)((r - 1) * Ns));
+                        w[r - 1] = gr_buf_ld2(twb, 8u * (unsigned)k, tofs + 8u * (unsigned)((r - 1) * Ns));
                 }
 #pragma unroll
                 for (int r = 0; r < 16; r++) v[c][r] = buf[gr_lds_idx(j + r * nb16)];
@@ -254,6 +267,45 @@ __device__ __forceinline__ bool gr_lds_fft(float2 *buf, int N, const float2 *__r
         if (Ns > 1) tofs += 8u * 15u * (unsigned)Ns;
         Ns <<= 4;
     }
+    if (max_radix >= 16 && Ns * 8 == N) {
+        const int nb8 = N >> 3;
+        constexpr int MAXB8 = (MAXB + 1) / 2;
+        float2 v[MAXB8][8];
+#pragma unroll
+        for (int c = 0; c < MAXB8; c++) {
+            const int j = tid + c * nthr;
+            if (j < nb8) {
+                const int k = j & (Ns - 1);
+                float2 w[7];
+                if (Ns > 1) {
+#pragma unroll
+                    for (int r = 0; r < 7; r++)
+                        w[r] = gr_buf_ld2(twb, 8u * (unsigned)k, tofs + 8u * (unsigned)(r * Ns));
+                }
+#pragma unroll
+                for (int r = 0; r < 8; r++) v[c][r] = buf[gr_lds_idx(j + r * nb8)];
+                if (Ns > 1) {
+#pragma unroll
+                    for (int r = 1; r < 8; r++) v[c][r] = gr_cmul(v[c][r], w[r - 1]);
+                }
+                gr_dft8<SIGN>(v[c]);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < MAXB8; c++) {
+            const int j = tid + c * nthr;
+            if (j < nb8) {
+                const int k = j & (Ns - 1);
+                const int base = ((j - k) << 3) + k;
+#pragma unroll
+                for (int r = 0; r < 8; r++) buf[gr_lds_idx(base + r * Ns)] = v[c][r];
+            }
+        }
+        __syncthreads();
+        if (Ns > 1) tofs += 8u * 7u * (unsigned)Ns;
+        Ns <<= 3;
+    }
     const int nb4 = N >> 2;
     while (Ns * 4 <= N) {
         float2 v[MAXB][4];
@@ -265,7 +317,8 @@ __device__ __forceinline__ bool gr_lds_fft(float2 *buf, int N, const float2 *__r
                 float2 w[3];
                 if (Ns > 1) {
 #pragma unroll
-                    for (int r = 0; r < 3; r++) w[r] = gr_buf_ld2(twb, 8u * (unsigned)k, tofs + 8u * (unsigned)(r * Ns));
+                    for (int r = 0; r < 3; r++)
+                        w[r] = gr_buf_ld2(twb, 8u * (unsigned)k, tofs + 8u * (unsigned)(r * Ns));
                 }
 #pragma unroll
                 for (int r = 0; r < 4; r++) v[c][r] = buf[gr_lds_idx(j + r * nb4)];
@@ -319,6 +372,15 @@ __device__ __forceinline__ bool gr_lds_fft(float2 *buf, int N, const float2 *__r
         __syncthreads();
     }
     return false;
+}
+
+// Output i of a closing radix-2 pass from its two inputs in buf (gr_lds_fft's
+// arithmetic), w = e^{SIGN 2 pi i k/N} for k = i mod N/2.
+__device__ __forceinline__ float2 gr_last2(const float2 *buf, int N, int i, float2 w) {
+    const int k = i & (N / 2 - 1);
+    const float2 x0 = buf[gr_lds_idx(k)];
+    const float2 x1 = gr_cmul(buf[gr_lds_idx(k + N / 2)], w);
+    return i < N / 2 ? make_float2(x0.x + x1.x, x0.y + x1.y) : make_float2(x0.x - x1.x, x0.y - x1.y);
 }
 
 // Threads per FFT block and the matching MAXB for a row of N points.

@@ -263,60 +263,150 @@ __global__ void __launch_bounds__(1024) k_ifft_cols(ColsArgs A) {
     }
 }
 
-// Persistent column transform for M = 4096 with 4 columns per item and
-// radix-16 passes (the plain 2048-detector geometry): the columns and the
-// 32 KiB of twiddles fill the CU's 160 KiB of LDS, so one workgroup of 1024
-// threads runs per CU and loops over (pair, column group) items, each one
-// contiguous 128 KB block of the column-blocked Z.  Each thread
-// loads rows j, j + 256, ..., j + 3840 of one column -- exactly the inputs of
+// ---- persistent transforms ----------------------------------------------------
+//
+// For M = 1024 .. 8192 with radix-16 passes: one workgroup of 1024 threads runs
+// per CU and loops over items of CW = 16384 / M neighbouring rows (columns),
+// which with the twiddles fill the CU's 160 KiB of LDS.  Each thread
+// loads elements j + r M/16, r < 16, of one row -- exactly the inputs of
 // the first radix-16 butterfly j -- so that pass runs from the registers that
 // received the loads; the next item's loads are issued into the same
-// registers right after, and stay in flight while passes 2 and 3 run on
+// registers right after, and stay in flight while the other passes run on
 // twiddles from LDS (no global load in between: the loads of all of a wave
-// complete in order, so any would wait for them).  The last pass ends in LDS
-// and an epilogue scales and stores the image row (an output hook would need
-// sixteen more registers for its deapodization factors: spills).  Same
-// arithmetic, twiddles and output values as k_ifft_cols: bitwise its images.
-// Needs 1 <= out_n <= 2048.
-constexpr int kPfM = 4096, kPfCw = 4, kPfThreads = 1024;
-constexpr int kPfNthr = kPfThreads / kPfCw;  // threads per column
-constexpr int kPfColStride = kPfM + 4;       // padded: the four columns' first-pass stores use different banks
-constexpr int kPfTw = 15 * 16 + 15 * 256;    // pass-ordered radix-16 twiddles of 4096 points
-constexpr size_t kPfLds = sizeof(float2) * ((size_t)kPfCw * kPfColStride + kPfTw);
+// complete in order, so any would wait for them).  The passes end in LDS
+// and an epilogue stores the window (an output hook would need
+// sixteen more registers for its deapodization factors: spills); the closing
+// radix-2 pass of M = 8192 happens there, a window's outputs needing half of
+// it each.  Same arithmetic, twiddles and output values as the one-shot
+// kernels: bitwise their images.
+//
+// Bound by HBM: at M = 4096 (32 pairs of 1500 x 2048) rows 1255 us and columns
+// 671, 4.4 and 4.8 TB/s, a copy's 4.7; M = 2048 (32 pairs of 720 x 1024) 323 and
+// 185 us, one-shot 607 and 383; M = 8192 (8 pairs of 1800 x 2560) 990 and 990,
+// one-shot 1980 (rows that hold only zeros included) and 1490; M = 1024 (16
+// pairs of 451 x 777, whole images) 52 and 57, one-shot 88 and 140.
+constexpr int kPfThreads = 1024;
+template <int LM>
+struct Pf {
+    static constexpr int M = 1 << LM, CW = 16384 / M, nthr = M / 16;  // threads per row
+    static constexpr int stride = M + 4;  // padded: neighbouring rows' first-pass stores use different banks
+    static constexpr bool last2 = LM == 13;                          // 16 16 16 2
+    static constexpr int r3 = last2 ? 16 : M / 256;                  // the third pass's radix
+    static constexpr int tw = 15 * 16 + (r3 - 1) * 256;              // twiddles of passes two and three
+    static constexpr size_t lds = sizeof(float2) * ((size_t)CW * stride + tw);
+    static constexpr int cpb = CW < 4 ? CW : 4;                      // columns of an item in a block of Z
+    static constexpr int blocks = CW < 4 ? 1 : CW / 4, tpb = kPfThreads / blocks;
+};
 
+// The passes on a row already loaded: the arithmetic of gr_lds_fft, with the
+// row's LDS places (gr_lds_idx) as a few addresses per thread plus constants:
+// for j < nthr, i = j + r nthr sits at (j ^ (j >> 4)) ^ (r nthr / 16 mod 32),
+// plus r nthr; an output of the first pass, i = 16 j + q, at (16 j ^ (j mod 32))
+// ^ q; one of the second, 256 J + k + 16 q, at (256 J + k + 16 (J mod 2)) ^ 17 q.
+// (With gr_lds_idx evaluated per access the addresses were half of the
+// kernels' VALU instructions, and those bound them.)
+__device__ __forceinline__ int pf_place(int j) { return j ^ ((j >> 4) & 31); }
+
+template <int LM>
+__device__ __forceinline__ void pf_first(float2 *buf, float2 (&v)[16], int j) {
+    gr_dft16<-1>(v);
+    const int b = (j << 4) ^ (j & 31);
+#pragma unroll
+    for (int q = 0; q < 16; q++) buf[b ^ q] = v[4 * (q & 3) + (q >> 2)];
+}
+
+template <int LM>
+__device__ __forceinline__ void pf_rest(float2 *buf, const float2 *tw, int tid) {
+    using F = Pf<LM>;
+    constexpr int NT = F::nthr;
+    float2 v[16], w[15];
+    {
+        const int k = tid & 15, J = tid >> 4, in = pf_place(tid), out = (J << 8) + k + ((J & 1) << 4);
+#pragma unroll
+        for (int r = 1; r < 16; r++) w[r - 1] = tw[(r - 1) * 16 + k];
+#pragma unroll
+        for (int r = 0; r < 16; r++) v[r] = buf[(in ^ ((r * (NT / 16)) & 31)) + r * NT];
+#pragma unroll
+        for (int r = 1; r < 16; r++) v[r] = gr_cmul(v[r], w[r - 1]);
+        gr_dft16<-1>(v);
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 16; q++) buf[out ^ (17 * q)] = v[4 * (q & 3) + (q >> 2)];
+        __syncthreads();
+    }
+    tw += 15 * 16;
+    if constexpr (F::r3 == 16) {
+        const int k = tid & 255, in = pf_place(tid), out = (tid & ~255) * 16 + pf_place(k);
+#pragma unroll
+        for (int r = 1; r < 16; r++) w[r - 1] = tw[(r - 1) * 256 + k];
+#pragma unroll
+        for (int r = 0; r < 16; r++) v[r] = buf[(in ^ ((r * (NT / 16)) & 31)) + r * NT];
+#pragma unroll
+        for (int r = 1; r < 16; r++) v[r] = gr_cmul(v[r], w[r - 1]);
+        gr_dft16<-1>(v);
+        if (LM != 12) __syncthreads();  // M = 4096: a thread writes the places it read
+#pragma unroll
+        for (int q = 0; q < 16; q++) buf[(out ^ ((q & 1) << 4)) + 256 * q] = v[4 * (q & 3) + (q >> 2)];
+    } else {  // 256 butterflies of radix 8 or 4, in place
+#pragma unroll
+        for (int c = 0; c < 256 / NT; c++) {
+            const int j = tid + c * NT, in = pf_place(j);
+            constexpr int R = F::r3;
+            float2 x[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) x[r] = buf[(in ^ ((r & 1) << 4)) + 256 * r];
+#pragma unroll
+            for (int r = 1; r < R; r++) x[r] = gr_cmul(x[r], tw[(r - 1) * 256 + j]);
+            if constexpr (R == 8) gr_dft8<-1>(x);
+            else gr_dft4<-1>(x[0], x[1], x[2], x[3]);
+#pragma unroll
+            for (int r = 0; r < R; r++) buf[(in ^ ((r & 1) << 4)) + 256 * r] = x[r];
+        }
+    }
+    __syncthreads();
+}
+
+// Columns: an item is CW neighbouring columns of one pair, contiguous blocks of
+// the column-blocked Z (M = 8192: half of one).
+// ALL: every row of Z was written.
+template <int LM, bool ALL>
 __global__ void __launch_bounds__(kPfThreads) k_ifft_cols_pf(ColsArgs A, int n_items) {
+    using F = Pf<LM>;
+    constexpr int M = F::M, CW = F::CW, NT = F::nthr;
     extern __shared__ float2 lds[];
-    float2 *tw = lds + kPfCw * kPfColStride;
-    const int out_n = (int)A.out_n, off = (int)A.out_off, m02 = (int)A.M02;
-    const int ngroups = (out_n + kPfCw - 1) / kPfCw;
-    for (int i = (int)threadIdx.x; i < kPfTw; i += kPfThreads) tw[i] = A.tw[i];
+    float2 *tw = lds + CW * F::stride;
+    const int out_n = (int)A.out_n, off = (int)A.out_off;
+    const int wrap = off + M - (int)A.M02;  // window output k is transform output (k + wrap) mod M
+    const int ngroups = (out_n + CW - 1) / CW;
+    for (int i = (int)threadIdx.x; i < F::tw; i += kPfThreads) tw[i] = A.tw[i];
     float2 v[16];
     float cu_next = 0.0f;
-    // the item's column loads: thread t reads rows t/4 + 256 r of column t % 4
-    // (the inputs of first-pass butterfly t/4); a column past the window (the
-    // last group only) reads zeros through the buffer bound, no branch
+    // the item's column loads: thread t reads rows j + r M/16 of column lc; a
+    // column past the window (the last group only) and rows that were not
+    // written read zeros through the buffer bound, no branch
+    auto column = [](int t) { return t % F::cpb + 4 * (t / F::tpb); };
+    auto first = [](int t) { return t % F::tpb / F::cpb; };  // j
     auto load = [&](int item) {
-        const int t = (int)threadIdx.x, lc = t % kPfCw;
+        const int t = (int)threadIdx.x, lc = column(t), j = first(t);
         const int p = item / ngroups, x = item - p * ngroups;
-        const int c0 = (int)column_group((unsigned)x, (unsigned)ngroups) * kPfCw;
-        // the group's column block: 4096 rows x 32 bytes, contiguous
-        const GrBuf zb = gr_buf(A.z + (long)p * kPfM * gr_z_cols(out_n) + (long)c0 * kPfM,
-                                (unsigned)(kPfM * kPfCw * sizeof(float2)));
+        const int c0 = (int)column_group((unsigned)x, (unsigned)ngroups) * CW;
+        const GrBuf zb = gr_buf(A.z + (long)p * M * gr_z_cols(out_n) + (long)(c0 & ~3) * M,
+                                (unsigned)(F::blocks * M * 4 * sizeof(float2)));
         const bool in = c0 + lc < out_n;
-        const int b0 = t / kPfCw;
-        if (A.row_hi - A.row_lo == kPfM) {
-            const unsigned o0 = in ? (unsigned)((b0 * kPfCw + lc) * sizeof(float2)) : kGrBufNone;
+        const unsigned o0 = (unsigned)(((lc / 4 * M + j) * 4 + (c0 + lc) % 4) * sizeof(float2));
+        if (ALL) {
+            const unsigned o = in ? o0 : kGrBufNone;
 #pragma unroll
-            for (int r = 0; r < 16; r++) v[r] = gr_buf_ld2(zb, o0, (unsigned)(r * kPfNthr * kPfCw * sizeof(float2)));
-        } else {  // rows outside [row_lo, row_hi) were not written
+            for (int r = 0; r < 16; r++) v[r] = gr_buf_ld2(zb, o, (unsigned)(r * NT * 4 * sizeof(float2)));
+        } else {
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                const int b = b0 + r * kPfNthr;
-                v[r] = gr_buf_ld2(zb, in && b >= A.row_lo && b < A.row_hi ? (unsigned)((b * kPfCw + lc) * sizeof(float2))
+                const int b = j + r * NT;
+                v[r] = gr_buf_ld2(zb, in && b >= A.row_lo && b < A.row_hi ? o0 + (unsigned)(r * NT * 4 * sizeof(float2))
                                                                           : kGrBufNone);
             }
         }
-        const int grp = t / kPfNthr;
+        const int grp = t / NT;
         cu_next = A.winv[off + (c0 + grp < out_n ? c0 + grp : out_n - 1)];
     };
     int item = (int)blockIdx.x;
@@ -328,108 +418,123 @@ __global__ void __launch_bounds__(kPfThreads) k_ifft_cols_pf(ColsArgs A, int n_i
         // 128 registers of a 1024-thread workgroup
         int t = (int)threadIdx.x;
         asm volatile("" : "+v"(t));
-        gr_fft_first_pass16<-1>(lds + (t % kPfCw) * kPfColStride, v, t / kPfCw);
+        pf_first<LM>(lds + column(t) * F::stride, v, first(t));
         const int cur = item;
         const float cu = cu_next;
         item += (int)gridDim.x;
         __syncthreads();
         if (item < n_items) load(item);
-        const int grp = t / kPfNthr, tid = t % kPfNthr;
+        const int grp = t / NT, tid = t % NT;
         const int p = cur / ngroups, x = cur - p * ngroups;
-        const long jj = column_group((unsigned)x, (unsigned)ngroups) * kPfCw + grp;
+        const long jj = (long)column_group((unsigned)x, (unsigned)ngroups) * CW + grp;
         const long s1 = 2L * (A.pair0 + p), s2 = s1 + 1;
         const bool live = jj < out_n;
         float *r1 = live ? A.out + s1 * A.out_slice_stride + jj * A.out_row_stride : nullptr;
         float *r2 = live && s2 < A.n_slices ? A.out + s2 * A.out_slice_stride + jj * A.out_row_stride : nullptr;
-        float2 *col = lds + grp * kPfColStride;
-        gr_lds_fft<-1, 4, GrFftToLds, true>(col, kPfM, tw, tid, kPfNthr, 16, GrFftToLds(), true);
-        // image row jj: output kk = tid + 256 r (r < 8 covers a window of up to 2048)
-        float wk[8];
-        float2 o[8];
+        float2 *col = lds + grp * F::stride;
+        pf_rest<LM>(col, tw, tid);
+        // image row jj: outputs kk = tid + r M/16, eight at a time
+        auto store = [&](int k0) {
+            float wk[8];
+            float2 o[8], w2[8];
 #pragma unroll
-        for (int r = 0; r < 8; r++) {
-            const int kk = tid + r * kPfNthr, k = off + (kk < out_n ? kk : 0);
-            wk[r] = A.winv[k];
-            o[r] = col[gr_lds_idx(k < m02 ? kPfM - m02 + k : k - m02)];
-        }
-#pragma unroll
-        for (int r = 0; r < 8; r++) {
-            const int kk = tid + r * kPfNthr;
-            if (r1 && kk < out_n) {
-                const float corrn = cu * wk[r];  // grid.cpp:401
-                r1[kk] = corrn * o[r].x;
-                if (r2) r2[kk] = corrn * o[r].y;
+            for (int r = 0; r < 8; r++) {
+                const int kk = k0 + tid + r * NT, i = (kk + wrap) & (M - 1);
+                wk[r] = A.winv[off + min(kk, out_n - 1)];
+                if (F::last2) w2[r] = A.tw[F::tw + (i & (M / 2 - 1))];
+                else o[r] = col[gr_lds_idx(i)];
             }
-        }
+#pragma unroll
+            for (int r = 0; r < 8; r++) {
+                const int kk = k0 + tid + r * NT;
+                if (F::last2) o[r] = gr_last2(col, M, (kk + wrap) & (M - 1), w2[r]);
+                if (r1 && kk < out_n) {
+                    const float corrn = cu * wk[r];  // grid.cpp:401
+                    r1[kk] = corrn * o[r].x;
+                    if (r2) r2[kk] = corrn * o[r].y;
+                }
+            }
+        };
+        store(0);  // all of a window of up to M/2
+        for (int k0 = 8 * NT; k0 < out_n; k0 += 8 * NT) store(k0);
         __syncthreads();  // the columns are free for the next item's first pass
     }
 }
 
-// Persistent row transform for the same geometry (M = 4096, radix 16, window
-// <= 2048): an item is four neighbouring rows b0 .. b0+3 of Ht (one 8-row tile
-// row: one active-tile interval), one per 256-thread group; each thread loads
-// elements j + 256 r of its row (buffer loads: inactive tiles read zeros, no
-// branch), runs the first radix-16 butterfly j from those registers, then
-// issues the next item's loads, which stay in flight through passes 2 and 3
-// (twiddles from LDS).  The epilogue writes Z column-blocked in whole lines:
-// sixteen consecutive lanes store one 128-byte line -- the four rows' four
-// columns of one column block.  Same arithmetic and output values as
-// k_ifft_rows: bitwise.
+// Rows: an item is CW neighbouring rows b0 .. of Ht (row_lo, a multiple of CW,
+// on), one per group of M/16 threads; inactive tiles read zeros.  The epilogue
+// writes Z column-blocked: 4 CW consecutive lanes store the rows' four columns
+// of one column block, CW * 32 contiguous bytes.
+template <int LM>
 __global__ void __launch_bounds__(kPfThreads) k_ifft_rows_pf(RowsArgs A, int n_items) {
+    using F = Pf<LM>;
+    constexpr int M = F::M, CW = F::CW, NT = F::nthr;
     extern __shared__ float2 lds[];
-    float2 *tw = lds + kPfCw * kPfColStride;
-    const int out_n = (int)A.out_n, off = (int)A.out_off, m02 = (int)A.M02;
-    const int groups = (A.row_hi - A.row_lo) / kPfCw;  // items per pair
-    for (int i = (int)threadIdx.x; i < kPfTw; i += kPfThreads) tw[i] = A.tw[i];
+    float2 *tw = lds + CW * F::stride;
+    const int out_n = (int)A.out_n, wrap = (int)A.out_off + M - (int)A.M02;  // as k_ifft_cols_pf
+    const int groups = (A.row_hi - A.row_lo) / CW;  // items per pair
+    for (int i = (int)threadIdx.x; i < F::tw; i += kPfThreads) tw[i] = A.tw[i];
     float2 v[16];
-    // the active-tile interval of an item's tile row (its four rows share
-    // one), fetched an item ahead: waited for only where the loads issued
-    // before it are waited for anyway
-    auto interval = [&](int item) {
+    // the active-tile interval of the thread's row (up to eight rows: the
+    // item's, one scalar load), fetched an item ahead:
+    // waited for only where the loads issued before it are waited for anyway
+    auto interval = [&](int item, int t) {
         const int p = item / groups;
-        return item < n_items ? A.row_tiles[(A.row_lo + (item - p * groups) * kPfCw) >> 3] : make_int2(1, 0);
+        return item < n_items ? A.row_tiles[(A.row_lo + (item - p * groups) * CW + (CW > 8 ? t / NT : 0)) >> 3] : make_int2(1, 0);
     };
     auto load = [&](int item, int2 lh, int t) {  // t: threadIdx.x (an opaque copy inside the loop)
-        const int grp = t / kPfNthr, tid = t % kPfNthr;
-        const int p = item / groups, b0 = A.row_lo + (item - p * groups) * kPfCw;
-        const GrBuf hb = gr_buf(A.ht + ((long)p * kPfM + b0) * kPfM, (unsigned)(kPfCw * kPfM * sizeof(float2)));
+        // a buffer over the active tiles of the wave's row: everything outside
+        // (an index before them wraps to one far past them) reads zeros
+        const int grp = __builtin_amdgcn_readfirstlane(t / NT), tid = t % NT;
+        const int lo = __builtin_amdgcn_readfirstlane(lh.x), hi = __builtin_amdgcn_readfirstlane(lh.y);
+        const int p = item / groups, b = A.row_lo + (item - p * groups) * CW + grp;
+        const GrBuf hb = gr_buf(A.ht + ((long)p * M + b) * M + 8 * lo, (unsigned)(max(hi - lo + 1, 0) * 8 * sizeof(float2)));
+        const unsigned o0 = (unsigned)((tid - 8 * lo) * (int)sizeof(float2));
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int i = tid + r * kPfNthr, tx = i >> 3;
-            const bool in = tx >= lh.x && tx <= lh.y;
-            v[r] = gr_buf_ld2(hb, in ? (unsigned)((grp * kPfM + i) * sizeof(float2)) : kGrBufNone);
-        }
+        for (int r = 0; r < 16; r++) v[r] = gr_buf_ld2(hb, o0 + (unsigned)(r * NT * sizeof(float2)));
     };
     int item = (int)blockIdx.x;
-    if (item < n_items) load(item, interval(item), (int)threadIdx.x);
-    int2 lh_next = interval(item + (int)gridDim.x);
+    if (item < n_items) load(item, interval(item, (int)threadIdx.x), (int)threadIdx.x);
+    int2 lh_next = interval(item + (int)gridDim.x, (int)threadIdx.x);
     __syncthreads();  // twiddles in place
     while (item < n_items) {  // the same trip count in every thread of the block
         int t = (int)threadIdx.x;
         asm volatile("" : "+v"(t));  // indices recomputed per item (as k_ifft_cols_pf)
-        const int grp = t / kPfNthr, tid = t % kPfNthr;
-        float2 *row = lds + grp * kPfColStride;
-        gr_fft_first_pass16<-1>(row, v, tid);
+        const int grp = t / NT, tid = t % NT;
+        float2 *row = lds + grp * F::stride;
+        pf_first<LM>(row, v, tid);
         const int cur = item;
         item += (int)gridDim.x;
         __syncthreads();
         if (item < n_items) {
             load(item, lh_next, t);
-            lh_next = interval(item + (int)gridDim.x);
+            lh_next = interval(item + (int)gridDim.x, t);
         }
-        gr_lds_fft<-1, 4, GrFftToLds, true>(row, kPfM, tw, tid, kPfNthr, 16, GrFftToLds(), true);
-        const int p = cur / groups, b0 = A.row_lo + (cur - p * groups) * kPfCw;
-        float2 *zp = A.z + (long)p * kPfM * gr_z_cols(out_n);
+        pf_rest<LM>(row, tw, tid);
+        const int p = cur / groups, b0 = A.row_lo + (cur - p * groups) * CW;
+        float2 *zp = A.z + (long)p * M * gr_z_cols(out_n);
+        const int n_out = CW * (int)gr_z_cols(out_n);
+        auto store = [&](int L0) {
+            float2 o[8], w2[8];
 #pragma unroll
-        for (int r = 0; r < 8; r++) {  // 4 rows x up to 2048 columns = 8192 outputs
-            const int L = t + r * kPfThreads, blk = L >> 4, rr = (L >> 2) & 3, c = L & 3;
-            const int jj = 4 * blk + c;
-            if (jj < out_n) {
-                const int k = off + jj;
-                zp[((long)blk * kPfM + b0 + rr) * 4 + c] =
-                    lds[rr * kPfColStride + gr_lds_idx(k < m02 ? kPfM - m02 + k : k - m02)];
+            for (int r = 0; r < 8; r++) {
+                const int L = L0 + t + r * kPfThreads, rr = (L >> 2) % CW, jj = 4 * (L / (4 * CW)) + (L & 3);
+                const int i = (jj + wrap) & (M - 1);
+                if (F::last2) w2[r] = A.tw[F::tw + (i & (M / 2 - 1))];
+                else o[r] = lds[rr * F::stride + gr_lds_idx(i)];
             }
-        }
+#pragma unroll
+            for (int r = 0; r < 8; r++) {
+                const int L = L0 + t + r * kPfThreads, blk = L / (4 * CW), rr = (L >> 2) % CW, c = L & 3;
+                const int jj = 4 * blk + c;
+                if (jj < out_n) {
+                    if (F::last2) o[r] = gr_last2(lds + rr * F::stride, M, (jj + wrap) & (M - 1), w2[r]);
+                    zp[((long)blk * M + b0 + rr) * 4 + c] = o[r];
+                }
+            }
+        };
+        store(0);  // all of a window of up to M/2
+        for (int L0 = 8 * kPfThreads; L0 < n_out; L0 += 8 * kPfThreads) store(L0);
         __syncthreads();  // the rows are free for the next item's first pass
     }
 }
@@ -470,8 +575,49 @@ int gr_max_lds_per_block() {
                     device_attr(hipDeviceAttributeMaxSharedMemoryPerBlock, plain));
 }
 
-// The persistent transforms need the whole 160 KiB of a CU's LDS.
-static bool pf_fits() { return gr_cu_count() > 0 && (size_t)gr_max_lds_per_block() >= kPfLds; }
+// Whether a launch of n_items items takes the persistent form: with fewer than
+// two per CU there is nothing to overlap and the one-shot kernels' smaller
+// workgroups fill the chip better.
+static bool pf_takes(long M, int radix, long n_items) {
+    const int cus = gr_cu_count();
+    return M >= 1024 && M <= 8192 && radix == 16 && cus > 0 && n_items >= 2L * cus &&
+           (size_t)gr_max_lds_per_block() >= std::max(Pf<12>::lds, Pf<13>::lds);
+}
+
+template <template <int> class Launch, class... Args>
+static hipError_t pf_launch(long M, Args... args) {
+    switch (M) {
+    case 1024: return Launch<10>::go(args...);
+    case 2048: return Launch<11>::go(args...);
+    case 4096: return Launch<12>::go(args...);
+    default: return Launch<13>::go(args...);
+    }
+}
+template <int LM>
+struct PfRows {
+    static hipError_t go(RowsArgs A, int pairs, hipStream_t s) {
+        const int n_items = (A.row_hi - A.row_lo) / Pf<LM>::CW * pairs;
+        const hipError_t e = gr_allow_lds(k_ifft_rows_pf<LM>, Pf<LM>::lds);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(k_ifft_rows_pf<LM>, dim3(std::min(n_items, gr_cu_count())), dim3(kPfThreads), Pf<LM>::lds, s,
+                           A, n_items);
+        return hipGetLastError();
+    }
+};
+template <int LM>
+struct PfCols {
+    static hipError_t go(ColsArgs A, int pairs, hipStream_t s) {
+        const int n_items = (int)((A.out_n + Pf<LM>::CW - 1) / Pf<LM>::CW) * pairs;
+        auto launch = [&](auto kernel) {
+            const hipError_t e = gr_allow_lds(kernel, Pf<LM>::lds);
+            if (e != hipSuccess) return e;
+            hipLaunchKernelGGL(kernel, dim3(std::min(n_items, gr_cu_count())), dim3(kPfThreads), Pf<LM>::lds, s, A,
+                               n_items);
+            return hipGetLastError();
+        };
+        return A.row_hi - A.row_lo == Pf<LM>::M ? launch(k_ifft_cols_pf<LM, true>) : launch(k_ifft_cols_pf<LM, false>);
+    }
+};
 
 hipError_t gr_launch_row_tiles(const GrGeom &g, int2 *out, hipStream_t s) {
     const int ntr = (int)(g.M >> 3);
@@ -489,13 +635,13 @@ hipError_t gr_launch_ifft_rows(const GrGeom &g, const GrDevTables &t, const floa
     RowsArgs A{ht, z, t.tw_grid, t.row_tiles, (int)g.M, g.fft_radix, g.M02, g.out_off, g.out_n,
                t.row_lo, t.row_hi};
     const int nthr = gr_fft_threads(g.M);
-    if (g.M == kPfM && nthr == kPfNthr && g.fft_radix == 16 && g.out_n <= 8 * kPfNthr && pf_fits()) {
-        const int n_items = (t.row_hi - t.row_lo) / kPfCw * pairs;
-        const int nblk = std::min(n_items, gr_cu_count());
-        hipError_t e = gr_allow_lds(k_ifft_rows_pf, kPfLds);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_ifft_rows_pf, dim3(nblk), dim3(kPfThreads), kPfLds, s, A, n_items);
-        return hipGetLastError();
+    const long pf_cw = 16384 / g.M;
+    if (g.M <= 16384) {
+        RowsArgs B = A;  // whole items: the rows added hold no active tile and read as zeros
+        B.row_lo = (int)(t.row_lo / std::max(pf_cw, 1L) * pf_cw);
+        B.row_hi = (int)((t.row_hi + pf_cw - 1) / std::max(pf_cw, 1L) * pf_cw);
+        if (pf_takes(g.M, g.fft_radix, (B.row_hi - B.row_lo) / std::max(pf_cw, 1L) * pairs))
+            return pf_launch<PfRows>(g.M, B, pairs, s);
     }
     int cw = kRowsPerBlock;  // rows side by side: a power of two dividing M, within 1024 threads and the LDS
     while (cw > 1 && ((long)cw * nthr > 1024 || (long)cw * g.M * 8 > 163840 || g.M % cw)) cw /= 2;
@@ -572,15 +718,10 @@ hipError_t gr_launch_ifft_cols(const GrGeom &g, const GrDevTables &t, const floa
     A.row_hi = t.row_hi;
     const int nthr = gr_fft_threads(g.M);
     const bool side = cols_side_by_side(g.M, A.cw);
-    if (side && A.cw == kPfCw && g.M == kPfM && nthr == kPfNthr && g.fft_radix == 16 && g.out_n <= 8 * kPfNthr &&
-        pf_fits()) {
-        const int n_items = (int)((g.out_n + kPfCw - 1) / kPfCw) * pairs;
-        const int nblk = std::min(n_items, gr_cu_count());
-        hipError_t e = gr_allow_lds(k_ifft_cols_pf, kPfLds);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_ifft_cols_pf, dim3(nblk), dim3(kPfThreads), kPfLds, s, A, n_items);
-        return hipGetLastError();
-    }
+    // at M = 4096 the persistent form is the width of four columns, too
+    if ((cols == 0 || (g.M == 4096 && A.cw == 4)) &&
+        pf_takes(g.M, g.fft_radix, (g.out_n + 16384 / g.M - 1) / (16384 / g.M) * pairs))
+        return pf_launch<PfCols>(g.M, A, pairs, s);
     const dim3 grid((unsigned)((g.out_n + A.cw - 1) / A.cw), pairs), block(side ? A.cw * nthr : nthr);
     const size_t lds = sizeof(float2) * A.cw * gr_lds_len(g.M);
 #define GR_COLS_K(MB, CW)                                                                \

@@ -450,3 +450,41 @@ def test_exec_pairs_host_rows_match_device_path():
     again = p.exec_pairs(sino, out=np.full_like(host, np.nan))  # staging reused
     assert np.array_equal(again, dev)
     p.close()
+
+
+# The persistent transforms at every size they take, against the one-shot
+# kernels (a launch of one pair has too few items for the persistent form, and
+# an explicit column width asks for the one-shot one): whole images (windows of
+# up to M - 1 columns: two rounds of the epilogue), ragged windows (a last column
+# group of one), grids with empty rows (an item of rows partly past them)
+PF_CASES = {
+    "1024-full": dict(n_ang=24, n_det=1000, center=500.3), "1024-ragged": dict(n_ang=20, n_det=300, center=150.0, pad="half", crop=(130, 601)),
+    "2048-full": dict(n_ang=20, n_det=1500, center=750.2), "2048-ragged": dict(n_ang=20, n_det=600, center=300.0, pad="half", crop=(700, 605)),
+    "4096-empty": dict(n_ang=16, n_det=1100, center=550.0, pad="half", crop=(1400, 1201)),
+    "8192-empty": dict(n_ang=12, n_det=2200, center=1100.0, pad="half", crop=(2500, 2049)),
+    "8192-wide": dict(n_ang=12, n_det=8100, center=4050.0, crop=(1000, 4111)),
+}
+
+
+@pytest.mark.parametrize("name", sorted(PF_CASES))
+def test_persistent_transforms_are_bitwise_the_one_shot_ones(name):
+    case = PF_CASES[name]
+    M = gr.Plan(**case, max_pairs=1).info["M"]
+    ns = {1024: 31, 2048: 17, 4096: 5, 8192: 3}[M]
+    sino = torch.from_numpy(np.random.default_rng(M).standard_normal((ns, case["n_ang"], case["n_det"])).astype(np.float32)).cuda()
+    out = gr.Plan(**case, max_pairs=(ns + 1) // 2, grid_op="off").recon(sino)
+    for s in (0, ns - 1):  # the last slice of an odd count is paired with zeros, as alone
+        p = gr.Plan(**case, max_pairs=1, grid_op="off")
+        p.set_cols_per_block(1)
+        one = p.recon(sino[s & ~1:(s & ~1) + 2])
+        torch.cuda.synchronize()
+        assert torch.equal(out[s], one[s & 1])
+    g = O.Geometry(**{k: v for k, v in case.items() if k not in ("pad", "crop")})
+    a, b = sino[0].cpu().numpy(), sino[1].cpu().numpy()
+    if case.get("pad") == "half":
+        g, a, b = g.padded(), O.pad_half(a), O.pad_half(b)
+    r1, _ = O.recon_f32(g, a, b)
+    M0 = r1.shape[0]
+    off, n = case.get("crop", (0, M0))
+    d = disk_mask(M0, 0.5)[off:off + n, off:off + n]
+    assert O.rel_l2(out[0].cpu().numpy()[d], r1[off:off + n, off:off + n][d]) < DISK_TOL

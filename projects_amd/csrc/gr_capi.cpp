@@ -67,6 +67,30 @@ int dev_alloc(gr_plan *pl, T **dst, size_t n) {
     return GR_OK;
 }
 
+// The small tables of a plan in one allocation and one copy: an allocation
+// and a blocking copy each cost plan creation tens of microseconds.  add()
+// notes a table (src null: space only) and commit() sets every pointer, on
+// 256-byte boundaries inside pl->d_small.
+struct TablePack {
+    std::vector<char> host;
+    std::vector<std::pair<void **, size_t>> at;
+
+    template <typename T>
+    void add(T **dst, const T *src, size_t n) {
+        const size_t off = host.size();
+        host.resize((off + sizeof(T) * n + 255) / 256 * 256);
+        if (src) memcpy(host.data() + off, src, sizeof(T) * n);
+        at.push_back({(void **)dst, off});
+    }
+
+    int commit(gr_plan *pl) {
+        const int rc = dev_upload(pl, &pl->d_small, host.data(), host.size());
+        if (rc) return rc;
+        for (const auto &a : at) *a.first = pl->d_small + a.second;
+        return GR_OK;
+    }
+};
+
 // Tables that depend only on a transform size -- twiddles and the gridding
 // tile order -- are built once per (device, kind, size) and shared by every
 // plan that needs them, reference-counted: a batch of hundreds of datasets
@@ -348,56 +372,52 @@ int build_gop(gr_plan *pl, hipStream_t s, bool required, size_t max_bytes) {
 // Whole, the four tiles at the centre walk every angle in one wave each and
 // the launch waits for them: one pair of 1500 x 2048 3.12 -> 0.87 ms split,
 // eight pairs 3.70 -> 1.80, one of 180 x 256 0.37 -> 0.08.
-// Two small kernels and two waits on stream s, at plan creation.
+// Two small kernels and one wait of their own on stream s, at plan creation.
 constexpr int kSplitSlots = 256;
 constexpr unsigned kSplitLines = 48;
 
-int build_split(gr_plan *pl, hipStream_t s) {
-    if (pl->prm.accum != GR_ACCUM_COMPENSATED) return GR_OK;
+int split_slots_of(const gr_plan *pl) { return std::min(kSplitSlots, pl->sector_len); }
+
+// Enqueue the count and its copy back; build_split reads it after a wait.
+hipError_t count_split(gr_plan *pl, std::vector<unsigned> &lines, hipStream_t s) {
+    if (pl->prm.accum != GR_ACCUM_COMPENSATED) return hipSuccess;
+    const int slots = split_slots_of(pl);
+    lines.resize((size_t)kGridSectors * slots);
+    hipError_t e = gr_launch_split_lines(pl->g, pl->tables(), pl->prm.n_ang, pl->prm.ltbl, slots, pl->d_slines, s);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(lines.data(), pl->d_slines, sizeof(unsigned) * lines.size(), hipMemcpyDeviceToHost, s);
+    return e;
+}
+
+int build_split(gr_plan *pl, const std::vector<unsigned> &lines, hipStream_t s) {
     const GrGeom &g = pl->g;
-    const int slots = std::min(kSplitSlots, pl->sector_len);
-    const GrDevTables t = pl->tables();
-    const int nw = kGridSectors * slots;
-    std::vector<unsigned> lines(nw), first(nw);
-    unsigned *d_w = nullptr;
-    if (hipMalloc((void **)&d_w, sizeof(unsigned) * nw) != hipSuccess) return fail(GR_ENOMEM, "device allocation failed");
-    auto run = [&]() -> int {
-        GR_HIP(gr_launch_split_lines(g, t, pl->prm.n_ang, pl->prm.ltbl, slots, d_w, s));
-        GR_HIP(hipMemcpyAsync(lines.data(), d_w, sizeof(unsigned) * nw, hipMemcpyDeviceToHost, s));
-        GR_HIP(hipStreamSynchronize(s));
-        int n_split = 0;
-        for (int w = 0; w < nw; w++)
-            if (lines[w] > kSplitLines) n_split = std::max(n_split, w % slots + 1);
-        if (n_split == 0) return GR_OK;
-        // nearest to the centre first, across the sectors
-        std::vector<uint4> meta;
-        unsigned long long items = 0;
-        for (int slot = 0; slot < n_split; slot++)
-            for (int sx = 0; sx < kGridSectors; sx++) {
-                const int w = sx * slots + slot;
-                const unsigned n = (lines[w] + kGridMergeLines - 1) / kGridMergeLines;
-                first[w] = (unsigned)items;
-                meta.push_back(make_uint4((unsigned)(sx * pl->sector_len + slot), first[w], n, 0u));
-                items += n;
-            }
-        if (items * 64 > (unsigned long long)g.M * g.out_n) return GR_OK;
-        int rc = dev_alloc(pl, &pl->d_sitems, (size_t)items);
-        if (rc == GR_OK) rc = dev_upload(pl, &pl->d_smeta, meta.data(), meta.size());
-        if (rc) return rc;
-        std::vector<unsigned> f2((size_t)kGridSectors * n_split);
-        for (int sx = 0; sx < kGridSectors; sx++)
-            for (int slot = 0; slot < n_split; slot++) f2[(size_t)sx * n_split + slot] = first[sx * slots + slot];
-        GR_HIP(hipMemcpyAsync(d_w, f2.data(), sizeof(unsigned) * f2.size(), hipMemcpyHostToDevice, s));
-        GR_HIP(gr_launch_split_items(g, t, pl->prm.n_ang, pl->prm.ltbl, n_split, d_w, pl->d_sitems, s));
-        GR_HIP(hipStreamSynchronize(s));
-        pl->n_sitems = (int)items;
-        pl->n_smeta = (int)meta.size();
-        pl->split_slots = n_split;
-        return GR_OK;
-    };
-    const int rc = run();
-    (void)hipFree(d_w);
-    return rc;
+    const int slots = split_slots_of(pl), nw = (int)lines.size();
+    int n_split = 0;
+    for (int w = 0; w < nw; w++)
+        if (lines[w] > kSplitLines) n_split = std::max(n_split, w % slots + 1);
+    if (n_split == 0) return GR_OK;
+    // nearest to the centre first, across the sectors
+    std::vector<uint4> meta;
+    std::vector<unsigned> first((size_t)kGridSectors * n_split);
+    unsigned long long items = 0;
+    for (int slot = 0; slot < n_split; slot++)
+        for (int sx = 0; sx < kGridSectors; sx++) {
+            const unsigned n = (lines[sx * slots + slot] + kGridMergeLines - 1) / kGridMergeLines;
+            first[(size_t)sx * n_split + slot] = (unsigned)items;
+            meta.push_back(make_uint4((unsigned)(sx * pl->sector_len + slot), (unsigned)items, n, 0u));
+            items += n;
+        }
+    if (items * 64 > (unsigned long long)g.M * g.out_n) return GR_OK;
+    int rc = dev_alloc(pl, &pl->d_sitems, (size_t)items);
+    if (rc == GR_OK) rc = dev_upload(pl, &pl->d_smeta, meta.data(), meta.size());
+    if (rc) return rc;
+    GR_HIP(hipMemcpyAsync(pl->d_slines, first.data(), sizeof(unsigned) * first.size(), hipMemcpyHostToDevice, s));
+    GR_HIP(gr_launch_split_items(g, pl->tables(), pl->prm.n_ang, pl->prm.ltbl, n_split, pl->d_slines, pl->d_sitems, s));
+    GR_HIP(hipStreamSynchronize(s));
+    pl->n_sitems = (int)items;
+    pl->n_smeta = (int)meta.size();
+    pl->split_slots = n_split;
+    return GR_OK;
 }
 
 // The gridding tile list: kGridSectors sectors of the polar angle of the
@@ -453,10 +473,9 @@ void free_staging(gr_plan *pl) {
 void free_plan(gr_plan *pl) {
     if (!pl) return;
     free_staging(pl);
-    void *ptrs[] = {pl->d_cose, pl->d_sine, pl->d_roi, pl->d_wtbl, pl->d_winv, pl->d_filphase, pl->d_akey,
-                    pl->d_aord, pl->d_ang, pl->d_gop, pl->d_gop_n, pl->d_gop_off, pl->d_dwtbl, pl->d_rowtiles,
-                    pl->d_sop_tile, pl->d_sop_ch, pl->d_sop_keys, pl->d_sop_ent, pl->d_hmeta, pl->d_hseg,
-                    pl->d_hsplit, pl->d_hitems, pl->d_sweep, pl->d_sitems, pl->d_smeta};
+    void *ptrs[] = {pl->d_small, pl->d_gop, pl->d_gop_n, pl->d_gop_off, pl->d_sop_tile, pl->d_sop_ch, pl->d_sop_keys,
+                    pl->d_sop_ent, pl->d_hmeta, pl->d_hseg, pl->d_hsplit, pl->d_hitems, pl->d_sweep, pl->d_sitems,
+                    pl->d_smeta};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     shared_release(pl->d_tw_row);
@@ -676,29 +695,16 @@ int gr_plan_create_impl(const gr_params *params, gr_plan **plan_out, bool alloc_
     std::vector<float> dwtbl(params->interp ? params->ltbl + 1 : 0);
     gr_host_tables(&pl->prm, g, sine.data(), cose.data(), filphase.data(), wtbl.data(), winv.data(), roi.data(),
                    params->interp ? dwtbl.data() : nullptr);
-    CK(dev_upload(pl, &pl->d_sine, sine.data(), n_ang));
-    CK(dev_upload(pl, &pl->d_cose, cose.data(), n_ang));
-    CK(dev_upload(pl, &pl->d_roi, roi.data(), n_ang));
-    CK(dev_upload(pl, &pl->d_filphase, (const float2 *)filphase.data(), g.half));
-    CK(dev_upload(pl, &pl->d_wtbl, wtbl.data(), wtbl.size()));
-    CK(dev_upload(pl, &pl->d_winv, winv.data(), winv.size()));
-    if (params->interp) CK(dev_upload(pl, &pl->d_dwtbl, dwtbl.data(), dwtbl.size()));
-    if (params->tables == GR_TABLES_FP64) {
-        hipStream_t ts;
-        CK(plan_stream(pl, &ts));
-        hipError_t e = gr_launch_tables_fp64(g, &pl->prm, pl->d_filphase, pl->d_wtbl, pl->d_winv, ts);
-        if (e == hipSuccess) e = hipStreamSynchronize(ts);
-        if (e != hipSuccess) {
-            free_plan(pl);
-            return hip_fail(e, "FP64 tables");
-        }
-    }
-    // twiddles (shared per size)
-    CK(shared_table(params->device, kTwPlus, g.pdim, [&] { return pass_twiddles(g.pdim, +1); }, &pl->d_tw_row, nullptr));
-    CK(shared_table(params->device, kTwMinus, g.M, [&] { return pass_twiddles(g.M, -1); }, &pl->d_tw_grid, nullptr));
-    pl->dev_bytes += sizeof(float2) * (gr_twp_len(g.pdim, 16) + gr_twp_len(g.pdim, 4) + gr_twp_len(g.M, 16) +
-                                       gr_twp_len(g.M, 4));
+    TablePack pack;
+    pack.add(&pl->d_sine, sine.data(), n_ang);
+    pack.add(&pl->d_cose, cose.data(), n_ang);
+    pack.add(&pl->d_roi, roi.data(), n_ang);
+    pack.add(&pl->d_filphase, (const float2 *)filphase.data(), g.half);
+    pack.add(&pl->d_wtbl, wtbl.data(), wtbl.size());
+    pack.add(&pl->d_winv, winv.data(), winv.size());
+    if (params->interp) pack.add(&pl->d_dwtbl, dwtbl.data(), dwtbl.size());
     // angle keys: direction of each sample line, atan2(SINE, COSE) mod pi, sorted
+    const int ts = gr_grid_tile_size(), nt = (int)((g.M + ts - 1) / ts);
     {
         std::vector<double> key(n_ang);
         for (int n = 0; n < n_ang; n++) {
@@ -714,23 +720,41 @@ int gr_plan_create_impl(const gr_params *params, gr_plan **plan_out, bool alloc_
         for (int i = 0; i < n_ang; i++) akey[i] = (float)key[ord[i]];
         // keep the float keys sorted after rounding
         for (int i = 1; i < n_ang; i++) akey[i] = std::max(akey[i], akey[i - 1]);
-        CK(dev_upload(pl, &pl->d_akey, akey.data(), n_ang));
-        CK(dev_upload(pl, &pl->d_aord, ord.data(), n_ang));
+        pack.add(&pl->d_akey, akey.data(), n_ang);
+        pack.add(&pl->d_aord, ord.data(), n_ang);
         std::vector<float4> ang(n_ang);
         for (int i = 0; i < n_ang; i++) {
             const float c = cose[ord[i]], sn = sine[ord[i]];
             ang[i] = make_float4(c, sn, fabsf(c) > 1e-6f ? 1.0f / c : 0.0f, fabsf(sn) > 1e-6f ? 1.0f / sn : 0.0f);
         }
-        CK(dev_upload(pl, &pl->d_ang, ang.data(), n_ang));
+        pack.add(&pl->d_ang, ang.data(), n_ang);
     }
+    // space for the row transform's active-tile interval of every tile row and
+    // for the line counts that the centre tiles are split by
+    pack.add(&pl->d_rowtiles, (const int2 *)nullptr, nt);
+    pack.add(&pl->d_slines, (const unsigned *)nullptr, kGridSectors * kSplitSlots);
+    CK(pack.commit(pl));
+    if (params->tables == GR_TABLES_FP64) {
+        hipStream_t ts;
+        CK(plan_stream(pl, &ts));
+        hipError_t e = gr_launch_tables_fp64(g, &pl->prm, pl->d_filphase, pl->d_wtbl, pl->d_winv, ts);
+        if (e == hipSuccess) e = hipStreamSynchronize(ts);
+        if (e != hipSuccess) {
+            free_plan(pl);
+            return hip_fail(e, "FP64 tables");
+        }
+    }
+    // twiddles (shared per size)
+    CK(shared_table(params->device, kTwPlus, g.pdim, [&] { return pass_twiddles(g.pdim, +1); }, &pl->d_tw_row, nullptr));
+    CK(shared_table(params->device, kTwMinus, g.M, [&] { return pass_twiddles(g.M, -1); }, &pl->d_tw_grid, nullptr));
+    pl->dev_bytes += sizeof(float2) * (gr_twp_len(g.pdim, 16) + gr_twp_len(g.pdim, 4) + gr_twp_len(g.M, 16) +
+                                       gr_twp_len(g.M, 4));
     // tiles of the gridding kernel over the M x M grid (shared per size):
     // eight sectors of the polar angle of the tile centre, each listed nearest
     // to the centre first and padded to a common length with kNoTile; the
     // kernels give sector x to the workgroups that the hardware places on
     // XCD x, so each XCD's L2 holds the samples of its own sector
     {
-        const int ts = gr_grid_tile_size();
-        const int nt = (int)((g.M + ts - 1) / ts);
         if ((long)nt * nt >= (1L << 24)) CK(fail(GR_EINVAL, "grid too large for the tile list"));
         int slots = 0;
         CK(shared_table(params->device, kTiles, g.M, [&] { return sector_tiles(nt, ts, g.M); }, &pl->d_tiles,
@@ -738,12 +762,12 @@ int gr_plan_create_impl(const gr_params *params, gr_plan **plan_out, bool alloc_
         pl->sector_len = slots / kGridSectors;
         pl->ntiles = slots;
         pl->dev_bytes += sizeof(unsigned) * (size_t)pl->ntiles;
-        // the row transform's active-tile interval of every tile row
-        CK(dev_alloc(pl, &pl->d_rowtiles, (size_t)nt));
         hipStream_t rs;
         CK(plan_stream(pl, &rs));
         std::vector<int2> rt(nt);
+        std::vector<unsigned> lines;
         hipError_t e = gr_launch_row_tiles(g, pl->d_rowtiles, rs);
+        if (e == hipSuccess) e = count_split(pl, lines, rs);
         if (e == hipSuccess) e = hipMemcpyAsync(rt.data(), pl->d_rowtiles, sizeof(int2) * nt, hipMemcpyDeviceToHost, rs);
         if (e == hipSuccess) e = hipStreamSynchronize(rs);
         // the disk of samples leaves the first and last rows of the grid empty
@@ -758,7 +782,7 @@ int gr_plan_create_impl(const gr_params *params, gr_plan **plan_out, bool alloc_
             free_plan(pl);
             return hip_fail(e, "row tile intervals");
         }
-        CK(build_split(pl, rs));
+        CK(build_split(pl, lines, rs));
     }
     // workspace
     const size_t spec_pp = (size_t)n_ang * g.half, ht_pp = (size_t)g.M * g.M, z_pp = (size_t)g.M * gr_z_cols(g.out_n);

@@ -12,6 +12,8 @@ struct gr_plan {
     std::vector<float> angles;  // copy of the caller's list (geom 0)
     hipStream_t stream = nullptr;
     // device tables
+    // the small tables share one allocation, d_small
+    char *d_small = nullptr;
     float *d_cose = nullptr, *d_sine = nullptr, *d_roi = nullptr, *d_wtbl = nullptr, *d_winv = nullptr;
     float *d_dwtbl = nullptr;  // INTERP only
     float2 *d_filphase = nullptr, *d_tw_row = nullptr, *d_tw_grid = nullptr;
@@ -46,6 +48,7 @@ struct gr_plan {
     int n_hitems = 0, n_split = 0, split_groups = 0;
     // the centre tiles' merge groups for the geometry kernel (GrDevTables::sitems)
     uint4 *d_sitems = nullptr, *d_smeta = nullptr;
+    unsigned *d_slines = nullptr;  // scratch of the split (in d_small)
     int n_sitems = 0, n_smeta = 0, split_slots = 0;
     long pairs_done = 0;  // pairs reconstructed so far (the automatic build's trigger)
     // workspace for max_pairs pairs: owned, or a region bound by a queue

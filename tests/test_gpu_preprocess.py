@@ -126,3 +126,26 @@ def test_ring_correction_sizes(ns, n_ang, n_det, row, zeros):
     for s in range(0, ns, max(1, ns // 3)):
         assert O.rel_l2(out[s], O.ring_correct(sino[s], 0.8, iterations=6)) < 1e-5, s
     assert torch.isnan(buf[:, :, n_det:]).all()
+
+
+@pytest.mark.parametrize("n_det,pad,ns", [(7, "half", 1), (65, "none", 3), (129, "half", 2), (1500, "half", 17),
+                                          (4097, "none", 5)])
+def test_raw_rows_at_odd_widths(n_det, pad, ns):
+    """Detector counts of one partial and several whole rounds of cells per
+    thread, an odd last slice, and a shift past both ends: bitwise the images
+    of the preprocessed rows."""
+    n_ang = 6
+    rng = np.random.default_rng(n_det)
+    raw = rng.integers(0, 65536, (ns, n_ang, n_det), dtype=np.uint16)
+    dark = rng.uniform(90, 110, (ns, n_det)).astype(np.float32)
+    w1 = rng.uniform(30000, 40000, (ns, n_det)).astype(np.float32)
+    w2 = rng.uniform(30000, 40000, (ns, n_det)).astype(np.float32)
+    plan = gr.Plan(n_ang=n_ang, n_det=n_det, center=n_det / 2.0, pad=pad)
+    g = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    for xoff in (-3.4, float(n_det + 2)):
+        out = plan.recon_raw(g(raw), g(dark), g(w1), g(w2), mode="flatdark", xoffset=xoff)
+        rows = np.stack([O.preprocess(1, raw[s], dark[s], w1[s], w2[s], xoffset=xoff) for s in range(ns)])
+        ref = plan.recon(g(rows))
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)
+    plan.close()

@@ -1066,8 +1066,10 @@ __device__ __forceinline__ void grid_sop_light(const GridArgs &A, const GopArgs 
 }
 
 // One tile (seg < 0) or one segment of a cut heavy tile for the P pairs of a
-// group from the streamed entries, software-pipelined: entries are loaded
-// four rows ahead, the samples of row k+1 are gathered while row k is added.
+// group from the streamed entries, software-pipelined: with P = 8 entries are
+// loaded four rows ahead and the samples of row k+1 are gathered while row k is
+// added; with fewer pairs a batch of rows is gathered while the next batch's
+// entries load.
 // A whole tile runs its rows to the end, merging into its sums, and stores
 // its cells.  A segment runs each lane's rows between its marks at the
 // segment's ends (segments start at merge points, so they hold whole merge
@@ -1131,21 +1133,44 @@ __device__ __forceinline__ void grid_op_tile(const GridArgs &A, const GopArgs &O
                 m++;
             }
         };
-        uint2 t0 = row(0), t1 = row(1), t2 = row(2), t3 = row(3);
-        float2 va[P], vb[P];
-        gop_gather<P>(t0, base1, base2, va);
-        for (unsigned k = 0; k < n; k += 2) {
-            // rows k (t0, samples in va) and k+1 (t1); t2, t3 hold rows k+2, k+3
-            const uint2 c1 = k + 1 < n ? t1 : zero;
-            gop_gather<P>(c1, base1, base2, vb);
-            const uint2 c0 = t0;
-            t0 = t2;
-            t2 = row(k + 4);
-            consume(c0, va);
-            gop_gather<P>(k + 2 < n ? t0 : zero, base1, base2, va);
-            t1 = t3;
-            t3 = row(k + 5);
-            consume(c1, vb);
+        if constexpr (P < 8) {
+            // few pairs leave registers for several rows at once, and a launch
+            // of few tiles waits for its longest chain of round trips: one
+            // pair of 180 x 256 33.1 -> 27.8 us of gridding, two 36.6 -> 33.2,
+            // four 41.7 -> 38.9 (one of 1500 x 2048 390 -> 389; sixteen rows
+            // for one pair 393)
+            constexpr int B = P == 1 ? 8 : 4;
+            uint2 t[B], tn[B];
+            float2 v[B][P];
+#pragma unroll
+            for (int i = 0; i < B; i++) t[i] = row(i);
+            for (unsigned k = 0; k < n; k += B) {
+#pragma unroll
+                for (int i = 0; i < B; i++) gop_gather<P>(t[i], base1, base2, v[i]);
+#pragma unroll
+                for (int i = 0; i < B; i++) tn[i] = row(k + B + i);
+#pragma unroll
+                for (int i = 0; i < B; i++) consume(t[i], v[i]);
+#pragma unroll
+                for (int i = 0; i < B; i++) t[i] = tn[i];
+            }
+        } else {
+            uint2 t0 = row(0), t1 = row(1), t2 = row(2), t3 = row(3);
+            float2 va[P], vb[P];
+            gop_gather<P>(t0, base1, base2, va);
+            for (unsigned k = 0; k < n; k += 2) {
+                // rows k (t0, samples in va) and k+1 (t1); t2, t3 hold rows k+2, k+3
+                const uint2 c1 = k + 1 < n ? t1 : zero;
+                gop_gather<P>(c1, base1, base2, vb);
+                const uint2 c0 = t0;
+                t0 = t2;
+                t2 = row(k + 4);
+                consume(c0, va);
+                gop_gather<P>(k + 2 < n ? t0 : zero, base1, base2, va);
+                t1 = t3;
+                t3 = row(k + 5);
+                consume(c1, vb);
+            }
         }
     }
     if (seg < 0) store_cells<ACCUM, P>(A, pair0, nvalid, a, b, acc);

@@ -64,7 +64,7 @@ struct GrDevTables {
     // entries, taps per tile, first entry of each tile
     const uint2 *gop = nullptr;
     const unsigned *gop_n = nullptr, *gop_off = nullptr;
-    int gop_heavy = 0;  // leading slots of every sector gridded one pair per wave
+    int gop_heavy = 0;  // leading slots of every sector on the heavy path
     // the heavy work: items {tile slot, segment}, the centre-most slots first;
     // heavy tiles cut into segments of kGopSegGroups merge groups, gridded by
     // one wave per (segment, pair) into partials that k_gop_merge sums:

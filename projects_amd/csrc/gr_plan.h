@@ -34,7 +34,7 @@ struct gr_plan {
     double gop_build_ms = 0.0;
     int gop_state = 0;
     int gop_aligned_tiles = 0;  // tiles in the aligned layout
-    int gop_heavy = 0;          // leading slots of each sector gridded one pair per wave
+    int gop_heavy = 0;          // leading slots of each sector on the heavy path
     // its staged form for the other tiles (null when the plan has none)
     uint4 *d_sop_tile = nullptr;
     uint2 *d_sop_ch = nullptr;

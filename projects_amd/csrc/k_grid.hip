@@ -848,7 +848,7 @@ __global__ void __launch_bounds__(256) k_sop_build(GridArgs A, int n_heavy, uint
 struct GopArgs {
     const uint2 *gop;
     const unsigned *tile_n, *tile_off;
-    int n_heavy;  // slots [0, n_heavy) of every sector take the one-pair-per-wave path
+    int n_heavy;  // slots [0, n_heavy) of every sector take the heavy path
     // the staged operator of the other slots (null: they stream the entries)
     const uint4 *sop_tile;
     const uint2 *sop_ch;
@@ -904,13 +904,12 @@ __device__ __forceinline__ void gop_consume(uint2 t, const float2 (&v)[P], float
 
 constexpr int kHeavyBatch = 16;  // rows loaded at once on the one-pair path
 
-// The one-pair-per-wave path for the tiles near the centre of the grid whose
-// cells take hundreds to thousands of taps: the P pairs of a group go to P
+// The one-pair-per-wave path, for compensated sums whose heavy tiles are not
+// cut (partials that the scratch does not hold): the P pairs of a group go to P
 // wavefronts, which stream the tile's rows kHeavyBatch at a time (the batch's
 // sample loads, then the next batch's entry loads, then the batch's adds), so
 // each wave has many loads in flight instead of a chain of dependent ones.
 // Per cell and pair the float operations are those of the wide path.
-template <int ACCUM>
 __device__ __forceinline__ void grid_op_heavy(const GridArgs &A, const GopArgs &O, int ti, int pair, int lane) {
     const unsigned tt = A.tiles[ti];
     const int tx = (int)(tt & 0xffffu), ty = (int)(tt >> 16);
@@ -925,7 +924,7 @@ __device__ __forceinline__ void grid_op_heavy(const GridArgs &A, const GopArgs &
         // a slot no sample reaches: no entry may be read (n - 1 would wrap and
         // the clamped prefetch below would run past the tile's entries); the
         // cells are still stored as zeros, which the row transform reads
-        store_cells<ACCUM, 1>(A, pair, 1, a, b, acc);
+        store_cells<GR_ACCUM_COMPENSATED, 1>(A, pair, 1, a, b, acc);
         return;
     }
     auto entry = [&](unsigned k) {
@@ -946,12 +945,90 @@ __device__ __forceinline__ void grid_op_heavy(const GridArgs &A, const GopArgs &
 #pragma unroll
         for (int i = 0; i < kHeavyBatch; i++) tn[i] = entry(k0 + kHeavyBatch + i);
 #pragma unroll
-        for (int i = 0; i < kHeavyBatch; i++) gop_consume<ACCUM, 1>(t[i], v[i], acc, part);
+        for (int i = 0; i < kHeavyBatch; i++) gop_consume<GR_ACCUM_COMPENSATED, 1>(t[i], v[i], acc, part);
 #pragma unroll
         for (int i = 0; i < kHeavyBatch; i++) t[i] = tn[i];
     }
-    store_cells<ACCUM, 1>(A, pair, 1, a, b, acc);
+    store_cells<GR_ACCUM_COMPENSATED, 1>(A, pair, 1, a, b, acc);
 }
+
+constexpr int kHeavyPlainBatch = 12;  // sixteen spill; eight cost 1% of the whole call
+
+// A heavy tile of plain sums, one pair per workgroup.  Plain sums are one
+// chain of adds per cell in tap order, so a tile's rows cannot be cut; the
+// chain itself is short, what a wave waits for is one memory round trip per
+// batch of rows (170 of them at the centre of 451 angles).  So the four waves
+// gather kHeavyPlainBatch rows each and put the products into LDS, and the first
+// adds all of them in order while the next ones arrive: the same products and
+// the same adds.  8 pairs of 451 x 777: k_grid_op<1, 8> 333 us with a pair per
+// wave, 146 this way.
+__device__ __forceinline__ void grid_op_heavy_plain(const GridArgs &A, const GopArgs &O, int ti, int pair, int wave,
+                                                    int lane, float2 *prod) {
+    const unsigned tt = A.tiles[ti];
+    const int tx = (int)(tt & 0xffffu), ty = (int)(tt >> 16);
+    const int a = tx * kTile + (lane & 7), b = ty * kTile + (lane >> 3);
+    const long group = spec_group_offset(A, pair);
+    const float2 *base1 = A.spec1 + group, *base2 = A.spec2 + group;
+    // wave-uniform, so that a row's address costs no vector registers
+    const unsigned n = __builtin_amdgcn_readfirstlane(O.tile_n[ti] & kGopRows);
+    const uint2 *e = O.gop + (unsigned)__builtin_amdgcn_readfirstlane(O.tile_off[ti]);
+    float4 acc[1] = {make_float4(0.0f, 0.0f, 0.0f, 0.0f)};
+    if (n) {  // else no entry may be read
+        constexpr int B = kHeavyPlainBatch;
+        constexpr unsigned R = 4 * B;  // rows of a round
+        const unsigned r0 = wave * B;
+        auto entry = [&](unsigned k) { return gop_load(e + 64ul * min(k, n - 1) + lane); };
+        uint2 t[B];
+        float2 v[B][1];
+        float w[B];
+#pragma unroll
+        for (int i = 0; i < B; i++) t[i] = entry(r0 + i);
+#pragma unroll
+        for (int i = 0; i < B; i++) {
+            gop_gather<1>(t[i], base1, base2, v[i]);
+            w[i] = __uint_as_float(t[i].y);
+        }
+#pragma unroll
+        for (int i = 0; i < B; i++) t[i] = entry(R + r0 + i);
+        for (unsigned k0 = 0; k0 < n; k0 += R) {
+            // rows past the tile's last repeat it; they are not added
+#pragma unroll
+            for (int i = 0; i < B; i++) prod[(r0 + i) * 64 + lane] = make_float2(w[i] * v[i][0].x, w[i] * v[i][0].y);
+#pragma unroll
+            for (int i = 0; i < B; i++) {
+                gop_gather<1>(t[i], base1, base2, v[i]);
+                w[i] = __uint_as_float(t[i].y);
+            }
+#pragma unroll
+            for (int i = 0; i < B; i++) t[i] = entry(k0 + 2 * R + r0 + i);
+            __syncthreads();
+            if (wave == 0) {
+                const unsigned m = min(R, n - k0);
+                const float2 *q = prod + lane;
+                unsigned k = 0;
+                for (; k + 8 <= m; k += 8) {
+                    float2 x[8];
+#pragma unroll
+                    for (int i = 0; i < 8; i++) x[i] = q[(k + i) * 64];
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        acc[0].x += x[i].x;
+                        acc[0].z += x[i].y;
+                    }
+                }
+                for (; k < m; k++) {
+                    acc[0].x += q[k * 64].x;
+                    acc[0].z += q[k * 64].y;
+                }
+            }
+            __syncthreads();
+        }
+    }
+    if (wave == 0) store_cells<GR_ACCUM_PLAIN, 1>(A, pair, 1, a, b, acc);
+}
+
+// LDS of one workgroup on that path.
+constexpr size_t kHeavyPlainLds = sizeof(float2) * 64 * 4 * kHeavyPlainBatch;
 
 template <int P>
 __device__ __forceinline__ void sop_stage(unsigned key, const float2 *base1, const float2 *base2, char *stg,
@@ -1205,17 +1282,22 @@ __global__ void __launch_bounds__(256) k_gop_merge(GridArgs A, GopArgs O, int pa
     }
     store_cells<GR_ACCUM_COMPENSATED, 1>(A, pair, 1, a, b, acc);
 }
-// Workgroups of k_grid_op given to the one-pair-per-wave path (a multiple of
-// the sector count, so the other workgroups keep their XCD-to-sector map).
+
+// Workgroups of k_grid_op given to the heavy items -- one a wave, plain sums
+// one a workgroup -- (a multiple of the sector count, so the other workgroups
+// keep their XCD-to-sector map).
+template <int ACCUM>
 __host__ __device__ __forceinline__ int heavy_blocks(int n_items) {
-    return (n_items + 4 * kGridSectors - 1) / (4 * kGridSectors) * kGridSectors;
+    constexpr int per = (ACCUM == GR_ACCUM_PLAIN ? 1 : 4) * kGridSectors;
+    return (n_items + per - 1) / per * kGridSectors;
 }
 
 // k_grid's accumulation, fed by the operator.  The first heavy_blocks
 // workgroups take the heavy work items (slots [0, n_heavy) of every sector)
 // from the streamed entries: with compensated sums one segment of a cut tile
 // per wave for the P pairs of the group (grid_op_tile; k_gop_merge sums the
-// partials afterwards), otherwise a tile one pair per wave (grid_op_heavy).
+// partials afterwards), otherwise a tile one pair per wave (grid_op_heavy) or,
+// with plain sums, per workgroup (grid_op_heavy_plain).
 // The others take one tile per wave for the P pairs -- SOP: from the staged
 // operator (grid_sop_light), otherwise from the streamed entries
 // (grid_op_tile).
@@ -1243,10 +1325,20 @@ __global__ void __launch_bounds__(256, 4) k_grid_op(GridArgs A, GopArgs O) {
     // SOP: the persistent light workgroups first (they start at once and
     // hold most of the machine), the heavy items after them in the slots
     // left; otherwise the heavy items first (their long chains start early)
-    const int hb = heavy_blocks(O.n_hitems);
+    const int hb = heavy_blocks<ACCUM>(O.n_hitems);
     const int nlight = SOP ? 2 * O.sop_waves : 0;  // kGridSectors * sop_waves / 4
     const int hbx = bx - nlight;
     if (hbx >= 0 && hbx < hb) {
+        if (ACCUM == GR_ACCUM_PLAIN) {
+            // workgroup: a heavy tile and one of its pairs
+            if (hbx >= O.n_hitems) return;
+            const uint2 it = O.hitems[hbx];
+            const int ti = (int)it.x, p = (int)it.y;
+            if (p >= nvalid || A.tiles[ti] == kGridNoTile) return;
+            grid_op_heavy_plain(A, O, ti, pair0 + p, __builtin_amdgcn_readfirstlane(wave), lane,
+                                reinterpret_cast<float2 *>(smem + (SOP ? A.lds_wtbl : 0)));
+            return;
+        }
         // wave: work item hbx * 4 + wave -- a cut tile's segment (the P pairs
         // into partials), or a heavy tile one pair per wave
         const int item = hbx * 4 + wave;
@@ -1257,7 +1349,7 @@ __global__ void __launch_bounds__(256, 4) k_grid_op(GridArgs A, GopArgs O) {
             grid_op_tile<ACCUM, P>(A, O, ti, (int)it.y, pair0, nvalid, lane);
         } else {
             const int p = (int)it.y;  // tiles not cut: one item per pair
-            if (p < nvalid) grid_op_heavy<ACCUM>(A, O, ti, pair0 + p, lane);
+            if (p < nvalid) grid_op_heavy(A, O, ti, pair0 + p, lane);
         }
         return;
     }
@@ -1287,9 +1379,10 @@ template <int ACCUM, int P>
 hipError_t launch(const GridArgs &A, const GopArgs *O, int groups, size_t lds_base, int wpb, hipStream_t s) {
     if (O) {
         const int light = (A.sector_len - O->n_heavy + 3) / 4;
-        const int blocks = heavy_blocks(O->n_hitems) + kGridSectors * light;
+        const int blocks = heavy_blocks<ACCUM>(O->n_hitems) + kGridSectors * light;
+        const size_t heavy_lds = ACCUM == GR_ACCUM_PLAIN ? kHeavyPlainLds : 0;
         if (!O->sop_tile) {
-            hipLaunchKernelGGL((k_grid_op<ACCUM, P, false>), dim3(blocks, groups), dim3(256), 0, s, A, *O);
+            hipLaunchKernelGGL((k_grid_op<ACCUM, P, false>), dim3(blocks, groups), dim3(256), heavy_lds, s, A, *O);
             return hipGetLastError();
         }
         // the staged light tiles: persistent workgroups, kSopBlocksPerSector
@@ -1297,12 +1390,12 @@ hipError_t launch(const GridArgs &A, const GopArgs *O, int groups, size_t lds_ba
         // interleaved), fewer when the sector has fewer slots
         const int G = groups <= 8 ? groups : 1;
         const int lb = std::max(1, std::min(light, kSopBlocksPerSector / G));
-        const int sblocks = heavy_blocks(O->n_hitems) + kGridSectors * lb;
+        const int sblocks = heavy_blocks<ACCUM>(O->n_hitems) + kGridSectors * lb;
         GopArgs o = *O;
         o.sop_waves = 4 * lb;
         o.sop_groups = G;
 
-        const size_t lds = lds_base + sizeof(float2) * 4 * kSopSlots * P;
+        const size_t lds = lds_base + std::max(heavy_lds, sizeof(float2) * 4 * kSopSlots * P);
         hipError_t e = gr_allow_lds(k_grid_op<ACCUM, P, true>, lds);
         if (e != hipSuccess) return e;
         if (G > 1)

@@ -211,3 +211,18 @@ def test_geometry_kernel_slot_rounds(name, ns, accum):
     disk = (yy * yy + xx * xx) < (0.45 * m) ** 2
     for img, r in ((ref[0], r1), (ref[1], r2)):
         assert O.rel_l2(img.cpu().numpy()[disk], r[disk]) < 1e-5
+
+
+@pytest.mark.parametrize("n_ang,n_det", [(9, 40), (31, 64), (200, 65)])
+@pytest.mark.parametrize("ns", [1, 9, 34])
+def test_plain_heavy_tiles(n_ang, n_det, ns):
+    """Plain sums of the tiles near the centre, gathered by four waves: from
+    tiles just over the line to ones of a thousand rows, one pair to several
+    groups with a partial one; in launches of 5 pairs too."""
+    case = dict(n_ang=n_ang, n_det=n_det, center=n_det / 2.0 + 0.3, accum="plain")
+    sino = sinos(case, ns, n_ang)
+    ref = gr.Plan(**case, grid_op="off").recon(sino)
+    out = gr.Plan(**case, grid_op="on").recon(sino)
+    out5 = gr.Plan(**case, grid_op="on", max_pairs=5).recon(sino)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref) and torch.equal(out5, ref)

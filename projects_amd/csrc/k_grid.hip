@@ -1370,10 +1370,22 @@ __global__ void __launch_bounds__(256, 4) k_grid_op(GridArgs A, GopArgs O) {
     grid_op_tile<ACCUM, P>(A, O, ti, -1, pair0, nvalid, lane);
 }
 
-// Persistent workgroups per sector (and group of pairs) of the staged light
-// path: 8 x 96 take three of the four workgroups an MI355X CU holds, the
-// fourth serves the heavy items.
-constexpr int kSopBlocksPerSector = 96;
+// Persistent workgroups per sector of the staged light path, shared by the
+// groups of pairs of a launch.  The light tiles wait for memory, so more of
+// them in flight help: 8 x 96 take three of the four workgroups an MI355X CU
+// holds, which leaves the fourth to the heavy items.  Several groups of a
+// large grid take all four (1500 x 2048, 32 pairs: 2.44 -> 2.27 ms; 720 x
+// 1024: 0.66 -> 0.60): the heavy items are then a short tail.  They are not
+// one in a small grid (360 x 512, 32 pairs: 0.18 -> 0.24), nor for a single
+// group (0.49 -> 0.51 at 1500 x 2048).  And a wave should have some ten tiles
+// to take, down to 48 workgroups: the heavy chains of a small grid run
+// faster beside fewer light waves (one pair of 180 x 256 27 -> 25 us, of
+// 360 x 512 46 -> 42).
+__host__ inline int sop_blocks_per_sector(int light, int groups) {
+    const int most = groups > 1 && light >= 1024 ? 128 : 96;
+    const int total = std::min(most, std::max(48, light * groups / 10));
+    return std::max(1, std::min(light, total / groups));
+}
 
 template <int ACCUM, int P>
 hipError_t launch(const GridArgs &A, const GopArgs *O, int groups, size_t lds_base, int wpb, hipStream_t s) {
@@ -1385,11 +1397,10 @@ hipError_t launch(const GridArgs &A, const GopArgs *O, int groups, size_t lds_ba
             hipLaunchKernelGGL((k_grid_op<ACCUM, P, false>), dim3(blocks, groups), dim3(256), heavy_lds, s, A, *O);
             return hipGetLastError();
         }
-        // the staged light tiles: persistent workgroups, kSopBlocksPerSector
-        // per sector shared by the launch's groups of pairs (up to 8 groups
-        // interleaved), fewer when the sector has fewer slots
+        // the staged light tiles: persistent workgroups (up to 8 groups of
+        // pairs interleaved)
         const int G = groups <= 8 ? groups : 1;
-        const int lb = std::max(1, std::min(light, kSopBlocksPerSector / G));
+        const int lb = sop_blocks_per_sector(light, G);
         const int sblocks = heavy_blocks<ACCUM>(O->n_hitems) + kGridSectors * lb;
         GopArgs o = *O;
         o.sop_waves = 4 * lb;

@@ -65,6 +65,12 @@ __device__ __forceinline__ uint16_t to_bf16(float f) {
     // MI355X: no difference).
     return __builtin_bit_cast(uint16_t, (__bf16)f);
 }
+// Two of them in one word, the first in its low half.
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
+}
 __device__ __forceinline__ float from_bf16(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 __device__ __forceinline__ float round_bf16(float f) { return from_bf16(to_bf16(f)); }
 __device__ __forceinline__ bool positive_bf16(uint16_t h) { return !(h & 0x8000u) && h != 0; }
@@ -709,134 +715,161 @@ __global__ void __launch_bounds__(256) k_conv_in_wgrad(const float *__restrict__
     block_sum_groups(acc, db, red, part + (long)blockIdx.x * IN_REC, true);
 }
 
-// Loss: dy = 2 (yn - t/scale) / N; per-block partial sums of (yn - t/scale)^2.
-__global__ void __launch_bounds__(256) k_loss(const float *__restrict__ yn, const float *__restrict__ target,
-                                              float scale, float *__restrict__ dy, float *__restrict__ part, long N) {
-    __shared__ float sred[256];
-    float s = 0.0f;
-    for (long p = (long)blockIdx.x * 256 + threadIdx.x; p < N; p += (long)gridDim.x * 256) {
-        const float e = yn[p] - target[p] / scale;
-        dy[p] = 2.0f * e / (float)N;
-        s += e * e;
-    }
-    sred[threadIdx.x] = s;
-    __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-        if (threadIdx.x < h) sred[threadIdx.x] += sred[threadIdx.x + h];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = sred[0];
-}
-
-// Input gradient of the 32 -> 1 layer, masked: dz4 = bf16(sum_t dy[p - off_t] W5[ci][t] * (a4 > 0)).
-__global__ void __launch_bounds__(256) k_conv_out_dgrad(const float *__restrict__ dy, const uint16_t *__restrict__ a4,
-                                                        const float *__restrict__ prm, uint16_t *__restrict__ dz4,
-                                                        int n, int H, int W) {
-    __shared__ float sw[9 * CH];
-    for (int i = threadIdx.x; i < 9 * CH; i += blockDim.x) sw[i] = round_bf16(prm[OFF_W5 + i]);
-    __syncthreads();
-    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (long)n * H * W) return;
-    const long img = p / ((long)H * W);
-    const int rem = (int)(p - img * H * W), py = rem / W, px = rem - py * W;
-    float d[9];
+// Loss, input and weight gradient of the 32 -> 1 layer in one pass over a4,
+// persistent over the tiles blockIdx.x, blockIdx.x + gridDim.x, ...:
+//   dy = 2 (yn - t/scale) / N, loss partial[block] = sum (yn - t/scale)^2
+//   dz4[q][ci] = bf16(sum_t dy[q - off_t] W5[ci][t] * (a4 > 0))
+//   partial[block] = (dW5[ci][t] = sum_q dy[q - off_t] a4[q][ci], db5 = sum dy)
+// The gradients take the same nine values of dy around a pixel q, from the tile
+// computed with its halo into LDS.  Thread tid takes the 4 channels (tid mod 8) * 4.. of
+// the tile's column tid / 8, KB rows at a time, so neighbouring rows share
+// their dy and four rows a tap's weights: one 8-byte load of a4 and one
+// 8-byte store of dz4 per pixel (a wave 8 whole records).  The next tile's loads
+// are issued (clamped, not guarded) as this tile's values are taken up, and the
+// weight sums stay in registers across tiles.  With 8 channels a thread the
+// sums, weights and values of a tile did not fit the registers; two waves a
+// SIMD, since a third has its sums spilled.  32 images of 512 x 512: 532 us as
+// three kernels (loss, weight gradient, input gradient), 289 as one; its 128 bytes
+// per pixel take 227.
+__global__ void __launch_bounds__(256, 2) k_conv_out_back(const float *__restrict__ yn,
+                                                          const float *__restrict__ target, float scale,
+                                                          float fN, const uint16_t *__restrict__ a4,
+                                                          const float *__restrict__ prm, uint16_t *__restrict__ dz4,
+                                                          float *__restrict__ part, float *__restrict__ lpart, int H,
+                                                          int W, int ntiles, TileMap tm) {
+    __shared__ float sdy[HS * WS];
+    __shared__ __align__(16) float sw[9 * CH];  // [t][ci]
+    __shared__ float red[4 * 9 * CH];
+    constexpr int KB = 4;                      // rows at a time
+    constexpr int ND = (HS * WS + 255) / 256;  // halo values per thread
+    static_assert(TW * 8 == 256 && TH % KB == 0, "a thread per column and 4 channels");
+    const int tid = threadIdx.x, cg = tid & 7, col = tid >> 3;
+    for (int i = tid; i < 9 * CH; i += 256) sw[i] = round_bf16(prm[OFF_W5 + (i % CH) * 9 + i / CH]);
+    float acc[9][4], dsum = 0.0f, lsum = 0.0f;
 #pragma unroll
-    for (int t = 0; t < 9; t++) {
-        const int yy = py - (t / 3 - 1), xx = px - (t % 3 - 1);
-        d[t] = (yy >= 0 && yy < H && xx >= 0 && xx < W) ? dy[(img * H + yy) * W + xx] : 0.0f;
-    }
-    const uint4 *m4 = reinterpret_cast<const uint4 *>(a4 + p * CH);
-    uint4 *o4 = reinterpret_cast<uint4 *>(dz4 + p * CH);
+    for (int t = 0; t < 9; t++)
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const uint4 m = m4[k];
-        const uint32_t mw[4] = {m.x, m.y, m.z, m.w};
-        uint32_t ow[4];
+        for (int e = 0; e < 4; e++) acc[t][e] = 0.0f;
+    struct At {
+        int y0, x0;
+        long ibase, base;  // first pixel of the image, of the tile
+        int col;           // this thread's column of the tile, inside the image
+    };
+    auto at = [&](int tile) {
+        At o;
+        int img;
+        tm.of(tile, img, o.y0, o.x0);
+        o.ibase = (long)img * H * W;
+        o.base = o.ibase + (long)o.y0 * W + o.x0;
+        o.col = min(col, W - 1 - o.x0);
+        return o;
+    };
+    uint2 v[TH];
+    float ne[ND];  // yn - t/scale, zero outside the image
+    // addresses: a wave-uniform tile base and offsets within the tile
+    auto load_a4 = [&](const At &o, int r) {
+        const long px = min(r, H - 1 - o.y0) * W + o.col;
+        v[r] = *reinterpret_cast<const uint2 *>(a4 + o.base * CH + px * CH + cg * 4);
+    };
+    auto load_err = [&](const At &o) {
 #pragma unroll
-        for (int e2 = 0; e2 < 4; e2++) {
-            uint32_t word = 0;
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int ci = k * 8 + e2 * 2 + h;
-                float s = 0.0f;
-#pragma unroll
-                for (int t = 0; t < 9; t++) s += d[t] * sw[ci * 9 + t];
-                const uint16_t mk = (uint16_t)(mw[e2] >> (16 * h));
-                word |= (uint32_t)to_bf16(positive_bf16(mk) ? s : 0.0f) << (16 * h);
-            }
-            ow[e2] = word;
+        for (int k = 0; k < ND; k++) {
+            const int i = min(tid + 256 * k, HS * WS - 1), gy = o.y0 + i / WS - 1, gx = o.x0 + i % WS - 1;
+            const long p = o.ibase + (long)min(max(gy, 0), H - 1) * W + min(max(gx, 0), W - 1);
+            const float d = yn[p] - target[p] / scale;
+            ne[k] = __int_as_float(__float_as_int(d) & -(int)(gy >= 0 && gy < H && gx >= 0 && gx < W));
         }
-        o4[k] = make_uint4(ow[0], ow[1], ow[2], ow[3]);
-    }
-}
-
-// Weight gradient of the 32 -> 1 layer: partial[block] = (dW5[ci][t], db5)
-// over the tiles blockIdx.x, blockIdx.x + gridDim.x, ...  dW5[ci][t] = sum_p
-// dy[p] a4[p + off_t][ci] is taken as a sum over the input pixels q of the
-// tile with its halo, dy[q - off_t] the output pixel each tap reaches: thread
-// tid takes the 8 channels (tid mod 4) * 8.. of the halo pixels tid / 4 +
-// 64 k (one 16-byte load per pixel, a wave 16 whole records, all six issued
-// before use) and dy of the tile from LDS; sums in registers across tiles.
-__global__ void __launch_bounds__(256) k_conv_out_wgrad(const float *__restrict__ dy, const uint16_t *__restrict__ a4,
-                                                        float *__restrict__ part, int H, int W, int ntiles,
-                                                        TileMap tm) {
-    __shared__ float sdy[TH * TW];
-    __shared__ float red[16 * 80];
-    constexpr int NQ = (HS * WS + 63) / 64;  // halo pixels per thread: 6
-    const int tid = threadIdx.x, cg = tid & 3, ps = tid >> 2;
-    float acc[9][8], db[8], dsum = 0.0f;
+    };
+    const At o0 = at(min((int)blockIdx.x, ntiles - 1));
+    load_err(o0);
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-        db[e] = 0.0f;
-#pragma unroll
-        for (int t = 0; t < 9; t++) acc[t][e] = 0.0f;
-    }
+    for (int r = 0; r < TH; r++) load_a4(o0, r);
     for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        int img, y0, x0;
-        tm.of(tile, img, y0, x0);
-        const long ibase = (long)img * H * W;
-        uint4 v[NQ];
-#pragma unroll
-        for (int k = 0; k < NQ; k++) {
-            const int q = ps + 64 * k, r = q / WS, c = q - r * WS, gy = y0 + r - 1, gx = x0 + c - 1;
-            v[k] = make_uint4(0u, 0u, 0u, 0u);
-            if (q < HS * WS && gy >= 0 && gy < H && gx >= 0 && gx < W)
-                v[k] = *reinterpret_cast<const uint4 *>(a4 + (ibase + (long)gy * W + gx) * CH + cg * 8);
-        }
+        const At o = at(tile), on = at(min(tile + (int)gridDim.x, ntiles - 1));
         __syncthreads();  // the previous tile's reads of sdy are done
-        {
-            const int r = tid / TW, c = tid - r * TW, gy = y0 + r, gx = x0 + c;
-            const float d = (gy < H && gx < W) ? dy[ibase + (long)gy * W + gx] : 0.0f;
-            sdy[tid] = d;
-            dsum += d;  // db5: thread tid takes pixel tid of every tile
+#pragma unroll
+        for (int k = 0; k < ND; k++) {
+            const int i = tid + 256 * k, r = i / WS - 1, c = i % WS - 1;
+            if (i < HS * WS) sdy[i] = 2.0f * ne[k] / fN;
+            if (r >= 0 && r < TH && c >= 0 && c < TW) lsum += ne[k] * ne[k];
         }
         __syncthreads();
+        load_err(on);
 #pragma unroll
-        for (int k = 0; k < NQ; k++) {
-            const int q = ps + 64 * k, qr = q / WS, qc = q - qr * WS;
-            const uint32_t w4[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
-            float a[8];
+        for (int r0 = 0; r0 < TH; r0 += KB) {
+            float a[KB][4], g[KB][4], d[KB + 2][3];
 #pragma unroll
-            for (int e = 0; e < 8; e++) a[e] = from_bf16((uint16_t)(w4[e >> 1] >> (16 * (e & 1))));
+            for (int k = 0; k < KB; k++) {
+                const uint32_t in = -(uint32_t)(o.y0 + r0 + k < H && col == o.col);  // a mask: no branch
+                const uint32_t w2[2] = {v[r0 + k].x & in, v[r0 + k].y & in};
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    a[k][e] = from_bf16((uint16_t)(w2[e >> 1] >> (16 * (e & 1))));
+                    g[k][e] = 0.0f;
+                }
+                load_a4(on, r0 + k);
+            }
+#pragma unroll
+            for (int k = 0; k < KB + 2; k++)
+#pragma unroll
+                for (int c = 0; c < 3; c++) d[k][c] = sdy[(r0 + k) * WS + col + c];
 #pragma unroll
             for (int t = 0; t < 9; t++) {
-                const int pr = qr - t / 3, pc = qc - t % 3;  // output pixel of tap t
-                const float d = (q < HS * WS && pr >= 0 && pr < TH && pc >= 0 && pc < TW) ? sdy[pr * TW + pc] : 0.0f;
+                const float4 w4 = *reinterpret_cast<const float4 *>(sw + t * CH + cg * 4);
+                const float w[4] = {w4.x, w4.y, w4.z, w4.w};
 #pragma unroll
-                for (int e = 0; e < 8; e++) acc[t][e] = __builtin_fmaf(d, a[e], acc[t][e]);
+                for (int k = 0; k < KB; k++) {
+                    const float dq = d[k + 2 - t / 3][2 - t % 3];  // dy[q - off_t]
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        g[k][e] = __builtin_fmaf(dq, w[e], g[k][e]);
+                        acc[t][e] = __builtin_fmaf(dq, a[k][e], acc[t][e]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < KB; k++) {
+                uint32_t ow[2];
+                // summed here, not in a branch of the mask with all operands alive
+#pragma unroll
+                for (int e = 0; e < 4; e++) asm volatile("" : "+v"(g[k][e]));
+#pragma unroll
+                for (int e = 0; e < 4; e += 2)  // positive_bf16, on the floats' bits
+                    ow[e >> 1] = pack_bf16(__float_as_int(a[k][e]) > 0 ? g[k][e] : 0.0f,
+                                           __float_as_int(a[k][e + 1]) > 0 ? g[k][e + 1] : 0.0f);
+                if (o.y0 + r0 + k < H && col == o.col)
+                    *reinterpret_cast<uint2 *>(dz4 + o.base * CH + (long)((r0 + k) * W + col) * CH + cg * 4) =
+                        make_uint2(ow[0], ow[1]);
             }
         }
+        dsum += sdy[(tid / TW + 1) * WS + tid % TW + 1];  // db5: thread tid takes pixel tid of every tile
     }
+    // the lanes of a channel group, then the waves, in a fixed order
+    const int lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+    for (int t = 0; t < 9; t++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+#pragma unroll
+            for (int x = 8; x < 64; x <<= 1) acc[t][e] += __shfl_xor(acc[t][e], x);
+            if (lane < 8) red[wave * 9 * CH + (cg * 4 + e) * 9 + t] = acc[t][e];
+        }
+    __syncthreads();
     float *out = part + (long)blockIdx.x * OUT_REC;
-    block_sum_groups(acc, db, red, out, false);
-    // db5: the threads' pixel sums in thread order
+    for (int i = tid; i < 9 * CH; i += 256)
+        out[i] = ((red[i] + red[9 * CH + i]) + red[2 * 9 * CH + i]) + red[3 * 9 * CH + i];
+    // db5 and the loss: the threads' sums in thread order
     __syncthreads();
     red[tid] = dsum;
+    red[256 + tid] = lsum;
     __syncthreads();
-    if (tid == 0) {
+    if (tid < 2) {
         float s5 = 0.0f;
-        for (int i = 0; i < 256; i++) s5 += red[i];
-        out[9 * CH] = s5;
+        for (int i = 0; i < 256; i++) s5 += red[tid * 256 + i];
+        if (tid == 0)
+            out[9 * CH] = s5;
+        else
+            lpart[blockIdx.x] = s5;
     }
 }
 
@@ -1007,7 +1040,6 @@ size_t gr_cnn_work_bytes(int n, int H, int W) {
     const size_t up = 256;
     auto al = [&](size_t b) { return (b + up - 1) / up * up; };
     return al(sizeof(float) * npx)                         // yn
-           + al(sizeof(float) * npx)                       // dy
            + 2 * al(sizeof(uint16_t) * npx * CH)           // dz ping-pong
            + al(sizeof(float) * (size_t)MAX_WG_BLOCKS * WG_REC)  // weight-gradient partials
            + al(sizeof(float) * 2 * (size_t)ntiles)        // forward statistics partials
@@ -1035,7 +1067,7 @@ int gr_cnn_forward(const float *params, const unsigned short *packed, const floa
         char *wb = (char *)work;
         const long npx = (long)n * H * W;
         auto al = [](size_t b) { return (b + 255) / 256 * 256; };
-        wb += 2 * al(sizeof(float) * npx) + 2 * al(sizeof(uint16_t) * npx * CH) +
+        wb += al(sizeof(float) * npx) + 2 * al(sizeof(uint16_t) * npx * CH) +
               al(sizeof(float) * (size_t)MAX_WG_BLOCKS * WG_REC);
         stats = (float *)wb;
     }
@@ -1075,8 +1107,6 @@ int gr_cnn_backward(const float *params, const unsigned short *packed, const flo
     auto al = [](size_t b) { return (b + 255) / 256 * 256; };
     char *wb = (char *)work;
     wb += al(sizeof(float) * npx);  // yn slot (the caller's yn may live there)
-    float *dy = (float *)wb;
-    wb += al(sizeof(float) * npx);
     uint16_t *dzA = (uint16_t *)wb;
     wb += al(sizeof(uint16_t) * npx * CH);
     uint16_t *dzB = (uint16_t *)wb;
@@ -1087,16 +1117,13 @@ int gr_cnn_backward(const float *params, const unsigned short *packed, const flo
     float *lpart = (float *)wb;
     const uint16_t *pk = reinterpret_cast<const uint16_t *>(packed);
     const int nwg = ntiles < MAX_WG_BLOCKS ? ntiles : MAX_WG_BLOCKS;
-    const int nloss = (int)std::min<long>(1024, (npx + 255) / 256);
 
-    hipLaunchKernelGGL(k_loss, dim3(nloss), dim3(256), 0, s, yn, target, scale, dy, lpart, npx);
-    if (loss) hipLaunchKernelGGL(k_sum_groups, dim3(1), dim3(256), 0, s, lpart, 1, nloss, 1, 1.0 / (double)npx, loss);
     // layer 5
-    hipLaunchKernelGGL(k_conv_out_wgrad, dim3(nwg), dim3(256), 0, s, dy, a4, part, H, W, ntiles, tm);
+    hipLaunchKernelGGL(k_conv_out_back, dim3(nwg), dim3(256), 0, s, yn, target, scale, (float)npx, a4, params, dzA, part,
+                       lpart, H, W, ntiles, tm);
+    if (loss) hipLaunchKernelGGL(k_sum_groups, dim3(1), dim3(256), 0, s, lpart, 1, nwg, 1, 1.0 / (double)npx, loss);
     hipLaunchKernelGGL(k_reduce, dim3((OUT_REC + 63) / 64), dim3(64 * RED_WAVES), 0, s, part, nwg, OUT_REC, 1,
                        grads + OFF_W5, grads + OFF_B5);
-    hipLaunchKernelGGL(k_conv_out_dgrad, dim3((unsigned)((npx + 255) / 256)), dim3(256), 0, s, dy, a4, params, dzA,
-                       n, H, W);
     // layers 4, 3, 2
     const unsigned short *acts[4] = {a1, a2, a3, a4};
     const int woff[3] = {OFF_W2, OFF_W3, OFF_W4}, boff[3] = {OFF_B2, OFF_B3, OFF_B4};

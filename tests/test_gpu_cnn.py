@@ -331,6 +331,26 @@ def test_backward_tile_edges(n, H, W):
         assert np.linalg.norm(gg[k] - g[k]) <= 2e-3 * np.linalg.norm(g[k]), k
 
 
+# the last layer's backward: 8 x 32 tiles, more of them than workgroups, with
+# ragged last rows and columns; a tile's rows and columns short of, exactly and
+# past one
+@pytest.mark.parametrize("n,H,W", [(1, 7, 31), (2, 8, 32), (1, 9, 33), (4, 130, 300)])
+def test_last_layer_backward_tiles(n, H, W):
+    """Loss and every gradient against the oracle's, within the bounds of
+    test_backward_tile_edges and for its reasons; a second run gives the same
+    bits."""
+    test_backward_tile_edges(n, H, W)
+    net, _, x, t = make(n + H + W, n, H, W)
+    xg, tg = torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda()
+    runs = []
+    for _ in range(2):
+        net.forward(xg, train=True)
+        net.backward(xg, tg)
+        torch.cuda.synchronize()
+        runs.append((net.grads.clone(), net.loss.clone()))
+    assert torch.equal(runs[0][0], runs[1][0]) and torch.equal(runs[0][1], runs[1][1])
+
+
 # the forward kernel's strips of 56 columns (16-column groups, guard columns)
 # and segments of rows (pairs of rows, odd ends): one short of, exactly and one
 # past a strip, several segments, images smaller than the halo

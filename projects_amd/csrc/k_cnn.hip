@@ -616,103 +616,132 @@ __global__ void __launch_bounds__(BK_THREADS, 2) k_conv32_back(const uint16_t *_
     }
 }
 
-// Sum acc[9][8] (tap, channel of the thread's group of 8) and extra[8] over
-// the threads of the block that share a channel group (tid mod 4), in a fixed
-// order: lanes of a wave by a butterfly over lane bits 2..5, then the four
-// waves in order through LDS; the block's record gets W[ch][t] at
-// ch * 9 + t (parameter order) and the extras at 9 * CH + ch.
-__device__ __forceinline__ void block_sum_groups(float (&acc)[9][8], float (&extra)[8], float *red, float *out,
-                                                 bool with_extra) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, cg = tid & 3;
+// The sums of a block of 256 threads over its lanes of equal channel group
+// tid mod 8 (4 channels each), then over its waves, in a fixed order: out[ch * 9
+// + t], ch = 4 (tid mod 8) + e.  red: 4 * 9 * CH floats.
+__device__ __forceinline__ void block_sum_taps(float (&acc)[9][4], float *red, float *out) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, cg = tid & 7;
 #pragma unroll
-    for (int o = 4; o < 64; o <<= 1) {
+    for (int t = 0; t < 9; t++)
 #pragma unroll
-        for (int t = 0; t < 9; t++)
+        for (int e = 0; e < 4; e++) {
 #pragma unroll
-            for (int e = 0; e < 8; e++) acc[t][e] += __shfl_xor(acc[t][e], o);
-#pragma unroll
-        for (int e = 0; e < 8; e++) extra[e] += __shfl_xor(extra[e], o);
-    }
-    // lanes 0..3 of each wave hold the wave's sums of groups 0..3
-    if (lane < 4) {
-#pragma unroll
-        for (int t = 0; t < 9; t++)
-#pragma unroll
-            for (int e = 0; e < 8; e++) red[(wave * 4 + cg) * 80 + t * 8 + e] = acc[t][e];
-#pragma unroll
-        for (int e = 0; e < 8; e++) red[(wave * 4 + cg) * 80 + 72 + e] = extra[e];
-    }
-    __syncthreads();
-    for (int i = tid; i < 4 * 80; i += blockDim.x) {  // i = group * 80 + slot
-        const int grp = i / 80, sl = i - grp * 80;
-        if (sl >= 72 && !with_extra) continue;
-        float v = 0.0f;
-        for (int w = 0; w < (int)(blockDim.x >> 6); w++) v += red[(w * 4 + grp) * 80 + sl];
-        if (sl < 72) {
-            const int t = sl >> 3, ch = grp * 8 + (sl & 7);
-            out[ch * 9 + t] = v;
-        } else {
-            out[9 * CH + grp * 8 + (sl - 72)] = v;
+            for (int x = 8; x < 64; x <<= 1) acc[t][e] += __shfl_xor(acc[t][e], x);
+            if (lane < 8) red[wave * 9 * CH + (cg * 4 + e) * 9 + t] = acc[t][e];
         }
-    }
+    __syncthreads();
+    for (int i = tid; i < 9 * CH; i += 256)
+        out[i] = ((red[i] + red[9 * CH + i]) + red[2 * 9 * CH + i]) + red[3 * 9 * CH + i];
 }
 
+// A tile of the first and last layers' gradients, for a thread of column col.
+struct GradTile {
+    int y0, x0;
+    long ibase, base;  // first pixel of the image, of the tile
+    int col;           // the thread's column of the tile, inside the image
+    __device__ GradTile(const TileMap &tm, int tile, int H, int W, int c) {
+        int img;
+        tm.of(tile, img, y0, x0);
+        ibase = (long)img * H * W;
+        base = ibase + (long)y0 * W + x0;
+        col = min(c, W - 1 - x0);
+    }
+    // halo value i's pixel, moved inside the image, and whether it was inside
+    __device__ long halo(int i, int H, int W, bool &in) const {
+        const int gy = y0 + i / WS - 1, gx = x0 + i % WS - 1;
+        in = gy >= 0 && gy < H && gx >= 0 && gx < W;
+        return ibase + (long)min(max(gy, 0), H - 1) * W + min(max(gx, 0), W - 1);
+    }
+};
+
 // Weight gradient of the 1 -> 32 layer: partial[block] = (dW1[co][t], db1[co])
-// over the tiles blockIdx.x, blockIdx.x + gridDim.x, ...  Thread tid takes the
-// 8 channels (tid mod 4) * 8.. of the output pixels tid / 4 + 64 k of a tile:
-// one 16-byte load of dz per pixel (four threads read a pixel's 64-byte
-// record, a wave 16 whole records), all four issued before use, and the nine
-// taps of bf16(x/scale) from the tile staged with its halo in LDS; the sums
-// stay in registers across the block's tiles.
-__global__ void __launch_bounds__(256) k_conv_in_wgrad(const float *__restrict__ x, float scale,
-                                                       const uint16_t *__restrict__ dz, float *__restrict__ part,
-                                                       int H, int W, int ntiles, TileMap tm) {
+// over the tiles blockIdx.x, blockIdx.x + gridDim.x, ...  As k_conv_out_back: thread
+// tid takes the 4 channels (tid mod 8) * 4.. of the tile's column tid / 8, four
+// rows at a time (one 8-byte load of dz per pixel), the nine taps of
+// bf16(x/scale) from the tile with its halo in LDS, the next tile's loads issued
+// as this one's values are taken up, the sums in registers across tiles.
+// Bound by reading dz, 114 us for 32 images of 512 x 512: 199 us with eight
+// channels a thread and the loads waited for, 161 this way.
+__global__ void __launch_bounds__(256, 2) k_conv_in_wgrad(const float *__restrict__ x, float scale,
+                                                          const uint16_t *__restrict__ dz, float *__restrict__ part,
+                                                          int H, int W, int ntiles, TileMap tm) {
     __shared__ float sx[HS * WS];
-    __shared__ float red[16 * 80];
-    const int tid = threadIdx.x, cg = tid & 3, ps = tid >> 2;
-    float acc[9][8], db[8];
+    __shared__ float red[4 * 9 * CH];
+    constexpr int KB = 4;                      // rows at a time
+    constexpr int ND = (HS * WS + 255) / 256;  // halo values per thread
+    const int tid = threadIdx.x, cg = tid & 7, col = tid >> 3;
+    float acc[9][4], db[4];
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
+    for (int e = 0; e < 4; e++) {
         db[e] = 0.0f;
 #pragma unroll
         for (int t = 0; t < 9; t++) acc[t][e] = 0.0f;
     }
+    uint2 v[TH];
+    float nx[ND];
+    auto load_dz = [&](const GradTile &o, int r) {
+        const long px = min(r, H - 1 - o.y0) * W + o.col;
+        v[r] = *reinterpret_cast<const uint2 *>(dz + o.base * CH + px * CH + cg * 4);
+    };
+    auto load_x = [&](const GradTile &o) {
+#pragma unroll
+        for (int k = 0; k < ND; k++) {
+            bool in;
+            const long p = o.halo(min(tid + 256 * k, HS * WS - 1), H, W, in);
+            nx[k] = __int_as_float(__float_as_int(x[p]) & -(int)in);
+        }
+    };
+    const GradTile o0(tm, min((int)blockIdx.x, ntiles - 1), H, W, col);
+    load_x(o0);
+#pragma unroll
+    for (int r = 0; r < TH; r++) load_dz(o0, r);
     for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        int img, y0, x0;
-        tm.of(tile, img, y0, x0);
-        const long ibase = (long)img * H * W;
-        uint4 v[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int p = ps + 64 * k, r = p / TW, c = p - r * TW, gy = y0 + r, gx = x0 + c;
-            v[k] = make_uint4(0u, 0u, 0u, 0u);
-            if (gy < H && gx < W) v[k] = *reinterpret_cast<const uint4 *>(dz + (ibase + (long)gy * W + gx) * CH + cg * 8);
-        }
+        const GradTile o(tm, tile, H, W, col), on(tm, min(tile + (int)gridDim.x, ntiles - 1), H, W, col);
         __syncthreads();  // the previous tile's reads of sx are done
-        for (int i = tid; i < HS * WS; i += 256) {
-            const int r = i / WS, c = i - r * WS, gy = y0 + r - 1, gx = x0 + c - 1;
-            sx[i] = (gy >= 0 && gy < H && gx >= 0 && gx < W) ? round_bf16(x[ibase + (long)gy * W + gx] / scale) : 0.0f;
-        }
+#pragma unroll
+        for (int k = 0; k < ND; k++)
+            if (tid + 256 * k < HS * WS) sx[tid + 256 * k] = round_bf16(nx[k] / scale);
         __syncthreads();
+        load_x(on);
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int p = ps + 64 * k, r = p / TW, c = p - r * TW;
-            const uint32_t w4[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
-            float d[8];
+        for (int r0 = 0; r0 < TH; r0 += KB) {
+            float a[KB][4], d[KB + 2][3];
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                d[e] = from_bf16((uint16_t)(w4[e >> 1] >> (16 * (e & 1))));
-                db[e] += d[e];
+            for (int k = 0; k < KB; k++) {
+                const uint32_t in = -(uint32_t)(o.y0 + r0 + k < H && col == o.col);  // a mask: no branch
+                const uint32_t w2[2] = {v[r0 + k].x & in, v[r0 + k].y & in};
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    a[k][e] = from_bf16((uint16_t)(w2[e >> 1] >> (16 * (e & 1))));
+                    db[e] += a[k][e];
+                }
+                load_dz(on, r0 + k);
             }
 #pragma unroll
-            for (int t = 0; t < 9; t++) {
-                const float xv = sx[(r + t / 3) * WS + c + t % 3];
+            for (int k = 0; k < KB + 2; k++)
 #pragma unroll
-                for (int e = 0; e < 8; e++) acc[t][e] = __builtin_fmaf(d[e], xv, acc[t][e]);
-            }
+                for (int c = 0; c < 3; c++) d[k][c] = sx[(r0 + k) * WS + col + c];
+#pragma unroll
+            for (int t = 0; t < 9; t++)
+#pragma unroll
+                for (int k = 0; k < KB; k++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        acc[t][e] = __builtin_fmaf(d[k + t / 3][t % 3], a[k][e], acc[t][e]);
         }
     }
-    block_sum_groups(acc, db, red, part + (long)blockIdx.x * IN_REC, true);
+    float *out = part + (long)blockIdx.x * IN_REC;
+    block_sum_taps(acc, red, out);
+    __syncthreads();
+    const int lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+#pragma unroll
+        for (int s = 8; s < 64; s <<= 1) db[e] += __shfl_xor(db[e], s);
+        if (lane < 8) red[wave * CH + cg * 4 + e] = db[e];
+    }
+    __syncthreads();
+    if (tid < CH) out[9 * CH + tid] = ((red[tid] + red[CH + tid]) + red[2 * CH + tid]) + red[3 * CH + tid];
 }
 
 // Loss, input and weight gradient of the 32 -> 1 layer in one pass over a4,
@@ -750,42 +779,28 @@ __global__ void __launch_bounds__(256, 2) k_conv_out_back(const float *__restric
     for (int t = 0; t < 9; t++)
 #pragma unroll
         for (int e = 0; e < 4; e++) acc[t][e] = 0.0f;
-    struct At {
-        int y0, x0;
-        long ibase, base;  // first pixel of the image, of the tile
-        int col;           // this thread's column of the tile, inside the image
-    };
-    auto at = [&](int tile) {
-        At o;
-        int img;
-        tm.of(tile, img, o.y0, o.x0);
-        o.ibase = (long)img * H * W;
-        o.base = o.ibase + (long)o.y0 * W + o.x0;
-        o.col = min(col, W - 1 - o.x0);
-        return o;
-    };
     uint2 v[TH];
     float ne[ND];  // yn - t/scale, zero outside the image
     // addresses: a wave-uniform tile base and offsets within the tile
-    auto load_a4 = [&](const At &o, int r) {
+    auto load_a4 = [&](const GradTile &o, int r) {
         const long px = min(r, H - 1 - o.y0) * W + o.col;
         v[r] = *reinterpret_cast<const uint2 *>(a4 + o.base * CH + px * CH + cg * 4);
     };
-    auto load_err = [&](const At &o) {
+    auto load_err = [&](const GradTile &o) {
 #pragma unroll
         for (int k = 0; k < ND; k++) {
-            const int i = min(tid + 256 * k, HS * WS - 1), gy = o.y0 + i / WS - 1, gx = o.x0 + i % WS - 1;
-            const long p = o.ibase + (long)min(max(gy, 0), H - 1) * W + min(max(gx, 0), W - 1);
+            bool in;
+            const long p = o.halo(min(tid + 256 * k, HS * WS - 1), H, W, in);
             const float d = yn[p] - target[p] / scale;
-            ne[k] = __int_as_float(__float_as_int(d) & -(int)(gy >= 0 && gy < H && gx >= 0 && gx < W));
+            ne[k] = __int_as_float(__float_as_int(d) & -(int)in);
         }
     };
-    const At o0 = at(min((int)blockIdx.x, ntiles - 1));
+    const GradTile o0(tm, min((int)blockIdx.x, ntiles - 1), H, W, col);
     load_err(o0);
 #pragma unroll
     for (int r = 0; r < TH; r++) load_a4(o0, r);
     for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const At o = at(tile), on = at(min(tile + (int)gridDim.x, ntiles - 1));
+        const GradTile o(tm, tile, H, W, col), on(tm, min(tile + (int)gridDim.x, ntiles - 1), H, W, col);
         __syncthreads();  // the previous tile's reads of sdy are done
 #pragma unroll
         for (int k = 0; k < ND; k++) {
@@ -844,20 +859,8 @@ __global__ void __launch_bounds__(256, 2) k_conv_out_back(const float *__restric
         }
         dsum += sdy[(tid / TW + 1) * WS + tid % TW + 1];  // db5: thread tid takes pixel tid of every tile
     }
-    // the lanes of a channel group, then the waves, in a fixed order
-    const int lane = tid & 63, wave = tid >> 6;
-#pragma unroll
-    for (int t = 0; t < 9; t++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-#pragma unroll
-            for (int x = 8; x < 64; x <<= 1) acc[t][e] += __shfl_xor(acc[t][e], x);
-            if (lane < 8) red[wave * 9 * CH + (cg * 4 + e) * 9 + t] = acc[t][e];
-        }
-    __syncthreads();
     float *out = part + (long)blockIdx.x * OUT_REC;
-    for (int i = tid; i < 9 * CH; i += 256)
-        out[i] = ((red[i] + red[9 * CH + i]) + red[2 * 9 * CH + i]) + red[3 * 9 * CH + i];
+    block_sum_taps(acc, red, out);
     // db5 and the loss: the threads' sums in thread order
     __syncthreads();
     red[tid] = dsum;

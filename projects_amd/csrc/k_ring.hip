@@ -18,8 +18,8 @@
 // sequential float sums only by rounding.
 //
 // The data of a slab that fits the 256 MB memory-side cache streams from
-// there: at 16 slices of 900 x 2048 an iteration takes 48 us (40 of them the
-// pass, 236 MB read and written: 5.9 TB/s) where row means, column means (a
+// there: at 16 slices of 900 x 2048 an iteration takes 53 us (about 43 of them
+// the pass, 236 MB read and written: 5.5 TB/s) where row means, column means (a
 // serial column per thread, eight workgroups per slice) and the correction as
 // three passes took 349 us.
 #include <algorithm>
@@ -38,7 +38,7 @@ struct RingArgs {
     int n_ang, n_det, rows, nblocks;  // rows per workgroup, workgroups per slice
     float coeff;
     float *row_mean;   // [n_slices][n_ang]
-    float *mt;         // [n_slices] mean of the row means
+    float2 *mt;        // [n_slices] mean of the row means: rounded, and the rest
     float *est;        // [n_slices][n_det] coeff (c_j - l_j)
     float *part;       // [n_slices][nblocks][n_det] sums of d / m over the workgroup's rows with m != 0
     float *part0;      // the same for d over the rows with m == 0, where flag0 is set
@@ -47,13 +47,13 @@ struct RingArgs {
 
 // Sum over the workgroup; red: two alternating sets of per-wave sums (one
 // barrier per call).
-template <int NT = kRingThreads>
-__device__ __forceinline__ float block_sum(float v, float *red) {
+template <int NT = kRingThreads, typename T>
+__device__ __forceinline__ T block_sum(T v, T *red) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    float s = red[0];
+    T s = red[0];
 #pragma unroll
     for (int w = 1; w < NT / 64; w++) s += red[w];
     return s;
@@ -73,17 +73,33 @@ __global__ void __launch_bounds__(kRingThreads) k_ring_pass(RingArgs A) {
     const long pb = ((long)s * A.nblocks + blockIdx.x) * n;
     float *base = A.sino + s * A.slice_stride;
     const float *est = A.est + (long)s * n;
-    const float mt = FIRST ? 0.0f : A.mt[s];
+    const float2 mt2 = FIRST ? make_float2(0.0f, 0.0f) : A.mt[s];
+    const float mt = mt2.x;
     float *rm = A.row_mean + (long)s * A.n_ang;
     bool zero_rows = false;
-    // value d of a row of mean m after the iteration; rs = mt / m, used where
-    // it is an ordinary number (one product instead of a division per value)
-    auto apply = [&](float d, float m, float rs, bool fast, float e) {
-        if (m != 0.0f) d = fast ? d * rs : d * mt / m;
-        const float t = d - e;
-        return t > 0.0f ? t : 0.0f;
+    // value d of a row of mean m after the iteration, d mt / m - e; where mt / m
+    // is an ordinary number it is taken once per row, with its rounding error
+    // and mt's (which would scale the whole slice, once per iteration), and a value costs two fused multiply-adds: one rounding, where a product,
+    // a quotient and a difference are three
+    struct Scale {
+        float rs, lo;
+        bool fast;
     };
     auto ordinary = [](float x) { return fabsf(x) > 1e-30f && fabsf(x) < 1e30f; };  // false for NaN
+    auto scale_of = [&](float m) {
+        const float rs = mt / m;
+        return Scale{rs, (__builtin_fmaf(-rs, m, mt) + mt2.y) / m, ordinary(rs) && ordinary(m)};
+    };
+    auto apply = [&](float d, float m, const Scale &f, float e) {
+        float t;
+        if (m != 0.0f && f.fast) {
+            t = __builtin_fmaf(d, f.rs, __builtin_fmaf(d, f.lo, -e));
+        } else {
+            if (m != 0.0f) d = d * mt / m;
+            t = d - e;
+        }
+        return t > 0.0f ? t : 0.0f;
+    };
     if constexpr (VPT > 0) {
         constexpr int W = V4 ? 4 : 1;
         auto col = [&](int k) { return W * (tid + kRingThreads * (k / W)) + k % W; };
@@ -113,11 +129,11 @@ __global__ void __launch_bounds__(kRingThreads) k_ring_pass(RingArgs A) {
         for (int i = i0; i < i1; i++) {
             if (i + 1 < i1) load(i + 1, nxt);
             if (!FIRST) {
-                const float m = rm[i], rs = mt / m;
-                const bool fast = ordinary(rs) && ordinary(m);
+                const float m = rm[i];
+                const Scale f = scale_of(m);
                 float *row = base + (long)i * A.row_stride;
 #pragma unroll
-                for (int k = 0; k < VPT; k++) cur[k] = apply(cur[k], m, rs, fast, e[k]);
+                for (int k = 0; k < VPT; k++) cur[k] = apply(cur[k], m, f, e[k]);
 #pragma unroll
                 for (int k = 0; k < VPT; k += W) {
                     const int j = col(k);
@@ -141,7 +157,7 @@ __global__ void __launch_bounds__(kRingThreads) k_ring_pass(RingArgs A) {
                 const float inv = 1.0f / m;
                 if (ordinary(m)) {
 #pragma unroll
-                    for (int k = 0; k < VPT; k++) acc[k] += cur[k] * inv;
+                    for (int k = 0; k < VPT; k++) acc[k] = __builtin_fmaf(cur[k], inv, acc[k]);
                 } else {
 #pragma unroll
                     for (int k = 0; k < VPT; k++) acc[k] += cur[k] / m;
@@ -169,9 +185,9 @@ __global__ void __launch_bounds__(kRingThreads) k_ring_pass(RingArgs A) {
             if (FIRST) {
                 for (int j = tid; j < n; j += kRingThreads) sum += row[j];
             } else {
-                const float m = rm[i], rs = mt / m;
-                const bool fast = ordinary(rs) && ordinary(m);
-                for (int j = tid; j < n; j += kRingThreads) sum += row[j] = apply(row[j], m, rs, fast, est[j]);
+                const float m = rm[i];
+                const Scale f = scale_of(m);
+                for (int j = tid; j < n; j += kRingThreads) sum += row[j] = apply(row[j], m, f, est[j]);
             }
             const float m = block_sum(sum, red[i & 1]) / (float)n;
             if (tid == 0) rm[i] = m;
@@ -190,48 +206,54 @@ __global__ void __launch_bounds__(kRingThreads) k_ring_pass(RingArgs A) {
 
 // The ring estimate coeff (c_j - l_j) of 62 columns of one slice from the
 // partials: 64 columns (one more each side) x 16 groups of workgroups'
-// partials, and the mean of the row means.
+// partials, and the mean of the row means.  In double up to the estimate:
+// c_j - l_j is a small difference of near equals, and an error of the mean scales
+// the whole slice: over 20 iterations 4.6e-7 in all with floats, 1.1e-7
+// so (16 slices of 900 x 2048).
 constexpr int kEstCols = 62, kEstGroups = 16;
 __global__ void __launch_bounds__(64 * kEstGroups) k_ring_columns(RingArgs A) {
-    __shared__ float red[kEstGroups];
-    __shared__ float sa[kEstGroups][64], sb[kEstGroups][64], sc[64];
+    __shared__ double red[kEstGroups];
+    __shared__ double sa[kEstGroups][64], sb[kEstGroups][64], sc[64];
     const int s = blockIdx.y, tid = threadIdx.x, n = A.n_det;
     const int c = tid & 63, g = tid >> 6;
     const int j = min(max((int)blockIdx.x * kEstCols + c - 1, 0), n - 1);
     const float *pa = A.part + (long)s * A.nblocks * n + j, *p0 = A.part0 + (long)s * A.nblocks * n + j;
     const int *f0 = A.flag0 + (long)s * A.nblocks;
-    float a = 0.0f, b = 0.0f;
+    double a = 0.0, b = 0.0;
     for (int k0 = g; k0 < A.nblocks; k0 += 8 * kEstGroups) {  // eight loads in flight
         float v[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) v[u] = k0 + u * kEstGroups < A.nblocks ? pa[(long)(k0 + u * kEstGroups) * n] : 0.0f;
 #pragma unroll
-        for (int u = 0; u < 8; u++) a += v[u];
+        for (int u = 0; u < 8; u++) a += (double)v[u];
     }
     for (int k = g; k < A.nblocks; k += kEstGroups)
-        if (f0[k]) b += p0[(long)k * n];
+        if (f0[k]) b += (double)p0[(long)k * n];
     sa[g][c] = a;
     sb[g][c] = b;
     const float *rm = A.row_mean + (long)s * A.n_ang;
-    float v = 0.0f;
-    for (int i = tid; i < A.n_ang; i += 64 * kEstGroups) v += rm[i];
-    const float mt = block_sum<64 * kEstGroups>(v, red) / (float)A.n_ang;  // its barrier covers sa and sb
-    if (tid == 0 && blockIdx.x == 0) A.mt[s] = mt;
+    double v = 0.0;
+    for (int i = tid; i < A.n_ang; i += 64 * kEstGroups) v += (double)rm[i];
+    const double mt = block_sum<64 * kEstGroups>(v, red) / (double)A.n_ang;  // its barrier covers sa and sb
+    if (tid == 0 && blockIdx.x == 0) {
+        const float hi = (float)mt, lo = (float)(mt - (double)hi);
+        A.mt[s] = make_float2(hi, fabsf(lo) < fabsf(hi) ? lo : 0.0f);  // none beside an infinity or a NaN
+    }
     if (tid < 64) {
-        a = b = 0.0f;
+        a = b = 0.0;
 #pragma unroll
         for (int k = 0; k < kEstGroups; k++) {
             a += sa[k][c];
             b += sb[k][c];
         }
-        sc[c] = (a * mt + b) / (float)A.n_ang;
+        sc[c] = (a * mt + b) / (double)A.n_ang;
     }
     __syncthreads();
     const int jo = (int)blockIdx.x * kEstCols + tid;
     if (tid < kEstCols && jo < n) {
-        const float cm = sc[tid + 1];
-        const float l = (jo == 0 || jo == n - 1) ? cm : (sc[tid] + cm + sc[tid + 2]) / 3.0f;
-        A.est[(long)s * n + jo] = (cm - l) * A.coeff;
+        const double cm = sc[tid + 1];
+        const double l = (jo == 0 || jo == n - 1) ? cm : (sc[tid] + cm + sc[tid + 2]) / 3.0;
+        A.est[(long)s * n + jo] = (float)((cm - l) * (double)A.coeff);
     }
 }
 
@@ -265,7 +287,7 @@ size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
 size_t gr_ring_scratch_bytes(int n_slices, int n_ang, int n_det) {
     const int rows = ring_rows(n_slices, n_ang), nb = (n_ang + rows - 1) / rows;
     const size_t ns = (size_t)n_slices;
-    return up256(4 * ns * n_ang) + up256(4 * ns) + up256(4 * ns * n_det) + 2 * up256(4 * ns * nb * n_det) +
+    return up256(4 * ns * n_ang) + up256(8 * ns) + up256(4 * ns * n_det) + 2 * up256(4 * ns * nb * n_det) +
            up256(4 * ns * nb);
 }
 
@@ -282,7 +304,7 @@ hipError_t gr_launch_ring(float *sino, long slice_stride, long row_stride, int n
         return q;
     };
     A.row_mean = (float *)take(ns * n_ang);
-    A.mt = (float *)take(ns);
+    A.mt = (float2 *)take(2 * ns);
     A.est = (float *)take(ns * n_det);
     A.part = (float *)take(ns * nb * n_det);
     A.part0 = (float *)take(ns * nb * n_det);

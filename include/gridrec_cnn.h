@@ -46,7 +46,9 @@ int gr_cnn_pack(const float *params, unsigned short *packed, void *stream);
  * consecutive ones must be distinct, and a buffer named for two layers ends
  * holding the later one (a3 may alias a1 and a4 a2).  y (may be NULL): the
  * corrected images in the input's units; yn (may be NULL): the same in network
- * units (x/scale + residual), needed by gr_cnn_backward.  slice_stats (may be
+ * units (x/scale + residual), needed by gr_cnn_backward.  y and yn may be x
+ * itself (the last layer is then a kernel of its own, from a4); where one lies
+ * over x otherwise, a stream-ordered copy of x is taken.  slice_stats (may be
  * NULL, needs work): per image, the sums of residual^2 and (x/scale)^2 in
  * network units (2n floats) -- the correction norm of the fallback test. */
 int gr_cnn_forward(const float *params, const unsigned short *packed, const float *x, int n, int H, int W,
@@ -55,7 +57,8 @@ int gr_cnn_forward(const float *params, const unsigned short *packed, const floa
 
 /* Inference: gr_cnn_forward's y and slice_stats (bitwise) with no activation
  * buffers.  work: gr_cnn_infer_work_bytes(n, H, W) bytes when slice_stats is
- * given, else may be NULL. */
+ * given, else may be NULL.  Where y lies over x, a stream-ordered copy of x is
+ * taken. */
 size_t gr_cnn_infer_work_bytes(int n, int H, int W);
 int gr_cnn_infer(const float *params, const unsigned short *packed, const float *x, int n, int H, int W,
                  float scale, float *y, float *slice_stats, void *work, void *stream);

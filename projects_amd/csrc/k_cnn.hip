@@ -410,6 +410,55 @@ __global__ void __launch_bounds__(FW_THREADS) k_forward(FwdArgs P) {
     }
 }
 
+// Layer 5 and the residual alone, from a4: for a forward pass whose y or yn is
+// x itself.  k_forward's workgroups read x around their pixels long after others
+// have written theirs, so there it stores the activations only, and here every
+// lane reads the x of a pixel before it writes that pixel.  A wave takes 16
+// columns and OUT_ROWS rows, the fragments of three rows of a4 in registers; the MFMAs
+// and the additions of an output are k_forward's: bitwise its values.
+constexpr int OUT_ROWS = 16;
+__global__ void __launch_bounds__(256) k_conv_out(const uint16_t *__restrict__ a4, const float *x, float scale,
+                                                  const float *__restrict__ prm, float *y, float *yn, int H, int W,
+                                                  int cols, int segs, long nwaves) {
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    const long w = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (w >= nwaves) return;
+    const long img = w / ((long)cols * segs), ibase = img * H * W;
+    const int r = (int)(w - img * cols * segs), y0 = r / cols * OUT_ROWS, gx = r % cols * 16 + j;
+    bf16x8 A[9];
+    conv_out_frag(prm + OFF_W5, lane, A);
+    const float b5 = prm[OFF_B5];
+    auto load = [&](int gy, bf16x8 (&B)[3]) {  // row gy at columns gx - 1 .. gx + 1, zero outside the image
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const int cx = gx + k - 1;
+            B[k] = bf16x8{};
+            if ((unsigned)gy < (unsigned)H && (unsigned)cx < (unsigned)W)
+                B[k] = *reinterpret_cast<const bf16x8 *>(a4 + (ibase + (long)gy * W + cx) * CH + 8 * g);
+        }
+    };
+    bf16x8 B[3][3];
+    load(y0 - 1, B[0]);
+    load(y0, B[1]);
+    for (int gy = y0; gy < min(y0 + OUT_ROWS, H); gy++) {
+        load(gy + 1, B[2]);
+        floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < 9; t++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[t], B[t / 3][t % 3], acc, 0, 0, 0);
+        if (lane < 16 && gx < W) {
+            const long p = ibase + (long)gy * W + gx;
+            const float v = x[p] / scale + (acc[0] + b5);
+            if (yn) yn[p] = v;
+            if (y) y[p] = v * scale;
+        }
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            B[0][k] = B[1][k];
+            B[1][k] = B[2][k];
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Backward of a 32 -> 32 layer in one pass: the input gradient
 // dzn = bf16(conv^T(dz) * (a > 0)) and the weight gradient's partial sums, from
@@ -1029,6 +1078,29 @@ int run_forward(const float *params, const unsigned short *packed, const float *
     return GR_OK;
 }
 
+// Whether a batch of npx values at p lies over the one at x.
+bool over(const float *x, const float *p, long npx) {
+    const uintptr_t a = (uintptr_t)x, b = (uintptr_t)p, bytes = sizeof(float) * (size_t)npx;
+    return p && a < b + bytes && b < a + bytes;
+}
+
+// run_forward on a copy of x, in stream-ordered memory: where what it writes
+// lies over x and nothing else is left to read x from.
+int run_forward_copy(const float *params, const unsigned short *packed, const float *x, int n, int H, int W,
+                     float scale, uint16_t *const (&act)[4], float *y, float *yn, float *slice_stats, float *stats,
+                     hipStream_t s) {
+    const size_t bytes = sizeof(float) * (size_t)n * H * W;
+    void *copy = nullptr;
+    if (hipMallocAsync(&copy, bytes, s) != hipSuccess)
+        return cnn_fail(GR_ENOMEM, "no device memory for a copy of the images (y or yn lies over x)");
+    const hipError_t e = hipMemcpyAsync(copy, x, bytes, hipMemcpyDeviceToDevice, s);
+    const int rc = e == hipSuccess ? run_forward(params, packed, (const float *)copy, n, H, W, scale, act, y, yn,
+                                                 slice_stats, stats, s)
+                                   : cnn_fail(GR_EHIP, hipGetErrorString(e));
+    (void)hipFreeAsync(copy, s);
+    return rc;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1076,7 +1148,20 @@ int gr_cnn_forward(const float *params, const unsigned short *packed, const floa
     }
     // a buffer named for two layers ends holding the later one
     uint16_t *act[4] = {a1 == a3 || a1 == a4 ? nullptr : a1, a2 == a4 ? nullptr : a2, a3, a4};
-    return run_forward(params, packed, x, n, H, W, scale, act, y, yn, slice_stats, stats, (hipStream_t)stream);
+    hipStream_t s = (hipStream_t)stream;
+    const long npx = (long)n * H * W;
+    if (!over(x, y, npx) && !over(x, yn, npx))
+        return run_forward(params, packed, x, n, H, W, scale, act, y, yn, slice_stats, stats, s);
+    if ((y != x && over(x, y, npx)) || (yn != x && over(x, yn, npx)))
+        return run_forward_copy(params, packed, x, n, H, W, scale, act, y, yn, slice_stats, stats, s);
+    rc = run_forward(params, packed, x, n, H, W, scale, act, nullptr, nullptr, slice_stats, stats, s);
+    if (rc) return rc;
+    const int cols = (W + 15) / 16, segs = (H + OUT_ROWS - 1) / OUT_ROWS;
+    const long nwaves = (long)n * cols * segs;
+    hipLaunchKernelGGL(k_conv_out, dim3((unsigned)((nwaves + 3) / 4)), dim3(256), 0, s, a4, x, scale, params, y, yn, H,
+                       W, cols, segs, nwaves);
+    CNN_HIP(hipGetLastError());
+    return GR_OK;
 }
 
 size_t gr_cnn_infer_work_bytes(int n, int H, int W) {
@@ -1091,6 +1176,9 @@ int gr_cnn_infer(const float *params, const unsigned short *packed, const float 
     if (rc) return rc;
     if (slice_stats && !work) return cnn_fail(GR_EINVAL, "slice statistics need the work buffer");
     uint16_t *act[4] = {nullptr, nullptr, nullptr, nullptr};
+    if (over(x, y, (long)n * H * W))
+        return run_forward_copy(params, packed, x, n, H, W, scale, act, y, nullptr, slice_stats, (float *)work,
+                                (hipStream_t)stream);
     return run_forward(params, packed, x, n, H, W, scale, act, y, nullptr, slice_stats, (float *)work,
                        (hipStream_t)stream);
 }

@@ -101,10 +101,25 @@ class Corrector:
                   "gr_cnn_pack")
 
     # -- passes -----------------------------------------------------------------
+    def _apart(self, x, out, stream):
+        """x, or a copy of it where out lies over it: the network reads x
+        around every pixel while others are written.  The copy is made, and
+        given back, on the stream that reads it."""
+        torch = self.torch
+        nbytes = 4 * x.numel()
+        if out is None or abs(out.data_ptr() - x.data_ptr()) >= nbytes:
+            return x
+        if stream is None:
+            return x.clone()
+        if not isinstance(stream, torch.cuda.Stream):
+            stream = torch.cuda.ExternalStream(gr._stream_handle(stream), device=self.dev)
+        with torch.cuda.stream(stream):
+            return x.clone()
+
     def forward(self, x, out=None, train=False, stream=None):
         """x: cuda float32 [n, H, W] gridrec images.  Returns (y, stats) with
-        y = the corrected images and stats [n, 2] = (sum residual^2, sum
-        (x/scale)^2) per image."""
+        y = the corrected images (in out, which may be x) and stats [n, 2] =
+        (sum residual^2, sum (x/scale)^2) per image."""
         if not train:
             return self.infer(x, out, stream)
         torch = self.torch
@@ -125,6 +140,7 @@ class Corrector:
         torch = self.torch
         assert x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.is_contiguous()
         n, H, W = x.shape
+        x = self._apart(x, out, stream)
         _, work, _, stats = self._buffers(n, H, W, False)
         if out is None:
             out = torch.empty_like(x)
@@ -159,8 +175,10 @@ class Corrector:
     def correct(self, x, out=None, stream=None):
         """Inference with the fallback: images whose relative correction norm
         ||residual|| / ||x/scale|| exceeds the threshold keep the plain image.
-        Returns (y, used) with used[i] True where the network's output was kept."""
+        Returns (y, used) with used[i] True where the network's output was kept;
+        out may be x."""
         torch = self.torch
+        x = self._apart(x, out, stream)
         y, stats = self.forward(x, out=out, stream=stream)
         s = torch.cuda.current_stream() if stream is None else stream
         with torch.cuda.stream(s):  # device-side selection, no host synchronisation

@@ -404,3 +404,111 @@ def test_forward_aliased_activations():
                                       p(b[0]), p(b[1]), p(y2), p(None), p(None), p(None), C.c_void_p(0)), "forward")
     torch.cuda.synchronize()
     assert torch.equal(y, y2) and torch.equal(b[0], acts[2]) and torch.equal(b[1], acts[3])
+
+
+# outputs over the input: the forward kernel reads x with a halo of five pixels
+# while other strips of 56 columns and segments of rows are written, so images of
+# several of both, and of one
+INPLACE_SHAPES = [(1, 20, 30), (2, 75, 130), (3, 300, 61), (1, 16, 300)]
+
+
+@pytest.mark.parametrize("shape", INPLACE_SHAPES)
+def test_forward_in_place(shape):
+    """forward, infer and correct with out=x: bitwise the images, sums and
+    choices of a separate output."""
+    net, _, x, _ = make(sum(shape), *shape)
+    xg = torch.from_numpy(x).cuda()
+    for train in (True, False):
+        y, s = net.forward(xg, train=train)
+        y, s = y.clone(), s.clone()
+        z = xg.clone()
+        out, s2 = net.forward(z, out=z, train=train)
+        torch.cuda.synchronize()
+        assert out is z and torch.equal(z, y) and torch.equal(s, s2)
+    z = xg.clone()
+    net.infer(z, out=z)
+    assert torch.equal(z, y)
+    rel_norm = torch.sqrt(s[:, 0] / s[:, 1])
+    for net.threshold in (float(rel_norm.min()), 0.0, 1e9):  # one, none, all kept
+        y, used = net.correct(xg)
+        z = xg.clone()
+        out, used2 = net.correct(z, out=z)
+        torch.cuda.synchronize()
+        assert out is z and torch.equal(z, y) and torch.equal(used, used2)
+        for i in range(shape[0]):
+            assert bool(used[i]) or torch.equal(z[i], xg[i])
+
+
+@pytest.mark.parametrize("shape", INPLACE_SHAPES)
+def test_c_entries_in_place(shape):
+    """The C entries with y or yn at x, or part of the way over it: bitwise the
+    outputs of separate buffers, the activations and sums among them."""
+    import ctypes as C
+
+    from projects_amd import gridrec as gr
+
+    net, _, x, _ = make(sum(shape), *shape)
+    n, H, W = shape
+    xg = torch.from_numpy(x).cuda()
+    y0, s0 = net.forward(xg, train=True)
+    acts, work, yn0, _ = net._buffers(n, H, W, True)
+    y0, s0, yn0 = y0.clone(), s0.clone(), yn0.clone()
+    a4 = acts[3].clone()
+    L = gr.lib()
+    p = lambda t: C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p(None)
+    npx = n * H * W
+
+    def forward(xv, y, yn, a, st=None, wk=None):
+        gr._check(L.gr_cnn_forward(p(net.params), p(net.packed), p(xv), n, H, W, net.scale, *[p(t) for t in a], p(y),
+                                   p(yn), p(st), p(wk), C.c_void_p(gr._stream_handle(None))), "gr_cnn_forward")
+        torch.cuda.synchronize()
+
+    def room(shift):  # a copy of x and an output `shift` floats further on
+        buf = torch.zeros(npx + abs(shift), device="cuda")
+        xv = buf[max(-shift, 0):max(-shift, 0) + npx].view(shape)
+        xv.copy_(xg)
+        return xv, buf[max(shift, 0):max(shift, 0) + npx].view(shape)
+
+    for shift in (0, 1, -W, npx // 2):
+        xv, out = room(shift)
+        forward(xv, out, None, acts)
+        assert torch.equal(out, y0) and torch.equal(acts[3], a4), shift
+        xv, out = room(shift)
+        other, st = torch.empty_like(xg), torch.empty_like(s0)
+        forward(xv, other, out, acts, st, work)
+        assert torch.equal(out, yn0) and torch.equal(other, y0) and torch.equal(st, s0), shift
+        xv, out = room(shift)
+        forward(xv, out, other, [acts[0], acts[1], acts[0], acts[1]])
+        assert torch.equal(out, y0) and torch.equal(other, yn0) and torch.equal(acts[1], a4), shift
+        xv, out = room(shift)
+        gr._check(L.gr_cnn_infer(p(net.params), p(net.packed), p(xv), n, H, W, net.scale, p(out), p(None), p(None),
+                                 C.c_void_p(gr._stream_handle(None))), "gr_cnn_infer")
+        torch.cuda.synchronize()
+        assert torch.equal(out, y0), shift
+
+
+def test_forward_in_place_captured():
+    """In-place inference as a graph on a stream of its own: every replay, with
+    other work in between, gives the eager images."""
+    net, _, x, _ = make(4, 2, 75, 130)
+    xg = torch.from_numpy(x).cuda()
+    y, _ = net.forward(xg)
+    y = y.clone()
+    s = torch.cuda.Stream()
+    z = xg.clone()
+    s.wait_stream(torch.cuda.current_stream())
+    net.forward(z, out=z, stream=s)
+    s.synchronize()
+    assert torch.equal(z, y)
+    z.copy_(xg)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        net.forward(z, out=z)
+    for _ in range(3):
+        z.copy_(xg)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(z, y)
+        torch.randn(1 << 20, device="cuda").mul_(2.0)
+        net.forward(torch.ones_like(xg))
+        torch.cuda.synchronize()

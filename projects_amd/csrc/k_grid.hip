@@ -1415,6 +1415,9 @@ hipError_t launch(const GridArgs &A, const GopArgs *O, int groups, size_t lds_ba
             hipLaunchKernelGGL((k_grid_op<ACCUM, P, true>), dim3(sblocks, groups), dim3(256), lds, s, A, o);
         return hipGetLastError();
     }
+    // fewer waves beside convolvent tables that leave no room for wpb of them
+    // (interp keeps two tables: ltbl above 16127 with four waves of eight pairs)
+    while (wpb > 1 && lds_base + grid_wave_lds<P>() * wpb > (size_t)gr_max_lds_per_block()) wpb /= 2;
     const size_t lds = lds_base + grid_wave_lds<P>() * wpb;
     hipError_t e = gr_allow_lds(k_grid<ACCUM, P>, lds);
     if (e != hipSuccess) return e;

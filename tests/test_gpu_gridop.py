@@ -226,3 +226,31 @@ def test_plain_heavy_tiles(n_ang, n_det, ns):
     out5 = gr.Plan(**case, grid_op="on", max_pairs=5).recon(sino)
     torch.cuda.synchronize()
     assert torch.equal(out, ref) and torch.equal(out5, ref)
+
+
+# the convolvent's two tables (interp) and the waves' sample slots in one
+# workgroup's LDS, whose four waves are a queue's default: 16127 is the last
+# table that leaves room for four waves of eight pairs, 16384 the largest
+@pytest.mark.parametrize("ltbl", [16126, 16127, 16128, 16383, 16384])
+@pytest.mark.parametrize("accum", ["compensated", "plain"])
+def test_geometry_kernel_largest_tables(ltbl, accum):
+    """A queue's images (one pair, four, a full and a partial group of eight)
+    bitwise the operator's."""
+    kw = dict(n_ang=60, n_det=50, center=25.2, interp=True, ltbl=ltbl, accum=accum)
+    p = gr.Plan(**kw, grid_op="on")
+    sets, ref = [], []
+    for ns in (2, 8, 10, 18):
+        sino = sinos(kw, ns, ns)
+        ref.append(p.recon(sino))
+        sets.append((dict(kw, grid_op="off"), sino, torch.full_like(ref[-1], float("nan"))))
+    for autotune in (False, True):
+        q = gr.Queue(sets, autotune=autotune)
+        q.run()
+        torch.cuda.synchronize()
+        for d, (r, (_, _, out)) in enumerate(zip(ref, sets)):
+            if q.settings(d)["fft_radix"] == 16:
+                assert torch.equal(r, out), d
+            else:
+                assert O.rel_l2(out.cpu().numpy(), r.cpu().numpy()) <= 1e-5, d
+        q.close()
+    p.close()

@@ -817,13 +817,15 @@ __global__ void __launch_bounds__(256, 2) k_conv_out_back(const float *__restric
                                                           int W, int ntiles, TileMap tm) {
     __shared__ float sdy[HS * WS];
     __shared__ __align__(16) float sw[9 * CH];  // [t][ci]
+    __shared__ double dred[2][4];
     __shared__ float red[4 * 9 * CH];
     constexpr int KB = 4;                      // rows at a time
     constexpr int ND = (HS * WS + 255) / 256;  // halo values per thread
     static_assert(TW * 8 == 256 && TH % KB == 0, "a thread per column and 4 channels");
     const int tid = threadIdx.x, cg = tid & 7, col = tid >> 3;
     for (int i = tid; i < 9 * CH; i += 256) sw[i] = round_bf16(prm[OFF_W5 + (i % CH) * 9 + i / CH]);
-    float acc[9][4], dsum = 0.0f, lsum = 0.0f;
+    float acc[9][4], dsum = 0.0f;
+    double lsum = 0.0;
 #pragma unroll
     for (int t = 0; t < 9; t++)
 #pragma unroll
@@ -855,7 +857,7 @@ __global__ void __launch_bounds__(256, 2) k_conv_out_back(const float *__restric
         for (int k = 0; k < ND; k++) {
             const int i = tid + 256 * k, r = i / WS - 1, c = i % WS - 1;
             if (i < HS * WS) sdy[i] = 2.0f * ne[k] / fN;
-            if (r >= 0 && r < TH && c >= 0 && c < TW) lsum += ne[k] * ne[k];
+            if (r >= 0 && r < TH && c >= 0 && c < TW) lsum += (double)ne[k] * (double)ne[k];
         }
         __syncthreads();
         load_err(on);
@@ -910,18 +912,26 @@ __global__ void __launch_bounds__(256, 2) k_conv_out_back(const float *__restric
     }
     float *out = part + (long)blockIdx.x * OUT_REC;
     block_sum_taps(acc, red, out);
-    // db5 and the loss: the threads' sums in thread order
-    __syncthreads();
-    red[tid] = dsum;
-    red[256 + tid] = lsum;
+    // db5 and the loss: pairwise over the lanes, then over the waves, in double
+    // -- one large error must not swallow a tile of small ones
+    const int lane = tid & 63, wave = tid >> 6;
+    double s5 = dsum, sl = lsum;
+#pragma unroll
+    for (int h = 32; h > 0; h >>= 1) {
+        s5 += __shfl_xor(s5, h);
+        sl += __shfl_xor(sl, h);
+    }
+    if (lane == 0) {
+        dred[0][wave] = s5;
+        dred[1][wave] = sl;
+    }
     __syncthreads();
     if (tid < 2) {
-        float s5 = 0.0f;
-        for (int i = 0; i < 256; i++) s5 += red[tid * 256 + i];
+        const float v = (float)((dred[tid][0] + dred[tid][1]) + (dred[tid][2] + dred[tid][3]));
         if (tid == 0)
-            out[9 * CH] = s5;
+            out[9 * CH] = v;
         else
-            lpart[blockIdx.x] = s5;
+            lpart[blockIdx.x] = v;
     }
 }
 

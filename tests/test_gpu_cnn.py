@@ -512,3 +512,23 @@ def test_forward_in_place_captured():
         torch.randn(1 << 20, device="cuda").mul_(2.0)
         net.forward(torch.ones_like(xg))
         torch.cuda.synchronize()
+
+
+# one value whose square no float sum of a workgroup's pixels can hold beside
+# theirs: 2^26 against squares below one
+@pytest.mark.parametrize("n,H,W,hot", [(1, 8, 32, 0), (1, 8, 32, 255), (3, 40, 70, 4321), (40, 128, 128, 77)])
+def test_loss_of_uneven_errors(n, H, W, hot):
+    """The loss against a sum in 64 bits.  Sums in double round twice, to a
+    workgroup's float partial and to the result, by 2^-24 each."""
+    net = Lrn.Corrector(params=np.zeros(28353, np.float32), scale=1.0)  # yn = x
+    x = np.random.default_rng(hot).uniform(0.5, 0.99, (n, H, W)).astype(np.float32)
+    x.reshape(-1)[hot] = 8192.0
+    xg, t = torch.from_numpy(x).cuda(), torch.zeros((n, H, W), device="cuda")
+    net.forward(xg, train=True)
+    net.backward(xg, t)
+    torch.cuda.synchronize()
+    loss = np.mean(x.astype(np.float64) ** 2)
+    assert abs(float(net.loss.cpu()) - loss) <= 2.0 ** -23 * loss
+    g = Lrn.unflatten(net.grads.cpu().numpy())
+    db5 = np.sum(2.0 * x.astype(np.float64)) / x.size
+    assert abs(float(g["b5"][0]) - db5) <= 2.0 ** -20 * np.sum(np.abs(2.0 * x)) / x.size

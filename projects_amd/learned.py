@@ -82,11 +82,13 @@ class Corrector:
         self.pack()
 
     # -- buffers ----------------------------------------------------------------
-    def _buffers(self, n, H, W, train):
-        key = (n, H, W, train)
+    def _buffers(self, n, H, W, train, infer=False):
+        """Buffers of forward() or (infer=True) infer(): each keeps its own, so
+        the sums one returned stay while the other runs."""
+        key = (n, H, W, train, infer)
         if key not in self._bufs:
             torch = self.torch
-            for k in [k for k in self._bufs if k[3] == train]:  # keep one shape per mode
+            for k in [k for k in self._bufs if k[3:] == key[3:]]:  # keep one shape per mode
                 del self._bufs[k]
             acts_l = [torch.empty((n, H, W, CH), dtype=torch.int16, device=self.dev) for _ in range(4 if train else 0)]
             wb = gr.lib().gr_cnn_work_bytes(n, H, W) if train else gr.lib().gr_cnn_infer_work_bytes(n, H, W)
@@ -121,7 +123,7 @@ class Corrector:
         y = the corrected images (in out, which may be x) and stats [n, 2] =
         (sum residual^2, sum (x/scale)^2) per image."""
         if not train:
-            return self.infer(x, out, stream)
+            return self._infer(x, out, stream, False)
         torch = self.torch
         assert x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.is_contiguous()
         n, H, W = x.shape
@@ -137,11 +139,14 @@ class Corrector:
     def infer(self, x, out=None, stream=None):
         """Inference: the training forward's kernel (bitwise its y and stats)
         writing no activations.  Returns (y, stats)."""
+        return self._infer(x, out, stream, True)
+
+    def _infer(self, x, out, stream, infer):
         torch = self.torch
         assert x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.is_contiguous()
         n, H, W = x.shape
         x = self._apart(x, out, stream)
-        _, work, _, stats = self._buffers(n, H, W, False)
+        _, work, _, stats = self._buffers(n, H, W, False, infer)
         if out is None:
             out = torch.empty_like(x)
         rc = gr.lib().gr_cnn_infer(_ptr(self.params), _ptr(self.packed), _ptr(x), n, H, W, self.scale, _ptr(out),

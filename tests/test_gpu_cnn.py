@@ -532,3 +532,18 @@ def test_loss_of_uneven_errors(n, H, W, hot):
     g = Lrn.unflatten(net.grads.cpu().numpy())
     db5 = np.sum(2.0 * x.astype(np.float64)) / x.size
     assert abs(float(g["b5"][0]) - db5) <= 2.0 ** -20 * np.sum(np.abs(2.0 * x)) / x.size
+
+
+def test_forward_and_infer_keep_their_sums():
+    """The sums forward() returned are still its image's after infer() on
+    another, and the other way round."""
+    net, _, x, _ = make(8, 2, 40, 70)
+    a, b = torch.from_numpy(x).cuda(), torch.from_numpy(3.0 * x).cuda()
+    want = [net.forward(v, train=True)[1].clone() for v in (a, b)]
+    s1 = net.forward(a)[1]
+    s2 = net.infer(b)[1]
+    torch.cuda.synchronize()
+    assert torch.equal(s1, want[0]) and torch.equal(s2, want[1])
+    net.forward(b)
+    torch.cuda.synchronize()
+    assert torch.equal(s2, want[1])

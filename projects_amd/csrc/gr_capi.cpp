@@ -148,7 +148,7 @@ int plan_stream(gr_plan *pl, hipStream_t *s) {
 
 // Tiles with more rows than this take the heavy path: a few dozen near the
 // centre of the grid, whose thousands of rows would otherwise make the launch
-// wait for their waves.  With plain sums, 8 pairs of 451 x 777 (whole call):
+// wait for their waves.  With plain sums, 16 pairs of 451 x 777 (whole call):
 // 350 us at 32 rows, 298 at 64, 299 at 96, 341 at 256.
 constexpr unsigned kGopHeavyRows = 64;
 

@@ -862,6 +862,7 @@ struct GopArgs {
     // (GrDevTables), and their partials
     const uint2 *hitems;
     int n_hitems;
+    int heavy_wide;  // plain sums: an item takes a workgroup, not a wave
     const uint4 *hmeta;
     const uint2 *hseg;
     const unsigned *hsplit;
@@ -904,12 +905,14 @@ __device__ __forceinline__ void gop_consume(uint2 t, const float2 (&v)[P], float
 
 constexpr int kHeavyBatch = 16;  // rows loaded at once on the one-pair path
 
-// The one-pair-per-wave path, for compensated sums whose heavy tiles are not
-// cut (partials that the scratch does not hold): the P pairs of a group go to P
+// The one-pair-per-wave path, for plain sums in launches of many heavy items and
+// for compensated sums whose heavy tiles are not cut (partials that the
+// scratch does not hold): the P pairs of a group go to P
 // wavefronts, which stream the tile's rows kHeavyBatch at a time (the batch's
 // sample loads, then the next batch's entry loads, then the batch's adds), so
 // each wave has many loads in flight instead of a chain of dependent ones.
 // Per cell and pair the float operations are those of the wide path.
+template <int ACCUM>
 __device__ __forceinline__ void grid_op_heavy(const GridArgs &A, const GopArgs &O, int ti, int pair, int lane) {
     const unsigned tt = A.tiles[ti];
     const int tx = (int)(tt & 0xffffu), ty = (int)(tt >> 16);
@@ -924,7 +927,7 @@ __device__ __forceinline__ void grid_op_heavy(const GridArgs &A, const GopArgs &
         // a slot no sample reaches: no entry may be read (n - 1 would wrap and
         // the clamped prefetch below would run past the tile's entries); the
         // cells are still stored as zeros, which the row transform reads
-        store_cells<GR_ACCUM_COMPENSATED, 1>(A, pair, 1, a, b, acc);
+        store_cells<ACCUM, 1>(A, pair, 1, a, b, acc);
         return;
     }
     auto entry = [&](unsigned k) {
@@ -945,11 +948,11 @@ __device__ __forceinline__ void grid_op_heavy(const GridArgs &A, const GopArgs &
 #pragma unroll
         for (int i = 0; i < kHeavyBatch; i++) tn[i] = entry(k0 + kHeavyBatch + i);
 #pragma unroll
-        for (int i = 0; i < kHeavyBatch; i++) gop_consume<GR_ACCUM_COMPENSATED, 1>(t[i], v[i], acc, part);
+        for (int i = 0; i < kHeavyBatch; i++) gop_consume<ACCUM, 1>(t[i], v[i], acc, part);
 #pragma unroll
         for (int i = 0; i < kHeavyBatch; i++) t[i] = tn[i];
     }
-    store_cells<GR_ACCUM_COMPENSATED, 1>(A, pair, 1, a, b, acc);
+    store_cells<ACCUM, 1>(A, pair, 1, a, b, acc);
 }
 
 constexpr int kHeavyPlainBatch = 12;  // sixteen spill; eight cost 1% of the whole call
@@ -960,8 +963,8 @@ constexpr int kHeavyPlainBatch = 12;  // sixteen spill; eight cost 1% of the who
 // batch of rows (170 of them at the centre of 451 angles).  So the four waves
 // gather kHeavyPlainBatch rows each and put the products into LDS, and the first
 // adds all of them in order while the next ones arrive: the same products and
-// the same adds.  8 pairs of 451 x 777: k_grid_op<1, 8> 333 us with a pair per
-// wave, 146 this way.
+// the same adds.  16 pairs of 451 x 777: k_grid_op<1, 8> 333 us with a pair per
+// wave, 146 this way (heavy_wide: which launches take which).
 __device__ __forceinline__ void grid_op_heavy_plain(const GridArgs &A, const GopArgs &O, int ti, int pair, int wave,
                                                     int lane, float2 *prod) {
     const unsigned tt = A.tiles[ti];
@@ -1283,12 +1286,11 @@ __global__ void __launch_bounds__(256) k_gop_merge(GridArgs A, GopArgs O, int pa
     store_cells<GR_ACCUM_COMPENSATED, 1>(A, pair, 1, a, b, acc);
 }
 
-// Workgroups of k_grid_op given to the heavy items -- one a wave, plain sums
-// one a workgroup -- (a multiple of the sector count, so the other workgroups
+// Workgroups of k_grid_op given to the heavy items -- one a wave, or (wide) one
+// a workgroup -- (a multiple of the sector count, so the other workgroups
 // keep their XCD-to-sector map).
-template <int ACCUM>
-__host__ __device__ __forceinline__ int heavy_blocks(int n_items) {
-    constexpr int per = (ACCUM == GR_ACCUM_PLAIN ? 1 : 4) * kGridSectors;
+__host__ __device__ __forceinline__ int heavy_blocks(int n_items, bool wide) {
+    const int per = (wide ? 1 : 4) * kGridSectors;
     return (n_items + per - 1) / per * kGridSectors;
 }
 
@@ -1297,7 +1299,7 @@ __host__ __device__ __forceinline__ int heavy_blocks(int n_items) {
 // from the streamed entries: with compensated sums one segment of a cut tile
 // per wave for the P pairs of the group (grid_op_tile; k_gop_merge sums the
 // partials afterwards), otherwise a tile one pair per wave (grid_op_heavy) or,
-// with plain sums, per workgroup (grid_op_heavy_plain).
+// with plain sums and heavy_wide, per workgroup (grid_op_heavy_plain).
 // The others take one tile per wave for the P pairs -- SOP: from the staged
 // operator (grid_sop_light), otherwise from the streamed entries
 // (grid_op_tile).
@@ -1325,11 +1327,12 @@ __global__ void __launch_bounds__(256, 4) k_grid_op(GridArgs A, GopArgs O) {
     // SOP: the persistent light workgroups first (they start at once and
     // hold most of the machine), the heavy items after them in the slots
     // left; otherwise the heavy items first (their long chains start early)
-    const int hb = heavy_blocks<ACCUM>(O.n_hitems);
+    const bool wide = ACCUM == GR_ACCUM_PLAIN && O.heavy_wide;
+    const int hb = heavy_blocks(O.n_hitems, wide);
     const int nlight = SOP ? 2 * O.sop_waves : 0;  // kGridSectors * sop_waves / 4
     const int hbx = bx - nlight;
     if (hbx >= 0 && hbx < hb) {
-        if (ACCUM == GR_ACCUM_PLAIN) {
+        if (wide) {
             // workgroup: a heavy tile and one of its pairs
             if (hbx >= O.n_hitems) return;
             const uint2 it = O.hitems[hbx];
@@ -1345,11 +1348,11 @@ __global__ void __launch_bounds__(256, 4) k_grid_op(GridArgs A, GopArgs O) {
         const uint2 it = O.hitems[min(item, O.n_hitems - 1)];
         const int ti = (int)it.x;
         if (item >= O.n_hitems || A.tiles[ti] == kGridNoTile) return;
-        if (O.hmeta) {
+        if (ACCUM == GR_ACCUM_COMPENSATED && O.hmeta) {
             grid_op_tile<ACCUM, P>(A, O, ti, (int)it.y, pair0, nvalid, lane);
         } else {
             const int p = (int)it.y;  // tiles not cut: one item per pair
-            if (p < nvalid) grid_op_heavy(A, O, ti, pair0 + p, lane);
+            if (p < nvalid) grid_op_heavy<ACCUM>(A, O, ti, pair0 + p, lane);
         }
         return;
     }
@@ -1387,22 +1390,40 @@ __host__ inline int sop_blocks_per_sector(int light, int groups) {
     return std::max(1, std::min(light, total / groups));
 }
 
+// Whether the heavy tiles of plain sums take a workgroup per tile and pair instead
+// of a wave.  While the launch waits for its longest chains of round trips --
+// the tiles at the centre -- four waves a chain shorten them; once the others
+// fill the chip for that long, the detour through LDS costs.  A tile at distance r
+// has 1/r of the centre's rows and the heavy ones reach as far as they have 64,
+// so n tiles are the work of some sqrt(n) centre tiles, and the line lies at a
+// multiple of pairs * sqrt(n).  Gridding wide and narrow, us: pairs * sqrt(n) =
+// 425 (8 pairs of 1800 x 1200) 1183 and 1871, 650 (16 of 1800 x 820) 1237 and
+// 1521, 794 (32 of 900 x 1470) 922 and 1013, 850 (16 of 1800 x 1300) 2042 and 2066;
+// 905 (32 of 1300 x 230) 802 and 780, 966 (32 of 1300 x 820) 1368 and 1272, 1032
+// (32 of 1800 x 500) 1500 and 1256, 1700 (32 of 1800 x 1300) 3981 and 3430.
+__host__ inline bool heavy_wide(int n_hitems, int pairs) {
+    const double tiles = n_hitems / kSpecGroup;
+    return tiles * pairs * pairs <= 870.0 * 870.0;
+}
+
 template <int ACCUM, int P>
 hipError_t launch(const GridArgs &A, const GopArgs *O, int groups, size_t lds_base, int wpb, hipStream_t s) {
     if (O) {
         const int light = (A.sector_len - O->n_heavy + 3) / 4;
-        const int blocks = heavy_blocks<ACCUM>(O->n_hitems) + kGridSectors * light;
-        const size_t heavy_lds = ACCUM == GR_ACCUM_PLAIN ? kHeavyPlainLds : 0;
+        GopArgs o = *O;
+        o.heavy_wide = ACCUM == GR_ACCUM_PLAIN && heavy_wide(O->n_hitems, std::min(groups * P, A.pair_end - A.pair_base));
+        const int hblocks = heavy_blocks(O->n_hitems, o.heavy_wide);
+        const size_t heavy_lds = o.heavy_wide ? kHeavyPlainLds : 0;
         if (!O->sop_tile) {
-            hipLaunchKernelGGL((k_grid_op<ACCUM, P, false>), dim3(blocks, groups), dim3(256), heavy_lds, s, A, *O);
+            hipLaunchKernelGGL((k_grid_op<ACCUM, P, false>), dim3(hblocks + kGridSectors * light, groups), dim3(256),
+                               heavy_lds, s, A, o);
             return hipGetLastError();
         }
         // the staged light tiles: persistent workgroups (up to 8 groups of
         // pairs interleaved)
         const int G = groups <= 8 ? groups : 1;
         const int lb = sop_blocks_per_sector(light, G);
-        const int sblocks = heavy_blocks<ACCUM>(O->n_hitems) + kGridSectors * lb;
-        GopArgs o = *O;
+        const int sblocks = hblocks + kGridSectors * lb;
         o.sop_waves = 4 * lb;
         o.sop_groups = G;
 

@@ -254,3 +254,18 @@ def test_geometry_kernel_largest_tables(ltbl, accum):
                 assert O.rel_l2(out.cpu().numpy(), r.cpu().numpy()) <= 1e-5, d
         q.close()
     p.close()
+
+
+@pytest.mark.parametrize("n_ang,n_det,ns", [(900, 140, 64), (905, 141, 75)])
+def test_plain_heavy_tiles_of_full_launches(n_ang, n_det, ns):
+    """Plain sums of so many heavy tiles and pairs (some thousand tiles of more
+    than 64 rows, 32 pairs and a partial group more) that each takes one wave:
+    in one launch, bitwise the geometry kernel's images and those of launches of
+    three pairs (a workgroup per tile and pair)."""
+    case = dict(n_ang=n_ang, n_det=n_det, center=n_det / 2.0 + 0.3, accum="plain", pad="half")
+    sino = sinos(case, ns, n_ang)
+    ref = gr.Plan(**case, grid_op="off").recon(sino)
+    for mp in ((ns + 1) // 2, 3):
+        out = gr.Plan(**case, grid_op="on", max_pairs=mp).recon(sino)
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref), mp

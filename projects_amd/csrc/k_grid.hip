@@ -862,7 +862,6 @@ struct GopArgs {
     // (GrDevTables), and their partials
     const uint2 *hitems;
     int n_hitems;
-    int heavy_wide;  // plain sums: an item takes a workgroup, not a wave
     const uint4 *hmeta;
     const uint2 *hseg;
     const unsigned *hsplit;
@@ -1299,11 +1298,11 @@ __host__ __device__ __forceinline__ int heavy_blocks(int n_items, bool wide) {
 // from the streamed entries: with compensated sums one segment of a cut tile
 // per wave for the P pairs of the group (grid_op_tile; k_gop_merge sums the
 // partials afterwards), otherwise a tile one pair per wave (grid_op_heavy) or,
-// with plain sums and heavy_wide, per workgroup (grid_op_heavy_plain).
+// WIDE (plain sums, where heavy_wide), per workgroup (grid_op_heavy_plain).
 // The others take one tile per wave for the P pairs -- SOP: from the staged
 // operator (grid_sop_light), otherwise from the streamed entries
 // (grid_op_tile).
-template <int ACCUM, int P, bool SOP>
+template <int ACCUM, int P, bool SOP, bool WIDE>
 __global__ void __launch_bounds__(256, 4) k_grid_op(GridArgs A, GopArgs O) {
     extern __shared__ float smem[];  // staged operator: wtbl, then the waves' record slots
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -1327,12 +1326,11 @@ __global__ void __launch_bounds__(256, 4) k_grid_op(GridArgs A, GopArgs O) {
     // SOP: the persistent light workgroups first (they start at once and
     // hold most of the machine), the heavy items after them in the slots
     // left; otherwise the heavy items first (their long chains start early)
-    const bool wide = ACCUM == GR_ACCUM_PLAIN && O.heavy_wide;
-    const int hb = heavy_blocks(O.n_hitems, wide);
+    const int hb = heavy_blocks(O.n_hitems, WIDE);
     const int nlight = SOP ? 2 * O.sop_waves : 0;  // kGridSectors * sop_waves / 4
     const int hbx = bx - nlight;
     if (hbx >= 0 && hbx < hb) {
-        if (wide) {
+        if (WIDE) {
             // workgroup: a heavy tile and one of its pairs
             if (hbx >= O.n_hitems) return;
             const uint2 it = O.hitems[hbx];
@@ -1383,10 +1381,17 @@ __global__ void __launch_bounds__(256, 4) k_grid_op(GridArgs A, GopArgs O) {
 // group (0.49 -> 0.51 at 1500 x 2048).  And a wave should have some ten tiles
 // to take, down to 48 workgroups: the heavy chains of a small grid run
 // faster beside fewer light waves (one pair of 180 x 256 27 -> 25 us, of
-// 360 x 512 46 -> 42).
-__host__ inline int sop_blocks_per_sector(int light, int groups) {
+// 360 x 512 46 -> 42) -- unless a few pairs' light tiles are what the launch
+// waits for: from some 640 angles on up to M = 1024 (one pair of 600 x 500 at M =
+// 512 43.6 us with 48 and 45.6 with 96, of 900 x 500 69 and 59; at M = 1024 400 x
+// 500 44 and 45, 900 x 500 84 and 75; eight pairs gain nothing, nor 1800 angles
+// at M = 512: four pairs of 1800 x 500 657 and 710), and at M = 1024 below some 160, where every tile is one round trip
+// (60 x 500 28 and 22, 180 x 500 36 and 36).
+__host__ inline int sop_blocks_per_sector(int light, int groups, int pairs, int n_ang) {
     const int most = groups > 1 && light >= 1024 ? 128 : 96;
-    const int total = std::min(most, std::max(48, light * groups / 10));
+    const bool waits_for_light = pairs < kSpecGroup && light < 1024 &&
+                                 (light > 300 ? n_ang > 640 || n_ang < 160 : n_ang > 640 && n_ang < 1500);
+    const int total = waits_for_light ? most : std::min(most, std::max(48, light * groups / 10));
     return std::max(1, std::min(light, total / groups));
 }
 
@@ -1406,35 +1411,39 @@ __host__ inline bool heavy_wide(int n_hitems, int pairs) {
     return tiles * pairs * pairs <= 870.0 * 870.0;
 }
 
+template <int ACCUM, int P, bool WIDE>
+hipError_t launch_op(const GridArgs &A, GopArgs o, int groups, size_t lds_base, hipStream_t s) {
+    const int light = (A.sector_len - o.n_heavy + 3) / 4;
+    const int heavy = heavy_blocks(o.n_hitems, WIDE);
+    const size_t heavy_lds = WIDE ? kHeavyPlainLds : 0;
+    if (!o.sop_tile) {
+        hipLaunchKernelGGL((k_grid_op<ACCUM, P, false, WIDE>), dim3(heavy + kGridSectors * light, groups), dim3(256),
+                           heavy_lds, s, A, o);
+        return hipGetLastError();
+    }
+    // the staged light tiles: persistent workgroups (up to 8 groups of
+    // pairs interleaved)
+    const int G = groups <= 8 ? groups : 1;
+    const int lb = sop_blocks_per_sector(light, G, P, A.n_ang);
+    const int blocks = heavy + kGridSectors * lb;
+    o.sop_waves = 4 * lb;
+    o.sop_groups = G;
+    const size_t lds = lds_base + std::max(heavy_lds, sizeof(float2) * 4 * kSopSlots * P);
+    hipError_t e = gr_allow_lds(k_grid_op<ACCUM, P, true, WIDE>, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((k_grid_op<ACCUM, P, true, WIDE>), G > 1 ? dim3(G * blocks, 1) : dim3(blocks, groups), dim3(256), lds,
+                       s, A, o);
+    return hipGetLastError();
+}
+
 template <int ACCUM, int P>
 hipError_t launch(const GridArgs &A, const GopArgs *O, int groups, size_t lds_base, int wpb, hipStream_t s) {
     if (O) {
-        const int light = (A.sector_len - O->n_heavy + 3) / 4;
-        GopArgs o = *O;
-        o.heavy_wide = ACCUM == GR_ACCUM_PLAIN && heavy_wide(O->n_hitems, std::min(groups * P, A.pair_end - A.pair_base));
-        const int hblocks = heavy_blocks(O->n_hitems, o.heavy_wide);
-        const size_t heavy_lds = o.heavy_wide ? kHeavyPlainLds : 0;
-        if (!O->sop_tile) {
-            hipLaunchKernelGGL((k_grid_op<ACCUM, P, false>), dim3(hblocks + kGridSectors * light, groups), dim3(256),
-                               heavy_lds, s, A, o);
-            return hipGetLastError();
+        if constexpr (ACCUM == GR_ACCUM_PLAIN) {
+            if (heavy_wide(O->n_hitems, std::min(groups * P, A.pair_end - A.pair_base)))
+                return launch_op<ACCUM, P, true>(A, *O, groups, lds_base, s);
         }
-        // the staged light tiles: persistent workgroups (up to 8 groups of
-        // pairs interleaved)
-        const int G = groups <= 8 ? groups : 1;
-        const int lb = sop_blocks_per_sector(light, G);
-        const int sblocks = hblocks + kGridSectors * lb;
-        o.sop_waves = 4 * lb;
-        o.sop_groups = G;
-
-        const size_t lds = lds_base + std::max(heavy_lds, sizeof(float2) * 4 * kSopSlots * P);
-        hipError_t e = gr_allow_lds(k_grid_op<ACCUM, P, true>, lds);
-        if (e != hipSuccess) return e;
-        if (G > 1)
-            hipLaunchKernelGGL((k_grid_op<ACCUM, P, true>), dim3(G * sblocks, 1), dim3(256), lds, s, A, o);
-        else
-            hipLaunchKernelGGL((k_grid_op<ACCUM, P, true>), dim3(sblocks, groups), dim3(256), lds, s, A, o);
-        return hipGetLastError();
+        return launch_op<ACCUM, P, false>(A, *O, groups, lds_base, s);
     }
     // fewer waves beside convolvent tables that leave no room for wpb of them
     // (interp keeps two tables: ltbl above 16127 with four waves of eight pairs)

@@ -368,8 +368,7 @@ __device__ __forceinline__ void pf_rest(float2 *buf, const float2 *tw, int tid) 
 
 // Columns: an item is CW neighbouring columns of one pair, contiguous blocks of
 // the column-blocked Z (M = 8192: half of one).
-// ALL: every row of Z was written.
-template <int LM, bool ALL>
+template <int LM>
 __global__ void __launch_bounds__(kPfThreads) k_ifft_cols_pf(ColsArgs A, int n_items) {
     using F = Pf<LM>;
     constexpr int M = F::M, CW = F::CW, NT = F::nthr;
@@ -390,22 +389,16 @@ __global__ void __launch_bounds__(kPfThreads) k_ifft_cols_pf(ColsArgs A, int n_i
         const int t = (int)threadIdx.x, lc = column(t), j = first(t);
         const int p = item / ngroups, x = item - p * ngroups;
         const int c0 = (int)column_group((unsigned)x, (unsigned)ngroups) * CW;
-        const GrBuf zb = gr_buf(A.z + (long)p * M * gr_z_cols(out_n) + (long)(c0 & ~3) * M,
-                                (unsigned)(F::blocks * M * 4 * sizeof(float2)));
-        const bool in = c0 + lc < out_n;
-        const unsigned o0 = (unsigned)(((lc / 4 * M + j) * 4 + (c0 + lc) % 4) * sizeof(float2));
-        if (ALL) {
-            const unsigned o = in ? o0 : kGrBufNone;
+        // a buffer over the written rows of the wave's block of four columns:
+        // a row before them wraps to one far past them
+        const int blk = (c0 >> 2) + __builtin_amdgcn_readfirstlane(t / F::tpb);
+        const GrBuf zb = gr_buf(A.z + (long)p * M * gr_z_cols(out_n) + ((long)blk * M + A.row_lo) * 4,
+                                (unsigned)((A.row_hi - A.row_lo) * 4 * sizeof(float2)));
+        // (a column past the window: past the buffer, whatever is added below)
+        const unsigned o0 = c0 + lc < out_n ? (unsigned)(((j - A.row_lo) * 4 + (c0 + lc) % 4) * (int)sizeof(float2))
+                                            : 0x80000000u;
 #pragma unroll
-            for (int r = 0; r < 16; r++) v[r] = gr_buf_ld2(zb, o, (unsigned)(r * NT * 4 * sizeof(float2)));
-        } else {
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int b = j + r * NT;
-                v[r] = gr_buf_ld2(zb, in && b >= A.row_lo && b < A.row_hi ? o0 + (unsigned)(r * NT * 4 * sizeof(float2))
-                                                                          : kGrBufNone);
-            }
-        }
+        for (int r = 0; r < 16; r++) v[r] = gr_buf_ld2(zb, o0 + (unsigned)(r * NT * 4 * sizeof(float2)));
         const int grp = t / NT;
         cu_next = A.winv[off + (c0 + grp < out_n ? c0 + grp : out_n - 1)];
     };
@@ -608,14 +601,11 @@ template <int LM>
 struct PfCols {
     static hipError_t go(ColsArgs A, int pairs, hipStream_t s) {
         const int n_items = (int)((A.out_n + Pf<LM>::CW - 1) / Pf<LM>::CW) * pairs;
-        auto launch = [&](auto kernel) {
-            const hipError_t e = gr_allow_lds(kernel, Pf<LM>::lds);
-            if (e != hipSuccess) return e;
-            hipLaunchKernelGGL(kernel, dim3(std::min(n_items, gr_cu_count())), dim3(kPfThreads), Pf<LM>::lds, s, A,
-                               n_items);
-            return hipGetLastError();
-        };
-        return A.row_hi - A.row_lo == Pf<LM>::M ? launch(k_ifft_cols_pf<LM, true>) : launch(k_ifft_cols_pf<LM, false>);
+        const hipError_t e = gr_allow_lds(k_ifft_cols_pf<LM>, Pf<LM>::lds);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(k_ifft_cols_pf<LM>, dim3(std::min(n_items, gr_cu_count())), dim3(kPfThreads), Pf<LM>::lds, s,
+                           A, n_items);
+        return hipGetLastError();
     }
 };
 
@@ -645,7 +635,12 @@ hipError_t gr_launch_ifft_rows(const GrGeom &g, const GrDevTables &t, const floa
     }
     int cw = kRowsPerBlock;  // rows side by side: a power of two dividing M, within 1024 threads and the LDS
     while (cw > 1 && ((long)cw * nthr > 1024 || (long)cw * g.M * 8 > 163840 || g.M % cw)) cw /= 2;
-    const dim3 grid((unsigned)((t.row_hi - t.row_lo) / cw), pairs), block(cw * nthr);
+    // whole groups of 32 rows, which row_group deals out (the rows added hold no
+    // active tile and read as zeros): with any other number the pieces of
+    // a line of Z come from several XCDs (4 pairs of 900 x 1000 28 -> 31 us)
+    A.row_lo = t.row_lo / 32 * 32;
+    A.row_hi = (int)std::min<long>((t.row_hi + 31) / 32 * 32, g.M);
+    const dim3 grid((unsigned)((A.row_hi - A.row_lo) / cw), pairs), block(cw * nthr);
     const size_t lds = sizeof(float2) * cw * gr_lds_len(g.M);
 #define GR_ROWS_K(MB, CW)                                                          \
     do {                                                                           \

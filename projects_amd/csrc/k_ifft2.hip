@@ -570,10 +570,12 @@ int gr_max_lds_per_block() {
 
 // Whether a launch of n_items items takes the persistent form: with fewer than
 // two per CU there is nothing to overlap and the one-shot kernels' smaller
-// workgroups fill the chip better.
+// workgroups fill the chip better -- but at M = 4096, where they take a CU each,
+// too (columns of a pair of 60 x 2000, 500 items: 28.9 us persistent, 41.2
+// one-shot).
 static bool pf_takes(long M, int radix, long n_items) {
     const int cus = gr_cu_count();
-    return M >= 1024 && M <= 8192 && radix == 16 && cus > 0 && n_items >= 2L * cus &&
+    return M >= 1024 && M <= 8192 && radix == 16 && cus > 0 && (M == 4096 || n_items >= 2L * cus) &&
            (size_t)gr_max_lds_per_block() >= std::max(Pf<12>::lds, Pf<13>::lds);
 }
 

@@ -488,3 +488,37 @@ def test_persistent_transforms_are_bitwise_the_one_shot_ones(name):
     off, n = case.get("crop", (0, M0))
     d = disk_mask(M0, 0.5)[off:off + n, off:off + n]
     assert O.rel_l2(out[0].cpu().numpy()[d], r1[off:off + n, off:off + n][d]) < DISK_TOL
+
+
+# fewer columns than two items per CU: one pair at M = 4096, whose columns take
+# the persistent form whatever their number (an explicit width of one column asks
+# for the one-shot one), down to a single column
+@pytest.mark.parametrize("crop", [(1400, 1201), (1548, 1025), (2000, 6), (2047, 1)])
+@pytest.mark.parametrize("ns", [1, 2, 3])
+def test_narrow_windows_of_one_pair(crop, ns):
+    case = dict(n_ang=16, n_det=1100, center=550.0, pad="half", crop=crop, max_pairs=1, grid_op="off")
+    sino = torch.from_numpy(np.random.default_rng(ns).standard_normal((ns, 16, 1100)).astype(np.float32)).cuda()
+    p = gr.Plan(**case)
+    assert p.info["M"] == 4096
+    out = p.recon(sino)
+    p.set_cols_per_block(1)
+    one = p.recon(sino)
+    torch.cuda.synchronize()
+    assert torch.equal(out, one)
+    p.close()
+
+
+# row ranges of every remainder modulo 32 (the rows dealt out in groups of 32),
+# one-shot sizes: grids without their first and last rows
+@pytest.mark.parametrize("n_det", [33, 40, 47, 57, 100, 104, 111, 127])
+def test_grids_without_their_outer_rows(n_det):
+    """Images against the oracle inside the disk, one pair and several."""
+    g = O.Geometry(n_ang=30, n_det=n_det, center=n_det / 2.0 + 0.2)
+    sino = np.random.default_rng(n_det).standard_normal((5, 30, n_det)).astype(np.float32)
+    p = plan_for(g)
+    out = p.recon(torch.from_numpy(sino).cuda()).cpu().numpy()
+    d = disk_mask(out.shape[1], 0.5)
+    for s in (0, 2):
+        r1, r2 = O.recon_f32(g, sino[s], sino[s + 1])
+        assert O.rel_l2(out[s][d], r1[d]) < DISK_TOL and O.rel_l2(out[s + 1][d], r2[d]) < DISK_TOL
+    p.close()

@@ -1382,15 +1382,16 @@ __global__ void __launch_bounds__(256, 4) k_grid_op(GridArgs A, GopArgs O) {
 // to take, down to 48 workgroups: the heavy chains of a small grid run
 // faster beside fewer light waves (one pair of 180 x 256 27 -> 25 us, of
 // 360 x 512 46 -> 42) -- unless a few pairs' light tiles are what the launch
-// waits for: from some 640 angles on up to M = 1024 (one pair of 600 x 500 at M =
-// 512 43.6 us with 48 and 45.6 with 96, of 900 x 500 69 and 59; at M = 1024 400 x
-// 500 44 and 45, 900 x 500 84 and 75; eight pairs gain nothing, nor 1800 angles
-// at M = 512: four pairs of 1800 x 500 657 and 710), and at M = 1024 below some 160, where every tile is one round trip
-// (60 x 500 28 and 22, 180 x 500 36 and 36).
+// waits for (96 against 48 and some, one pair, us): from some 640 angles on (M =
+// 512: 600 x 500 45.6 and 43.6, 900 x 500 59 and 69; M = 1024: 400 x 500 45 and 43, 900
+// x 500 75 and 84; but four pairs of 1800 x 500 at M = 512 710 and 657, and eight pairs
+// of 900 x 230 94 and 90), and at M = 1024 below some 160, where every tile is one
+// round trip (60 x 500 22 and 26, 180 x 500 36 and 34).
 __host__ inline int sop_blocks_per_sector(int light, int groups, int pairs, int n_ang) {
     const int most = groups > 1 && light >= 1024 ? 128 : 96;
     const bool waits_for_light = pairs < kSpecGroup && light < 1024 &&
-                                 (light > 300 ? n_ang > 640 || n_ang < 160 : n_ang > 640 && n_ang < 1500);
+                                 (light > 300 ? n_ang > 640 || n_ang < 160
+                                              : n_ang > 640 && (pairs <= 2 || n_ang < 1500));
     const int total = waits_for_light ? most : std::min(most, std::max(48, light * groups / 10));
     return std::max(1, std::min(light, total / groups));
 }
@@ -1431,8 +1432,8 @@ hipError_t launch_op(const GridArgs &A, GopArgs o, int groups, size_t lds_base, 
     const size_t lds = lds_base + std::max(heavy_lds, sizeof(float2) * 4 * kSopSlots * P);
     hipError_t e = gr_allow_lds(k_grid_op<ACCUM, P, true, WIDE>, lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_grid_op<ACCUM, P, true, WIDE>), G > 1 ? dim3(G * blocks, 1) : dim3(blocks, groups), dim3(256), lds,
-                       s, A, o);
+    hipLaunchKernelGGL((k_grid_op<ACCUM, P, true, WIDE>), G > 1 ? dim3(G * blocks, 1) : dim3(blocks, groups), dim3(256),
+                       lds, s, A, o);
     return hipGetLastError();
 }
 

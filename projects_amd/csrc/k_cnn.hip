@@ -1057,12 +1057,14 @@ int check_dims(int n, int H, int W) {
 // Segments of rows a strip is cut into: the fewest steps of the busiest CU
 // (one workgroup each at a time); a segment of k rows takes k / 2 + 8 steps,
 // the pipeline's fill and the four halo rows on either side among them.  At
-// least 16 rows each (what gr_cnn_infer_work_bytes counts on).
+// least 8 rows each (what the work sizes count on): at 16 an image of up to 256 x
+// 256 kept most CUs idle for 16 steps (33.8 us a call, 29.5 at 8), as one of 4096 x 64
+// did in 64 segments at most (66 us; 49).
 int forward_segments(int n, int H, int strips) {
     const long cus = gr_cu_count() > 0 ? gr_cu_count() : 256;
     int best = 1;
     long best_cost = 0;
-    for (int v = 1; v <= std::min(64, (H + 15) / 16); v++) {
+    for (int v = 1; v <= std::min(256, (H + 7) / 8); v++) {
         const long rows = (H + v - 1) / v, groups = (long)n * strips * ((H + rows - 1) / rows);
         const long cost = (groups + cus - 1) / cus * ((rows + 1) / 2 + 8);
         if (v == 1 || cost < best_cost) {
@@ -1175,8 +1177,8 @@ int gr_cnn_forward(const float *params, const unsigned short *packed, const floa
 }
 
 size_t gr_cnn_infer_work_bytes(int n, int H, int W) {
-    // two floats per workgroup: at most one per 16 rows and 32 columns
-    return sizeof(float) * 2 * (size_t)((W + 31) / 32) * ((H + 15) / 16) * (n > 0 ? n : 0);
+    // two floats per workgroup: at most one per 8 rows and 32 columns
+    return sizeof(float) * 2 * (size_t)((W + 31) / 32) * ((H + 7) / 8) * (n > 0 ? n : 0);
 }
 
 int gr_cnn_infer(const float *params, const unsigned short *packed, const float *x, int n, int H, int W, float scale,

@@ -547,3 +547,9 @@ def test_forward_and_infer_keep_their_sums():
     net.forward(b)
     torch.cuda.synchronize()
     assert torch.equal(s2, want[1])
+
+
+# segments of eight rows at least, and more than 64 of them
+@pytest.mark.parametrize("shape", [(1, 8, 8), (1, 9, 60), (2, 15, 57), (1, 2100, 20)])
+def test_forward_short_segments(shape):
+    test_forward_strips_and_segments(shape)

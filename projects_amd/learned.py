@@ -107,10 +107,9 @@ class Corrector:
         """x, or a copy of it where out lies over it: the network reads x
         around every pixel while others are written.  The copy is made, and
         given back, on the stream that reads it."""
-        torch = self.torch
-        nbytes = 4 * x.numel()
-        if out is None or abs(out.data_ptr() - x.data_ptr()) >= nbytes:
+        if out is None or abs(out.data_ptr() - x.data_ptr()) >= 4 * x.numel():
             return x
+        torch = self.torch
         if stream is None:
             return x.clone()
         if not isinstance(stream, torch.cuda.Stream):
@@ -123,7 +122,7 @@ class Corrector:
         y = the corrected images (in out, which may be x) and stats [n, 2] =
         (sum residual^2, sum (x/scale)^2) per image."""
         if not train:
-            return self._infer(x, out, stream, False)
+            return self._infer(self._apart(x, out, stream), out, stream, False)
         torch = self.torch
         assert x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.is_contiguous()
         n, H, W = x.shape
@@ -139,13 +138,12 @@ class Corrector:
     def infer(self, x, out=None, stream=None):
         """Inference: the training forward's kernel (bitwise its y and stats)
         writing no activations.  Returns (y, stats)."""
-        return self._infer(x, out, stream, True)
+        return self._infer(self._apart(x, out, stream), out, stream, True)
 
-    def _infer(self, x, out, stream, infer):
+    def _infer(self, x, out, stream, infer):  # out: not over x
         torch = self.torch
         assert x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.is_contiguous()
         n, H, W = x.shape
-        x = self._apart(x, out, stream)
         _, work, _, stats = self._buffers(n, H, W, False, infer)
         if out is None:
             out = torch.empty_like(x)
@@ -184,7 +182,7 @@ class Corrector:
         out may be x."""
         torch = self.torch
         x = self._apart(x, out, stream)
-        y, stats = self.forward(x, out=out, stream=stream)
+        y, stats = self._infer(x, out, stream, False)
         s = torch.cuda.current_stream() if stream is None else stream
         with torch.cuda.stream(s):  # device-side selection, no host synchronisation
             rel = torch.sqrt(stats[:, 0] / torch.clamp(stats[:, 1], min=1e-30))

@@ -269,3 +269,28 @@ def test_plain_heavy_tiles_of_full_launches(n_ang, n_det, ns):
         out = gr.Plan(**case, grid_op="on", max_pairs=mp).recon(sino)
         torch.cuda.synchronize()
         assert torch.equal(out, ref), mp
+
+
+# angles within a few degrees, so many that tiles along their lines are heavy:
+# in the sectors across the lines the slots next to the centre hold tiles no
+# sample reaches, which have to be written as zeros like any other
+@pytest.mark.parametrize("accum", ["compensated", "plain"])
+@pytest.mark.parametrize("spread,n_ang,n_det", [(0.0, 50, 187), (15.0, 60, 128), (1.0, 400, 100)])
+def test_heavy_tiles_no_sample_reaches(spread, n_ang, n_det, accum):
+    """Bitwise the geometry kernel's images whatever the grid's memory held
+    before: here a centre sweep's images."""
+    case = dict(n_ang=n_ang, n_det=n_det, center=n_det / 2.0 + 0.2, geom=0, pad="half", accum=accum,
+                angles=(33.0 + np.linspace(0.0, spread, n_ang)).astype(np.float32))
+    sino = sinos(case, 10, 6)
+    ref = gr.Plan(**case, grid_op="off").recon(sino)
+    shifts = np.linspace(-2, 2, 11).astype(np.float32)
+    e = {}
+    for op in ("on", "off"):
+        p = gr.Plan(**case, grid_op=op, max_pairs=5)
+        for _ in range(2):
+            e[op] = p.center_entropy(sino[:2].contiguous(), shifts, -1.0, 2.0, 400)
+            out = p.recon(sino)
+            torch.cuda.synchronize()
+            assert torch.equal(out, ref), op
+        p.close()
+    assert np.array_equal(e["on"], e["off"])

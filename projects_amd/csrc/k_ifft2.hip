@@ -47,7 +47,10 @@ struct WindowRow {
     __device__ __forceinline__ void prep(int, int) {}
     __device__ __forceinline__ void operator()(int i, float2 v, int) const {
         const int jp = i >= M - m02 ? i - (M - m02) : i + m02;
-        const int jj = jp - off;
+        put(jp - off, v);
+        if (i >= M - m02 && i <= m02) put(i + m02 - off, v);  // an image wider than the grid (sampl < 1) repeats it
+    }
+    __device__ __forceinline__ void put(int jj, float2 v) const {
         if (jj >= 0 && jj < out_n) dst[(long)(jj >> 2) * M * 4 + (jj & 3)] = v;
     }
 };
@@ -109,6 +112,8 @@ __global__ void __launch_bounds__(1024) k_ifft_rows(RowsArgs A) {
         const int jj = tid + r * nthr;
         if (jj < out_n) dst[(long)(jj >> 2) * M * 4 + (jj & 3)] = o[r];
     }
+    for (int jj = tid + EPT * nthr; jj < out_n; jj += nthr)  // a window wider than the grid
+        dst[(long)(jj >> 2) * M * 4 + (jj & 3)] = row[gr_lds_idx((int)corner_index(off + jj, M, m02))];
 }
 
 struct ColsArgs {
@@ -139,9 +144,12 @@ struct WindowCol {
     __device__ __forceinline__ int kprime(int i) const { return i >= M - m02 ? i - (M - m02) : i + m02; }
     __device__ __forceinline__ void prep(int i, int s) { wv[s] = winv[kprime(i)]; }
     __device__ __forceinline__ void operator()(int i, float2 v, int s) const {
-        const int kk = kprime(i) - off;
+        put(kprime(i) - off, v, wv[s]);
+        if (i >= M - m02 && i <= m02) put(i + m02 - off, v, winv[i + m02]);  // as WindowRow
+    }
+    __device__ __forceinline__ void put(int kk, float2 v, float w) const {
         if (r1 && kk >= 0 && kk < out_n) {
-            const float corrn = cu * wv[s];
+            const float corrn = cu * w;
             r1[kk] = corrn * v.x;
             if (r2) r2[kk] = corrn * v.y;
         }
@@ -251,9 +259,9 @@ __global__ void __launch_bounds__(1024) k_ifft_cols(ColsArgs A) {
                     if (r2) r2[kk] = corrn * v[r].y;
                 }
             }
-            continue;
         }
-        for (int kk = tid; kk < out_n; kk += nthr) {
+        // (CW: a window wider than the grid)
+        for (int kk = CW ? tid + EPT * nthr : tid; kk < out_n; kk += nthr) {
             const int k = off + kk;
             const float corrn = cu * A.winv[k];  // grid.cpp:401
             const float2 v = col[gr_lds_idx(k < m02 ? M - m02 + k : k - m02)];

@@ -522,3 +522,37 @@ def test_grids_without_their_outer_rows(n_det):
         r1, r2 = O.recon_f32(g, sino[s], sino[s + 1])
         assert O.rel_l2(out[s][d], r1[d]) < DISK_TOL and O.rel_l2(out[s + 1][d], r2[d]) < DISK_TOL
     p.close()
+
+
+# sampl < 1: an image larger than the grid, whose outer rows and columns repeat
+# the grid's -- at one-shot sizes that end in a radix-16 pass (outputs from its
+# registers) and in others, and at persistent ones
+@pytest.mark.parametrize("sampl,n_det,ns", [(0.9, 90, 3), (0.9, 45, 2), (0.6, 50, 5), (0.55, 20, 1), (0.9, 180, 4), (0.8, 900, 33),
+                                            (0.9, 1500, 2)])
+def test_image_larger_than_the_grid(sampl, n_det, ns):
+    """Against the oracle over the whole image, divided by the deapodization of
+    each pixel (which grows without bound outwards): rel-L2 1e-5, the parity
+    gate.  Windows at the far end are those of the whole image, bitwise."""
+    g = O.Geometry(n_ang=24, n_det=n_det, center=n_det / 2.0 + 0.3, sampl=sampl)
+    sino = np.random.default_rng(n_det).standard_normal((ns, 24, n_det)).astype(np.float32)
+    x = torch.from_numpy(sino).cuda()
+    for op in ("off", "on"):
+        p = plan_for(g, grid_op=op)
+        M, M0 = p.info["M"], p.info["M0"]
+        assert M0 > M
+        w = p.tables()["winv"].astype(np.float64)
+        out = p.recon(x, torch.full((ns, M0, M0), float("nan"), device="cuda"))
+        torch.cuda.synchronize()
+        img = out.cpu().numpy()
+        r = O.recon_f32(g, sino[0], sino[1] if ns > 1 else np.zeros_like(sino[0]))
+        keep = np.abs(np.outer(w, w)) > 0
+        for s in range(min(ns, 2)):
+            a, b = (np.where(keep, v.astype(np.float64) / np.where(keep, np.outer(w, w), 1.0), 0.0) for v in (img[s], r[s]))
+            assert O.rel_l2(a, b) < 1e-5, (op, s)
+        p.close()
+        for off, n in ((M0 - 7, 7), (M - 3, 5), (0, M0 - 1)):
+            q = plan_for(g, grid_op=op, crop=(off, n))
+            win = q.recon(x, torch.full((ns, n, n), float("nan"), device="cuda"))
+            torch.cuda.synchronize()
+            assert torch.equal(win, out[:, off:off + n, off:off + n]), (op, off)
+            q.close()

@@ -1093,9 +1093,16 @@ int gr_center_entropy(gr_plan *pl, const float *sino, long sino_slice_stride, lo
     if (!pl->d_spec1) return fail(GR_EINVAL, "plan has no workspace");
     const long on = g.out_n, nb1 = n_bins + 1;
     // shifts and histograms: kept by the plan (allocated and freed per call
-    // they are given back to the system at every synchronisation)
+    // they are given back to the system at every synchronisation).  A chunk's
+    // images go to the gridding step's grid, which is free once the row
+    // transform has read it, and are counted before the next chunk; where sampl < 1
+    // makes an image larger than the grid (out_n > M: 8 out_n^2 bytes per pair
+    // against 8 M^2), they have room of their own.
     const size_t shift_bytes = (sizeof(float) * n_shifts + 255) / 256 * 256;
-    const size_t sweep_bytes = shift_bytes + sizeof(unsigned) * nb1 * n_shifts;
+    const size_t hist_bytes = (sizeof(unsigned) * nb1 * n_shifts + 255) / 256 * 256;
+    const bool own = on > g.M;
+    const size_t img_bytes = own ? sizeof(float) * 2 * on * on * std::min(pl->max_pairs, n_shifts) : 0;
+    const size_t sweep_bytes = shift_bytes + hist_bytes + img_bytes;
     if (sweep_bytes > pl->sweep_bytes) {
         if (pl->d_sweep) {
             GR_HIP(hipFree(pl->d_sweep));
@@ -1109,12 +1116,9 @@ int gr_center_entropy(gr_plan *pl, const float *sino, long sino_slice_stride, lo
     }
     float *d_shift = (float *)pl->d_sweep;
     unsigned *d_hist = (unsigned *)((char *)pl->d_sweep + shift_bytes);
+    float *img = own ? (float *)((char *)pl->d_sweep + shift_bytes + hist_bytes) : (float *)pl->d_ht;
     GR_HIP(hipMemcpyAsync(d_shift, shifts, sizeof(float) * n_shifts, hipMemcpyHostToDevice, s));
     int rc = count_pairs(pl, n_shifts, s);
-    // a chunk's images go to the gridding step's grid, which is free once the
-    // row transform has read it and larger than the images (M > out_n: 8 M^2
-    // bytes per pair against 8 out_n^2), and are counted before the next chunk
-    float *img = (float *)pl->d_ht;
     hipError_t e = hipSuccess;
     for (int c0 = 0; c0 < n_shifts && rc == GR_OK && e == hipSuccess; c0 += pl->max_pairs) {
         const int np = std::min(pl->max_pairs, n_shifts - c0);

@@ -89,3 +89,25 @@ def test_entropy_sweep_chunks_and_bins(n, max_pairs, nb):
     assert np.max(np.abs(ent - ref)) <= 1e-5 * np.max(ref)
     plan.close()
     one.close()
+
+
+@pytest.mark.parametrize("max_pairs", [1, 2, 5])
+@pytest.mark.parametrize("sampl,n", [(0.9, 45), (0.55, 20)])
+def test_sweep_of_images_larger_than_the_grid(sampl, n, max_pairs):
+    """sampl < 1: each candidate's images are larger than its grid.  Unshifted
+    candidates have the plain reconstruction's images, so its entropy, and the
+    plan's own reconstructions are as before."""
+    sino = torch.from_numpy(np.random.default_rng(n).standard_normal((2, 30, n)).astype(np.float32)).cuda()
+    plan = gr.Plan(n_ang=30, n_det=n, center=n / 2.0, sampl=sampl, max_pairs=max_pairs, grid_op="off")
+    assert plan.info["M0"] > plan.info["M"]
+    img = plan.recon(sino)
+    torch.cuda.synchronize()
+    v = img.cpu().numpy()
+    lo, hi, nb = float(np.percentile(v, 2)), float(np.percentile(v, 98)), 300
+    ent = plan.center_entropy(sino, np.zeros(7, np.float32), lo, hi, nb)
+    ref = O.entropy(v.ravel(), lo, hi, nb)
+    assert np.all(ent == ent[0]) and abs(ent[0] - ref) <= 1e-5 * ref
+    again = plan.recon(sino)
+    torch.cuda.synchronize()
+    assert torch.equal(again, img)
+    plan.close()

@@ -250,10 +250,12 @@ int build_gop(gr_plan *pl, hipStream_t s, bool required, size_t max_bytes) {
     if (pl->prm.accum == GR_ACCUM_COMPENSATED) {
         hmeta.assign(nt, make_uint4(0u, 0u, 0u, 0u));
         for (int i = 0; i < nt; i++) {
-            // a tile without groups (no sample line reaches it) has no segments,
-            // but is among those whose cells k_gop_merge stores: the row
-            // transform reads them
+            // a tile without rows -- no sample line reaches it, or lines that
+            // deposit into none of its cells do: its marks are not filled --
+            // has no segments, but is among those whose cells k_gop_merge
+            // stores: the row transform reads them
             if (i % pl->sector_len >= pl->gop_heavy) continue;
+            if ((cnt[i] & ~kGopAlignedBit) == 0) groups[i] = 0;
             const unsigned S = (groups[i] + kGopSegGroups - 1) / kGopSegGroups;
             hmeta[i] = make_uint4(S, (unsigned)seg_total, (unsigned)part_total, (unsigned)hsplit.size());
             seg_total += 64ull * (S + 1);

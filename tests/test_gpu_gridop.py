@@ -294,3 +294,23 @@ def test_heavy_tiles_no_sample_reaches(spread, n_ang, n_det, accum):
             assert torch.equal(out, ref), op
         p.close()
     assert np.array_equal(e["on"], e["off"])
+
+
+# heavy slots with a tile that sample lines pass (within the tests' margins) but
+# that no sample deposits into: one at the edge of a grid of half a cell per
+# sample, one beside a bundle of 259 directions within a degree
+@pytest.mark.parametrize("ns", [1, 3, 18])
+@pytest.mark.parametrize("case", [
+    dict(n_ang=214, n_det=36, center=17.937523509860704, pad="half", C_=4.2, sampl=1.3, R=0.5, ltbl=2048),
+    dict(n_ang=259, n_det=235, center=116.75638071216909, geom=0, pad="half", C_=4.0, sampl=1.3,
+         angles=np.full(259, 33.0, np.float32) + np.linspace(0, 1, 259).astype(np.float32)),
+], ids=["edge", "bundle"])
+def test_heavy_tiles_lines_only_pass(case, ns):
+    """Such a tile has neither entries nor marks: bitwise the geometry kernel's
+    images, in launches of all pairs and of two."""
+    sino = sinos(case, ns, ns)
+    ref = gr.Plan(**case, grid_op="off").recon(sino)
+    for mp in (0, 2):
+        out = gr.Plan(**case, grid_op="on", max_pairs=mp).recon(sino)
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref), mp

@@ -1057,14 +1057,20 @@ int check_dims(int n, int H, int W) {
 // Segments of rows a strip is cut into: the fewest steps of the busiest CU
 // (one workgroup each at a time); a segment of k rows takes k / 2 + 8 steps,
 // the pipeline's fill and the four halo rows on either side among them.  At
-// least 8 rows each (what the work sizes count on): at 16 an image of up to 256 x
-// 256 kept most CUs idle for 16 steps (33.8 us a call, 29.5 at 8), as one of 4096 x 64
-// did in 64 segments at most (66 us; 49).
-int forward_segments(int n, int H, int strips) {
+// least 8 rows each, and per image no more workgroups than its tiles of 16 x 32,
+// what the work sizes hold partial sums for.  A strip is wider than a tile, so 256 x 256
+// still goes in segments of 12 rows (31.4 us a call; 34.0 with 16), 4096 x 64 in 128
+// of them (44.6 us; 65.7 with 64).
+long infer_tiles(int H, int W) {
+    return (long)((W + 31) / 32) * ((H + 15) / 16);
+}
+
+int forward_segments(int n, int H, int W, int strips) {
     const long cus = gr_cu_count() > 0 ? gr_cu_count() : 256;
+    const int most = (int)std::min({256L, (H + 7) / 8L, infer_tiles(H, W) / strips});
     int best = 1;
     long best_cost = 0;
-    for (int v = 1; v <= std::min(256, (H + 7) / 8); v++) {
+    for (int v = 1; v <= most; v++) {
         const long rows = (H + v - 1) / v, groups = (long)n * strips * ((H + rows - 1) / rows);
         const long cost = (groups + cus - 1) / cus * ((rows + 1) / 2 + 8);
         if (v == 1 || cost < best_cost) {
@@ -1077,7 +1083,7 @@ int forward_segments(int n, int H, int strips) {
 
 int run_forward(const float *params, const unsigned short *packed, const float *x, int n, int H, int W, float scale,
                 uint16_t *const (&act)[4], float *y, float *yn, float *slice_stats, float *stats, hipStream_t s) {
-    const int strips = (W + FW_OUT - 1) / FW_OUT, v = forward_segments(n, H, strips);
+    const int strips = (W + FW_OUT - 1) / FW_OUT, v = forward_segments(n, H, W, strips);
     const int rows = (H + v - 1) / v, segs = (H + rows - 1) / rows;
     if ((long)n * strips * segs > (1L << 31) - 1) return cnn_fail(GR_EINVAL, "too many tiles");
     FwdArgs A{x, params, reinterpret_cast<const uint16_t *>(packed), {act[0], act[1], act[2], act[3]}, y, yn,
@@ -1177,8 +1183,8 @@ int gr_cnn_forward(const float *params, const unsigned short *packed, const floa
 }
 
 size_t gr_cnn_infer_work_bytes(int n, int H, int W) {
-    // two floats per workgroup: at most one per 8 rows and 32 columns
-    return sizeof(float) * 2 * (size_t)((W + 31) / 32) * ((H + 7) / 8) * (n > 0 ? n : 0);
+    // two floats per workgroup: at most one per 16 rows and 32 columns
+    return sizeof(float) * 2 * (size_t)infer_tiles(H, W) * (n > 0 ? n : 0);
 }
 
 int gr_cnn_infer(const float *params, const unsigned short *packed, const float *x, int n, int H, int W, float scale,

@@ -553,3 +553,28 @@ def test_forward_and_infer_keep_their_sums():
 @pytest.mark.parametrize("shape", [(1, 8, 8), (1, 9, 60), (2, 15, 57), (1, 2100, 20)])
 def test_forward_short_segments(shape):
     test_forward_strips_and_segments(shape)
+
+
+# the sums' partials stay within the documented work sizes, short segments or not
+@pytest.mark.parametrize("shape", [(1, 8, 8), (3, 16, 32), (2, 40, 57), (1, 64, 64), (1, 256, 256), (1, 2100, 20), (2, 1100, 64)])
+def test_infer_work_stays_in_its_size(shape):
+    import ctypes as C
+
+    from projects_amd import gridrec as gr
+
+    net, _, x, _ = make(sum(shape), *shape)
+    n, H, W = shape
+    L = gr.lib()
+    size = L.gr_cnn_infer_work_bytes(n, H, W)
+    assert size == 8 * n * ((W + 31) // 32) * ((H + 15) // 16)
+    xg = torch.from_numpy(x).cuda()
+    work = torch.full((size + 65536,), 0x5A, dtype=torch.uint8, device="cuda")
+    y, st = torch.empty_like(xg), torch.empty((n, 2), dtype=torch.float32, device="cuda")
+    p = lambda t: C.c_void_p(t.data_ptr())
+    gr._check(L.gr_cnn_infer(p(net.params), p(net.packed), p(xg), n, H, W, net.scale, p(y), p(st), p(work),
+                             C.c_void_p(gr._stream_handle(None))), "gr_cnn_infer")
+    torch.cuda.synchronize()
+    assert bool((work[size:] == 0x5A).all())
+    y1, s1 = net.forward(xg, train=True)
+    torch.cuda.synchronize()
+    assert torch.equal(y, y1) and torch.equal(st, s1)

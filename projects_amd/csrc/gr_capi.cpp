@@ -375,8 +375,8 @@ int build_gop(gr_plan *pl, hipStream_t s, bool required, size_t max_bytes) {
 // transform's output buffer, which must hold them; a plan whose buffer does
 // not (or whose sums are plain: they have no merge points) is not split.
 // Whole, the four tiles at the centre walk every angle in one wave each and
-// the launch waits for them: one pair of 1500 x 2048 3.12 -> 0.87 ms split,
-// eight pairs 3.70 -> 1.80, one of 180 x 256 0.37 -> 0.08.
+// the launch waits for them: one pair of half-padded 1500 x 2048 3.12 ms, 0.60
+// split, eight pairs 3.70 and 1.09, one of 180 x 256 0.37 and 0.05.
 // Two small kernels and one wait of their own on stream s, at plan creation.
 constexpr int kSplitSlots = 256;
 constexpr unsigned kSplitLines = 48;

@@ -56,7 +56,8 @@ struct gr_plan {
     bool owns_workspace = true;
     float2 *d_spec1 = nullptr, *d_spec2 = nullptr, *d_ht = nullptr, *d_z = nullptr;
     size_t dev_bytes = 0;
-    // centre sweeps: shifts and histograms, grown to the largest sweep so far
+    // centre sweeps: shifts, histograms and, where the grid is smaller than the
+    // images, a chunk of them; grown to the largest sweep so far
     void *d_sweep = nullptr;
     size_t sweep_bytes = 0;
     // launch tuning (0 = automatic)

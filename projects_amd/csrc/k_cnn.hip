@@ -143,7 +143,7 @@ struct TileMap {
 // Per output the MFMAs run tap by tap into one accumulator, then bias, ReLU
 // and rounding, whichever buffers are written.  Bound by MFMA (130 per step and
 // SIMD, half of the time) and what a barrier per step leaves exposed around
-// them: 4 x 2048^2 inference 1.05 ms where five layer kernels took 1.93, of
+// them: 4 x 2048^2 inference 0.96 ms where five layer kernels took 1.93, of
 // which 6.4 GB of activations 1.36 at the rate of a copy; 32 x 512^2 training
 // 0.87 ms (2.2 GB written) against 1.02.
 constexpr int FW_COLS = 64, FW_OUT = 56, FW_RING = 6, FW_PITCH = FW_COLS + 2;
@@ -1109,8 +1109,10 @@ int run_forward_copy(const float *params, const unsigned short *packed, const fl
                      hipStream_t s) {
     const size_t bytes = sizeof(float) * (size_t)n * H * W;
     void *copy = nullptr;
-    if (hipMallocAsync(&copy, bytes, s) != hipSuccess)
+    if (hipMallocAsync(&copy, bytes, s) != hipSuccess) {
+        (void)hipGetLastError();
         return cnn_fail(GR_ENOMEM, "no device memory for a copy of the images (y or yn lies over x)");
+    }
     const hipError_t e = hipMemcpyAsync(copy, x, bytes, hipMemcpyDeviceToDevice, s);
     const int rc = e == hipSuccess ? run_forward(params, packed, (const float *)copy, n, H, W, scale, act, y, yn,
                                                  slice_stats, stats, s)

@@ -226,10 +226,9 @@ __device__ __forceinline__ unsigned long long batch_lines(const GridArgs &A, con
 // Walk the sample lines that can reach the wave's tile, in the kernel's fixed
 // order (sorted angle keys, the window's two ranges in turn; per line the
 // direct samples, then the mirrored ones, in chunks of at most 64 ascending
-// j), calling on_chunk(mirror, row_off, c0, nj, j0, j1, C, S) per chunk --
-// [c0, c0+nj) the tile's samples of the chunk, [j0, j1] the lane's own
-// candidates among them -- and on_line() after each line that passed the
-// tile tests.  Tiles beyond the largest sample radius visit nothing.  The
+// j), calling on_chunk(mirror, row_off, j0, j1, C, S) per chunk -- [j0, j1]
+// the lane's own candidates in it -- and on_line() after each line that
+// passed the tile tests.  Tiles beyond the largest sample radius visit nothing.  The
 // lines are tested 64 at a time, one per lane.
 template <class ChunkFn, class LineFn>
 __device__ __forceinline__ void walk_tile(const GridArgs &A, int tx, int ty, bool valid, float du, float dv,
@@ -249,11 +248,9 @@ __device__ __forceinline__ void walk_tile(const GridArgs &A, int tx, int ty, boo
             }
             const long row_off = (long)l.ang * A.half;
             for (int c0 = l.td0; c0 <= l.td1; c0 += 64)
-                on_chunk(0, row_off, c0, min(64, l.td1 - c0 + 1), max(jd0, c0), min(min(jd1, l.td1), c0 + 63), l.cs.x,
-                         l.cs.y);
+                on_chunk(0, row_off, max(jd0, c0), min(min(jd1, l.td1), c0 + 63), l.cs.x, l.cs.y);
             for (int c0 = l.tm0; c0 <= l.tm1; c0 += 64)
-                on_chunk(1, row_off, c0, min(64, l.tm1 - c0 + 1), max(jm0, c0), min(min(jm1, l.tm1), c0 + 63), l.cs.x,
-                         l.cs.y);
+                on_chunk(1, row_off, max(jm0, c0), min(min(jm1, l.tm1), c0 + 63), l.cs.x, l.cs.y);
             on_line();
         }
     }
@@ -693,7 +690,7 @@ __global__ void __launch_bounds__(256) k_gop_build(GridArgs A, unsigned *tile_n,
     int lines = 0;
     walk_tile(
         A, tx, ty, valid, pa - M2, pb - M2,
-        [&](int mirror, long row_off, int c0, int nj, int j0, int j1, float C, float S) {
+        [&](int mirror, long row_off, int j0, int j1, float C, float S) {
             for (int j = j0; j <= j1; j++) {
                 float w;
                 const float qa = mirror ? ma : pa, qb = mirror ? mb : pb;
@@ -802,7 +799,7 @@ __global__ void __launch_bounds__(256) k_sop_build(GridArgs A, int n_heavy, uint
     int lines = 0;
     walk_tile(
         A, tx, ty, valid, pa - M2, pb - M2,
-        [&](int mirror, long row_off, int c0, int nj, int j0, int j1, float C, float S) {
+        [&](int mirror, long row_off, int j0, int j1, float C, float S) {
             // stage only the samples some lane taps: [lo, hi] of the run
             const float qa = mirror ? ma : pa, qb = mirror ? mb : pb;
             unsigned lo = 0xffffffffu, hi = 0u;
@@ -816,9 +813,7 @@ __global__ void __launch_bounds__(256) k_sop_build(GridArgs A, int n_heavy, uint
             lo = wave_min(lo);
             hi = wave_max(hi);
             if (hi < lo) return;  // no lane taps this run (j >= 1, so hi = 0 means none)
-            (void)c0;
-            (void)nj;
-            const unsigned n = hi - lo + 1u;  // <= nj <= 64
+            const unsigned n = hi - lo + 1u;  // <= 64
             if (slots + n > (unsigned)kSopSlots) close(false);
             const unsigned sb = slots - lo;  // slot of sample j: sb + j
             if (MODE == 1 && (unsigned)lane < n)

@@ -315,7 +315,6 @@ struct Pf {
 // kernels' VALU instructions, and those bound them.)
 __device__ __forceinline__ int pf_place(int j) { return j ^ ((j >> 4) & 31); }
 
-template <int LM>
 __device__ __forceinline__ void pf_first(float2 *buf, float2 (&v)[16], int j) {
     gr_dft16<-1>(v);
     const int b = (j << 4) ^ (j & 31);
@@ -419,7 +418,7 @@ __global__ void __launch_bounds__(kPfThreads) k_ifft_cols_pf(ColsArgs A, int n_i
         // 128 registers of a 1024-thread workgroup
         int t = (int)threadIdx.x;
         asm volatile("" : "+v"(t));
-        pf_first<LM>(lds + column(t) * F::stride, v, first(t));
+        pf_first(lds + column(t) * F::stride, v, first(t));
         const int cur = item;
         const float cu = cu_next;
         item += (int)gridDim.x;
@@ -503,7 +502,7 @@ __global__ void __launch_bounds__(kPfThreads) k_ifft_rows_pf(RowsArgs A, int n_i
         asm volatile("" : "+v"(t));  // indices recomputed per item (as k_ifft_cols_pf)
         const int grp = t / NT, tid = t % NT;
         float2 *row = lds + grp * F::stride;
-        pf_first<LM>(row, v, tid);
+        pf_first(row, v, tid);
         const int cur = item;
         item += (int)gridDim.x;
         __syncthreads();

@@ -355,6 +355,8 @@ int build_gop(gr_plan *pl, hipStream_t s, bool required, size_t max_bytes) {
         GR_HIP(hipMemcpyAsync(pl->d_hmeta, hmeta.data(), sizeof(uint4) * nt, hipMemcpyHostToDevice, s));
         GR_HIP(hipMemcpyAsync(pl->d_hsplit, hsplit.data(), sizeof(unsigned) * hsplit.size(), hipMemcpyHostToDevice,
                               s));
+        // (the fill pass leaves the marks of a tile without segments: none)
+        GR_HIP(hipMemsetAsync(pl->d_hseg, 0, sizeof(uint2) * seg_total, s));
         pl->n_split = (int)hsplit.size();
         pl->split_groups = (int)part_total;
     }

@@ -1260,12 +1260,10 @@ __global__ void __launch_bounds__(256) k_gop_merge(GridArgs A, GopArgs O, int pa
     const int h = w / pairs, pair = w % pairs;
     const unsigned ti = O.hsplit[h];
     const unsigned tt = A.tiles[ti];
-    if (tt == kGridNoTile) return;
     const int tx = (int)(tt & 0xffffu), ty = (int)(tt >> 16);
     const int a = tx * kTile + (lane & 7), b = ty * kTile + (lane >> 3);
     const uint4 hm = O.hmeta[ti];
-    // (a tile without segments has no marks: zeros)
-    const unsigned total = hm.x ? O.hseg[hm.y + 64ul * hm.x + lane].y : 0u, n = wave_max(total);
+    const unsigned total = O.hseg[hm.y + 64ul * hm.x + lane].y, n = wave_max(total);  // (no segments: 0)
     const float2 *in = O.part + (size_t)hm.z * O.part_pairs * 64 + (size_t)pair * 64 + lane;
     const size_t gstride = (size_t)O.part_pairs * 64;
     float4 acc[1] = {make_float4(0.0f, 0.0f, 0.0f, 0.0f)};
@@ -1279,7 +1277,7 @@ __global__ void __launch_bounds__(256) k_gop_merge(GridArgs A, GopArgs O, int pa
             merge<1>(acc, part);
         }
     }
-    store_cells<GR_ACCUM_COMPENSATED, 1>(A, pair, 1, a, b, acc);
+    if (tt != kGridNoTile) store_cells<GR_ACCUM_COMPENSATED, 1>(A, pair, 1, a, b, acc);
 }
 
 // Workgroups of k_grid_op given to the heavy items -- one a wave, or (wide) one
